@@ -275,9 +275,9 @@ void *dnnrtConvBiasActivMaxPool(dnnrtHandle_t handle, const void *X,
  * padding, the first with stride 1, over 64 + 64 or 128 + 256 input channels
  * (every element is then what the two calls would store: each conv + bias
  * rounded to fp16 on its own, the sum and the activation in fp32); fp32
- * DNNRT_NCHW, both 1x1 without padding, on problems small enough for the
- * batch-1 kernels (the two reductions are then one sum, rounded once: within
- * an fp32 ulp or two of the chain).  Everywhere else the call runs the two
+ * DNNRT_NCHW, both 1x1 without padding, with C,R,S,K filters or on problems
+ * small enough for the batch-1 kernels (the two reductions are then one sum,
+ * rounded once: within an fp32 ulp or two of the chain).  Everywhere else the call runs the two
  * convolutions one after the other with the shortcut's result passing through
  * Y, which gives the chain's bits; `algo` and `algo2` are then the `algo`
  * operands of the first (closing) and the second (shortcut) convolution. */

@@ -547,8 +547,10 @@ void *dnnrtConvBiasAddConvBiasActiv(dnnrtHandle_t handle, const void *X, const i
     a.Kdim2 = s2.C; a.H2 = s2.H; a.W2 = s2.W; a.sh2 = s2.sh; a.sw2 = s2.sw; a.x2_img_stride = (int64_t)s2.C * s2.H * s2.W;
     a.magic_rs = dnnrt::magic_of(1); a.magic_s = dnnrt::magic_of(1);
     const auto wgs64 = dnnrt::ceil_div(a.M, 64) * dnnrt::ceil_div(a.Ncols, 64);
+    bool launched = false;
+    if (!dnnrt::launch_conv_f32_dma(handle, a, wgs64 < handle->num_cu ? dnnrt::small_f32_estimate_us(a) : 1e30, launched)) return nullptr;
+    if (launched) return Y;
     if (wgs64 < handle->num_cu) {  // where a convolution of its own would take the small kernels as well
-      bool launched = false;
       if (!dnnrt::launch_igemm_f32_small(handle, a, 1, crsk ? 2 : 0, launched)) return nullptr;
       if (launched) return Y;
     }

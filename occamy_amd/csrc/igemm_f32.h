@@ -71,6 +71,19 @@ bool launch_igemm_f32(const dnnrtContext *ctx, const IgemmArgs &a);
 bool launch_igemm_f32_direct(const dnnrtContext *ctx, const IgemmArgs &a, int rsmode, int layout);
 // 3x3 convolutions large enough for LDS-staged tiles (igemm_f32_3x3.hip); `launched` says whether it applied.
 bool launch_conv3x3_f32_tiled(const dnnrtContext *ctx, const IgemmArgs &a, int layout, bool &launched);
+// Convolutions with C,R,S,K filters on tiles whose operands go straight into LDS (conv_f32_dma.hip), if they take no longer
+// than `at_most_us` by its estimate; `launched` says whether it applied.
+bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &a, double at_most_us, bool &launched);
+// What the small-problem kernels take for a convolution, estimated in microseconds: single launches of 0.1 .. 2 GFLOP
+// (counting whole 32x32 tiles) measure 5 + 18 per GFLOP for 3x3 filters, 5 + 15.5 for 1x1, 60 and more per GFLOP on the
+// general kernel.  0 below a quarter of a GFLOP: there either way is launch and latency, and inside a network, with its
+// operands further away, the small kernels have the shorter chain (56x56 layers of a ResNet-50 at batch 1: 8.1 against 8.6).
+inline double small_f32_estimate_us(const IgemmArgs &a) {
+  const double gflop = 2e-9 * 1024 * (double)ceil_div(a.M, 32) * (double)ceil_div(a.Ncols, 32) * (a.Kdim + (a.A2 ? a.Kdim2 : 0));
+  const bool pointwise = a.R == 1 && a.S == 1 && a.ph == 0 && a.pw == 0;
+  if (gflop < 0.25 && (pointwise || (a.R == 3 && a.S == 3))) return 0;
+  return 5.0 + (pointwise ? 15.5 : a.R == 3 && a.S == 3 ? 18.0 : 60.0) * gflop;
+}
 // Row-major products with a few hundred rows (gemm_f32_rows.hip); `launched` says whether it applied.
 bool launch_gemm_f32_rows(const dnnrtContext *ctx, const IgemmArgs &a, bool &launched);
 // Zeroes the first n arrival counters of the context's split-reduction scratch on its stream.  For scratch that

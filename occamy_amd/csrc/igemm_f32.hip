@@ -299,6 +299,12 @@ bool launch_igemm_f32(const dnnrtContext *ctx, const IgemmArgs &args) {
   const int layout = (a.b_kcontig ? 1 : 0) | (a.a_mcontig ? 2 : 0);
   if ((layout & 1) && rsmode != 1) { set_error("igemm_f32: a k-contiguous right operand needs a 1x1 geometry"); return false; }
 
+  const bool fills_chip = ceil_div(a.M, 64) * ceil_div(a.Ncols, 64) * a.Z >= ctx->num_cu;
+  if (layout == 2) {  // C,R,S,K filters: always where 64x64 tiles fill the chip, below that where it beats the small kernels
+    bool launched = false;
+    if (!launch_conv_f32_dma(ctx, a, fills_chip ? 1e30 : small_f32_estimate_us(a), launched)) return false;
+    if (launched) return true;
+  }
   if (rsmode == 3) {  // the 3x3 specialisation takes the problems the tiles below would get
     bool launched = false;
     if (!launch_conv3x3_f32_tiled(ctx, a, layout, launched)) return false;

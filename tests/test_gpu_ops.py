@@ -141,6 +141,36 @@ def test_conv_f32_random_shapes(gpu, cpu):
         np.testing.assert_array_equal(oc.conv(gpu, x, w, b, (ph, pw), (sh, sw), grp, activ, z=z, coef=coef, inplace=True), gotz, err_msg=what + " in place")
 
 
+# N, C, H, W, K, R, stride, pad: the tiles whose operands go straight into LDS (C,R,S,K filters, problems that fill the
+# chip).  K off the tile and off multiples of four, pixels per image odd (pairs of pixels that straddle two images) and
+# in fours (16-byte loads), channels fewer than a step, not a multiple of a step, not a multiple of four, filters of one
+# tap with padding, 16 to 32 filters, tiles left over and split along the reduction, one reduction step.
+DMA_F32_CASES = [(3, 20, 75, 75, 66, 3, 1, 1), (2, 64, 90, 117, 130, 3, 1, 1), (4, 4, 80, 80, 64, 3, 2, 1), (1, 12, 130, 131, 70, 5, 1, 2),
+                 (2, 3, 190, 190, 64, 7, 2, 3), (1, 5, 150, 120, 64, 4, 1, 0), (4, 64, 56, 56, 128, 1, 1, 0), (3, 36, 75, 75, 96, 1, 1, 0),
+                 (2, 30, 75, 75, 132, 1, 1, 1), (8, 16, 32, 32, 256, 1, 2, 0), (3, 256, 38, 38, 24, 3, 1, 1), (3, 512, 19, 19, 486, 3, 1, 1),
+                 (16, 256, 14, 14, 256, 3, 1, 1), (33, 8, 24, 24, 64, 1, 1, 0)]
+
+
+@pytest.mark.parametrize("case", DMA_F32_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_conv_f32_direct_to_lds_tiles(gpu, cpu, case):
+    """fp32 convolutions on the direct-to-LDS tiles against the oracle, plain, with a residual and over it; twice (the
+    arrival counters of split tiles must be back at zero), the second result bit-identical."""
+    N, C, H, W, K, R, st, pd = case
+    r = rng(sum(case))
+    x = r.standard_normal((N, C, H, W)).astype(np.float32)
+    w = (r.standard_normal((K, C, R, R)) * np.sqrt(2.0 / (C * R * R))).astype(np.float32)
+    b = r.uniform(-0.3, 0.3, K).astype(np.float32)
+    args = ((pd, pd), (st, st), 1)
+    got = oc.conv(gpu, x, w, b, *args, _abi.ACT_LEAKY_RELU, crsk=True, coef=0.1)
+    ref = oc.conv(cpu, x, w, b, *args, _abi.ACT_IDENTITY)
+    np.testing.assert_allclose(got, np.where(ref < 0, np.float32(0.1) * ref, ref), rtol=RTOL, atol=ATOL)
+    np.testing.assert_array_equal(oc.conv(gpu, x, w, b, *args, _abi.ACT_LEAKY_RELU, crsk=True, coef=0.1), got)
+    z = r.standard_normal(ref.shape).astype(np.float32)
+    gotz = oc.conv(gpu, x, w, b, *args, _abi.ACT_RELU, crsk=True, z=z)
+    np.testing.assert_allclose(gotz, np.maximum(ref + z, 0), rtol=RTOL, atol=ATOL)
+    np.testing.assert_array_equal(oc.conv(gpu, x, w, b, *args, _abi.ACT_RELU, crsk=True, z=z, inplace=True), gotz)
+
+
 def test_conv_f16_random_shapes(gpu, cpu):
     """120 seeded shapes through the fp16 convolution, channels-last (every fast path's boundary: channel counts
     around the multiples of 8 / 32 / 64, a few steps or many, padded or not, grouped and depthwise) and, every
