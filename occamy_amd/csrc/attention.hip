@@ -1,13 +1,13 @@
 // Multi-head attention core for transformer encoders:
 //   Y[b, q, h*DH + d] = sum_k softmax_k(scale * <Q[b,q,h,:], K[b,k,h,:]>) * V[b,k,h,d]
 // with Q, K, V, Y stored [batch, seq, heads * DH] (the layout the Linear layers
-// write), fp32 or fp16 (widened on the way into LDS, everything in between in
-// fp32, one rounding on the way out).  It stands for the chain the reference runs call by call --
+// write), fp32 or fp16 (a kernel each; everything between the fp16 tensors is
+// in fp32, one rounding on the way out).  It stands for the chain the reference runs call by call --
 // Reshape + Transpose of each operand (CUDAReshapeFunc, CUDATranspose4DFloatFunc),
 // CUDAMatmulNdFunc, the scaling Mul, CUDASoftmaxFunc, CUDAMatmulNdFunc, Transpose
 // + Reshape back -- twelve launches and eleven round trips through memory.
 //
-// One workgroup = 32 queries of one head; its four wavefronts split every block
+// fp32: one workgroup = 32 queries of one head; its four wavefronts split every block
 // of 128 keys (32 each).  Scores are computed transposed (keys x queries) so
 // that a lane owns one query: the soft-max statistics are per lane, and the
 // exponentiated scores already sit in the register layout the second product
@@ -19,25 +19,18 @@
 namespace dnnrt {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef _Float16 att_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 att_half4 __attribute__((ext_vector_type(4)));
+typedef short att_short4 __attribute__((ext_vector_type(4)));
 
-// four consecutive elements of a stored tensor as fp32, and back
 __device__ __forceinline__ float4 load4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
-__device__ __forceinline__ float4 load4(const __half *p) {
-  const att_half4 h = *reinterpret_cast<const att_half4 *>(p);
-  return make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
-}
 __device__ __forceinline__ void store4(float *p, float4 v) { *reinterpret_cast<float4 *>(p) = v; }
-__device__ __forceinline__ void store4(__half *p, float4 v) {
-  const att_half4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
-  *reinterpret_cast<att_half4 *>(p) = h;
-}
 
 constexpr int ATT_QB = 32, ATT_KB = 128;
 
-template <int DH, typename T>
-__global__ __launch_bounds__(256) void attention_kernel(const T *__restrict__ Q, const T *__restrict__ K,
-                                                        const T *__restrict__ V, T *__restrict__ Y, int Sq,
+template <int DH>
+__global__ __launch_bounds__(256) void attention_kernel(const float *__restrict__ Q, const float *__restrict__ K,
+                                                        const float *__restrict__ V, float *__restrict__ Y, int Sq,
                                                         int Sk, int ld_in, int ld, float scale) {
   constexpr int ROW = DH + 4;       // LDS row stride in floats: 16-byte aligned rows, 16-byte reads spread over the banks
   constexpr int TD = DH / 32;       // 32-wide tiles of the head dimension
@@ -49,9 +42,9 @@ __global__ __launch_bounds__(256) void attention_kernel(const T *__restrict__ Q,
   float *sm = mx + 4 * 32;          // [4][32] final sums per wavefront
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, half = lane >> 5;
   const int q0 = blockIdx.x * ATT_QB, head = blockIdx.y, b = blockIdx.z;
-  const T *Qg = Q + (int64_t)b * Sq * ld_in + head * DH;
-  const T *Kg = K + (int64_t)b * Sk * ld_in + head * DH;
-  const T *Vg = V + (int64_t)b * Sk * ld_in + head * DH;
+  const float *Qg = Q + (int64_t)b * Sq * ld_in + head * DH;
+  const float *Kg = K + (int64_t)b * Sk * ld_in + head * DH;
+  const float *Vg = V + (int64_t)b * Sk * ld_in + head * DH;
 
   // the query tile (rows past the end repeat the last query; they are not stored)
   // All of a tile's loads are requested before the first value goes to LDS (as a load-then-store loop the
@@ -164,7 +157,7 @@ __global__ __launch_bounds__(256) void attention_kernel(const T *__restrict__ Q,
       *reinterpret_cast<float4 *>(red + (wave * 32 + l32) * ROW + 32 * t + 8 * g + 4 * half) =
           make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
   __syncthreads();
-  T *Yg = Y + (int64_t)b * Sq * ld + head * DH;
+  float *Yg = Y + (int64_t)b * Sq * ld + head * DH;
   for (int i = tid; i < ATT_QB * (DH / 4); i += 256) {
     const int q = i / (DH / 4), c4 = i - q * (DH / 4);
     if (q0 + q >= Sq) continue;
@@ -179,19 +172,185 @@ __global__ __launch_bounds__(256) void attention_kernel(const T *__restrict__ Q,
   }
 }
 
-template <int DH, typename T>
-static void launch_attention(const dnnrtContext *ctx, const T *Q, const T *K, const T *V, T *Y, int B,
+// fp16.  A workgroup is 32 queries of one head; its NW wavefronts take every NW-th block of 32 keys, each on its own: its
+// own running maximum and sum, no barrier until the partial results meet.  A block's scores are DH / 16 MFMAs of
+// 32x32x16 (keys x queries, exact products, fp32 sums; K and Q straight from global memory in the operands' shape), and
+// the register order of the scores is again the reduction order of the second product.  There the probabilities
+// enter as two fp16 numbers each, p = hi + lo, scaled by 2^14 so that both keep their bits (22 in all, down to
+// probabilities of 2^-28): two MFMAs for what fp32 ones take eight times as long for.  V's operand, four consecutive keys of one d
+// per read, comes out of the wavefront's LDS tile by transposing reads (ds_read_b64_tr_b16).
+// Bound by latency (0.04 .. 0.8 GFLOP): 12 heads of 64, sequence 384: 19.3 us on fp32 MFMAs with fp16 storage -> 11.2 us
+// (a pair of timestamps included in both).
+template <int DH, int NW>
+__global__ __launch_bounds__(64 * NW) void attention_f16_kernel(const _Float16 *__restrict__ Q, const _Float16 *__restrict__ K,
+                                                                const _Float16 *__restrict__ V, _Float16 *__restrict__ Y, int Sq,
+                                                                int Sk, int ld_in, int ld, float scale) {
+  constexpr int TD = DH / 32, SUB = DH / 16, VROW = DH + 8;  // V rows in LDS: 16-byte aligned, neighbouring rows in different banks
+  constexpr int OROW = DH + 4;                               // rows of the partial results, floats
+  constexpr int V_L = DH / 16;                               // 16-byte loads per lane for 32 rows of V
+  extern __shared__ float smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+  const int q0 = blockIdx.x * 32, head = blockIdx.y, b = blockIdx.z;
+  const _Float16 *Qg = Q + (int64_t)b * Sq * ld_in + head * DH;
+  const _Float16 *Kg = K + (int64_t)b * Sk * ld_in + head * DH;
+  const _Float16 *Vg = V + (int64_t)b * Sk * ld_in + head * DH;
+  _Float16 *Vs = reinterpret_cast<_Float16 *>(smem) + wave * 32 * VROW;
+  // eight halfs of a row; rows are 16-byte aligned if the row stride allows it
+  const bool wide = (ld_in & 7) == 0;
+  auto load8 = [&](const _Float16 *p) -> att_half8 {
+    if (wide) return *reinterpret_cast<const att_half8 *>(p);
+    const att_half4 lo = *reinterpret_cast<const att_half4 *>(p), hi = *reinterpret_cast<const att_half4 *>(p + 4);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  att_half8 qf[SUB], kf[SUB], vr[V_L];
+#pragma unroll
+  for (int s = 0; s < SUB; s++) qf[s] = load8(Qg + (int64_t)min(q0 + l32, Sq - 1) * ld_in + 16 * s + 8 * half);
+  auto fetch = [&](int k0) {  // 32 keys from k0; rows past the end repeat the last key, masked below
+    const _Float16 *krow = Kg + (int64_t)min(k0 + l32, Sk - 1) * ld_in + 8 * half;
+#pragma unroll
+    for (int s = 0; s < SUB; s++) kf[s] = load8(krow + 16 * s);
+#pragma unroll
+    for (int u = 0; u < V_L; u++) {
+      const int i = lane + 64 * u, r = i / (DH / 8), c = i - r * (DH / 8);
+      vr[u] = load8(Vg + (int64_t)min(k0 + r, Sk - 1) * ld_in + 8 * c);
+    }
+  };
+  floatx16 o[TD];
+#pragma unroll
+  for (int t = 0; t < TD; t++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) o[t][r] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  int k0 = 32 * wave;
+  if (k0 < Sk) fetch(k0);
+  for (; k0 < Sk; k0 += 32 * NW) {
+    floatx16 s;
+#pragma unroll
+    for (int r = 0; r < 16; r++) s[r] = 0.f;
+#pragma unroll
+    for (int u = 0; u < SUB; u++) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[u], qf[u], s, 0, 0, 0);
+    asm volatile("" ::: "memory");  // the transposing reads of the block before are behind us
+#pragma unroll
+    for (int u = 0; u < V_L; u++) {
+      const int i = lane + 64 * u, r = i / (DH / 8), c = i - r * (DH / 8);
+      *reinterpret_cast<att_half8 *>(Vs + r * VROW + 8 * c) = vr[u];
+    }
+    asm volatile("" ::: "memory");  // a wavefront's LDS accesses are carried out in order
+    if (k0 + 32 * NW < Sk) fetch(k0 + 32 * NW);
+    // register r of lane (l32, half): key k0 + 8 * (r / 4) + 4 * half + r % 4, query l32
+    float m_new = m_run;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < Sk ? s[r] * scale : -INFINITY;
+      m_new = fmaxf(m_new, s[r]);
+    }
+    m_new = fmaxf(m_new, __shfl_xor(m_new, 32, 64));  // finite: every block that is entered holds a key
+    const float alpha = expf(m_run - m_new);          // 0 on the first block
+    float lsum = 0.f;
+    att_half8 hi[2], lo[2];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const float p = expf(s[r] - m_new) * 16384.f;
+      lsum += p;
+      const _Float16 h = (_Float16)p;
+      hi[r >> 3][r & 7] = h;
+      lo[r >> 3][r & 7] = (_Float16)(p - (float)h);
+    }
+    l_run = l_run * alpha + lsum;  // this lane's keys; the halves are added at the end
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < TD; t++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) o[t][r] *= alpha;
+    // O^T[d][query] += V^T[d][key] P^T[key][query]: element e of lane half h is key 16 u + 8 (e / 4) + 4 h + e % 4
+#if __HIP_DEVICE_COMPILE__
+    typedef __attribute__((address_space(3))) att_short4 *tr_ptr;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int t = 0; t < TD; t++) {
+        const _Float16 *at = Vs + (16 * u + 4 * half + ((lane & 15) >> 2)) * VROW + 32 * t + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+        const att_short4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)at), v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(at + 8 * VROW));
+        const att_half8 vf = __builtin_bit_cast(att_half8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, hi[u], o[t], 0, 0, 0);
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, lo[u], o[t], 0, 0, 0);
+      }
+#endif
+  }
+  // the wavefronts' results: [NW][32 queries][OROW], then maxima and sums [NW][32] each
+  __syncthreads();
+  float *red = smem, *mx = red + NW * 32 * OROW, *sm = mx + NW * 32;
+  l_run += __shfl_xor(l_run, 32, 64);
+  if (half == 0) { mx[wave * 32 + l32] = m_run; sm[wave * 32 + l32] = l_run; }
+#pragma unroll
+  for (int t = 0; t < TD; t++)
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      store4(red + (wave * 32 + l32) * OROW + 32 * t + 8 * g + 4 * half, make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]));
+  __syncthreads();
+  _Float16 *Yg = Y + (int64_t)b * Sq * ld + head * DH;
+  for (int i = tid; i < 32 * (DH / 8); i += 64 * NW) {
+    const int q = i / (DH / 8), c = i - q * (DH / 8);
+    if (q0 + q >= Sq) continue;
+    float m = mx[q];
+#pragma unroll
+    for (int w = 1; w < NW; w++) m = fmaxf(m, mx[w * 32 + q]);
+    float sum = 0.f, v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float f = expf(mx[w * 32 + q] - m);  // 0 for a wavefront that had no keys
+      sum += f * sm[w * 32 + q];
+      const float4 a = load4(red + (w * 32 + q) * OROW + 8 * c), d = load4(red + (w * 32 + q) * OROW + 8 * c + 4);
+      v[0] += f * a.x; v[1] += f * a.y; v[2] += f * a.z; v[3] += f * a.w;
+      v[4] += f * d.x; v[5] += f * d.y; v[6] += f * d.z; v[7] += f * d.w;
+    }
+    const float inv = 1.0f / sum;
+    att_half8 out;
+#pragma unroll
+    for (int e = 0; e < 8; e++) out[e] = (_Float16)(v[e] * inv);
+    *reinterpret_cast<att_half8 *>(Yg + (int64_t)(q0 + q) * ld + 8 * c) = out;
+  }
+}
+
+// More than 64 KiB of dynamic LDS must be asked for once per kernel.
+template <typename F>
+static void raise_lds(F *kernel, size_t lds, bool &raised) {
+  if (raised) return;
+  (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  raised = true;
+}
+
+template <int DH>
+static void launch_attention(const dnnrtContext *ctx, const float *Q, const float *K, const float *V, float *Y, int B,
                              int Sq, int Sk, int H, int ld_in, float scale) {
   constexpr int ROW = DH + 4;
   const size_t lds = (size_t)((ATT_QB + 2 * ATT_KB) * ROW + 8 * 32) * sizeof(float);
-  static bool raised = false;  // per instantiation: more than 64 KiB of dynamic LDS must be asked for once
-  if (!raised) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_kernel<DH, T>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    raised = true;
-  }
-  hipLaunchKernelGGL((attention_kernel<DH, T>), dim3((unsigned)ceil_div(Sq, ATT_QB), (unsigned)H, (unsigned)B), dim3(256),
+  static bool raised = false;
+  raise_lds(&attention_kernel<DH>, lds, raised);
+  hipLaunchKernelGGL((attention_kernel<DH>), dim3((unsigned)ceil_div(Sq, ATT_QB), (unsigned)H, (unsigned)B), dim3(256),
                      lds, ctx->stream, Q, K, V, Y, Sq, Sk, ld_in, H * DH, scale);
+}
+
+template <int DH, int NW>
+static void launch_attention_f16(const dnnrtContext *ctx, const __half *Q, const __half *K, const __half *V, __half *Y, int B,
+                                 int Sq, int Sk, int H, int ld_in, float scale) {
+  const size_t lds = (size_t)NW * 32 * (DH + 4 + 2) * sizeof(float);  // the partial results; the V tiles lie under them
+  static_assert((DH + 8) * 2 <= (DH + 4) * 4, "V tiles fit");
+  static bool raised = false;
+  raise_lds(&attention_f16_kernel<DH, NW>, lds, raised);
+  hipLaunchKernelGGL((attention_f16_kernel<DH, NW>), dim3((unsigned)ceil_div(Sq, 32), (unsigned)H, (unsigned)B), dim3(64 * NW), lds, ctx->stream,
+                     (const _Float16 *)Q, (const _Float16 *)K, (const _Float16 *)V, (_Float16 *)Y, Sq, Sk, ld_in, H * DH, scale);
+}
+
+template <int DH>
+static void launch_attention(const dnnrtContext *ctx, const __half *Q, const __half *K, const __half *V, __half *Y, int B,
+                             int Sq, int Sk, int H, int ld_in, float scale) {
+  // eight wavefronts where four would leave SIMDs idle and there are keys for more
+  const bool more = DH <= 64 && Sk > 128 && ceil_div(Sq, 32) * H * B < 2 * (int64_t)ctx->num_cu;
+  if (more) launch_attention_f16<DH, DH <= 64 ? 8 : 4>(ctx, Q, K, V, Y, B, Sq, Sk, H, ld_in, scale);
+  else launch_attention_f16<DH, 4>(ctx, Q, K, V, Y, B, Sq, Sk, H, ld_in, scale);
 }
 
 }  // namespace dnnrt

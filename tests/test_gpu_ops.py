@@ -624,6 +624,53 @@ def test_attention(gpu, cpu):
                                oc.attention_packed(cpu, qkv, 4, 0.125).astype(np.float32), rtol=2e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("case", [(1, 384, 384, 12, 64), (2, 31, 257, 3, 64), (1, 70, 129, 2, 32), (1, 64, 160, 5, 32), (1, 45, 513, 2, 128),
+                                  (1, 1, 1, 1, 64), (3, 33, 32, 2, 64), (1, 600, 600, 16, 64)], ids=str)
+def test_attention_f16_blocks_and_wavefronts(gpu, cpu, case):
+    """Key counts around the 32-key blocks and what four and eight wavefronts take, sharp and flat soft-maxima, rows of
+    Q, K and V that are 16-byte aligned and rows that are not."""
+    B, Sq, Sk, H, D = case
+    r = rng(sum(case))
+    q, k, v = (r.standard_normal((B, S, H * D)).astype(np.float16) for S in (Sq, Sk, Sk))
+    for scale in (1.0 / np.sqrt(D), 1.0, 1e-3):
+        ref = oc.attention(cpu, q, k, v, H, scale).astype(np.float32)
+        np.testing.assert_allclose(oc.attention(gpu, q, k, v, H, scale).astype(np.float32), ref, rtol=2e-3, atol=2e-3)
+        wide = [np.zeros((B, S, H * D + 4), np.float16) for S in (Sq, Sk, Sk)]
+        for w, t in zip(wide, (q, k, v)):
+            w[:, :, :H * D] = t
+        Q, K, V = (gpu.put(w) for w in wide)
+        Y = gpu.empty((B, Sq, H * D), np.float16)
+        gpu.ops.attention(gpu.ptr(Q), gpu.ptr(K), gpu.ptr(V), gpu.ptr(Y), B, Sq, Sk, H, D, float(scale), _abi.F16, ld_in=H * D + 4)
+        gpu.sync()
+        np.testing.assert_allclose(gpu.get(Y).astype(np.float32), ref, rtol=2e-3, atol=2e-3)
+
+
+# M, K, N: rows, columns and a reduction off the tiles, the reduction's last step partial, fewer steps than ring stages and
+# as many, one more, odd and even counts; split reductions; both tile shapes
+@pytest.mark.parametrize("case", [(1, 8, 8), (5, 64, 72), (64, 192, 64), (65, 256, 136), (33, 320, 64), (130, 1000, 328), (16, 3072, 768), (197, 768, 2304),
+                                  (100, 384, 3072), (1030, 448, 1160)], ids=str)
+def test_matmul_f16_direct_to_lds_tiles(gpu, cpu, case):
+    """fp16 products on the direct-to-LDS tiles against the oracle: right operand [K,N] with bias, residual and GELU, twice
+    (the arrival counters of split tiles must be back at zero), batched, and stored [N,K]."""
+    M, K, N = case
+    r = rng(sum(case))
+    a = r.standard_normal((1, M, K)).astype(np.float16)
+    b = (r.standard_normal((K, N)) / np.sqrt(K)).astype(np.float16)
+    bias, z = r.standard_normal(N).astype(np.float16), r.standard_normal((1, M, N)).astype(np.float16)
+    exact = a[0].astype(np.float64) @ b.astype(np.float64) + bias.astype(np.float64)
+    tol = dict(rtol=2e-3, atol=2e-3)
+    got = oc.matmul_nd_bias(gpu, a, b, bias)
+    np.testing.assert_allclose(got[0].astype(np.float64), exact, **tol)
+    np.testing.assert_array_equal(oc.matmul_nd_bias(gpu, a, b, bias), got)
+    np.testing.assert_allclose(oc.matmul_nd_bias(gpu, a, b, bias, z=z)[0].astype(np.float64), exact + z[0], **tol)
+    np.testing.assert_allclose(oc.matmul_nd_bias(gpu, a, b, bias, gelu=True).astype(np.float32), oc.matmul_nd_bias(cpu, a, b, bias, gelu=True).astype(np.float32),
+                               rtol=1e-2, atol=1e-2)
+    np.testing.assert_allclose(oc.matmul2d(gpu, a[0], np.ascontiguousarray(b.T), transB=1, alpha=0.5).astype(np.float64), 0.5 * (exact - bias), **tol)
+    if M * K * N < 1 << 22:
+        a3, b3 = r.standard_normal((3, M, K)).astype(np.float16), (r.standard_normal((3, K, N)) / np.sqrt(K)).astype(np.float16)
+        np.testing.assert_allclose(oc.matmul_nd(gpu, a3, b3).astype(np.float64), a3.astype(np.float64) @ b3.astype(np.float64), **tol)
+
+
 # ---- data movement -------------------------------------------------------------------------
 
 def test_data_movement(gpu, cpu):
