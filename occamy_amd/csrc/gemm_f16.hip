@@ -17,22 +17,6 @@ namespace dnnrt {
 typedef _Float16 g_half8 __attribute__((ext_vector_type(8)));
 typedef float g_floatx16 __attribute__((ext_vector_type(16)));
 
-struct GemmF16Args {
-  const __half *A, *B, *C, *bias;
-  __half *Out;
-  int M, N, K;
-  int64_t a_sm, a_sk, b_sk, b_sn;   // element strides of A along m and k, of B along k and n
-  int64_t az, bz, yz;               // batch strides (0: shared)
-  int64_t c_sm, cz;                 // C: row stride (0: one row for every m), batch stride
-  float alpha, beta;
-  int act;
-  float act_coef;
-  bool a_vec, b_vec;                // the contiguous direction of A / B may be read eight elements (16 bytes) at a time
-  int steps_per_split;              // 64-k steps per workgroup along gridDim.y (the reduction split over workgroups)
-  float *partials;                  // the handle's scratch: one 64 x 64 fp32 tile per (tile, split)
-  unsigned *counters;               // ... and one arrival counter per tile, zero between kernels
-};
-
 constexpr int G_BK = 64, G_ROW = 72;  // k per step; halfs per LDS row (64 + 8 of padding)
 
 // Tile: 64 columns n x 64 rows m; the MFMA's row operand is the B side (n), its column operand the A side (m), so
@@ -253,6 +237,11 @@ bool gemm_f16(const dnnrtContext *ctx, const __half *A, const __half *B, const _
   const int64_t a_other = transA ? g.a_sk : g.a_sm, b_other = transB ? g.b_sn : g.b_sk;
   g.a_vec = aligned16(A) && a_other % 8 == 0 && az % 8 == 0;
   g.b_vec = aligned16(B) && b_other % 8 == 0 && bz % 8 == 0;
+  g.partials = ctx->splitk_partials;
+  g.counters = ctx->splitk_counters;
+  bool launched = false;
+  if (!launch_gemm_f16_dma(ctx, g, Z, launched)) return false;
+  if (launched) return true;
   // Few tiles and a long reduction (a transformer's Linear layers at batch 1: 128 rows): the reduction is split over
   // workgroups up to about one workgroup per CU, a split keeping at least four 64-k steps (all of them in flight
   // at once), as far as the handle's scratch holds the partial tiles.  Measured on the fp16 BERT-base encoder:
@@ -270,8 +259,6 @@ bool gemm_f16(const dnnrtContext *ctx, const __half *A, const __half *B, const _
   }
   g.steps_per_split = (int)ceil_div(steps, splits);
   splits = ceil_div(steps, g.steps_per_split);  // no empty split: every arrival carries a partial tile
-  g.partials = ctx->splitk_partials;
-  g.counters = ctx->splitk_counters;
   hipLaunchKernelGGL(gemm_f16_generic_kernel, dim3((unsigned)tiles, (unsigned)splits, (unsigned)Z), dim3(256), 0, ctx->stream, g);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("matmul(fp16): launch failed: %s", hipGetErrorString(e)); return false; }
