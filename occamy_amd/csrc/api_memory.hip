@@ -2,6 +2,7 @@
 // (reference: src/Tools/dnn-wrapper/cuda/wrapDNN*.cpp and the
 // cudnnCreate/cudaStreamCreate rows of DNNAPISpecs.inc:92-95).
 #include "common.h"
+#include "dnnrt_exec.h"
 
 #include <stdarg.h>
 #include <string.h>
@@ -71,6 +72,19 @@ constexpr int MAX_DEVICES = 64;
 static unsigned char *g_scratch_at[MAX_DEVICES];      // this device's copy of handle_scratch
 static const dnnrtContext *g_scratch_holder[MAX_DEVICES];
 static std::mutex g_scratch_mutex;
+}  // namespace dnnrt
+
+namespace dnnrt {
+// Host (pinned) to device.  The link bounds it: 32 workgroups with 16 bytes per thread in flight move 9 MB in 168 us
+// (56 GB/s; 8 workgroups 366, 1024 of them 201), and leave the other compute units to the kernels beside it.  A copy
+// through the DMA engine takes as long for large sizes and 7 to 20 us more in a stream that also runs kernels:
+// 256 KB 7.4 us against 14.2, 64 KB 3.7 against 10.8, alone.
+constexpr int UPLOAD_WORKGROUPS = 32;
+__global__ __launch_bounds__(256) void upload_kernel(uint4 *dst, const uint4 *src, int64_t n16, int tail) {
+  const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  for (int64_t i = first; i < n16; i += UPLOAD_WORKGROUPS * 256) dst[i] = src[i];
+  if (first < tail) reinterpret_cast<unsigned char *>(dst + n16)[first] = reinterpret_cast<const unsigned char *>(src + n16)[first];
+}
 }  // namespace dnnrt
 
 #define HIP_RET(call, what)                                                    \
@@ -285,6 +299,28 @@ int32_t dnnrtEventElapsedMs(void *start, void *stop, float *ms) {
 
 int32_t dnnrtEventDestroy(void *event) {
   if (event) HIP_RET(hipEventDestroy((hipEvent_t)event), "dnnrtEventDestroy");
+  return 0;
+}
+
+int32_t dnnrtExecFenceCreate(void **event) {
+  if (!event) { set_error("dnnrtExecFenceCreate: null pointer"); return 1; }
+  hipEvent_t e;
+  HIP_RET(hipEventCreateWithFlags(&e, hipEventDisableTiming), "dnnrtExecFenceCreate");
+  *event = e;
+  return 0;
+}
+
+int32_t dnnrtExecStreamWait(dnnrtStream_t stream, void *event) {
+  HIP_RET(hipStreamWaitEvent((hipStream_t)stream, (hipEvent_t)event, 0), "dnnrtExecStreamWait");
+  return 0;
+}
+
+int32_t dnnrtExecUpload(void *dst, const void *src, int64_t bytes, dnnrtStream_t stream) {
+  if (bytes <= 0) return 0;
+  if (!dst || !src || !dnnrt::aligned16(dst) || !dnnrt::aligned16(src)) { set_error("dnnrtExecUpload: bad arguments"); return 1; }
+  hipLaunchKernelGGL(dnnrt::upload_kernel, dim3(dnnrt::UPLOAD_WORKGROUPS), dim3(256), 0, (hipStream_t)stream, static_cast<uint4 *>(dst),
+                     static_cast<const uint4 *>(src), bytes / 16, (int)(bytes % 16));
+  HIP_RET(hipGetLastError(), "dnnrtExecUpload");
   return 0;
 }
 

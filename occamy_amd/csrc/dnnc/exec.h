@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "../../../include/dnnrt.h"
+#include "../dnnrt_exec.h"
 #include "ir.h"
 
 namespace dnnc {
@@ -74,6 +75,10 @@ struct RuntimeApi {
   decltype(&::dnnrtSqueeze) dnnrtSqueeze = nullptr;
   decltype(&::dnnrtUnsqueeze) dnnrtUnsqueeze = nullptr;
   decltype(&::dnnrtExpand) dnnrtExpand = nullptr;
+  // null in a host-only build
+  decltype(&::dnnrtExecFenceCreate) dnnrtExecFenceCreate = nullptr;
+  decltype(&::dnnrtExecStreamWait) dnnrtExecStreamWait = nullptr;
+  decltype(&::dnnrtExecUpload) dnnrtExecUpload = nullptr;
 };
 
 bool load_runtime(const std::string &path, RuntimeApi &rt, std::string &err);
@@ -146,6 +151,21 @@ class Session {
   std::map<size_t, void *> arg_home;  // resident mode: value id of a function argument's pool slot -> its address in the pool
   std::vector<const Op *> direct_out;  // the result copies of the current run that are not needed for that reason
   std::map<size_t, void *> out_home;  // ... and of a result's pool tensor, when results are written where the caller wants them
+  // Per-inference mode on the GPU runtime: the constants as they go to the device on a second stream, ahead of the
+  // operations that read them (plan_uploads).  Compute operations are counted in program order.
+  struct Upload {
+    int64_t host_off, dev_off, bytes;  // in upload_host, in the pool
+    int first;                         // the first operation that reads it
+    int after;                         // these bytes of the pool are free once this many operations are done
+    void *landed;                      // recorded behind the copy; null where the next entry completes the same constants
+  };
+  std::vector<Upload> uploads;
+  std::vector<std::pair<size_t, int64_t>> upload_slots;  // value id of a constant's device tensor, its offset in the pool
+  std::map<int, void *> op_done;                         // recorded when that many operations are issued
+  void *upload_host = nullptr;
+  dnnrtStream_t upload_stream = nullptr;
+  bool plan_uploads(std::string &err);
+  bool run_uploading(const void *const *inputs, void *const *outputs, std::string &err);
   std::map<std::string, void *> host_const;
   std::vector<void *> host_out, host_in;
   // resident mode: results produced mid-program, whose pool bytes a later

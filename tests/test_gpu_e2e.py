@@ -76,6 +76,20 @@ def test_device_memory_is_the_planned_pool(name):
     s.close()
 
 
+@pytest.mark.parametrize("model,batch,image", [("resnet50", 1, 64), ("resnet50", 3, 97), ("mobilenet_v2", 1, 224), ("mobilenet_v2", 5, 131), ("alexnet", 2, 224)])
+def test_uploaded_constants_arrive_before_their_readers(model, batch, image):
+    """Per inference the constants are uploaded on a second stream into whatever bytes of the pool are free: bit for bit
+    the resident program's results, on inputs that change from run to run."""
+    kw = {} if model == "alexnet" else dict(image=image)
+    g, _ = getattr(models, model)(batch, **kw)
+    p = g.compile(fusion=True)
+    s, res = p.session(compiler.MODE_OCCAMY), p.session(compiler.MODE_RESIDENT)
+    (shape, _), = g.input_shapes.values()
+    for seed in range(4):
+        x = np.random.default_rng(seed).standard_normal(shape, dtype=np.float32)
+        np.testing.assert_array_equal(s.run(x)[0], res.run(x)[0])
+
+
 @pytest.mark.parametrize("name", list(CONFIGS))
 def test_fused_program_matches_oracle(name, oracle_outputs):
     out, _ = run(CONFIGS[name], fusion=True)
