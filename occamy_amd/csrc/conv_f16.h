@@ -84,3 +84,10 @@ bool c64_conv_applies(const ConvF16Args &a);
 bool launch_conv_f16_c64(const dnnrtContext *ctx, const ConvF16Args &a);
 
 }  // namespace dnnrt
+
+struct dnnrtExecBlock;
+namespace dnnrt {
+// A whole inverted residual block (conv_f16_block.hip).
+bool block_f16_applies(const dnnrtContext *ctx, const dnnrtExecBlock &k);
+bool launch_block_f16(const dnnrtContext *ctx, const dnnrtExecBlock &k);
+}  // namespace dnnrt

@@ -46,6 +46,9 @@ bool load_runtime(const std::string &path, RuntimeApi &rt, std::string &err) {
   *(void **)(&rt.dnnrtExecFenceCreate) = dlsym(rt.dl, "dnnrtExecFenceCreate");
   *(void **)(&rt.dnnrtExecStreamWait) = dlsym(rt.dl, "dnnrtExecStreamWait");
   *(void **)(&rt.dnnrtExecUpload) = dlsym(rt.dl, "dnnrtExecUpload");
+  *(void **)(&rt.dnnrtExecBlockApplies) = dlsym(rt.dl, "dnnrtExecBlockApplies");
+  *(void **)(&rt.dnnrtExecRunBlock) = dlsym(rt.dl, "dnnrtExecRunBlock");
+  *(void **)(&rt.dnnrtExecBlockFilter) = dlsym(rt.dl, "dnnrtExecBlockFilter");
   return true;
 }
 #undef LOAD
@@ -224,10 +227,220 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
       if (rt.dnnrtMalloc(&stage, op->bytes)) { err = rt_error("dnnrtMalloc(result staging)"); return false; }
       staged_out[op] = stage;
     }
-  } else if (!host_backend && rt.dnnrtExecFenceCreate && rt.dnnrtExecStreamWait && rt.dnnrtExecUpload) {
-    return plan_uploads(err);
   }
-  return true;
+  plan_blocks();
+  // Both modes take the same blocks (the same bits): those that a per-inference program can have with its constants uploaded
+  // ahead; in the reference's order a block's first filter is gone when the block runs.
+  const bool ahead = !host_backend && rt.dnnrtExecFenceCreate && rt.dnnrtExecStreamWait && rt.dnnrtExecUpload;
+  std::vector<UploadChunk> chunks;
+  bool placed = ahead && (mode == MODE_OCCAMY || !blocks.empty()) && place_constants(chunks);
+  if (!placed && !blocks.empty()) {
+    blocks.clear();
+    block_of.clear();
+    moved_results.clear();
+    placed = ahead && mode == MODE_OCCAMY && place_constants(chunks);
+  }
+  for (const Block &b : blocks)
+    for (const Op *op : {b.expand, b.project})
+      if (op && op->operands.back()->dtype == F16) block_filters[op->operands[1]] = {op->dimB[0], op->dimB[1]};
+  if (mode == MODE_RESIDENT) {
+    use_blocks = true;
+    block_base = pool;
+    for (const Op *op : prog->ops) {  // once more, in the block call's layout
+      if (op->kind != OP_MEMCPY || op->mode != 1) continue;
+      const auto f = block_filters.find(op->operands[0]);
+      if (f == block_filters.end()) continue;
+      uint8_t *host = (uint8_t *)ptr[(size_t)op->operands[1]->id];
+      const std::vector<uint8_t> rows(host, host + op->bytes);
+      rt.dnnrtExecBlockFilter(host, rows.data(), f->second.first, f->second.second);
+      if (rt.dnnrtMemcpy(ptr[(size_t)op->operands[0]->id], host, op->bytes, 1, stream)) { err = rt_error("dnnrtMemcpy(constant)"); return false; }
+    }
+    if (!block_filters.empty() && rt.dnnrtSync(handle)) { err = rt_error("dnnrtSync"); return false; }
+    return true;
+  }
+  return !placed || plan_uploads(chunks, err);
+}
+
+static bool is_conv_call(const Op *op) { return op->kind == OP_CONV_BIAS_ACTIV || op->kind == OP_CONV_BIAS_ADD_ACTIV; }
+
+void Session::fill_block(const Block &b, dnnrtExecBlock &k) const {
+  auto P = [&](const Op *op, size_t i) { return ptr[(size_t)op->operands[i]->id]; };
+  const Op *first = b.expand ? b.expand : b.dw;
+  k = dnnrtExecBlock{};
+  k.expand = b.expand != nullptr;
+  k.x = P(first, 0);
+  if (b.expand) { k.w1 = P(b.expand, 1); k.b1 = P(b.expand, 2); k.act1 = b.expand->mode; k.coef1 = b.expand->coef; }
+  k.wd = P(b.dw, 1); k.bd = P(b.dw, 2); k.actd = b.dw->mode; k.coefd = b.dw->coef;
+  k.w3 = P(b.project, 1); k.b3 = P(b.project, 2); k.act = b.project->mode; k.coef = b.project->coef;
+  k.z = b.project->kind == OP_CONV_BIAS_ADD_ACTIV ? P(b.project, 4) : nullptr;
+  k.y = b.y_off >= 0 ? (char *)block_base + b.y_off : P(b.project, b.project->operands.size() - 1);
+  k.n = first->dimA[0]; k.cin = first->dimA[1]; k.h = first->dimA[2]; k.w = first->dimA[3];
+  k.ch = b.dw->dimB[0]; k.r = b.dw->dimB[2]; k.s = b.dw->dimB[3]; k.stride = b.dw->strides[0]; k.pad_h = b.dw->pads[0]; k.pad_w = b.dw->pads[1];
+  k.p = b.project->dimA[2]; k.q = b.project->dimA[3]; k.cout = b.project->dimB[0];
+  k.dtype = (int32_t)b.project->operands.back()->dtype;
+  k.format = format_for(first);
+  k.filter_layout = filter_crsk[(size_t)b.dw->operands[1]->id] ? DNNRT_FILTER_CRSK : DNNRT_FILTER_KCRS;
+}
+
+// The slots of everything but constants: from the first operation that uses one to the last.  A block's inner tensors
+// have none, and its operands are read where its last convolution stands.
+std::map<const Value *, Session::Range> Session::live_slots() const {
+  std::map<const Value *, Range> live;
+  std::map<const Value *, const Value *> home;  // value -> the slot it lives in
+  std::map<const Value *, bool> constant;
+  int n = 0;
+  auto touch = [&](const Value *v, int at) {
+    const auto h = home.find(v);
+    if (h == home.end() || h->second->def->bytes <= 0 || constant.count(h->second)) return;
+    const Value *s = h->second;
+    const auto l = live.emplace(s, Range{s->def->offset, s->def->offset + s->def->bytes, at, at}).first;
+    l->second.last = std::max(l->second.last, at);
+  };
+  for (const Op *op : prog->ops) {
+    if (op->kind == OP_MEM_OFFSET) {
+      home[op->result] = op->result;
+    } else if (op->kind == OP_MEMCPY && op->mode == 1) {
+      const Value *src = op->operands[1];
+      if (src->def && src->def->kind == OP_HOST_CONST) constant[op->operands[0]] = true;
+      else touch(op->operands[0], 0);  // an argument: from the start
+    } else if (op->kind == OP_MEMCPY) {
+      for (const Value *v : op->operands) touch(v, n);
+    } else if (is_compute(op->kind)) {
+      const auto b = block_of.find(op);
+      const int at = b == block_of.end() ? n : blocks[(size_t)b->second].at;
+      const bool inner = b != block_of.end() && op != blocks[(size_t)b->second].project;
+      for (size_t i = 0; i < op->operands.size(); i++)
+        if (!inner || i + 1 < op->operands.size()) touch(op->operands[i], at);
+      if (!inner && !op->operands.empty()) {
+        const auto h = home.find(op->operands.back());
+        if (h != home.end()) home[op->result] = h->second;
+      }
+      n++;
+    }
+  }
+  return live;
+}
+
+// Which runs of two or three convolutions are one inverted residual block, and where its result goes.
+//
+// The planner may have put the result over the block's input (free once the expansion has read it) or, in place, over its
+// residual; a kernel whose workgroups read the input while others write the result cannot have that, so the result then
+// gets bytes that are free from here to its last reader: those of the two wide tensors that are not stored any more, as
+// a rule.  Nothing else moves.
+void Session::plan_blocks() {
+  if (host_backend || !rt.dnnrtExecBlockApplies || !rt.dnnrtExecRunBlock || !rt.dnnrtExecBlockFilter) return;
+  std::vector<const Op *> ops;
+  std::map<const Op *, int> number;
+  for (const Op *op : prog->ops)
+    if (is_compute(op->kind)) { number[op] = (int)ops.size(); ops.push_back(op); }
+  auto pointwise = [](const Op *op) {
+    return op->group == 1 && op->dimB.size() == 4 && op->dimB[2] == 1 && op->dimB[3] == 1 && op->pads[0] == 0 && op->pads[1] == 0 && op->strides[0] == 1 && op->strides[1] == 1;
+  };
+  auto only_reader = [](const Value *v, const Op *reader) { return v->uses.size() == 1 && v->uses[0].first == reader && v->uses[0].second == 0; };
+  // the buffer is named by its writers alone (nobody reads it past the result, no copy to the host)
+  auto plain_buffer = [](const Op *op) {
+    const Value *s = op->operands.back();
+    if (!s->def || s->def->kind != OP_MEM_OFFSET) return false;
+    for (const auto &u : s->uses)
+      if (!is_compute(u.first->kind) || u.second + 1 != (int)u.first->operands.size()) return false;
+    return true;
+  };
+  for (size_t i = 1; i < ops.size(); i++) {
+    const Op *dw = ops[i - 1], *pr = ops[i];
+    if (dw->kind != OP_CONV_BIAS_ACTIV || !is_conv_call(pr) || pr->operands[0] != dw->result || !pointwise(pr) || !only_reader(dw->result, pr)) continue;
+    if (dw->dimB.size() != 4 || dw->group != dw->dimB[0] || dw->dimA[1] != dw->group || dw->group < 2 || dw->strides[0] != dw->strides[1]) continue;
+    if (!plain_buffer(dw) || !plain_buffer(pr)) continue;
+    const Op *ex = i >= 2 ? ops[i - 2] : nullptr;
+    if (ex && (block_of.count(ex) || ex->kind != OP_CONV_BIAS_ACTIV || ex->result != dw->operands[0] || !pointwise(ex) || !only_reader(ex->result, dw) || !plain_buffer(ex))) ex = nullptr;
+    // a filter that nothing else reads: its constant may be laid out for the block
+    auto own_filter = [](const Op *op) {
+      const Value *w = op->operands[1];
+      if (!w->def || w->def->kind != OP_MEM_OFFSET) return false;
+      int uploads_of_it = 0;
+      for (const auto &u : w->uses) {
+        if (u.first == op) continue;
+        const Value *src = u.first->kind == OP_MEMCPY && u.first->mode == 1 && u.second == 0 ? u.first->operands[1] : nullptr;
+        if (!src || !src->def || src->def->kind != OP_HOST_CONST || src->uses.size() != 1) return false;
+        uploads_of_it++;
+      }
+      return uploads_of_it == 1;
+    };
+    if (!own_filter(pr)) continue;
+    if (ex && !own_filter(ex)) ex = nullptr;
+    bool read_later = true;  // by operations that launch something
+    for (const auto &u : pr->result->uses) read_later = read_later && is_compute(u.first->kind) && launches(u.first);
+    const char lay = filter_crsk[(size_t)dw->operands[1]->id];
+    if (!read_later || filter_crsk[(size_t)pr->operands[1]->id] != lay || (ex && filter_crsk[(size_t)ex->operands[1]->id] != lay)) continue;
+    Block b{ex, dw, pr, (int)i, -1};
+    dnnrtExecBlock k;
+    fill_block(b, k);
+    if (!rt.dnnrtExecBlockApplies(handle, &k)) continue;
+    for (const Op *op : {ex, dw, pr})
+      if (op) block_of[op] = (int)blocks.size();
+    blocks.push_back(b);
+  }
+  // Results that would meet the block's input or residual get a place of their own.  One that cannot takes its block out,
+  // and as the other places rest on what is not stored, the search starts again.
+  for (bool again = true; again;) {
+    again = false;
+    moved_results.clear();
+    const std::map<const Value *, Range> live = live_slots();
+    std::map<const Value *, Range> moved;  // by result value
+    auto bytes_of = [&](const Value *v, Range &r) -> bool {
+      const auto m = moved.find(v);
+      if (m != moved.end()) { r = m->second; return true; }
+      const Value *s = v->def && is_compute(v->def->kind) ? v->def->operands.back() : v;
+      const auto l = live.find(s);
+      if (l == live.end()) return false;
+      r = l->second;
+      return true;
+    };
+    for (size_t q = 0; q < blocks.size() && !again; q++) {
+      Block &b = blocks[q];
+      b.y_off = -1;
+      const Value *slot = b.project->operands.back();
+      const int64_t size = slot->def->bytes;
+      std::vector<const Value *> reads{(b.expand ? b.expand : b.dw)->operands[0]};
+      if (b.project->kind == OP_CONV_BIAS_ADD_ACTIV) reads.push_back(b.project->operands[4]);
+      bool meets = false, known = true;
+      for (const Value *v : reads) {
+        Range r;
+        if (!bytes_of(v, r)) { known = false; break; }
+        meets = meets || (r.lo < slot->def->offset + size && slot->def->offset < r.hi);
+      }
+      if (known && !meets) continue;
+      int last = b.at;
+      for (const auto &u : b.project->result->uses) {
+        const auto o = block_of.find(u.first);
+        last = std::max(last, o == block_of.end() ? number[u.first] : blocks[(size_t)o->second].at);
+      }
+      std::vector<Range> taken = moved_results;
+      for (const auto &l : live) taken.push_back(l.second);
+      std::vector<int64_t> at{0};
+      for (const Range &r : taken) at.push_back(align_up(r.hi, 256));
+      std::sort(at.begin(), at.end());
+      for (const int64_t o : at) {
+        if (!known || o + size > prog->pool_bytes) continue;
+        bool ok = true;
+        for (const Range &r : taken) ok = ok && !(r.lo < o + size && o < r.hi && r.first <= last && r.last >= b.at);
+        if (!ok) continue;
+        b.y_off = o;
+        break;
+      }
+      if (b.y_off >= 0) {
+        const Range r{b.y_off, b.y_off + size, b.at, last};
+        moved_results.push_back(r);
+        moved[b.project->result] = r;
+      } else {
+        blocks.erase(blocks.begin() + (long)q);
+        block_of.clear();
+        for (size_t i = 0; i < blocks.size(); i++)
+          for (const Op *op : {blocks[i].expand, blocks[i].dw, blocks[i].project})
+            if (op) block_of[op] = (int)i;
+        again = true;
+      }
+    }
+  }
 }
 
 // Per-inference mode: where and when each constant is uploaded.
@@ -242,166 +455,195 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
 // bytes, a wait of one stream for the other 15); the first chunks are small so that the first operations start early.
 // (128 KB, 1.5 MB: within 2 %.)  ResNet-50 3.51 -> 2.56 ms, of which the link 1.85; MobileNetV2 1.52 -> 0.87.
 static constexpr int64_t UPLOAD_PART_BYTES = 512 << 10;
-bool Session::plan_uploads(std::string &err) {
-  struct Range { int64_t lo, hi; int first, last; };
-  struct Item { const Op *copy; int64_t bytes; int first, last; };
-  std::vector<Range> taken;
-  std::vector<Item> items;
-  std::map<const Value *, Range> live;  // the slots of everything but constants
+bool Session::place_constants(std::vector<UploadChunk> &chunks) const {
+  std::vector<UploadItem> items;
   std::map<const Value *, size_t> item_of;
-  std::map<const Value *, const Value *> home;  // value -> the slot it lives in
-  auto slot_of = [&](const Value *v) -> const Value * {
-    const auto it = home.find(v);
-    return it == home.end() ? nullptr : it->second;
-  };
   int n = 0;
-  auto touch = [&](const Value *v, int at) {
-    const Value *s = slot_of(v);
-    if (!s || s->def->bytes <= 0) return;
-    const auto it = item_of.find(s);
-    if (it != item_of.end()) {
-      Item &c = items[it->second];
-      if (c.first < 0) c.first = at;
-      c.last = std::max(c.last, at);
-      return;
-    }
-    const auto l = live.emplace(s, Range{s->def->offset, s->def->offset + s->def->bytes, at, at}).first;
-    l->second.last = std::max(l->second.last, at);
-  };
   for (const Op *op : prog->ops) {
-    if (op->kind == OP_MEM_OFFSET) {
-      home[op->result] = op->result;
-    } else if (op->kind == OP_MEMCPY && op->mode == 1) {
+    if (op->kind == OP_MEMCPY && op->mode == 1) {
       const Value *src = op->operands[1], *dst = op->operands[0];
-      if (src->def && src->def->kind == OP_HOST_CONST) {
-        if (op->bytes <= 0) continue;
-        if (item_of.count(dst)) return true;  // uploaded twice into one slot: not planned
-        item_of[dst] = items.size();
-        items.push_back({op, op->bytes, -1, n});
-      } else {
-        touch(dst, 0);  // an argument: from the start
-      }
-    } else if (op->kind == OP_MEMCPY) {
-      for (const Value *v : op->operands) touch(v, n);
+      if (!src->def || src->def->kind != OP_HOST_CONST || op->bytes <= 0) continue;
+      if (item_of.count(dst)) return false;  // uploaded twice into one slot: not planned
+      item_of[dst] = items.size();
+      items.push_back({op, op->bytes, -1, n});
     } else if (is_compute(op->kind)) {
-      for (const Value *v : op->operands) touch(v, n);
-      if (!op->operands.empty())
-        if (const Value *s = slot_of(op->operands.back())) home[op->result] = s;
+      const auto b = block_of.find(op);
+      const int at = b == block_of.end() ? n : blocks[(size_t)b->second].at;
+      for (const Value *v : op->operands) {
+        const auto it = item_of.find(v);
+        if (it == item_of.end()) continue;
+        UploadItem &c = items[it->second];
+        if (c.first < 0) c.first = at;
+        c.last = std::max(c.last, at);
+      }
       n++;
     }
   }
-  for (const auto &l : live) taken.push_back(l.second);
-  for (Item &c : items)
+  for (UploadItem &c : items)
     if (c.first < 0) c.first = c.last;  // nothing reads it
-  std::stable_sort(items.begin(), items.end(), [](const Item &a, const Item &b) { return a.first < b.first; });
+  std::stable_sort(items.begin(), items.end(), [](const UploadItem &a, const UploadItem &b) { return a.first < b.first; });
+  std::vector<Range> slots = moved_results;
+  for (const auto &l : live_slots()) slots.push_back(l.second);
 
-  // chunks: consecutive constants, side by side in the pool
-  struct Part { int64_t lo, hi; int after; };
-  struct Chunk { size_t lo, hi; int64_t bytes, off; int first, last; std::vector<Part> parts; };
-  std::vector<Chunk> chunks;
-  auto place = [&](Chunk &k) -> bool {
-    k.bytes = 0; k.first = items[k.lo].first; k.last = 0;
-    for (size_t i = k.lo; i < k.hi; i++) {
-      k.bytes += i + 1 < k.hi ? align_up(items[i].bytes, 256) : items[i].bytes;
-      k.last = std::max(k.last, items[i].last);
+  std::vector<Range> taken;
+  // The bytes [o, o + k.bytes) for the chunk: its parts, or false if something else holds them while it is read.
+  auto parts_at = [&](const UploadChunk &k, int64_t o, std::vector<UploadPart> &parts) -> bool {
+    const int64_t end = o + k.bytes;
+    if (end > prog->pool_bytes) return false;
+    std::vector<int64_t> cut{o, end};
+    std::vector<const Range *> met;
+    for (const Range &r : taken)
+      if (r.lo < end && o < r.hi && r.first <= k.last) {
+        if (r.last >= k.first) return false;
+        met.push_back(&r);
+        cut.push_back(std::max(o, r.lo));
+        cut.push_back(std::min(end, align_up(r.hi, 16)));
+      }
+    std::sort(cut.begin(), cut.end());
+    parts.clear();
+    for (size_t i = 0; i + 1 < cut.size(); i++) {
+      if (cut[i] == cut[i + 1]) continue;
+      int after = 0;
+      for (const Range *r : met)
+        if (r->lo < cut[i + 1] && cut[i] < r->hi) after = std::max(after, r->last + 1);
+      if (!parts.empty() && parts.back().after == after) parts.back().hi = cut[i + 1];
+      else parts.push_back({cut[i], cut[i + 1], after});
     }
+    return true;
+  };
+  auto candidates = [&](int64_t bytes) {
     std::vector<int64_t> at{0};
     for (const Range &r : taken) {
       at.push_back(align_up(r.hi, 256));
-      if (r.lo >= k.bytes) at.push_back((r.lo - k.bytes) / 256 * 256);
+      if (r.lo >= bytes) at.push_back((r.lo - bytes) / 256 * 256);
     }
-    bool found = false;
-    int64_t best = 0;
-    for (const int64_t o : at) {
-      const int64_t end = o + k.bytes;
-      if (end > prog->pool_bytes) continue;
-      std::vector<int64_t> cut{o, end};
-      std::vector<const Range *> met;
-      bool ok = true;
-      for (const Range &r : taken)
-        if (r.lo < end && o < r.hi && r.first <= k.last) {
-          if (r.last >= k.first) { ok = false; break; }
-          met.push_back(&r);
-          cut.push_back(std::max(o, r.lo));
-          cut.push_back(std::min(end, align_up(r.hi, 16)));
-        }
-      if (!ok) continue;
-      std::sort(cut.begin(), cut.end());
-      std::vector<Part> parts;
-      int64_t cost = 0;
-      for (size_t i = 0; i + 1 < cut.size(); i++) {
-        if (cut[i] == cut[i + 1]) continue;
-        int after = 0;
-        for (const Range *r : met)
-          if (r->lo < cut[i + 1] && cut[i] < r->hi) after = std::max(after, r->last + 1);
-        if (!parts.empty() && parts.back().after == after) parts.back().hi = cut[i + 1];
-        else parts.push_back({cut[i], cut[i + 1], after});
-        cost += after * (cut[i + 1] - cut[i]);
-      }
-      if (!found || cost < best || (cost == best && o < k.off)) { found = true; best = cost; k.off = o; k.parts = parts; }
-    }
-    // bytes that come free a little before the rest of the chunk are not worth a copy of their own
+    std::sort(at.begin(), at.end());
+    return at;
+  };
+  auto finish_parts = [&](UploadChunk &k) {  // bytes that come free a little before the rest are not worth a copy of their own
     std::map<int, int64_t> sizes;
-    for (const Part &q : k.parts) sizes[q.after] += q.hi - q.lo;
+    for (const UploadPart &q : k.parts) sizes[q.after] += q.hi - q.lo;
     for (auto it = sizes.begin(); it != sizes.end() && std::next(it) != sizes.end(); ++it) {
       if (it->second >= UPLOAD_PART_BYTES) continue;
       const int later = std::next(it)->first;
-      for (Part &q : k.parts)
+      for (UploadPart &q : k.parts)
         if (q.after == it->first) q.after = later;
       std::next(it)->second += it->second;
     }
-    for (const Part &q : k.parts) taken.push_back({q.lo, q.hi, q.after, k.last});
-    std::stable_sort(k.parts.begin(), k.parts.end(), [](const Part &a, const Part &b) { return a.after < b.after; });
     for (size_t i = 0; i + 1 < k.parts.size();) {
-      if (k.parts[i].after == k.parts[i + 1].after && k.parts[i].hi == k.parts[i + 1].lo) {
+      if (k.parts[i].after == k.parts[i + 1].after) {
         k.parts[i].hi = k.parts[i + 1].hi;
         k.parts.erase(k.parts.begin() + (long)i + 1);
       } else {
         i++;
       }
     }
-    return found;
+    std::stable_sort(k.parts.begin(), k.parts.end(), [](const UploadPart &a, const UploadPart &b) { return a.after < b.after; });
   };
+  auto chunk_of = [&](size_t lo, size_t hi) {
+    UploadChunk k{{items.begin() + (long)lo, items.begin() + (long)hi}, 0, 0, items[lo].first, 0, {}};
+    for (size_t i = lo; i < hi; i++) {
+      k.bytes += i + 1 < hi ? align_up(items[i].bytes, 256) : items[i].bytes;
+      k.last = std::max(k.last, items[i].last);
+    }
+    return k;
+  };
+  auto place_early = [&](UploadChunk &k) -> bool {
+    bool found = false;
+    int64_t best = 0;
+    std::vector<UploadPart> parts;
+    for (const int64_t o : candidates(k.bytes)) {
+      if (!parts_at(k, o, parts)) continue;
+      int64_t cost = 0;
+      for (const UploadPart &q : parts) cost += q.after * (q.hi - q.lo);
+      if (!found || cost < best) { found = true; best = cost; k.off = o; k.parts = parts; }
+    }
+    if (!found) return false;
+    finish_parts(k);
+    for (const UploadPart &q : k.parts) taken.push_back({q.lo, q.hi, q.after, k.last});
+    return true;
+  };
+  chunks.clear();
+  taken = slots;
+  bool ok = true;
   int64_t target = 32 << 10;
-  for (size_t i = 0; i < items.size();) {
+  for (size_t i = 0; ok && i < items.size();) {
     size_t j = i;
     int64_t sum = 0;
     do sum += items[j++].bytes;
     while (j < items.size() && (sum + items[j].bytes <= target || items[j].bytes <= 8192));
-    Chunk k{i, j, 0, 0, 0, 0, {}};
-    if (place(k)) {
+    UploadChunk k = chunk_of(i, j);
+    if (place_early(k)) {
       chunks.push_back(k);
     } else {
-      for (size_t q = i; q < j; q++) {
-        Chunk one{q, q + 1, 0, 0, 0, 0, {}};
-        if (!place(one)) return true;  // the planned slots are then used, one constant after the other
-        chunks.push_back(one);
+      for (size_t q = i; ok && q < j; q++) {
+        UploadChunk one = chunk_of(q, q + 1);
+        ok = place_early(one);
+        if (ok) chunks.push_back(one);
       }
     }
     i = j;
     target = std::min<int64_t>(2 * target, 1 << 20);
   }
+  if (ok) return true;
+  // A pool too tight for that: each constant has its bytes only while it is read, the largest are placed first.
+  chunks.clear();
+  taken = slots;
+  for (size_t i = 0; i < items.size(); i++) chunks.push_back(chunk_of(i, i + 1));
+  std::vector<size_t> order(chunks.size());
+  for (size_t i = 0; i < order.size(); i++) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return chunks[a].bytes > chunks[b].bytes; });
+  for (const size_t i : order) {
+    UploadChunk &k = chunks[i];
+    bool found = false;
+    for (const int64_t o : candidates(k.bytes)) {
+      if (!parts_at(k, o, k.parts)) continue;
+      k.off = o;
+      found = true;
+      break;
+    }
+    if (!found) return false;
+    taken.push_back({k.off, k.off + k.bytes, k.first, k.last});
+  }
+  for (UploadChunk &k : chunks) {  // what was placed since counts too
+    for (Range &r : taken)
+      if (r.lo == k.off && r.hi == k.off + k.bytes && r.first == k.first && r.last == k.last) { std::swap(r, taken.back()); break; }
+    const Range mine = taken.back();
+    taken.pop_back();
+    if (!parts_at(k, k.off, k.parts)) return false;
+    taken.push_back(mine);
+    finish_parts(k);
+  }
+  return true;
+}
 
+bool Session::plan_uploads(const std::vector<UploadChunk> &chunks, std::string &err) {
   int64_t total = 0;
-  for (const Chunk &k : chunks) total += align_up(k.bytes, 256);
+  for (const UploadChunk &k : chunks) total += align_up(k.bytes, 256);
   if (!total) return true;
   if (rt.dnnrtHostAlloc(&upload_host, total)) { err = rt_error("dnnrtHostAlloc(constants)"); return false; }
   if (rt.dnnrtStreamCreate(&upload_stream)) { err = rt_error("dnnrtStreamCreate"); return false; }
   int64_t host = 0;
   std::map<size_t, void *> moved;
   int waited = 0;
-  for (const Chunk &k : chunks) {
+  for (const UploadChunk &k : chunks) {
     int64_t in = 0;
-    for (size_t i = k.lo; i < k.hi; i++) {
-      const Op *copy = items[i].copy;
+    for (const UploadItem &item : k.items) {
+      const Op *copy = item.copy;
       void *at = (char *)upload_host + host + in;
-      std::memcpy(at, ptr[(size_t)copy->operands[1]->id], (size_t)items[i].bytes);
-      moved[(size_t)copy->operands[1]->id] = at;
+      const void *from = ptr[(size_t)copy->operands[1]->id];
+      const auto f = block_filters.find(copy->operands[0]);
+      if (f != block_filters.end()) {  // run_occamy's other path still needs the rows
+        rt.dnnrtExecBlockFilter(at, from, f->second.first, f->second.second);
+      } else {
+        std::memcpy(at, from, (size_t)item.bytes);
+        moved[(size_t)copy->operands[1]->id] = at;
+      }
       upload_slots.push_back({(size_t)copy->operands[0]->id, k.off + in});
-      in += align_up(items[i].bytes, 256);
+      in += align_up(item.bytes, 256);
     }
     for (size_t i = 0; i < k.parts.size(); i++) {
-      const Part &q = k.parts[i];
+      const UploadPart &q = k.parts[i];
       uploads.push_back({host + q.lo - k.off, q.lo, q.hi - q.lo, k.first, q.after, nullptr});
       if (i + 1 == k.parts.size() && rt.dnnrtExecFenceCreate(&uploads.back().landed)) { err = rt_error("dnnrtExecFenceCreate"); return false; }
       if (q.after > waited) {
@@ -437,6 +679,18 @@ int Session::format_for(const Op *op) const {
 
 // One compute operation -> one runtime call.
 bool Session::issue(const Op *op, std::string &err) {
+  if (use_blocks) {
+    const auto it = block_of.find(op);
+    if (it != block_of.end()) {
+      const Block &b = blocks[(size_t)it->second];
+      if (op != b.project) return true;
+      dnnrtExecBlock k;
+      fill_block(b, k);
+      if (rt.dnnrtExecRunBlock(handle, &k)) { err = rt_error("dnnrtExecRunBlock"); return false; }
+      ptr[(size_t)op->result->id] = k.y;
+      return true;
+    }
+  }
   auto P = [&](size_t i) { return ptr[(size_t)op->operands[i]->id]; };
   void *out = op->operands.empty() ? nullptr : P(op->operands.size() - 1);
   const Value *ov = op->operands.empty() ? nullptr : op->operands.back();
@@ -651,6 +905,7 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
       case OP_MEMPOOL_INIT:
         if (rt.dnnrtMemPoolInit(&run_pool, op->bytes)) return fail("dnnrtMemPoolInit");
         ptr[(size_t)op->result->id] = run_pool;
+        block_base = run_pool;
         last_pool_bytes = op->bytes;
         for (const Op *o : prog->ops)
           if (o->kind == OP_MEM_OFFSET && rt.dnnrtMemOffset(&ptr[(size_t)o->result->id], run_pool, o->offset, o->bytes)) return fail("dnnrtMemOffset");
@@ -712,7 +967,8 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
 
 // The reference's per-inference sequence, call for call.
 bool Session::run_occamy(const void *const *inputs, void *const *outputs, std::string &err) {
-  if (!uploads.empty() && debug_fill < 0) return run_uploading(inputs, outputs, err);
+  use_blocks = !uploads.empty() && debug_fill < 0;  // the fill would go over results that are not where the planner put them
+  if (use_blocks) return run_uploading(inputs, outputs, err);
   void *run_pool = nullptr;
   for (size_t i = 0; i < prog->args.size(); i++) {
     std::memcpy(host_in[i], inputs[i], (size_t)(shape_numel(prog->args[i]->shape) * dtype_bytes(prog->args[i]->dtype)));
@@ -723,7 +979,7 @@ bool Session::run_occamy(const void *const *inputs, void *const *outputs, std::s
     switch (op->kind) {
       case OP_MEMPOOL_INIT:
         if (rt.dnnrtMemPoolInit(&run_pool, op->bytes)) { err = rt_error("dnnrtMemPoolInit"); ok = false; }
-        ptr[(size_t)op->result->id] = run_pool;
+        ptr[(size_t)op->result->id] = block_base = run_pool;
         last_pool_bytes = op->bytes;
         if (ok && debug_fill >= 0 && rt.dnnrtMemFill(run_pool, debug_fill, op->bytes, stream)) { err = rt_error("dnnrtMemFill"); ok = false; }
         break;

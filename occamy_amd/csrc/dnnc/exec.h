@@ -79,6 +79,9 @@ struct RuntimeApi {
   decltype(&::dnnrtExecFenceCreate) dnnrtExecFenceCreate = nullptr;
   decltype(&::dnnrtExecStreamWait) dnnrtExecStreamWait = nullptr;
   decltype(&::dnnrtExecUpload) dnnrtExecUpload = nullptr;
+  decltype(&::dnnrtExecBlockApplies) dnnrtExecBlockApplies = nullptr;
+  decltype(&::dnnrtExecRunBlock) dnnrtExecRunBlock = nullptr;
+  decltype(&::dnnrtExecBlockFilter) dnnrtExecBlockFilter = nullptr;
 };
 
 bool load_runtime(const std::string &path, RuntimeApi &rt, std::string &err);
@@ -151,6 +154,23 @@ class Session {
   std::map<size_t, void *> arg_home;  // resident mode: value id of a function argument's pool slot -> its address in the pool
   std::vector<const Op *> direct_out;  // the result copies of the current run that are not needed for that reason
   std::map<size_t, void *> out_home;  // ... and of a result's pool tensor, when results are written where the caller wants them
+  // Bytes of the pool and the compute operations (counted in program order) between which they hold something.
+  struct Range { int64_t lo, hi; int first, last; };
+  // Inverted residual blocks that run as one call (plan_blocks): issued where their last convolution stands.
+  struct Block {
+    const Op *expand, *dw, *project;  // expand may be null
+    int at;                           // the last convolution's number
+    int64_t y_off;                    // where in the pool the result goes, or -1: its planned slot
+  };
+  std::vector<Block> blocks;
+  std::map<const Op *, int> block_of;  // their operations; the block's number
+  std::vector<Range> moved_results;    // the places y_off names
+  bool use_blocks = false;
+  void *block_base = nullptr;          // the pool of the current run
+  void fill_block(const Block &b, dnnrtExecBlock &k) const;
+  std::map<const Value *, std::pair<int64_t, int64_t>> block_filters;  // device tensors uploaded in the block call's layout; rows, columns
+  void plan_blocks();
+  std::map<const Value *, Range> live_slots() const;
   // Per-inference mode on the GPU runtime: the constants as they go to the device on a second stream, ahead of the
   // operations that read them (plan_uploads).  Compute operations are counted in program order.
   struct Upload {
@@ -164,7 +184,12 @@ class Session {
   std::map<int, void *> op_done;                         // recorded when that many operations are issued
   void *upload_host = nullptr;
   dnnrtStream_t upload_stream = nullptr;
-  bool plan_uploads(std::string &err);
+  // Constants that travel together, side by side in the pool; `parts` have places that come free at different times.
+  struct UploadItem { const Op *copy; int64_t bytes; int first, last; };
+  struct UploadPart { int64_t lo, hi; int after; };
+  struct UploadChunk { std::vector<UploadItem> items; int64_t bytes, off; int first, last; std::vector<UploadPart> parts; };
+  bool place_constants(std::vector<UploadChunk> &chunks) const;
+  bool plan_uploads(const std::vector<UploadChunk> &chunks, std::string &err);
   bool run_uploading(const void *const *inputs, void *const *outputs, std::string &err);
   std::map<std::string, void *> host_const;
   std::vector<void *> host_out, host_in;

@@ -15,6 +15,25 @@ int32_t dnnrtExecStreamWait(dnnrtStream_t stream, void *event);
 /* Copies pinned host memory to the device with a kernel: dst and src 16-byte aligned. */
 int32_t dnnrtExecUpload(void *dst, const void *src, int64_t bytes, dnnrtStream_t stream);
 
+/* An inverted residual block: y = act(conv1x1(actd(dwconv(act1(conv1x1(x, w1) + b1), wd) + bd), w3) + b3 [+ z]), square
+ * stride, group of the middle convolution = its channels.  Results as from the separate calls.
+ * fp16: w1 and w3 in blocks, dnnrtExecBlockFilter. */
+typedef struct dnnrtExecBlock {
+  const void *x, *w1, *b1, *wd, *bd, *w3, *b3, *z; /* w1, b1: not read without expansion; z: residual laid out like y, or null */
+  void *y;
+  int64_t n, cin, h, w, ch, r, s, stride, pad_h, pad_w, p, q, cout;
+  int64_t act1, actd, act; /* activation modes of the three convolutions and their coefficients */
+  float coef1, coefd, coef;
+  int32_t expand, dtype, format, filter_layout;
+} dnnrtExecBlock;
+/* 1 if dnnrtExecRunBlock takes the block (pointers aside) and is meant to be faster than the three calls. */
+int32_t dnnrtExecBlockApplies(dnnrtHandle_t handle, const dnnrtExecBlock *block);
+/* The layout of a 1x1 filter (rows x cols, fp16) for the block call, on the host: for every 32 rows, every 8 columns, the
+ * rows' 8 values each. */
+void dnnrtExecBlockFilter(void *dst, const void *src, int64_t rows, int64_t cols);
+/* y must not overlap x or z. */
+int32_t dnnrtExecRunBlock(dnnrtHandle_t handle, const dnnrtExecBlock *block);
+
 #ifdef __cplusplus
 }
 #endif

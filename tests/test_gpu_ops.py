@@ -6,6 +6,8 @@ add/mul, reciprocal and sqrt (no reassociation is involved); fp32 reductions
 and transcendental functions within rtol 1e-4 / atol 1e-5 of the oracle
 (which accumulates in double); fp16 storage within rtol 2e-2.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -1427,3 +1429,63 @@ def test_matmul2d_f16(gpu, cpu):
                 if not tA:
                     np.testing.assert_allclose(oc.matmul2d_row(gpu, a, b, row, beta=0.5, transB=tB).astype(np.float32),
                                                oc.matmul2d_row(cpu, a, b, row, beta=0.5, transB=tB).astype(np.float32), rtol=4e-3, atol=6e-3)
+
+
+class ExecBlock(C.Structure):
+    _fields_ = ([(n, C.c_void_p) for n in ("x", "w1", "b1", "wd", "bd", "w3", "b3", "z", "y")] +
+                [(n, C.c_int64) for n in ("n", "cin", "h", "w", "ch", "r", "s", "stride", "pad_h", "pad_w", "p", "q", "cout", "act1", "actd", "act")] +
+                [(n, C.c_float) for n in ("coef1", "coefd", "coef")] + [(n, C.c_int32) for n in ("expand", "dtype", "format", "filter_layout")])
+
+
+@pytest.mark.parametrize("n,cin,h,w,ch,cout,stride,expand,residual", [
+    (1, 8, 5, 7, 48, 8, 1, True, False),       # less than one tile, channels short of every block
+    (2, 16, 33, 17, 96, 24, 2, True, False),   # one step of input channels, stride 2, ragged tiles
+    (1, 24, 28, 29, 144, 24, 1, True, True),   # half a step, half a group of channels, residual
+    (3, 64, 14, 14, 384, 64, 1, True, True),
+    (1, 96, 7, 9, 576, 160, 2, True, False),   # most steps, five blocks of output channels
+    (2, 40, 11, 10, 200, 328, 1, True, False),  # output channels over two workgroups
+    (1, 32, 30, 31, 32, 16, 1, False, False),  # no expansion
+    (1, 24, 13, 12, 24, 24, 2, False, False),
+])
+def test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, residual):
+    """The block call of the executor against fp32 arithmetic on the same operands, rounded to fp16 where the three
+    separate calls round."""
+    import torch
+    import torch.nn.functional as F
+    g = torch.Generator().manual_seed(n * 1000 + cin)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    x = rnd(n, cin, h, w).half()
+    w1, b1 = (rnd(ch, cin) * (2 / cin) ** 0.5).half(), rnd(ch).half() * 0.5
+    wd, bd = (rnd(ch, 1, 3, 3) * 0.4).half(), rnd(ch).half() * 0.5
+    w3, b3 = (rnd(cout, ch) * (1 / ch) ** 0.5).half(), rnd(cout).half() * 0.5
+    r16 = lambda t: t.half().float()  # noqa: E731
+    t = x.float()
+    if expand:
+        t = r16(F.conv2d(t, w1.float()[:, :, None, None], b1.float()).clamp(0, 6))
+    t = r16(F.conv2d(t, wd.float(), bd.float(), stride, 1, groups=ch).clamp(0, 6))
+    want = F.conv2d(t, w3.float()[:, :, None, None], b3.float())
+    p, q = want.shape[2:]
+    z = rnd(n, cout, p, q).half() if residual else None
+    want = r16(r16(want) + z.float()) if residual else r16(want)
+
+    lib = C.CDLL(_abi.RUNTIME_PATH)
+    handle = C.c_void_p()
+    assert lib.dnnrtCreate(C.byref(handle)) == 0
+    lib.dnnrtExecBlockFilter.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64]
+
+    def blocked(m):
+        out = torch.empty_like(m)
+        lib.dnnrtExecBlockFilter(out.data_ptr(), m.contiguous().data_ptr(), m.shape[0], m.shape[1])
+        return out.cuda()
+    keep = dict(x=x.permute(0, 2, 3, 1).contiguous().cuda(), w1=blocked(w1) if expand else None, b1=b1.cuda() if expand else None,
+                wd=wd.cuda(), bd=bd.cuda(), w3=blocked(w3), b3=b3.cuda(), z=None if z is None else z.permute(0, 2, 3, 1).contiguous().cuda(),
+                y=torch.full((n, p, q, cout), float("nan"), dtype=torch.half, device="cuda"))
+    k = ExecBlock(n=n, cin=cin, h=h, w=w, ch=ch, r=3, s=3, stride=stride, pad_h=1, pad_w=1, p=p, q=q, cout=cout, act1=3, actd=3, act=5,
+                  coef1=6.0, coefd=6.0, expand=int(expand), dtype=_abi.F16, format=1, **{m: v.data_ptr() for m, v in keep.items() if v is not None})
+    torch.cuda.synchronize()
+    lib.dnnrtLastError.restype = C.c_char_p
+    assert lib.dnnrtExecRunBlock(handle, C.byref(k)) == 0, lib.dnnrtLastError()
+    torch.cuda.synchronize()
+    got = keep["y"].permute(0, 3, 1, 2).float().cpu()
+    lib.dnnrtDestroy(handle)
+    np.testing.assert_allclose(got.numpy(), want.numpy(), rtol=4e-3, atol=8e-3)
