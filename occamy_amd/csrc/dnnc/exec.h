@@ -1,5 +1,6 @@
 #pragma once
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -165,7 +166,10 @@ class Session {
   std::vector<Block> blocks;
   std::map<const Op *, int> block_of;  // their operations; the block's number
   std::vector<Range> moved_results;    // the places y_off names
-  bool use_blocks = false;
+  bool use_blocks = false;             // ... and `elided`: not while a debug fill marks the planned slots
+  // Flatten, Reshape, Squeeze and Unsqueeze whose readers read the input where it is (plan_elided_copies)
+  std::set<const Op *> elided;
+  void plan_elided_copies();
   void *block_base = nullptr;          // the pool of the current run
   void fill_block(const Block &b, dnnrtExecBlock &k) const;
   std::map<const Value *, std::pair<int64_t, int64_t>> block_filters;  // device tensors uploaded in the block call's layout; rows, columns
