@@ -98,6 +98,31 @@ def test_conv_f32(gpu, cpu, case):
     np.testing.assert_array_equal(oc.conv(cpu, x, w, b, *args, _abi.ACT_RELU, z=z, inplace=True), oc.conv(cpu, x, w, b, *args, _abi.ACT_RELU, z=z))
 
 
+# N, C, H, W, K, stride, pad: 3x3 depthwise layers with outputs enough for strips of four rows (N K ceil(P/4) Q from
+# 2048 threads per compute unit on): rows that leave one, two or three over, one row, no padding and more than needed,
+# two results per channel, stride 2 with even and odd sides, the last strip and image together.
+DW_ROWS_CASES = [(4, 96, 113, 111, 96, 1, 1), (3, 160, 78, 79, 160, 1, 0), (2, 64, 119, 121, 128, 1, 2), (600, 64, 1, 14, 64, 1, 1),
+                 (6, 64, 150, 149, 64, 2, 1), (4, 96, 151, 152, 96, 2, 0), (257, 576, 14, 14, 576, 2, 1)]
+
+
+@pytest.mark.parametrize("case", DW_ROWS_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_conv_f32_depthwise_strips(gpu, cpu, case):
+    """Depthwise layers computed in strips of rows against the oracle, both filter layouts, with a residual and over it."""
+    N, C, H, W, K, st, pd = case
+    r = rng(sum(case))
+    x = r.standard_normal((N, C, H, W)).astype(np.float32)
+    w = (r.standard_normal((K, 1, 3, 3)) / 3).astype(np.float32)
+    b = r.uniform(-0.3, 0.3, K).astype(np.float32)
+    args = ((pd, pd), (st, st), C)
+    lin = oc.conv(cpu, x, w, b, *args, _abi.ACT_IDENTITY)
+    close(oc.conv(gpu, x, w, None, *args), lin - b[:, None, None], atol=1e-5)
+    z = r.standard_normal(lin.shape).astype(np.float32)
+    for crsk in (False, True):
+        gotz = oc.conv(gpu, x, w, b, *args, _abi.ACT_RELU, crsk=crsk, z=z)
+        close(gotz, np.maximum(lin + z, 0))
+        np.testing.assert_array_equal(oc.conv(gpu, x, w, b, *args, _abi.ACT_RELU, crsk=crsk, z=z, inplace=True), gotz)
+
+
 def random_conv_cases(seed, count, f16):
     """Seeded shapes around the kernels' boundaries: channel counts on both sides of the multiples of 8, 32 and
     64 the fast paths ask for, filter sizes 1 / 2 / 3 / 5 / 7, strides 1-3 (different along the two axes now and
