@@ -62,7 +62,9 @@ __device__ __forceinline__ void d32_barrier() {
 
 // TAPS: the filter has more than one tap, or padding.  Reduction order: with C4 (C a multiple of 4) tap by tap, the
 // channels of a tap in a row, so that the four k a wavefront loads per step share their tap; without it (a first layer
-// of three channels) in the filter's own order c, r, s, the taps looked up per k.
+// of three channels) in the filter's own order c, r, s, the taps looked up per k.  POINTWISE and C4 test the reduction's
+// end once for a wavefront's four k, so both need C a multiple of 4 (of either convolution of a pair); ANY masks each k
+// and takes the rest, one-tap filters among them.
 enum { D32_POINTWISE = 0, D32_TAPS_C4 = 1, D32_TAPS_ANY = 2 };
 
 template <int BM, int BN, int WM, int WN, int NS, int U, int AV, int BV, int MODE, bool DUAL>
@@ -542,11 +544,11 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
   const bool pointwise = a.R == 1 && a.S == 1 && a.ph == 0 && a.pw == 0;
   if (dual && (!pointwise || a.Kdim % 4 || a.Kdim2 % 4 || 4 * images * a.x2_img_stride > lim || 4 * (int64_t)a.Kdim2 * a.a_ld > lim)) return true;
   const int RS = a.R * a.S, C = a.Kdim / RS;
-  const bool av4 = a.M % 4 == 0 && a.a_ld % 4 == 0 && aligned16(a.A) && (!dual || aligned16(a.A2)) && (!pointwise || C % 4 == 0);
+  const bool av4 = a.M % 4 == 0 && a.a_ld % 4 == 0 && aligned16(a.A) && (!dual || aligned16(a.A2));
   if (dual && !av4) return true;
   const bool bv4 = pointwise && a.sh == 1 && a.sw == 1 && PQ % 4 == 0 && C % 4 == 0 && aligned16(a.X) &&
                    (!dual || (a.sh2 == 1 && a.sw2 == 1 && aligned16(a.X2)));
-  const int mode = pointwise ? D32_POINTWISE : C % 4 == 0 ? D32_TAPS_C4 : D32_TAPS_ANY;
+  const int mode = C % 4 ? D32_TAPS_ANY : pointwise ? D32_POINTWISE : D32_TAPS_C4;
   a.magic_pq = magic_of(PQ);
   a.magic_q = magic_of(a.Q);
   a.magic_rs = magic_of(RS);

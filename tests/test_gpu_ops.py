@@ -198,6 +198,31 @@ def test_conv_f32_direct_to_lds_tiles(gpu, cpu, case):
     np.testing.assert_array_equal(oc.conv(gpu, x, w, b, *args, _abi.ACT_RELU, crsk=True, z=z, inplace=True), gotz)
 
 
+# channel counts around the four rows a wavefront loads at a time; sizes that fill the chip, whole tiles and split ones
+@pytest.mark.parametrize("C", [1, 2, 3, 5, 29, 30, 33, 47])
+@pytest.mark.parametrize("N,H,W,K,stride", [(3, 75, 75, 66, 1), (6, 56, 56, 64, 1), (10, 60, 60, 128, 2)])
+def test_pointwise_conv_f32_any_channel_count(gpu, cpu, C, N, H, W, K, stride):
+    """fp32 1x1 layers without padding whose channels are no multiple of four: against the oracle, and an image of
+    infinities leaves the images beside it as they are, bit for bit (the rows past an image's last channel are the next
+    image's first ones)."""
+    r = rng(100 * C + H)
+    x = r.standard_normal((N, C, H, W)).astype(np.float32)
+    w = (r.standard_normal((K, C, 1, 1)) * np.sqrt(1.0 / C)).astype(np.float32)
+    b = r.uniform(-0.3, 0.3, K).astype(np.float32)
+    args = ((0, 0), (stride, stride), 1, _abi.ACT_IDENTITY)
+    got = oc.conv(gpu, x, w, b, *args, crsk=True)
+    np.testing.assert_allclose(got, oc.conv(cpu, x, w, b, *args), rtol=RTOL, atol=ATOL)
+    for bad in (np.inf, np.nan):
+        xi = x.copy()
+        xi[N - 2] = bad
+        goti = oc.conv(gpu, xi, w, b, *args, crsk=True)
+        for n in range(N):
+            if n == N - 2:
+                assert not np.isfinite(goti[n]).any()
+            else:
+                np.testing.assert_array_equal(goti[n], got[n])
+
+
 def test_conv_f16_random_shapes(gpu, cpu):
     """120 seeded shapes through the fp16 convolution, channels-last (every fast path's boundary: channel counts
     around the multiples of 8 / 32 / 64, a few steps or many, padded or not, grouped and depthwise) and, every
