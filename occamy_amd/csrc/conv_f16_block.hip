@@ -345,6 +345,10 @@ constexpr int BLOCK_PER_GROUP = 2 * 32 * 4 + 32 * 9 * 2;  // biases and depthwis
 static bool plan_block_f16(int num_cu, const dnnrtExecBlock &k, bool faster, BlockF16Args &a, int &kc, int &grid_y, int &G) {
   if (k.dtype != DNNRT_F16 || k.format != DNNRT_NHWC || k.r != 3 || k.s != 3 || (k.stride != 1 && k.stride != 2) || k.cin % 8 || k.ch % 8 || k.cout % 8) return false;
   if (!k.expand && k.cin != k.ch) return false;
+  // Every tile's patch must hold a row and a column of the image (the kernel divides by their number, and with none it would
+  // compute padding from what lies beside the image): tiles are two pixels or more, so a padding of up to two leaves one.
+  if (k.n < 1 || k.h < 1 || k.w < 1 || k.pad_h < 0 || k.pad_h > 2 || k.pad_w < 0 || k.pad_w > 2) return false;
+  if (k.h + 2 * k.pad_h < 3 || k.w + 2 * k.pad_w < 3 || k.p != (k.h + 2 * k.pad_h - 3) / k.stride + 1 || k.q != (k.w + 2 * k.pad_w - 3) / k.stride + 1) return false;
   const int64_t lim = 1ll << 29;  // elements of a buffer
   if (k.h * k.w * k.cin > lim || k.p * k.q * k.cout > lim || k.ch * std::max(k.cin, k.cout) > lim || k.n * k.p * k.q > lim || k.ch > 4096 || k.cout > 4096) return false;
   if ((k.expand && !clamp_of(k.act1, k.coef1, a.lo1, a.hi1)) || !clamp_of(k.actd, k.coefd, a.lod, a.hid)) return false;
