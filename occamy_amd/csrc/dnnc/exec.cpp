@@ -354,9 +354,7 @@ void Session::plan_elided_copies() {
     if (!moves_nothing(op) || !launches(op) || !plain_buffer(op)) continue;
     bool read = true;
     for (const auto &u : op->result->uses) read = read && is_compute(u.first->kind) && u.second + 1 < (int)u.first->operands.size();
-    const Value *x = op->operands[0];
-    while (x->def && elided.count(x->def)) x = x->def->operands[0];
-    const Value *slot = x->def && is_compute(x->def->kind) && !x->def->operands.empty() ? x->def->operands.back() : x;
+    const Value *slot = buffer_of(op->operands[0]);
     if (!read || !slot->def || slot->def->kind != OP_MEM_OFFSET) continue;
     elided.insert(op);
     const std::map<const Value *, Range> live = live_slots();
@@ -370,6 +368,12 @@ void Session::plan_elided_copies() {
       if (is_compute(u.first->kind) && u.second + 1 == (int)u.first->operands.size() && number[u.first] > number[op]) ok = false;
     if (!ok) elided.erase(op);
   }
+}
+
+// The tensor that a value lies in: its producer's output buffer, its input's where the producer moves nothing.
+const Value *Session::buffer_of(const Value *v) const {
+  while (v->def && elided.count(v->def)) v = v->def->operands[0];
+  return v->def && is_compute(v->def->kind) && !v->def->operands.empty() ? v->def->operands.back() : v;
 }
 
 // Which runs of two or three convolutions are one inverted residual block, and where its result goes.
@@ -386,6 +390,18 @@ void Session::plan_blocks() {
     if (is_compute(op->kind)) { number[op] = (int)ops.size(); ops.push_back(op); }
   auto pointwise = [](const Op *op) {
     return op->group == 1 && op->dimB.size() == 4 && op->dimB[2] == 1 && op->dimB[3] == 1 && op->pads[0] == 0 && op->pads[1] == 0 && op->strides[0] == 1 && op->strides[1] == 1;
+  };
+  // The tensors that a run in place has at the caller's addresses (run_resident), aligned to an element: arguments and the
+  // buffers that results are computed into.  The block call needs 16-byte aligned operands, the three calls take any.
+  std::set<const Value *> callers;
+  for (const Op *op : prog->ops) {
+    if (op->kind == OP_MEMCPY && op->mode == 1 && op->operands[1]->arg_index >= 0) callers.insert(op->operands[0]);
+    if (op->kind == OP_MEMCPY && op->mode == 2) callers.insert(buffer_of(op->operands[1]));
+  }
+  auto in_pool = [&](const Op *op, bool first, bool stored) {
+    for (size_t i = first ? 0 : 1; i < op->operands.size() - (stored ? 0 : 1); i++)
+      if (callers.count(buffer_of(op->operands[i]))) return false;
+    return true;
   };
   auto only_reader = [](const Value *v, const Op *reader) { return v->uses.size() == 1 && v->uses[0].first == reader && v->uses[0].second == 0; };
   for (size_t i = 1; i < ops.size(); i++) {
@@ -408,8 +424,9 @@ void Session::plan_blocks() {
       }
       return uploads_of_it == 1;
     };
-    if (!own_filter(pr)) continue;
-    if (ex && !own_filter(ex)) ex = nullptr;
+    if (!own_filter(pr) || !in_pool(pr, false, true)) continue;
+    if (ex && (!own_filter(ex) || !in_pool(ex, true, false))) ex = nullptr;
+    if (!in_pool(dw, !ex, false)) continue;
     bool read_later = true;  // by operations that launch something
     for (const auto &u : pr->result->uses) read_later = read_later && is_compute(u.first->kind) && launches(u.first) && !elided.count(u.first);
     const char lay = filter_crsk[(size_t)dw->operands[1]->id];

@@ -170,6 +170,7 @@ class Session {
   // Flatten, Reshape, Squeeze and Unsqueeze whose readers read the input where it is (plan_elided_copies)
   std::set<const Op *> elided;
   void plan_elided_copies();
+  const Value *buffer_of(const Value *v) const;
   void *block_base = nullptr;          // the pool of the current run
   void fill_block(const Block &b, dnnrtExecBlock &k) const;
   std::map<const Value *, std::pair<int64_t, int64_t>> block_filters;  // device tensors uploaded in the block call's layout; rows, columns

@@ -46,7 +46,7 @@ def test_which_blocks_the_call_takes():
     ops.close()
 
 
-def small_net(batch, height, width, stride, pads, dtype=np.float16, cin=24, hidden=144, cout=32, residual=False):
+def small_net(batch, height, width, stride, pads, dtype=np.float16, cin=24, hidden=144, cout=32):
     """A 3x3 layer, one inverted residual block with the given depthwise padding, a 1x1 layer and a pooled result."""
     r = np.random.default_rng(batch * height + width + stride)
     g = compiler.Graph()
@@ -60,12 +60,10 @@ def small_net(batch, height, width, stride, pads, dtype=np.float16, cin=24, hidd
     def relu6(v):
         return g.node("Clip", [v, g.constant(np.array(0.0, dtype)), g.constant(np.array(6.0, dtype))])
 
-    v = y = relu6(conv(x, 3, cin, 3, 1, (1, 1)))
+    v = relu6(conv(x, 3, cin, 3, 1, (1, 1)))
     v = relu6(conv(v, cin, hidden, 1, 1, (0, 0)))
     v = relu6(conv(v, hidden, hidden, 3, stride, pads, hidden))
     v = conv(v, hidden, cout, 1, 1, (0, 0))
-    if residual:
-        v = g.node("Add", [v, y])
     v = relu6(conv(v, cout, 48, 1, 1, (0, 0)))
     g.output(g.node("Flatten", [g.node("GlobalAveragePool", [v])], axis=1))
     return g, [r.standard_normal((batch, 3, height, width)).astype(dtype)]
@@ -75,11 +73,76 @@ def small_net(batch, height, width, stride, pads, dtype=np.float16, cin=24, hidd
 @pytest.mark.parametrize("pads", [(0, 0), (1, 2), (2, 0), (2, 2), (3, 1), (1, 3), (4, 4), (5, 3)], ids=str)
 def test_any_depthwise_padding(pads, stride):
     """Paddings the block call takes and paddings it leaves to the three calls; images down to a pixel or two."""
-    for batch, height, width in ((8, 28, 31), (16, 9, 2), (16, 1, 12)):
+    ops = Ops()
+    for batch, height, width in ((128, 28, 31), (512, 9, 2), (512, 1, 12)):
         if height + 2 * pads[0] < 3 or width + 2 * pads[1] < 3:
             continue
-        build = lambda: small_net(batch, height, width, stride, pads)  # noqa: E731
+        sizes = dict(cin=16, hidden=96, cout=24)
+        if stride == 1 or height == 28:
+            b = block(batch, 16, height, width, 96, 24, stride, *pads)
+            assert ops.lib.dnnrtExecBlockApplies(ops.handle, C.byref(b)) == (max(pads) <= 2)
+        build = lambda: small_net(batch, height, width, stride, pads, **sizes)  # noqa: E731
         ref, _ = run(lambda: as_fp32_graph(*build()), ORACLE_PATH, fusion=True)
         for mode in (compiler.MODE_OCCAMY, compiler.MODE_RESIDENT):
             got, _ = run(build, mode=mode, **FLAGS)
             close16(got[0], ref[0])
+    ops.close()
+
+
+def test_operands_at_any_address():
+    """A block some of whose operands are the program's arguments, or whose result lies in the tensor that is returned: a
+    run in place hands those over at the caller's addresses, which are aligned to an element only."""
+    import torch
+    batch, cin, hidden, cout, side = 32, 24, 144, 24, 28
+    r = np.random.default_rng(5)
+    half = lambda *s, f=1.0: (r.standard_normal(s) * f).astype(np.float16)  # noqa: E731
+    values = {"x": half(batch, 3, side, side), "b1": half(hidden), "wd": half(hidden, 1, 3, 3, f=0.4), "bd": half(hidden), "b3": half(cout)}
+
+    def build(args, dtype=np.float16):
+        r2 = np.random.default_rng(6)
+        g = compiler.Graph()
+        c = lambda *s: g.constant((r2.standard_normal(s) * np.sqrt(2.0 / np.prod(s[1:]))).astype(np.float16).astype(dtype))  # noqa: E731
+        v = {n: g.input(n, a.shape, dtype) if n == "x" or n in args else g.constant(a.astype(dtype)) for n, a in values.items()}
+        clip = lambda t: g.node("Clip", [t, g.constant(np.array(0.0, dtype)), g.constant(np.array(6.0, dtype))])  # noqa: E731
+        one = dict(kernel_shape=[1, 1], pads=[0] * 4, strides=[1, 1], group=1)
+        t = clip(g.node("Conv", [v["x"], c(cin, 3, 3, 3), g.constant(np.zeros(cin, dtype))], kernel_shape=[3, 3], pads=[1] * 4, strides=[1, 1], group=1))
+        t = clip(g.node("Conv", [t, c(hidden, cin, 1, 1), v["b1"]], **one))
+        t = clip(g.node("Conv", [t, v["wd"], v["bd"]], kernel_shape=[3, 3], pads=[1] * 4, strides=[1, 1], group=hidden))
+        t = g.node("Conv", [t, c(cout, hidden, 1, 1), v["b3"]], **one)
+        t = clip(g.node("Conv", [t, c(40, cout, 1, 1), g.constant(np.zeros(40, dtype))], **one))
+        g.output(g.node("Flatten", [g.node("GlobalAveragePool", [t])], axis=1))
+        return g, [values[n] for n in g.input_shapes]
+
+    def closing_layer(dtype=np.float16):  # a block's result is added to in place by the layer whose result is returned
+        r2 = np.random.default_rng(7)
+        g = compiler.Graph()
+        c = lambda *s: g.constant((r2.standard_normal(s) * 0.2).astype(np.float16).astype(dtype))  # noqa: E731
+        clip = lambda t: g.node("Clip", [t, g.constant(np.array(0.0, dtype)), g.constant(np.array(6.0, dtype))])  # noqa: E731
+        conv = lambda t, ci, co, k=1, group=1: g.node("Conv", [t, c(co, ci // group, k, k), c(co)], kernel_shape=[k, k], pads=[k // 2] * 4, strides=[1, 1], group=group)  # noqa: E731
+        y = clip(conv(g.input("x", (64, 16, 1, 1), dtype), 16, 24))
+        y = conv(clip(conv(clip(conv(y, 24, 48)), 48, 48, 3, 48)), 48, 24)
+        g.output(g.node("Add", [conv(y, 24, 24), y]))
+        return g, [np.random.default_rng(8).standard_normal((64, 16, 1, 1)).astype(dtype)]
+
+    ops = Ops()
+    for b in (block(batch, cin, side, side, hidden, cout, 1, 1, 1), block(64, 24, 1, 1, 48, 24, 1, 1, 1)):
+        assert ops.lib.dnnrtExecBlockApplies(ops.handle, C.byref(b))
+    ops.close()
+    nets = [lambda args=args: build(args) for args in ((), ("b1",), ("wd",), ("bd",), ("b3",), ("b1", "wd", "bd", "b3"))]
+    for net in nets + [closing_layer]:
+        ref, _ = run(lambda: as_fp32_graph(*net()), ORACLE_PATH, fusion=True)
+        g, inputs = net()
+        s = g.compile(inplace_residual=True, **FLAGS).session(compiler.MODE_RESIDENT)
+        n = ref[0].size
+        for off in (0, 1):
+            bufs = [torch.zeros(a.size + 8, dtype=torch.float16, device="cuda") for a in inputs]
+            for b, a in zip(bufs, inputs):
+                b[off:off + a.size] = torch.from_numpy(a.reshape(-1)).cuda()
+            out = torch.zeros(n + 8, dtype=torch.float16, device="cuda")
+            for use_graph in (False, True, True):
+                out.zero_()
+                torch.cuda.synchronize()
+                s.run_device([b.data_ptr() + 2 * off for b in bufs], [out.data_ptr() + 2 * off], use_graph=use_graph, in_place=True)
+                s.sync()
+                close16(out[off:off + n].cpu().numpy().reshape(ref[0].shape), ref[0])
+        s.close()
