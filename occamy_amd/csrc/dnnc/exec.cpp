@@ -228,6 +228,10 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
       staged_out[op] = stage;
     }
   }
+  for (const Op *op : prog->ops) {
+    if (op->kind == OP_MEMCPY && op->mode == 1 && op->operands[1]->arg_index >= 0) callers.insert(op->operands[0]);
+    if (op->kind == OP_MEMCPY && op->mode == 2) callers.insert(buffer_of(op->operands[1]));
+  }
   if (mode == MODE_RESIDENT) plan_elided_copies();  // per inference, the longer lives would stand in the way of the uploads
   plan_blocks();
   // Both modes take the same blocks (the same bits): those that a per-inference program can have with its constants uploaded
@@ -341,8 +345,9 @@ static bool plain_buffer(const Op *op) {
   return true;
 }
 
-// Copies that move no element need not run where their input's bytes stay as they are until the copy's last reader: the
-// planner's lifetimes say so.  (The alias_copies pass does the same to the program; one compiled without it still has the
+// Copies that move no element need not run where their input's bytes stay as they are until the copy's last reader (the
+// planner's lifetimes say so) and lie in the pool: what a run in place has at the caller's address need not be aligned as
+// the copy is.  (The alias_copies pass does the same to the program; one compiled without it still has the
 // calls and the slots, a launch of 4.5 us or a pass over memory each.)  SRGAN's generator at 90x117 0.779 -> 0.759 ms,
 // SSD300 1.622 -> 1.609, AlexNet at batch 1 0.136 -> 0.131; what is left is overwritten by the next operation's result.
 void Session::plan_elided_copies() {
@@ -355,7 +360,7 @@ void Session::plan_elided_copies() {
     bool read = true;
     for (const auto &u : op->result->uses) read = read && is_compute(u.first->kind) && u.second + 1 < (int)u.first->operands.size();
     const Value *slot = buffer_of(op->operands[0]);
-    if (!read || !slot->def || slot->def->kind != OP_MEM_OFFSET) continue;
+    if (!read || !slot->def || slot->def->kind != OP_MEM_OFFSET || callers.count(slot)) continue;
     elided.insert(op);
     const std::map<const Value *, Range> live = live_slots();
     const auto mine = live.find(slot);
@@ -391,13 +396,7 @@ void Session::plan_blocks() {
   auto pointwise = [](const Op *op) {
     return op->group == 1 && op->dimB.size() == 4 && op->dimB[2] == 1 && op->dimB[3] == 1 && op->pads[0] == 0 && op->pads[1] == 0 && op->strides[0] == 1 && op->strides[1] == 1;
   };
-  // The tensors that a run in place has at the caller's addresses (run_resident), aligned to an element: arguments and the
-  // buffers that results are computed into.  The block call needs 16-byte aligned operands, the three calls take any.
-  std::set<const Value *> callers;
-  for (const Op *op : prog->ops) {
-    if (op->kind == OP_MEMCPY && op->mode == 1 && op->operands[1]->arg_index >= 0) callers.insert(op->operands[0]);
-    if (op->kind == OP_MEMCPY && op->mode == 2) callers.insert(buffer_of(op->operands[1]));
-  }
+  // The block call needs 16-byte aligned operands, the three calls take any.
   auto in_pool = [&](const Op *op, bool first, bool stored) {
     for (size_t i = first ? 0 : 1; i < op->operands.size() - (stored ? 0 : 1); i++)
       if (callers.count(buffer_of(op->operands[i]))) return false;

@@ -171,6 +171,9 @@ class Session {
   std::set<const Op *> elided;
   void plan_elided_copies();
   const Value *buffer_of(const Value *v) const;
+  // The tensors that a run in place has at the caller's addresses (run_resident), which are aligned to an element only:
+  // arguments, and the buffers that results are computed into.
+  std::set<const Value *> callers;
   void *block_base = nullptr;          // the pool of the current run
   void fill_block(const Block &b, dnnrtExecBlock &k) const;
   std::map<const Value *, std::pair<int64_t, int64_t>> block_filters;  // device tensors uploaded in the block call's layout; rows, columns

@@ -505,6 +505,60 @@ def test_resident_run_reads_device_inputs_in_place():
         s.close()
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_resident_run_in_place_of_reshaped_arguments_at_any_address(dtype):
+    """Arguments that a Reshape turns into attention operands, and a result that is read on after a Reshape, with the
+    caller's buffers aligned to an element only: a copy that moves no element still gives its reader an aligned tensor."""
+    import torch
+    seq, heads, dh = 40, 2, 32
+    hidden = heads * dh
+
+    def build(dtype=dtype):
+        g = compiler.Graph()
+        r = np.random.default_rng(9)
+        ins = {n: r.standard_normal((seq, hidden)).astype(np.float16).astype(dtype) for n in "qkv"}
+        shp = lambda *s: g.constant(np.array(s, np.int64))  # noqa: E731
+
+        def attention(q, k, v):
+            split = lambda t, perm: g.node("Transpose", [g.node("Reshape", [g.node("Reshape", [t, shp(1, seq, hidden)]), shp(1, seq, heads, dh)])], perm=perm)  # noqa: E731
+            q, k, v = split(q, [0, 2, 1, 3]), split(k, [0, 2, 3, 1]), split(v, [0, 2, 1, 3])
+            p = g.node("Softmax", [g.node("Div", [g.node("MatMul", [q, k]), g.constant(np.array(np.sqrt(dh), dtype))])], axis=-1)
+            c = g.node("Transpose", [g.node("MatMul", [p, v])], perm=[0, 2, 1, 3])
+            return g.node("Reshape", [g.node("Reshape", [c, shp(1, seq, hidden)]), shp(seq, hidden)])
+
+        q, k, v = (g.input(n, a.shape, dtype) for n, a in ins.items())
+        y = g.node("Relu", [g.node("MatMul", [attention(q, k, v), g.constant((r.standard_normal((hidden, hidden)) / 8).astype(np.float16).astype(dtype))])])
+        g.output(y)
+        g.output(g.node("Relu", [attention(y, y, y)]))
+        return g, list(ins.values())
+
+    ref, _ = run(lambda: build(np.float32), ORACLE_PATH)
+    tol = dict(rtol=1e-4, atol=1e-5) if dtype == np.float32 else dict(rtol=5e-3, atol=5e-3)
+    for alias in (False, True):
+        g, inputs = build()
+        p = g.compile(fuse_attention=True, alias_copies=alias)
+        assert p.text.count("dnn.attention") == 2 and "dnn.reshape" in p.text
+        s = p.session(compiler.MODE_RESIDENT)
+        dt = torch.from_numpy(inputs[0]).dtype
+        for off in (0, 1):
+            if alias and off:
+                continue  # the program itself has the attention read its arguments: 16-byte aligned ones
+            ins = [torch.zeros(a.size + 8, dtype=dt, device="cuda") for a in inputs]
+            for b, a in zip(ins, inputs):
+                b[off:off + a.size] = torch.from_numpy(a.reshape(-1)).cuda()
+            outs = [torch.zeros(seq * hidden + 8, dtype=dt, device="cuda") for _ in ref]
+            es = ins[0].element_size()
+            for use_graph in (False, True, True):
+                for t in outs:
+                    t.zero_()
+                torch.cuda.synchronize()
+                s.run_device([t.data_ptr() + es * off for t in ins], [t.data_ptr() + es * off for t in outs], use_graph=use_graph, in_place=True)
+                s.sync()
+                for t, want in zip(outs, ref):
+                    np.testing.assert_allclose(t[off:off + seq * hidden].cpu().numpy().reshape(seq, hidden).astype(np.float32), want, **tol)
+        s.close()
+
+
 def test_resident_run_in_place_with_two_results():
     """Two results, the first of them produced before the last operation and read again by it: with
     run_device(in_place=True) both land in the caller's buffers with the bits of the copying mode, eager and
