@@ -91,6 +91,12 @@ __global__ __launch_bounds__(256) void attention_kernel(const float *__restrict_
         *reinterpret_cast<float4 *>(Ks + r * ROW + c4 * 4) = kv[u];
         *reinterpret_cast<float4 *>(Vs + r * ROW + c4 * 4) = vv[u];
       }
+      if (kb + ATT_KB > Sk)  // past the end the probability is zero, which times a repeated infinity would be NaN
+#pragma unroll
+        for (int u = 0; u < KV_CHUNK; u++) {
+          const int i = tid + 256 * (u0 + u), r = i / (DH / 4), c4 = i - r * (DH / 4);
+          if (kb + r >= Sk) *reinterpret_cast<float4 *>(Vs + r * ROW + c4 * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
     }
     __syncthreads();
 

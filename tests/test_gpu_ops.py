@@ -697,13 +697,14 @@ def test_attention_f16_blocks_and_wavefronts(gpu, cpu, case):
         np.testing.assert_allclose(gpu.get(Y).astype(np.float32), ref, rtol=2e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
 @pytest.mark.parametrize("case", [(1, 33, 384, 2, 64), (1, 20, 129, 2, 32), (2, 32, 97, 1, 128), (1, 7, 32, 3, 64), (1, 600, 300, 16, 64)], ids=str)
-def test_attention_f16_infinities(gpu, cpu, case):
+def test_attention_infinities(gpu, cpu, case, dtype):
     """A probability times an infinity is that infinity: an Inf in V, at any key, the last one and a lone one among them,
     gives Inf in its column for every query, opposite ones and NaN give NaN, and the other columns and heads stay."""
     B, Sq, Sk, H, D = case
     r = rng(sum(case))
-    q, k, v = (r.standard_normal((B, S, H * D)).astype(np.float16) for S in (Sq, Sk, Sk))
+    q, k, v = (r.standard_normal((B, S, H * D)).astype(dtype) for S in (Sq, Sk, Sk))
     scale = 1.0 / np.sqrt(D)
     plain = oc.attention(gpu, q, k, v, H, scale).astype(np.float32)
     for key in sorted({0, Sk // 2, Sk - 1}):
@@ -718,7 +719,7 @@ def test_attention_f16_infinities(gpu, cpu, case):
         got = oc.attention(gpu, q, k, vi, H, scale).astype(np.float32)
         np.testing.assert_array_equal(np.where(np.isfinite(got), 0, got), np.where(np.isfinite(want), 0, want))
         fine = np.isfinite(want)
-        np.testing.assert_allclose(got[fine], want[fine], rtol=1e-3, atol=1e-6)  # one rounding to fp16 apart
+        np.testing.assert_allclose(got[fine], want[fine], rtol=1e-3 if dtype == np.float16 else RTOL, atol=1e-6)  # fp16: one rounding apart
 
 
 # M, K, N: rows, columns and a reduction off the tiles, the reduction's last step partial, fewer steps than ring stages and
