@@ -152,9 +152,10 @@ int32_t dnncSessionSetConvTile(dnncSession *s, int32_t tile);
 int64_t dnncSessionTune(dnncSession *s, const void *const *inputs, int32_t on_device, int32_t reps);
 int64_t dnncSessionGetAlgos(const dnncSession *s, int64_t *algos, int64_t cap);
 int32_t dnncSessionSetAlgos(dnncSession *s, const int64_t *algos, int64_t n);
-/* Debugging, per-inference (occamy) mode: fill the pool when it is allocated, and every tensor's slot when it
- * is carved out of the pool, with `byte` (0..255; -1 switches it off).  With 0xFF a byte that a kernel leaves
- * unwritten, or that is read before its producer ran, shows up as NaN in the results. */
+/* Debugging, per-inference (occamy) mode: fill the pool when it is allocated, and every tensor's bytes in it once
+ * its last reader is issued (where constants are uploaded in program order, as on the host build: when its slot is
+ * carved out), with `byte` (0..255; -1 switches it off).  With 0xFF a byte that a kernel leaves unwritten, or
+ * that is read before its producer ran, shows up as NaN in the results. */
 int32_t dnncSessionSetDebugFill(dnncSession *s, int32_t byte);
 /* resident mode: one eager pass with device timestamps around every compute
  * operation; ms[i] belongs to dnncProgramComputeOp(i).  Returns the count.

@@ -325,7 +325,7 @@ class Session:
         return list(ms[:n])
 
     def set_debug_fill(self, byte):
-        """Per-inference mode: fill the pool and every tensor's slot with `byte` before use (-1: off)."""
+        """Per-inference mode: fill the pool, and every tensor's bytes between uses, with `byte` (-1: off)."""
         if lib().dnncSessionSetDebugFill(self._s, byte):
             raise RuntimeError("set_debug_fill: " + _err())
 

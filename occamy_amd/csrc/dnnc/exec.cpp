@@ -692,18 +692,15 @@ bool Session::plan_uploads(const std::vector<UploadChunk> &chunks, std::string &
       void *at = (char *)upload_host + host + in;
       const void *from = ptr[(size_t)copy->operands[1]->id];
       const auto f = block_filters.find(copy->operands[0]);
-      if (f != block_filters.end()) {  // run_occamy's other path still needs the rows
-        rt.dnnrtExecBlockFilter(at, from, f->second.first, f->second.second);
-      } else {
-        std::memcpy(at, from, (size_t)item.bytes);
-        moved[(size_t)copy->operands[1]->id] = at;
-      }
+      if (f != block_filters.end()) rt.dnnrtExecBlockFilter(at, from, f->second.first, f->second.second);
+      else std::memcpy(at, from, (size_t)item.bytes);
+      moved[(size_t)copy->operands[1]->id] = at;
       upload_slots.push_back({(size_t)copy->operands[0]->id, k.off + in});
       in += align_up(item.bytes, 256);
     }
     for (size_t i = 0; i < k.parts.size(); i++) {
       const UploadPart &q = k.parts[i];
-      uploads.push_back({host + q.lo - k.off, q.lo, q.hi - q.lo, k.first, q.after, nullptr});
+      uploads.push_back({host + q.lo - k.off, q.lo, q.hi - q.lo, k.first, k.last, q.after, nullptr});
       if (i + 1 == k.parts.size() && rt.dnnrtExecFenceCreate(&uploads.back().landed)) { err = rt_error("dnnrtExecFenceCreate"); return false; }
       if (q.after > waited) {
         waited = q.after;
@@ -944,11 +941,38 @@ bool Session::issue(const Op *op, std::string &err) {
   return true;
 }
 
+// debug_fill with the constants uploaded ahead: what held something until compute operation `n`, just issued, and is not
+// read any more is filled, so that whoever reads it before it is written again gets the fill.  `held`: every tensor's and
+// every constant's bytes.  In front of op_done, so that an upload into these bytes comes behind it.
+bool Session::fill_dead(const std::vector<Range> &held, int n, void *base) const {
+  for (const Range &dead : held) {
+    if (dead.last != n) continue;
+    int64_t lo = dead.lo;
+    while (lo < dead.hi) {  // the pieces between what lives on
+      int64_t hi = dead.hi, next = dead.hi;
+      for (const Range &r : held) {
+        if (r.first > n || r.last <= n || r.hi <= lo || r.lo >= hi) continue;
+        if (r.lo <= lo) { hi = lo; next = r.hi; }
+        else { hi = r.lo; next = r.lo; }
+      }
+      if (hi > lo && rt.dnnrtMemFill((char *)base + lo, debug_fill, hi - lo, stream)) return false;
+      lo = next;
+    }
+  }
+  return true;
+}
+
 // The per-inference sequence with the constants uploaded on a stream of their own (plan_uploads).
 bool Session::run_uploading(const void *const *inputs, void *const *outputs, std::string &err) {
   void *run_pool = nullptr;
   size_t next = 0, landed = 0;  // the next upload to issue; those that the compute stream has waited for
   int n = 0, waited = 0;
+  std::vector<Range> held;
+  if (debug_fill >= 0) {
+    held = moved_results;
+    for (const auto &l : live_slots()) held.push_back(l.second);
+    for (const Upload &u : uploads) held.push_back({u.dev_off, u.dev_off + u.bytes, u.after, u.last});
+  }
   auto fail = [&](const char *what) { err = rt_error(what); return false; };
   // The uploads whose place is free when n operations are done.  In program order: one that has to wait holds back the rest.
   auto pump = [&]() -> bool {
@@ -970,6 +994,7 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
         ptr[(size_t)op->result->id] = run_pool;
         block_base = run_pool;
         last_pool_bytes = op->bytes;
+        if (debug_fill >= 0 && (rt.dnnrtMemFill(run_pool, debug_fill, op->bytes, stream) || rt.dnnrtSync(handle))) return fail("dnnrtMemFill");
         for (const Op *o : prog->ops)
           if (o->kind == OP_MEM_OFFSET && rt.dnnrtMemOffset(&ptr[(size_t)o->result->id], run_pool, o->offset, o->bytes)) return fail("dnnrtMemOffset");
         for (const auto &s : upload_slots) ptr[s.first] = (char *)run_pool + s.second;
@@ -1005,6 +1030,7 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
       if (rt.dnnrtExecStreamWait(stream, uploads[need - 1].landed)) return fail("dnnrtExecStreamWait");
     }
     if (!issue(op, err)) return false;
+    if (debug_fill >= 0 && !fill_dead(held, n, run_pool)) return fail("dnnrtMemFill");
     n++;
     const auto done = op_done.find(n);
     if (done != op_done.end() && rt.dnnrtEventRecord(done->second, stream)) return fail("dnnrtEventRecord");
@@ -1028,9 +1054,9 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
   return true;
 }
 
-// The reference's per-inference sequence, call for call.
+// The reference's per-inference sequence, call for call: where the constants are not uploaded ahead.
 bool Session::run_occamy(const void *const *inputs, void *const *outputs, std::string &err) {
-  use_blocks = !uploads.empty() && debug_fill < 0;  // the fill would go over results that are not where the planner put them
+  use_blocks = !uploads.empty();
   if (use_blocks) return run_uploading(inputs, outputs, err);
   void *run_pool = nullptr;
   for (size_t i = 0; i < prog->args.size(); i++) {

@@ -123,9 +123,9 @@ class Session {
   const Program *prog = nullptr;
   int mode = MODE_OCCAMY;
   int64_t weights_bytes = 0;     // bytes of the constants arena (resident mode)
-  // Debugging (the reference's per-inference mode): fill the pool when it is allocated and every tensor's slot when
-  // it is carved out with this byte (-1: off); 0xFF makes any byte a kernel leaves unwritten, or reads before its
-  // producer ran, a NaN in the results.
+  // Debugging (the reference's per-inference mode): fill the pool when it is allocated, and a tensor's bytes whenever
+  // nothing is to read them any more (fill_dead; in the reference's order, its slot when it is carved out), with this
+  // byte (-1: off); 0xFF makes any byte a kernel leaves unwritten, or reads before its producer ran, a NaN in the results.
   int debug_fill = -1;
   int64_t last_pool_bytes = -1;  // bytes the last occamy-mode run asked the runtime for
   // the bound runtime library's device-memory accounting (dnnrtDeviceMemoryStats)
@@ -166,7 +166,7 @@ class Session {
   std::vector<Block> blocks;
   std::map<const Op *, int> block_of;  // their operations; the block's number
   std::vector<Range> moved_results;    // the places y_off names
-  bool use_blocks = false;             // ... and `elided`: not while a debug fill marks the planned slots
+  bool use_blocks = false;             // ... and `elided`: not in the reference's order of calls
   // Flatten, Reshape, Squeeze and Unsqueeze whose readers read the input where it is (plan_elided_copies)
   std::set<const Op *> elided;
   void plan_elided_copies();
@@ -183,7 +183,7 @@ class Session {
   // operations that read them (plan_uploads).  Compute operations are counted in program order.
   struct Upload {
     int64_t host_off, dev_off, bytes;  // in upload_host, in the pool
-    int first;                         // the first operation that reads it
+    int first, last;                   // the first and the last operation that read it
     int after;                         // these bytes of the pool are free once this many operations are done
     void *landed;                      // recorded behind the copy; null where the next entry completes the same constants
   };
@@ -198,6 +198,7 @@ class Session {
   struct UploadChunk { std::vector<UploadItem> items; int64_t bytes, off; int first, last; std::vector<UploadPart> parts; };
   bool place_constants(std::vector<UploadChunk> &chunks) const;
   bool plan_uploads(const std::vector<UploadChunk> &chunks, std::string &err);
+  bool fill_dead(const std::vector<Range> &held, int n, void *base) const;
   bool run_uploading(const void *const *inputs, void *const *outputs, std::string &err);
   std::map<std::string, void *> host_const;
   std::vector<void *> host_out, host_in;

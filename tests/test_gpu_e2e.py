@@ -126,9 +126,12 @@ def test_resident_mode_and_graph_replay(name, oracle_outputs):
 
 
 def test_poisoned_pool_changes_nothing_on_the_gpu():
-    """Every kernel writes all of its output and no operator reads a slot before its producer ran: with the pool and
-    every freshly carved slot filled with 0xFF bytes (NaN) the results are those of the plain run, bit for bit.
-    fp32 networks with and without the fused calls, BERT with its fused paths, fp16 channels-last."""
+    """Every kernel writes all of its output and no operator reads bytes before their producer ran: with the pool, and
+    every tensor's and constant's bytes once their last reader is issued, filled with 0xFF bytes (NaN) the results are
+    those of the plain run, bit for bit (the same path: constants uploaded ahead into bytes other tensors used, blocks
+    with results of their own place).  fp32 networks with and without the fused calls, BERT with its fused paths, fp16
+    channels-last, MobileNetV2 with inverted residual blocks in one launch."""
+    mobile = dict(fusion=True, fuse_residual=True, fuse_activations=True, fuse_matmul_bias=True, channels_last=True, alias_copies=True)
     cases = [(lambda: models.resnet50(image=64, classes=100), dict()),
              (lambda: models.resnet50(image=64, classes=100), dict(fusion=True, fuse_residual=True, fuse_matmul_bias=True)),
              (lambda: models.mobilenet_v2(image=64, classes=100), dict(fusion=True, fuse_residual=True, fuse_activations=True)),
@@ -138,7 +141,9 @@ def test_poisoned_pool_changes_nothing_on_the_gpu():
               dict(fusion=True, fuse_residual=True, fuse_matmul_bias=True, channels_last=True, fuse_first_layer_maxpool=True)),
              (lambda: models.resnet50(image=64, classes=100),
               dict(fusion=True, fuse_residual=True, fuse_matmul_bias=True, fuse_first_layer_maxpool=True, fuse_projection_shortcut=True)),
-             (lambda: models.srgan_generator(1, np.float32, height=24, width=16), dict(fusion=True, fuse_activations=True))]
+             (lambda: models.srgan_generator(1, np.float32, height=24, width=16), dict(fusion=True, fuse_activations=True)),
+             (lambda: models.mobilenet_v2(16, np.float16, seed=4, classes=100), dict(mobile)),
+             (lambda: models.mobilenet_v2(16, np.float16, seed=4, classes=100), dict(mobile, inplace_residual=True, compact_pool=True))]
     for builder, flags in cases:
         g, inputs = builder()
         s = g.compile(**flags).session(compiler.MODE_OCCAMY)
