@@ -137,7 +137,7 @@ def measure(name, steps, warmup, profile_only=False, tune=True, reference_leg=Tr
     torch.cuda.synchronize()
     dt = timed_steps(sess, ip, op, steps, warmup)
     res = dict(name=name, batch=batch, unit=unit, dtype=dtype, pool_bytes=prog.pool_bytes, weights_bytes=sess.weights_bytes,
-               kernels_per_step=prog.num_ops(compute_only=True), flags=flags)
+               kernels_per_step=sum(i == op[4] for i, op in enumerate(sess.compute_ops())), flags=flags)
     now, _, static = sess.device_bytes()
     res["device_bytes"] = dict(allocated=now, static=static, total=now + static,
                                what="everything the runtime library holds on the device during the timed steps: the pool and the "
@@ -187,7 +187,7 @@ def measure(name, steps, warmup, profile_only=False, tune=True, reference_leg=Tr
     # device timestamps on the session's own stream, eager launches: one pair per operation
     # class around that class's launches issued back to back (a timestamp between two kernels
     # of a few microseconds costs about as much as the kernels themselves)
-    ops = prog.compute_ops()
+    ops = sess.compute_ops()
     acc = np.zeros(len(ops))
     reps = 20
     sess.profile(ip, on_device=True, by_class=True)
@@ -195,7 +195,9 @@ def measure(name, steps, warmup, profile_only=False, tune=True, reference_leg=Tr
         acc += np.array(sess.profile(ip, on_device=True, by_class=True))
     acc /= reps
     by_class = {}
-    for (mn, cls, fl, by), ms in zip(ops, acc):
+    for i, ((mn, cls, fl, by, launch), ms) in enumerate(zip(ops, acc)):
+        if launch != i:  # runs in another operation's launch, or is a copy that is not launched
+            continue
         c = by_class.setdefault(cls, dict(launches=0, flops=0.0, bytes=0.0, ms=0.0))
         c["launches"] += 1
         c["flops"] += fl
@@ -349,7 +351,10 @@ def layer_table(res):
            f"the measured column sums to {sum(res['per_op_ms']) * 1e3:.0f} us); frac = bound / measured.", "",
            f"{'#':>3s} {'operation':28s} {'result':22s} {'red.':>5s} {'attrs':28s} {'MFLOP':>9s} {'KB':>9s} {'t_mfma':>7s} {'t_hbm':>7s} "
            f"{'by':>4s} {'meas_us':>8s} {'frac':>5s} {'TF/s':>7s} {'GB/s':>7s}"]
-    for i, ((mn, cls, fl, by), ms) in enumerate(zip(res["ops"], res["per_op_ms"])):
+    for i, ((mn, cls, fl, by, launch), ms) in enumerate(zip(res["ops"], res["per_op_ms"])):
+        if launch != i:
+            out.append(f"{i:3d} {mn[4:]:28s} " + ("not launched" if launch < 0 else f"in the launch of {launch}"))
+            continue
         line = lines[i] if len(lines) == len(res["ops"]) else ""
         shape = re.search(r": \w+(\[[^\]]*\])\s*$", line)
         attrs = re.search(r"\{([^}]*)\}", line)
@@ -363,7 +368,7 @@ def layer_table(res):
         out.append(f"{i:3d} {mn[4:]:28s} {shape.group(1) if shape else '':22s} {red:>5s} {a[:28]:28s} {fl / 1e6:9.1f} {by / 1e3:9.1f} "
                    f"{t_m:7.2f} {t_h:7.2f} {'mfma' if t_m >= t_h else 'hbm':>4s} {us:8.2f} {bound / max(us, 1e-9):5.2f} "
                    f"{fl / max(us, 1e-9) / 1e6:7.1f} {by / max(us, 1e-9) / 1e3:7.1f}")
-    tot_b = sum(max(fl / peak, by / PEAK["hbm"]) for _, _, fl, by in res["ops"]) * 1e6
+    tot_b = sum(max(fl / peak, by / PEAK["hbm"]) for _, _, fl, by, _ in res["ops"]) * 1e6
     out.append("")
     out.append(f"sum of bounds {tot_b:.0f} us; sum of measured {sum(res['per_op_ms']) * 1e3:.0f} us")
     return "\n".join(out) + "\n"

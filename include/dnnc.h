@@ -148,7 +148,9 @@ int32_t dnncSessionSetConvTile(dnncSession *s, int32_t tile);
  * common tolerance; recorded graphs are dropped.
  * dnncSessionGetAlgos / SetAlgos: the choices as two variant ids per operation that launches
  * (dnncProgramComputeOp order; the second is for the second convolution of a fused shortcut pair; 0 = the
- * runtime's own choice), so that a tuning can be kept beside the model and applied to a later session. */
+ * runtime's own choice), so that a tuning can be kept beside the model and applied to a later session.
+ * Convolutions that run in a block's launch have no variants: what is set for them is not kept (GetAlgos gives 0),
+ * nor does dnncSessionSetConvTile reach them. */
 int64_t dnncSessionTune(dnncSession *s, const void *const *inputs, int32_t on_device, int32_t reps);
 int64_t dnncSessionGetAlgos(const dnncSession *s, int64_t *algos, int64_t cap);
 int32_t dnncSessionSetAlgos(dnncSession *s, const int64_t *algos, int64_t n);
@@ -157,8 +159,15 @@ int32_t dnncSessionSetAlgos(dnncSession *s, const int64_t *algos, int64_t n);
  * carved out), with `byte` (0..255; -1 switches it off).  With 0xFF a byte that a kernel leaves unwritten, or
  * that is read before its producer ran, shows up as NaN in the results. */
 int32_t dnncSessionSetDebugFill(dnncSession *s, int32_t byte);
-/* resident mode: one eager pass with device timestamps around every compute
- * operation; ms[i] belongs to dnncProgramComputeOp(i).  Returns the count.
+/* What the session launches for the program's i-th compute operation (dnncProgramComputeOp order): `launch` is the
+ * operation in whose launch it runs: i itself; the last one of an inverted residual block that runs as one call;
+ * -1 for a copy that moves no element and is not launched.  Where launch == i, work_class, flops and bytes are
+ * those of that launch: a block's three convolutions together ("inverted_block"), without the tensors between
+ * them; flops and bytes are 0 elsewhere. */
+int32_t dnncSessionComputeOp(const dnncSession *s, int64_t i, int64_t *launch, const char **work_class, double *flops, double *bytes);
+/* resident mode: one eager pass with device timestamps around every launch;
+ * ms[i] belongs to dnncProgramComputeOp(i) and is 0 where the session launches
+ * nothing for it (dnncSessionComputeOp).  Returns the count.
  * on_device bit 0: the inputs are device buffers; bit 1: one pair of
  * timestamps per operation class around that class's launches issued back to
  * back, ms[i] = the class average (a timestamp between kernels of a few

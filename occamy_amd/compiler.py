@@ -73,6 +73,7 @@ def lib():
         "dnncSessionProfile": (C.c_int64, [P, C.POINTER(P), C.c_int32, C.POINTER(C.c_float), C.c_int64]),
         "dnncPlanPool": (C.c_int64, [C.c_int64, I32P, I64P, I64P, I64P]),
         "dnncPlanFreeList": (C.c_int64, [C.c_int64, I32P, I64P, I64P, C.c_int64, I64P, C.c_int64]),
+        "dnncSessionComputeOp": (C.c_int32, [P, C.c_int64, I64P, C.POINTER(C.c_char_p), C.POINTER(C.c_double), C.POINTER(C.c_double)]),
         "dnncSessionCreate": (P, [P, C.c_char_p, C.c_int32]),
         "dnncSessionDestroy": (None, [P]),
         "dnncSessionRun": (C.c_int32, [P, C.POINTER(P), C.POINTER(P)]),
@@ -312,7 +313,8 @@ class Session:
             raise RuntimeError("run_device: " + _err())
 
     def profile(self, in_ptrs_or_arrays, on_device=False, by_class=False):
-        """Resident mode: milliseconds per compute op (device timestamps), program order."""
+        """Resident mode: milliseconds per compute op (device timestamps), program order; 0 where the session launches
+        nothing for it (compute_ops)."""
         if on_device:
             ip = (C.c_void_p * max(len(in_ptrs_or_arrays), 1))(*in_ptrs_or_arrays)
         else:
@@ -323,6 +325,18 @@ class Session:
         if lib().dnncSessionProfile(self._s, ip, int(on_device) | (2 if by_class else 0), ms, n) < 0:
             raise RuntimeError("profile: " + _err())
         return list(ms[:n])
+
+    def compute_ops(self):
+        """[(mnemonic, work class, FLOPs, bytes, launch)] per compute op of the program, for what this session launches:
+        `launch` is the index of the op in whose launch it runs (its own; the last one's of an inverted residual block,
+        which carries the block's work; -1: a copy that is not launched)."""
+        out = []
+        for i, (name, _, _, _) in enumerate(self.program.compute_ops()):
+            launch, cls, fl, by = C.c_int64(), C.c_char_p(), C.c_double(), C.c_double()
+            if lib().dnncSessionComputeOp(self._s, i, C.byref(launch), C.byref(cls), C.byref(fl), C.byref(by)):
+                raise RuntimeError(_err())
+            out.append((name, cls.value.decode(), fl.value, by.value, launch.value))
+        return out
 
     def set_debug_fill(self, byte):
         """Per-inference mode: fill the pool, and every tensor's bytes between uses, with `byte` (-1: off)."""
@@ -348,8 +362,8 @@ class Session:
         return n
 
     def algos(self):
-        """[(variant of the convolution, variant of a fused pair's second convolution)] per operation that launches;
-        0 = the runtime's own choice."""
+        """[(variant of the convolution, variant of a fused pair's second convolution)] per compute op; 0 = the runtime's
+        own choice, always where the op's launch has no variants (an inverted residual block's)."""
         n = lib().dnncSessionGetAlgos(self._s, None, 0)
         buf = (C.c_int64 * max(n, 1))()
         lib().dnncSessionGetAlgos(self._s, buf, n)

@@ -364,6 +364,11 @@ int64_t dnncSessionProfile(dnncSession *s, const void *const *inputs, int32_t on
   return (int64_t)t.size();
 }
 
+int32_t dnncSessionComputeOp(const dnncSession *s, int64_t i, int64_t *launch, const char **work_class, double *flops, double *bytes) {
+  if (!s || !launch || !work_class || !flops || !bytes) return fail("dnncSessionComputeOp: bad arguments");
+  return s->s.compute_op(i, *launch, *work_class, *flops, *bytes) ? 0 : fail("dnncSessionComputeOp: index out of range");
+}
+
 int64_t dnncSessionWeightsBytes(const dnncSession *s) { return s ? s->s.weights_bytes : -1; }
 int64_t dnncSessionLastPoolBytes(const dnncSession *s) { return s ? s->s.last_pool_bytes : -1; }
 int32_t dnncSessionDeviceBytes(const dnncSession *s, int64_t *allocated_now, int64_t *allocated_peak, int64_t *static_bytes, int32_t reset_peak) {

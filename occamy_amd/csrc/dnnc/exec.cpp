@@ -1126,6 +1126,39 @@ bool Session::issue_all_compute(std::string &err) {
   return true;
 }
 
+// Whether the session makes a runtime call for the operation: not for copies it elides, nor for a block's operations in
+// front of its last one.
+bool Session::issues(const Op *op) const {
+  const auto b = block_of.find(op);
+  return launches(op) && !elided.count(op) && (b == block_of.end() || op == blocks[(size_t)b->second].project);
+}
+
+const char *Session::launch_class(const Op *op) const { return block_of.count(op) ? "inverted_block" : op_class(op); }
+
+bool Session::compute_op(int64_t i, int64_t &launch, const char *&work_class, double &flops, double &bytes) const {
+  std::vector<const Op *> compute;
+  for (const Op *op : prog->ops)
+    if (launches(op)) compute.push_back(op);
+  if (i < 0 || i >= (int64_t)compute.size()) return false;
+  const Op *op = compute[(size_t)i];
+  const auto at = block_of.find(op);
+  const Block *b = at == block_of.end() ? nullptr : &blocks[(size_t)at->second];
+  launch = elided.count(op) ? -1 : b ? std::find(compute.begin(), compute.end(), b->project) - compute.begin() : i;
+  work_class = launch_class(op);
+  flops = bytes = 0;
+  if (!issues(op)) return true;
+  if (!b) { op_work(op, flops, bytes); return true; }
+  for (const Op *o : {b->expand, b->dw, b->project}) {
+    if (!o) continue;
+    double f, by;
+    op_work(o, f, by);
+    flops += f;
+    bytes += by;
+    if (o != b->project) bytes -= 2.0 * (double)shape_numel(o->result->shape) * (double)dtype_bytes(o->result->dtype);  // stays on the chip
+  }
+  return true;
+}
+
 // Resident inference.  `on_device` != 0: inputs/outputs are device pointers and
 // the call returns without waiting (sync() does).
 bool Session::run_resident(const void *const *inputs, void *const *outputs, int on_device, int use_graph, std::string &err) {
@@ -1207,7 +1240,7 @@ bool Session::run_resident(const void *const *inputs, void *const *outputs, int 
   // A graph launch costs the host about as much as half a dozen kernel launches: a program of up to three kernels
   // (the single convolution block: 19 us per pass replayed, 8 us launched directly) is issued as it is.
   int launching = 0;
-  for (const Op *op : prog->ops) launching += launches(op) ? 1 : 0;
+  for (const Op *op : prog->ops) launching += issues(op) ? 1 : 0;
   const bool graphed = use_graph && !host_backend && launching > 3;
   if (graphed && !graph) {
     // One eager pass on real data first: it validates every call outside of
@@ -1267,10 +1300,10 @@ bool Session::profile_resident(const void *const *inputs, int on_device, bool by
       break;
     }
   if (by_class) return profile_classes(inputs, on_device, compute, ms, err);
-  std::vector<void *> ev(compute.size() + 1, nullptr);
+  std::vector<void *> ev(compute.size() + 1, nullptr);  // [0]: the start; [i + 1]: behind operation i, if it launches in this session
   bool ok = true;
-  for (void *&e : ev)
-    if (rt.dnnrtEventCreate(&e)) { err = rt_error("dnnrtEventCreate"); ok = false; break; }
+  for (size_t i = 0; ok && i < ev.size(); i++)
+    if ((i == 0 || issues(compute[i - 1])) && rt.dnnrtEventCreate(&ev[i])) { err = rt_error("dnnrtEventCreate"); ok = false; }
   if (ok) {
     for (const Op *op : prog->ops) {  // inputs into their pool slots
       if (op->kind != OP_MEMCPY || op->mode != 1 || op->operands[1]->arg_index < 0) continue;
@@ -1285,13 +1318,17 @@ bool Session::profile_resident(const void *const *inputs, int on_device, bool by
   if (ok && rt.dnnrtEventRecord(ev[0], stream)) { err = rt_error("dnnrtEventRecord"); ok = false; }
   for (size_t i = 0; ok && i < compute.size(); i++) {
     ok = issue(compute[i], err);
-    if (ok && rt.dnnrtEventRecord(ev[i + 1], stream)) { err = rt_error("dnnrtEventRecord"); ok = false; }
+    if (ok && ev[i + 1] && rt.dnnrtEventRecord(ev[i + 1], stream)) { err = rt_error("dnnrtEventRecord"); ok = false; }
   }
   if (rt.dnnrtSync(handle) && ok) { err = rt_error("dnnrtSync"); ok = false; }
   ms.assign(compute.size(), 0.f);
-  for (size_t i = 0; ok && i < compute.size(); i++)
-    if (rt.dnnrtEventElapsedMs(ev[i], ev[i + 1], &ms[i])) { err = rt_error("dnnrtEventElapsedMs"); ok = false; }
-  for (void *e : ev) rt.dnnrtEventDestroy(e);
+  for (size_t i = 0, before = 0; ok && i < compute.size(); i++) {
+    if (!ev[i + 1]) continue;
+    if (rt.dnnrtEventElapsedMs(ev[before], ev[i + 1], &ms[i])) { err = rt_error("dnnrtEventElapsedMs"); ok = false; }
+    before = i + 1;
+  }
+  for (void *e : ev)
+    if (e) rt.dnnrtEventDestroy(e);
   return ok;
 }
 
@@ -1304,10 +1341,11 @@ bool Session::profile_resident(const void *const *inputs, int on_device, bool by
 // a little faster here than inside the whole program).
 bool Session::profile_classes(const void *const *inputs, int on_device, const std::vector<const Op *> &compute,
                               std::vector<float> &ms, std::string &err) {
+  auto class_of = [&](const Op *op) -> std::string { return issues(op) ? launch_class(op) : ""; };
   std::vector<std::string> classes;
   for (const Op *op : compute) {
-    const std::string c = op_class(op);
-    if (std::find(classes.begin(), classes.end(), c) == classes.end()) classes.push_back(c);
+    const std::string c = class_of(op);
+    if (!c.empty() && std::find(classes.begin(), classes.end(), c) == classes.end()) classes.push_back(c);
   }
   bool ok = true;
   for (const Op *op : prog->ops) {  // inputs into their pool slots
@@ -1328,18 +1366,18 @@ bool Session::profile_classes(const void *const *inputs, int on_device, const st
     // a class of one or two launches is repeated: behind an idle stream the first dispatch alone takes
     // longer to reach the GPU than such a kernel runs
     size_t members = 0, n = 0;
-    for (const Op *op : compute) members += c == op_class(op);
+    for (const Op *op : compute) members += c == class_of(op);
     const size_t reps = members >= 32 ? 1 : (32 + members - 1) / members;
     if (rt.dnnrtEventRecord(e0, stream)) { err = rt_error("dnnrtEventRecord"); ok = false; break; }
     for (size_t r = 0; ok && r < reps; r++)
       for (size_t i = 0; ok && i < compute.size(); i++)
-        if (c == op_class(compute[i])) { ok = issue(compute[i], err); n++; }
+        if (c == class_of(compute[i])) { ok = issue(compute[i], err); n++; }
     if (ok && rt.dnnrtEventRecord(e1, stream)) { err = rt_error("dnnrtEventRecord"); ok = false; }
     if (ok && rt.dnnrtSync(handle)) { err = rt_error("dnnrtSync"); ok = false; }
     float total = 0.f;
     if (ok && rt.dnnrtEventElapsedMs(e0, e1, &total)) { err = rt_error("dnnrtEventElapsedMs"); ok = false; }
     for (size_t i = 0; ok && i < compute.size(); i++)
-      if (c == op_class(compute[i])) ms[i] = total / (float)n;
+      if (c == class_of(compute[i])) ms[i] = total / (float)n;
   }
   rt.dnnrtEventDestroy(e0);
   rt.dnnrtEventDestroy(e1);
@@ -1352,9 +1390,10 @@ int64_t Session::algo_operand(const Op *op, int which, int64_t reference_value) 
   return id > 0 ? DNNRT_CONV_ALGO_BASE + id : reference_value;
 }
 
-static bool tunable(const Op *op) {
+// Convolutions with a call of their own; a block's launch has no variants.
+bool Session::tunable(const Op *op) const {
   return (op->kind == OP_CONVFWD || op->kind == OP_CONV_BIAS_ACTIV || op->kind == OP_CONV_BIAS_ADD_ACTIV || op->kind == OP_CONV_ADD_CONV_ACTIV) &&
-         !op->operands.empty() && op->operands.back()->dtype == F16;
+         !op->operands.empty() && op->operands.back()->dtype == F16 && !block_of.count(op);
 }
 
 std::vector<int64_t> Session::algos() const {

@@ -99,12 +99,17 @@ class Session {
   // Tuning: dnnrtSetConvTile on the session's handle; a captured graph is dropped (it holds the old variants).
   bool set_conv_tile(int tile, std::string &err);
   // Resident mode: one eager pass with a device timestamp around every compute
-  // operation; ms[i] is the time of the i-th compute op in program order.
+  // operation; ms[i] is the time of the i-th compute op in program order, 0 where the session launches nothing for it.
   // by_class: timestamps only around each operation class's launches issued
   // back to back; ms[i] is then the class average.
   bool profile_resident(const void *const *inputs, int on_device, bool by_class, std::vector<float> &ms, std::string &err);
   bool profile_classes(const void *const *inputs, int on_device, const std::vector<const Op *> &compute,
                        std::vector<float> &ms, std::string &err);
+
+  // What the session makes of the program's i-th compute operation (dnncProgramComputeOp order): the operation in whose
+  // launch it runs (itself, the last one of its block, -1 for a copy that is not launched), and the class and work of
+  // that launch where it is itself, a block's counted whole ("inverted_block").
+  bool compute_op(int64_t i, int64_t &launch, const char *&work_class, double &flops, double &bytes) const;
 
   // The measured choice of convolution variant, where the reference times cuDNN's algorithms at compile time
   // and passes the winner as the call's `algo` operand (src/Conversion/ONNXToDNN/ONNXToDNNCommonCUDA.cu:57-111).
@@ -116,7 +121,8 @@ class Session {
   // has nothing to tune (changed = 0).
   bool tune(const void *const *inputs, int on_device, int reps, int64_t &changed, std::string &err);
   // The choices, two per operation that launches (dnncProgramComputeOp order): the `algo` operand and, for a
-  // fused shortcut pair, that of its second convolution; 0 = the runtime's own choice.
+  // fused shortcut pair, that of its second convolution; 0 = the runtime's own choice.  An operation whose launch has no
+  // variants (a block's convolutions among them) keeps 0 whatever is set.
   std::vector<int64_t> algos() const;
   bool set_algos(const int64_t *a, int64_t n, std::string &err);
 
@@ -175,6 +181,9 @@ class Session {
   // arguments, and the buffers that results are computed into.
   std::set<const Value *> callers;
   void *block_base = nullptr;          // the pool of the current run
+  bool issues(const Op *op) const;
+  const char *launch_class(const Op *op) const;
+  bool tunable(const Op *op) const;
   void fill_block(const Block &b, dnnrtExecBlock &k) const;
   std::map<const Value *, std::pair<int64_t, int64_t>> block_filters;  // device tensors uploaded in the block call's layout; rows, columns
   void plan_blocks();

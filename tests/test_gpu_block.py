@@ -146,3 +146,59 @@ def test_operands_at_any_address():
                 s.sync()
                 close16(out[off:off + n].cpu().numpy().reshape(ref[0].shape), ref[0])
         s.close()
+
+
+def test_profile_and_variants_know_blocks():
+    """MobileNetV2 with blocks: the session says which operations run in whose launch, times are those of launches, a
+    block's work is its three convolutions' without the tensors between them, and variants are kept only for
+    convolutions that have a call of their own."""
+    import torch
+    from occamy_amd import models
+    g, inputs = models.mobilenet_v2(32, np.float16, seed=4, classes=100)
+    p = g.compile(inplace_residual=True, **FLAGS)
+    s = p.session(compiler.MODE_RESIDENT)
+    plain = s.run(*inputs)[0]
+    ops, prog = s.compute_ops(), p.compute_ops()
+    assert [o[0] for o in ops] == [o[0] for o in prog]
+    blocks = [i for i, o in enumerate(ops) if o[1] == "inverted_block" and o[4] == i]
+    inner = [i for i, o in enumerate(ops) if o[4] != i]
+    assert len(blocks) >= 5 and all(ops[i][4] in blocks and ops[i][2:4] == (0.0, 0.0) for i in inner) and len(inner) >= len(blocks)
+    for b in blocks:
+        members = [i for i, o in enumerate(ops) if o[4] == b]
+        assert members == list(range(members[0], b + 1)) and len(members) in (2, 3)
+        assert ops[b][2] == sum(prog[i][2] for i in members) and 0 < ops[b][3] < 0.6 * sum(prog[i][3] for i in members)
+    for by_class in (False, True):
+        for _ in range(2):
+            ms = s.profile(inputs, by_class=by_class)
+        assert all((m > 0) == (o[4] == i) for i, (m, o) in enumerate(zip(ms, ops)))
+    rates = [ops[b][3] / ms[b] / 1e6 for b in blocks]  # GB/s
+    assert max(rates) < 8000, rates
+    np.testing.assert_array_equal(s.run(*inputs)[0], plain)
+    s.set_algos([(3, 0)] * len(ops))
+    kept = s.algos()
+    assert all(kept[i] == (0, 0) for i in [*inner, *blocks]) and (3, 0) in kept
+    close16(s.run(*inputs)[0], plain.astype(np.float32))
+    s.set_algos([(0, 0)] * len(ops))
+    np.testing.assert_array_equal(s.run(*inputs)[0], plain)
+    changed = s.tune(inputs, reps=3)
+    kept = s.algos()
+    assert changed == sum(a != (0, 0) for a in kept) and all(kept[i] == (0, 0) for i in [*inner, *blocks])
+    x = [torch.from_numpy(a).cuda() for a in inputs]
+    out = torch.empty(plain.shape, dtype=torch.float16, device="cuda")
+    for _ in range(2):
+        s.run_device([t.data_ptr() for t in x], [out.data_ptr()], in_place=True)
+        s.sync()
+        close16(out.cpu().numpy(), plain.astype(np.float32))
+    s.close()
+
+
+def test_profile_knows_copies_that_are_not_launched():
+    from occamy_amd import models
+    g, inputs = models.alexnet(2, np.float32, image=224)
+    s = g.compile(fusion=True, fuse_matmul_bias=True).session(compiler.MODE_RESIDENT)
+    s.run(*inputs)
+    ops, ms = s.compute_ops(), s.profile(inputs)
+    elided = [i for i, o in enumerate(ops) if o[4] < 0]
+    assert elided and all(ops[i][0] in ("dnn.flatten", "dnn.reshape", "dnn.squeeze", "dnn.unsqueeze") for i in elided)
+    assert all((m > 0) == (o[4] == i) for i, (m, o) in enumerate(zip(ms, ops)))
+    s.close()

@@ -142,8 +142,8 @@ def test_poisoned_pool_changes_nothing_on_the_gpu():
              (lambda: models.resnet50(image=64, classes=100),
               dict(fusion=True, fuse_residual=True, fuse_matmul_bias=True, fuse_first_layer_maxpool=True, fuse_projection_shortcut=True)),
              (lambda: models.srgan_generator(1, np.float32, height=24, width=16), dict(fusion=True, fuse_activations=True)),
-             (lambda: models.mobilenet_v2(16, np.float16, seed=4, classes=100), dict(mobile)),
-             (lambda: models.mobilenet_v2(16, np.float16, seed=4, classes=100), dict(mobile, inplace_residual=True, compact_pool=True))]
+             (lambda: models.mobilenet_v2(32, np.float16, seed=4, classes=100), dict(mobile)),
+             (lambda: models.mobilenet_v2(32, np.float16, seed=4, classes=100), dict(mobile, inplace_residual=True, compact_pool=True))]
     for builder, flags in cases:
         g, inputs = builder()
         s = g.compile(**flags).session(compiler.MODE_OCCAMY)
