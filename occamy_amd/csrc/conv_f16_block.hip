@@ -14,9 +14,9 @@
 //            Results replace the slab.
 //   project  after a barrier, the G slabs are the right operand of the projection: blocks of 32 output channels x 32 pixels
 //            dealt over the wavefronts, accumulators kept over the rounds.
-// Values are rounded where the three separate calls round them.  The two 1x1 filters are read in blocks of 32 rows and 8
-// columns (512 contiguous bytes), the order the executor uploads them in: rows of the plain matrix would cost a cache line
-// per lane and load, and took longer than everything else.
+// Values are rounded where the three separate calls round them, from fp32 sums that start at the bias.  The two 1x1 filters
+// are read in blocks of 32 rows and 8 columns (512 contiguous bytes), the order the executor uploads them in: rows of the
+// plain matrix would cost a cache line per lane and load, and took longer than everything else.
 //
 // What bounds it: vector instructions and LDS accesses about evenly where tiles are many, at three wavefronts per SIMD; where
 // they are few, a launch's own 8 us and the 3.5 to 5 us of a round.

@@ -247,7 +247,7 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
   }
   for (const Block &b : blocks)
     for (const Op *op : {b.expand, b.project})
-      if (op && op->operands.back()->dtype == F16) block_filters[op->operands[1]] = {op->dimB[0], op->dimB[1]};
+      if (op) block_filters[op->operands[1]] = {op->dimB[0], op->dimB[1]};
   if (mode == MODE_RESIDENT) {
     use_blocks = true;
     block_base = pool;
@@ -284,7 +284,6 @@ void Session::fill_block(const Block &b, dnnrtExecBlock &k) const {
   k.p = b.project->dimA[2]; k.q = b.project->dimA[3]; k.cout = b.project->dimB[0];
   k.dtype = (int32_t)b.project->operands.back()->dtype;
   k.format = format_for(first);
-  k.filter_layout = filter_crsk[(size_t)b.dw->operands[1]->id] ? DNNRT_FILTER_CRSK : DNNRT_FILTER_KCRS;
 }
 
 // The slots of everything but constants: from the first operation that uses one to the last.  A block's inner tensors
@@ -428,8 +427,7 @@ void Session::plan_blocks() {
     if (!in_pool(dw, !ex, false)) continue;
     bool read_later = true;  // by operations that launch something
     for (const auto &u : pr->result->uses) read_later = read_later && is_compute(u.first->kind) && launches(u.first) && !elided.count(u.first);
-    const char lay = filter_crsk[(size_t)dw->operands[1]->id];
-    if (!read_later || filter_crsk[(size_t)pr->operands[1]->id] != lay || (ex && filter_crsk[(size_t)ex->operands[1]->id] != lay)) continue;
+    if (!read_later) continue;
     Block b{ex, dw, pr, (int)i, -1};
     dnnrtExecBlock k;
     fill_block(b, k);

@@ -16,7 +16,9 @@ int32_t dnnrtExecStreamWait(dnnrtStream_t stream, void *event);
 int32_t dnnrtExecUpload(void *dst, const void *src, int64_t bytes, dnnrtStream_t stream);
 
 /* An inverted residual block: y = act(conv1x1(actd(dwconv(act1(conv1x1(x, w1) + b1), wd) + bd), w3) + b3 [+ z]), square
- * stride, group of the middle convolution = its channels.  Results as from the separate calls.
+ * stride, group of the middle convolution = its channels.  Rounded to fp16 where the separate calls round, behind each bias
+ * and behind the sum with z; in front of that the fp32 sums start at the bias, which the separate calls add last, and run
+ * in another order, so single results are another fp16 step than theirs.
  * fp16: w1 and w3 in blocks, dnnrtExecBlockFilter. */
 typedef struct dnnrtExecBlock {
   const void *x, *w1, *b1, *wd, *bd, *w3, *b3, *z; /* w1, b1: not read without expansion; z: residual laid out like y, or null */
@@ -24,7 +26,7 @@ typedef struct dnnrtExecBlock {
   int64_t n, cin, h, w, ch, r, s, stride, pad_h, pad_w, p, q, cout;
   int64_t act1, actd, act; /* activation modes of the three convolutions and their coefficients */
   float coef1, coefd, coef;
-  int32_t expand, dtype, format, filter_layout;
+  int32_t expand, dtype, format;
 } dnnrtExecBlock;
 /* 1 if dnnrtExecRunBlock takes the block (pointers aside) and is meant to be faster than the three calls. */
 int32_t dnnrtExecBlockApplies(dnnrtHandle_t handle, const dnnrtExecBlock *block);

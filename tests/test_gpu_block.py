@@ -18,7 +18,7 @@ FLAGS = dict(fusion=True, fuse_residual=True, fuse_activations=True, fuse_matmul
 class ExecBlock(C.Structure):
     _fields_ = ([(n, C.c_void_p) for n in ("x", "w1", "b1", "wd", "bd", "w3", "b3", "z", "y")]
                 + [(n, C.c_int64) for n in ("n", "cin", "h", "w", "ch", "r", "s", "stride", "pad_h", "pad_w", "p", "q", "cout", "act1", "actd", "act")]
-                + [(n, C.c_float) for n in ("coef1", "coefd", "coef")] + [(n, C.c_int32) for n in ("expand", "dtype", "format", "filter_layout")])
+                + [(n, C.c_float) for n in ("coef1", "coefd", "coef")] + [(n, C.c_int32) for n in ("expand", "dtype", "format")])
 
 
 def block(n, cin, h, w, ch, cout, stride, pad_h, pad_w, **kw):
