@@ -365,7 +365,7 @@ def layer_table(res):
         t_m, t_h = fl / peak * 1e6, by / PEAK["hbm"] * 1e6
         bound = max(t_m, t_h)
         us = ms * 1e3
-        out.append(f"{i:3d} {mn[4:]:28s} {shape.group(1) if shape else '':22s} {red:>5s} {a[:28]:28s} {fl / 1e6:9.1f} {by / 1e3:9.1f} "
+        out.append(f"{i:3d} {cls if cls == 'inverted_block' else mn[4:]:28s} {shape.group(1) if shape else '':22s} {red:>5s} {a[:28]:28s} {fl / 1e6:9.1f} {by / 1e3:9.1f} "
                    f"{t_m:7.2f} {t_h:7.2f} {'mfma' if t_m >= t_h else 'hbm':>4s} {us:8.2f} {bound / max(us, 1e-9):5.2f} "
                    f"{fl / max(us, 1e-9) / 1e6:7.1f} {by / max(us, 1e-9) / 1e3:7.1f}")
     tot_b = sum(max(fl / peak, by / PEAK["hbm"]) for _, _, fl, by, _ in res["ops"]) * 1e6
