@@ -23,7 +23,7 @@
 //
 // Measured against the three calls at batch 64 (us): 16 -> 96 -> 24 channels, 112x112 stride 2: 104 -> 54; 24 -> 144 -> 24 at
 // 56x56: 85 -> 48; 24 -> 144 -> 32 stride 2: 52 -> 30; 32 -> 192 -> 32 at 28x28: 34 -> 17; 64 -> 384 -> 64 at 14x14: 34 -> 15.5;
-// 96 -> 576 -> 96: 38 -> 22.5; 32 -> 16 behind a depthwise layer at 112x112, no expansion: 49 -> 36.5.  MobileNetV2 0.77 -> 0.53 ms.
+// 96 -> 576 -> 96: 38 -> 22.5; 32 -> 16 behind a depthwise layer at 112x112, no expansion: 49 -> 36.5.  MobileNetV2 0.77 -> 0.50 ms.
 // 160 -> 960 -> 160 at 7x7 was slower (64 workgroups, 34 against 30) and is left to the three calls.
 #include "conv_f16.h"
 #include "dnnrt_exec.h"
