@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void attention_kernel(const float *__restrict_
 // that is more (with V at fp16's limits, a step of the smallest fp16 result); two MFMAs for what fp32 ones take eight times as
 // long for.  Before its rounding the result is nearer to 64 bits than the fp32 kernel's on the same values: 384 keys, normal
 // Q, K and V, relative error in the 2-norm at scales 0.001, 1/8, 1 and 4: 1.9e-7, 3.2e-7, 9.4e-7, 1.8e-6 -> 1.2e-7, 1.6e-7,
-// 3.9e-7, 7.2e-7, and 0.3 to 1.0 of it over 16 to 2048 keys, head sizes 32 to 128, V positive or spread over 24 octaves (the
+// 3.9e-7, 7.2e-7, and 0.25 to 1.0 of it over 16 to 2048 keys, head sizes 32 to 128, V positive or spread over 24 octaves (the
 // scores' error decides, and their sums are shorter chains here).  A third part, all 24 bits, takes 1 % off that and adds 0.7
 // us to 7.9.  V's operand, four consecutive keys of one d per read, comes out of the wavefront's LDS tile by transposing
 // reads (ds_read_b64_tr_b16).
