@@ -593,6 +593,9 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
       }
     }
   }
+  // 3x3 layers with stride 1: by Winograd's method where that is estimated to be faster
+  if (!launch_conv_f32_winograd(ctx, args, best_shape < 0 || best + 1.5 > at_most_us ? at_most_us - 1.5 : best, launched)) return false;
+  if (launched) return true;
   if (best_shape < 0 || best + 1.5 > at_most_us) return true;
   pl.magic_tiles_m = magic_of(pl.tiles_m);
   pl.magic_rest = magic_of(pl.rest > 0 ? pl.rest : 1);

@@ -74,6 +74,8 @@ bool launch_conv3x3_f32_tiled(const dnnrtContext *ctx, const IgemmArgs &a, int l
 // Convolutions with C,R,S,K filters on tiles whose operands go straight into LDS (conv_f32_dma.hip), if they take no longer
 // than `at_most_us` by its estimate; `launched` says whether it applied.
 bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &a, double at_most_us, bool &launched);
+// 3x3 convolutions with stride 1 and C,R,S,K filters by Winograd's method (conv_f32_winograd.hip), likewise.
+bool launch_conv_f32_winograd(const dnnrtContext *ctx, const IgemmArgs &a, double at_most_us, bool &launched);
 // What the small-problem kernels take for a convolution, estimated in microseconds: single launches of 0.1 .. 2 GFLOP
 // (counting whole 32x32 tiles) measure 5 + 18 per GFLOP for 3x3 filters, 5 + 15.5 for 1x1, 60 and more per GFLOP on the
 // general kernel.  0 below a quarter of a GFLOP: there either way is launch and latency, and inside a network, with its

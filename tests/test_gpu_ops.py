@@ -1564,3 +1564,61 @@ def test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, re
     got = keep["y"].permute(0, 3, 1, 2).float().cpu()
     lib.dnnrtDestroy(handle)
     np.testing.assert_allclose(got.numpy(), want.numpy(), rtol=4e-3, atol=8e-3)
+
+
+@pytest.mark.parametrize("case", [
+    # N, C, H, W, K, pad, residual, activation: sizes at which the launcher picks the tiles of conv_f32_winograd.hip
+    (11, 64, 56, 56, 64, 1, False, _abi.ACT_RELU),          # 270 tiles: 14 left over, one stage of four channels per part
+    (6, 48, 75, 77, 100, 1, True, _abi.ACT_LEAKY_RELU),     # odd image, filters off the 64 grid
+    (3, 512, 19, 19, 486, 1, False, _abi.ACT_IDENTITY),     # filter rows off the 16-byte grid
+    (2, 128, 64, 63, 128, 0, True, _abi.ACT_RELU),          # two stages per part, no padding
+    (1, 256, 50, 51, 256, 2, False, _abi.ACT_CLIPPED_RELU),
+    (2, 512, 28, 28, 256, 1, True, _abi.ACT_RELU),
+])
+def test_conv_3x3_by_minimal_filtering(gpu, case):
+    """Against 64-bit sums: no further from them than a chain of 9 C fp32 additions, whose relative error in the 2-norm is about
+    2^-25 sqrt(9 C) / 2.4 for independent products, and the transforms' few roundings beside it."""
+    import torch
+    N, Cc, H, W, K, pad, residual, activ = case
+    r = rng(N * 100 + Cc)
+    x = np.maximum(r.standard_normal((N, Cc, H, W)), 0).astype(np.float32)
+    w = (r.standard_normal((K, Cc, 3, 3)) * np.sqrt(2.0 / (9 * Cc))).astype(np.float32)
+    b = r.uniform(-0.5, 0.5, K).astype(np.float32)
+    ref = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), torch.from_numpy(b).double(), padding=pad).numpy()
+    z = r.standard_normal(ref.shape).astype(np.float32) if residual else None
+    if residual:
+        ref = ref + z
+    coef = {_abi.ACT_LEAKY_RELU: 0.1, _abi.ACT_CLIPPED_RELU: 1.5}.get(activ)
+    if activ == _abi.ACT_LEAKY_RELU:
+        ref = np.where(ref < 0, 0.1 * ref, ref)
+    elif activ != _abi.ACT_IDENTITY:
+        ref = np.clip(ref, 0, 1.5 if activ == _abi.ACT_CLIPPED_RELU else None)
+    bound = 2.0 ** -25 * (np.sqrt(9 * Cc) / 2.4 + 4)
+    for _ in range(2):  # twice: the split reduction's counters must be back at zero
+        got = oc.conv(gpu, x, w, b, (pad, pad), (1, 1), 1, activ, crsk=True, z=z, coef=coef, inplace=residual)
+        assert np.linalg.norm(got - ref) <= bound * np.linalg.norm(ref)
+        np.testing.assert_allclose(got, ref, rtol=RTOL, atol=ATOL)
+
+
+def test_conv_3x3_by_minimal_filtering_keeps_infinities_in_their_place(gpu, cpu):
+    """The transforms take differences within a 4x4 patch: an infinity, a NaN and values whose differences leave fp32's range
+    must reach the results that use them and no others, as they do tap by tap."""
+    r = rng(9)
+    x = r.standard_normal((6, 48, 75, 77)).astype(np.float32)
+    w = (r.standard_normal((64, 48, 3, 3)) * 0.1).astype(np.float32)
+    b = r.uniform(-0.5, 0.5, 64).astype(np.float32)
+    x[0, 3, 10, 20] = np.inf
+    x[1, 5, 0, 0] = -np.inf
+    x[2, 7, 74, 76] = np.nan
+    x[3, 9, 30, 31], x[3, 9, 30, 33] = 3e38, -3e38
+    w[5, 11, 1, 1] = np.inf
+    ref = oc.conv(cpu, x, w, b, (1, 1), (1, 1), 1, _abi.ACT_IDENTITY)
+    got = oc.conv(gpu, x, w, b, (1, 1), (1, 1), 1, _abi.ACT_IDENTITY, crsk=True)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(ref))
+    np.testing.assert_array_equal(np.isneginf(got), np.isneginf(ref))
+    ok = np.isfinite(ref)
+    ok[3] = False  # its values of 3e38 are summed in another order, and so rounded differently
+    np.testing.assert_allclose(got[ok], ref[ok], rtol=RTOL, atol=ATOL)
+    far = np.isfinite(ref[3]) & (np.abs(ref[3]) > 1e30)
+    np.testing.assert_allclose(got[3][far], ref[3][far], rtol=RTOL)
