@@ -90,11 +90,35 @@ inline unsigned magic_of(int d) {  // ceil(2^32 / d), saturated (d == 1)
   return (unsigned)(m > 0xffffffffull ? 0xffffffffull : m);
 }
 
+// v / 2 (1 + erf(v / sqrt 2)) without a branch: erff's two ranges, both taken by some lane of nearly every wavefront, made an
+// epilogue of sixteen values 2.2 us long.  |v| >= 1: erfc(a) = t P(t) exp(-a^2), t = 1 / (1 + 0.44 a) (the form of Abramowitz
+// and Stegun 7.1.26), below: erf(v / sqrt 2) = v R(v^2); P and R are minimax fits (2.2e-9 and 2.6e-10 absolute).  Relative error
+// in the 2-norm against 64 bits over normal v of deviation 0.1, 0.5, 1, 4: 3.7e-8, 4.0e-8, 3.5e-8, 2.1e-8; by way of erff
+// 3.8e-8, 4.2e-8, 3.9e-8, 2.3e-8.
+__device__ __forceinline__ float gelu(float v) {
+  const float a = fabsf(v) * 0.70710678118654752f, t = __builtin_amdgcn_rcpf(fmaf(0.44f, a, 1.0f)), u = v * v;
+  float p = 0.09016146510839462f;
+  p = fmaf(p, t, -0.5130200386047363f);
+  p = fmaf(p, t, 0.9627975821495056f);
+  p = fmaf(p, t, -0.4957951605319977f);
+  p = fmaf(p, t, 0.5246581435203552f);
+  p = fmaf(p, t, 0.17550785839557648f);
+  p = fmaf(p, t, 0.2556901276111603f) * t;
+  float r = -1.506052831246052e-05f;
+  r = fmaf(r, u, 0.0002262870839331299f);
+  r = fmaf(r, u, -0.0023719691671431065f);
+  r = fmaf(r, u, 0.019946342334151268f);
+  r = fmaf(r, u, -0.13298065960407257f);
+  r = fmaf(r, u, 0.7978845834732056f);
+  const float e = __builtin_amdgcn_exp2f(a * (a * -1.4426950408889634f));
+  const float outer = v < 0.f ? p * e : fmaf(-p, e, 2.0f);
+  return (0.5f * v) * (a < 0.70710678f ? fmaf(v, r, 1.0f) : outer);
+}
 __device__ __forceinline__ float apply_act(float v, int act, float coef) {
   if (act == DNNRT_ACT_RELU) return v < 0.f ? 0.f : v;
   if (act == DNNRT_ACT_CLIPPED_RELU) { v = v < 0.f ? 0.f : v; return v > coef ? coef : v; }
   if (act == DNNRT_ACT_LEAKY_RELU) return v < 0.f ? coef * v : v;
-  if (act == ACT_GELU) return 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
+  if (act == ACT_GELU) return gelu(v);
   return v;
 }
 __host__ __device__ inline bool fusable_act(int64_t act) {

@@ -748,6 +748,18 @@ def test_matmul_f16_direct_to_lds_tiles(gpu, cpu, case):
         np.testing.assert_allclose(oc.matmul_nd(gpu, a3, b3).astype(np.float64), a3.astype(np.float64) @ b3.astype(np.float64), **tol)
 
 
+def test_gelu_epilogue_against_64_bits(gpu):
+    """A product with the identity is its left operand, so this is the epilogue's Gelu of chosen values: to 3 units of the last
+    place of its argument (the formula's last two roundings and the fits' 2e-9), infinities and NaN as 0.5 x (1 + erf) has them."""
+    from scipy.special import erfc
+    r = rng(21)
+    x = np.concatenate([r.standard_normal(4000) * s for s in (1e-6, 0.05, 0.7, 1.0, 3.0, 20.0)] + [np.linspace(-1.1, 1.1, 575)]).astype(np.float32)
+    x = np.concatenate([x, [0.0]]).astype(np.float32).reshape(-1, 64)
+    got = oc.matmul_nd_bias(gpu, x[None], np.eye(64, dtype=np.float32), np.zeros(64, np.float32), gelu=True)[0]
+    x64 = x.astype(np.float64)
+    assert (np.abs(got - 0.5 * x64 * erfc(-x64 / np.sqrt(2))) <= 3 * 2.0 ** -24 * np.abs(x64)).all()
+
+
 # ---- data movement -------------------------------------------------------------------------
 
 def test_data_movement(gpu, cpu):
