@@ -24,6 +24,10 @@ struct GemmF16Args {
 // whether it applied.  steps_per_split is set there.
 bool launch_gemm_f16_dma(const dnnrtContext *ctx, const GemmF16Args &g, int Z, bool &launched);
 
+// ... and on tiles whose four wavefronts share the reduction (gemm_f16_waves.hip); launch_gemm_f16_dma, its caller, has checked
+// the forms.
+bool launch_gemm_f16_waves(const dnnrtContext *ctx, const GemmF16Args &g, int Z, int splits);
+
 // Out[z][M,N] = alpha * op(A[z]) op(B[z]) + beta * C[z]; strides in elements,
 // 0 = operand shared by every z.
 // bias: one value per column n, added to every row (may be null); act: an activation mode of apply_act applied last;

@@ -10,12 +10,13 @@
 //
 // What bounds it: at a transformer's sizes (16 to a few hundred rows, 0.1 .. 2 GFLOP) a chain of latencies per step, its
 // barrier, LDS reads and requests; the matrix pipes are busy for a tenth of the time.  Hence 64x64 tiles, all of a step's
-// operands read one step ahead (0.56 -> 0.37 us per step against reads a 16-k sub-step ahead; rings of 6 and 9 stages
-// changed nothing), and reductions split over workgroups where tiles are few (partial tiles through the handle's scratch,
+// operands read one step ahead (0.56 -> 0.37 us per step against reads a 16-k sub-step ahead; 0.30 since the transposing reads
+// no longer wait for the whole ring, gd_read_tr), and reductions split over workgroups where tiles are few (partial tiles through the handle's scratch,
 // the last to arrive adds them in split order; nobody waits).  128x128 tiles on eight wavefronts take the products of
 // thousands of rows (4096 cubed: 650 TFLOP/s, 333 us on 64x64 tiles, 212 on these).
-// Against gemm_f16.hip's kernel, which keeps what is not aligned (K x N -> us before, now): 384 rows, 768 x 2304 19.4 -> 8.1,
-// 768 x 768 15.9 -> 7.0, 768 x 3072 + GELU 24.7 -> 11.0, 3072 x 768 26.7 -> 11.5; 16 rows, 3072 x 768 20.6 -> 9.3.
+// Against gemm_f16.hip's kernel, which keeps what is not aligned (K x N -> us before, now): 384 rows, 768 x 2304 19.4 -> 7.2,
+// 768 x 768 15.9 -> 7.3, 768 x 3072 + GELU 24.7 -> 9.7, 3072 x 768 26.7 -> 11.5; 2048 rows, 768 x 2304 20.4.  Products of at most a tile per
+// compute unit go to gemm_f16_waves.hip.
 #include "gemm_f16.h"
 
 #include <type_traits>
@@ -40,6 +41,22 @@ __device__ __forceinline__ void gd_barrier() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+}
+
+#if __HIP_DEVICE_COMPILE__
+// ds_read_b64_tr_b16 at LDS address `at` + OFFSET.  By hand: ahead of the builtin the compiler waits for every load into LDS
+// that is still on its way (vmcnt 0), and so for the whole ring.  It knows nothing of this read either: the value is there
+// behind the next wait for lgkmcnt, and gd_arrived() ties it to that place.
+template <int OFFSET>
+__device__ __forceinline__ gd_short4 gd_read_tr(unsigned at) {
+  gd_short4 v;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(at), "i"(OFFSET) : "memory");
+  return v;
+}
+#endif
+template <class T>
+__device__ __forceinline__ void gd_arrived(T &v) {
+  asm volatile("" : "+v"(v));
 }
 
 // FN x FM: columns n and rows m of a workgroup's tile, over WN x WM wavefronts; NS ring stages; B_KC: B stored [N,K].
@@ -141,6 +158,7 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
       tr_off[i][t] = (unsigned)(k * 2 * FN + (((n >> 3) ^ swz(k)) * 16) + (n & 7) * 2);
     }
   gd_half8 fn[2][4][TN], fm[2][4][TM];  // two steps' operands
+  [[maybe_unused]] gd_short4 tr[2][4][TN][2];  // [K,N]: the halves of fn
   auto read_step = [&](const char *stage, auto set_c) {
     constexpr int S = decltype(set_c)::value;
 #pragma unroll
@@ -150,11 +168,12 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
         if constexpr (B_KC) {
           fn[S][sub][i] = *reinterpret_cast<const gd_half8 *>(stage + ((ld_n0 ^ (32u * sub)) + i * 4096));
         } else {
-          // sixteen rows further on the swizzle is the same
-          typedef __attribute__((address_space(3))) gd_short4 *tr_ptr;
-          const gd_short4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(stage + tr_off[i][0] + sub * 32 * FN));
-          const gd_short4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(stage + tr_off[i][1] + sub * 32 * FN));
-          fn[S][sub][i] = __builtin_bit_cast(gd_half8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          const unsigned at = (unsigned)(size_t)(gd_lds)const_cast<char *>(stage);  // sixteen rows further on the swizzle is the same
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            const unsigned from = at + tr_off[i][t];
+            tr[S][sub][i][t] = sub == 0 ? gd_read_tr<0>(from) : sub == 1 ? gd_read_tr<32 * FN>(from) : sub == 2 ? gd_read_tr<64 * FN>(from) : gd_read_tr<96 * FN>(from);
+          }
         }
       }
 #pragma unroll
@@ -169,15 +188,29 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
   constexpr std::integral_constant<int, 0> set0{};
   constexpr std::integral_constant<int, 1> set1{};
   int c_stage = 0;
-  auto step_body = [&](auto set_c, auto g_c, auto loads_c) {
-    constexpr int S = decltype(set_c)::value, G = decltype(g_c)::value;  // G: steps in flight behind this one
-    constexpr bool LOADS = decltype(loads_c)::value;
-    if constexpr (G > 0) {
-      gd_wait<(G - 1) * L, 0>();
+  auto step_body = [&](auto set_c, auto full_c, int ahead) {  // `ahead` steps follow this one; FULL: NS or more
+    constexpr int S = decltype(set_c)::value;
+    constexpr bool FULL = decltype(full_c)::value;
+    // the next step has landed, NS - 2 behind it may still be on their way; this one's operands are here
+    if (FULL) gd_wait<(NS - 2) * L, 0>();
+    else if (NS > 3 && ahead > 2) gd_wait<(NS > 3 ? 2 : 0) * L, 0>();
+    else if (NS > 2 && ahead > 1) gd_wait<(NS > 2 ? 1 : 0) * L, 0>();
+    else gd_wait<0, 0>();
+    if constexpr (!B_KC) {
+#pragma unroll
+      for (int sub = 0; sub < 4; sub++)
+#pragma unroll
+        for (int i = 0; i < TN; i++) {
+          gd_arrived(tr[S][sub][i][0]);
+          gd_arrived(tr[S][sub][i][1]);
+          fn[S][sub][i] = __builtin_bit_cast(gd_half8, __builtin_shufflevector(tr[S][sub][i][0], tr[S][sub][i][1], 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    }
+    if (FULL || ahead > 0) {
       gd_barrier();
       c_stage = c_stage + 1 == NS ? 0 : c_stage + 1;
       read_step(smem + c_stage * STAGE, std::integral_constant<int, 1 - S>{});
-      if constexpr (LOADS) issue_loads();
+      if (FULL || ahead >= NS) issue_loads();
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -201,40 +234,18 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
     gd_barrier();
     read_step(smem, set0);
   }
-  // the last steps (NS of them, or fewer): nothing left to load
-  auto drain = [&](auto set_c) {
-    constexpr int S = decltype(set_c)::value;
-    auto one = [&](auto g_c) {
-      constexpr int G = decltype(g_c)::value;  // NS - 1 - G of the full drain's steps come before: the set alternates
-      step_body(std::integral_constant<int, (S + NS - 1 - G) % 2>{}, g_c, std::false_type{});
-    };
-    if constexpr (NS > 3) one(std::integral_constant<int, 3>{});
-    if constexpr (NS > 2) one(std::integral_constant<int, 2>{});
-    one(std::integral_constant<int, 1>{});
-    one(set0);
-  };
-  if (nk >= NS) {
-    constexpr std::integral_constant<int, NS - 1> full{};
-    int it = 0;
-    for (; it + 2 <= nk - NS; it += 2) {
-      step_body(set0, full, std::true_type{});
-      step_body(set1, full, std::true_type{});
+  {
+    int ahead = nk - 1;
+    for (; ahead > NS; ahead -= 2) {
+      step_body(set0, std::true_type{}, ahead);
+      step_body(set1, std::true_type{}, ahead - 1);
     }
-    if (it < nk - NS) {
-      step_body(set0, full, std::true_type{});
-      drain(set1);
-    } else {
-      drain(set0);
+#pragma unroll 1
+    for (; ahead > 0; ahead -= 2) {
+      step_body(set0, std::false_type{}, ahead);
+      step_body(set1, std::false_type{}, ahead - 1);
     }
-  } else {  // fewer steps than stages
-    for (int it = 0; it < nk; it++) {
-      // in flight behind this one: nk - 1 - it; waiting for all of them costs nothing the first of them does not
-      if (it + 1 < nk) step_body(set0, set1, std::false_type{});
-      else step_body(set0, set0, std::false_type{});
-      if (++it >= nk) break;
-      if (it + 1 < nk) step_body(set1, set1, std::false_type{});
-      else step_body(set1, set0, std::false_type{});
-    }
+    if (ahead == 0) step_body(set0, std::false_type{}, 0);
   }
   gd_barrier();  // nobody reads the operand stages any more
 
@@ -372,7 +383,7 @@ bool launch_gemm_f16_dma(const dnnrtContext *ctx, const GemmF16Args &args, int Z
     return true;
   // Estimated microseconds, fitted on 16 .. 4096 rows and 768 / 3072 columns and channels: a step of 64 k takes a compute
   // unit t1 with one workgroup, tm per workgroup with several; a split's hand-over takes 3 and more with its parts.
-  static const struct { int fn, fm; double t1, tm; } shapes[] = {{64, 64, 0.37, 0.23}, {128, 128, 0.56, 0.80}};
+  static const struct { int fn, fm; double t1, tm; } shapes[] = {{64, 64, 0.30, 0.23}, {128, 128, 0.56, 0.80}};
   const int steps = (int)ceil_div(g.K, 64);
   int best = -1, best_splits = 1;
   double best_cost = 0;
@@ -388,8 +399,22 @@ bool launch_gemm_f16_dma(const dnnrtContext *ctx, const GemmF16Args &args, int Z
       if (best < 0 || cost < best_cost) { best = i; best_cost = cost; best_splits = s; g.steps_per_split = per; }
     }
   }
+  // The kernel whose wavefronts share the reduction: a stage of 32 k takes each of the four 0.43, what comes before and after
+  // them 0.3 more than here, a split's hand-over 2.3 and 0.25 per part.  One workgroup per compute unit: with two it is the
+  // slower one (384 x 768 x 3072 9.7 us here, 10.3 there).
+  const int stages = (int)ceil_div(g.K, 32);
+  const int64_t tiles = ceil_div(g.M, 64) * ceil_div(g.N, 64) * Z;
+  int waves_splits = 0;
+  for (int s = 1; s <= 16 && s <= stages && tiles * s <= ctx->num_cu; s++) {
+    if (s > 1 && (ctx->splitk_shared || tiles > ctx->splitk_max_tiles || tiles * s * 16384 > ctx->splitk_partial_bytes)) break;
+    const int per = (int)ceil_div(stages, s);
+    if (ceil_div(stages, per) != s) continue;
+    const double cost = 0.3 + 0.43 * (double)ceil_div(per, 4) + (s > 1 ? 2.3 + 0.25 * s : 0);
+    if (best < 0 || cost < best_cost) { best = 2; best_cost = cost; waves_splits = s; }
+  }
   if (best < 0) return true;
   launched = true;
+  if (waves_splits) return launch_gemm_f16_waves(ctx, g, Z, waves_splits);
   switch (best) {
     case 0: return launch_gd<64, 64, 2, 2, 4>(ctx, g, Z, best_splits);
     default: return launch_gd<128, 128, 2, 4, 4>(ctx, g, Z, best_splits);

@@ -748,6 +748,25 @@ def test_matmul_f16_direct_to_lds_tiles(gpu, cpu, case):
         np.testing.assert_allclose(oc.matmul_nd(gpu, a3, b3).astype(np.float64), a3.astype(np.float64) @ b3.astype(np.float64), **tol)
 
 
+# The kernel whose wavefronts share the reduction: stages of 32 k for one to four wavefronts, a partial last one, one to many
+# stages each, parts of a split; and the tiles it leaves to the other kernel (more than one per compute unit), with fewer
+# steps than ring stages, as many, and odd and even counts beyond, on 64x64 and 128x128
+@pytest.mark.parametrize("case", [(3, 8, 16), (64, 40, 64), (63, 104, 72), (65, 136, 136), (70, 264, 64), (20, 520, 200), (40, 1288, 64), (129, 6000, 128),
+                                  (1100, 64, 1024), (1100, 192, 1024), (1090, 320, 1032), (1100, 392, 1024), (2100, 136, 2056)], ids=str)
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_matmul_f16_shared_reduction(gpu, case, trans_b):
+    """Against 64-bit sums of the same fp16 operands: fp32 sums and one rounding to fp16 (2^-11), whatever the kernel."""
+    M, K, N = case
+    r = rng(sum(case) + trans_b)
+    a, b = r.standard_normal((M, K)).astype(np.float16), (r.standard_normal((K, N)) / np.sqrt(K)).astype(np.float16)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    if trans_b:
+        got = oc.matmul2d(gpu, a, np.ascontiguousarray(b.T), transB=1).astype(np.float64)
+    else:
+        got = oc.matmul_nd_bias(gpu, a[None], b, np.zeros(N, np.float16))[0].astype(np.float64)
+    np.testing.assert_allclose(got, exact, rtol=2.0 ** -11, atol=2.0 ** -16)
+
+
 def test_gelu_epilogue_against_64_bits(gpu):
     """A product with the identity is its left operand, so this is the epilogue's Gelu of chosen values: to 3 units of the last
     place of its argument (the formula's last two roundings and the fits' 2e-9), infinities and NaN as 0.5 x (1 + erf) has them."""
