@@ -86,8 +86,8 @@ inline double small_f32_estimate_us(const IgemmArgs &a) {
   if (gflop < 0.25 && (pointwise || (a.R == 3 && a.S == 3))) return 0;
   return 5.0 + (pointwise ? 15.5 : a.R == 3 && a.S == 3 ? 18.0 : 60.0) * gflop;
 }
-// Row-major products with a few hundred rows (gemm_f32_rows.hip); `launched` says whether it applied.
-bool launch_gemm_f32_rows(const dnnrtContext *ctx, const IgemmArgs &a, bool &launched);
+// Row-major products (gemm_f32_waves.hip); `launched` says whether it applied.
+bool launch_gemm_f32_waves(const dnnrtContext *ctx, const IgemmArgs &a, bool &launched);
 // Zeroes the first n arrival counters of the context's split-reduction scratch on its stream.  For scratch that
 // is shared beyond one handle (splitk_shared): whoever used the counters last may have died half-way.
 void clear_split_counters(const dnnrtContext *ctx, int n);

@@ -107,7 +107,7 @@ static bool gemm_f32(const dnnrtContext *ctx, const float *A, const float *B, co
   a.a_vec4 = !transA && (K % 4 == 0) && aligned16(A) && (az % 4 == 0);
   a.b_vec4 = transB && (K % 4 == 0) && aligned16(B) && (bz % 4 == 0);
   bool launched = false;
-  if (!launch_gemm_f32_rows(ctx, a, launched)) return false;
+  if (!launch_gemm_f32_waves(ctx, a, launched)) return false;
   if (launched) return true;
   return launch_igemm_f32(ctx, a);
 }

@@ -767,6 +767,29 @@ def test_matmul_f16_shared_reduction(gpu, case, trans_b):
     np.testing.assert_allclose(got, exact, rtol=2.0 ** -11, atol=2.0 ** -16)
 
 
+# rows and columns off the tiles, one stage of 16 k (three wavefronts without any), a few, odd and even counts, whole tiles
+# beside split ones, a handful of split tiles
+@pytest.mark.parametrize("case", [(4100, 16, 3104), (1030, 48, 4100), (300, 336, 2052), (161, 1296, 1000), (384, 768, 3072), (128, 3072, 768), (65, 6160, 132)], ids=str)
+def test_matmul_f32_shared_reduction(gpu, case):
+    """Against 64-bit sums: no further from them than a chain of K fp32 additions (2^-25 sqrt(K) / 2.4 in the 2-norm for
+    independent products) and a few roundings; bias, residual and Gelu; twice, the arrival counters must be back at zero."""
+    M, K, N = case
+    r = rng(sum(case))
+    a, b = r.standard_normal((M, K)).astype(np.float32), (r.standard_normal((K, N)) / np.sqrt(K)).astype(np.float32)
+    bias, z = r.standard_normal(N).astype(np.float32), r.standard_normal((1, M, N)).astype(np.float32)
+    exact = a.astype(np.float64) @ b.astype(np.float64) + bias.astype(np.float64)
+    bound = 2.0 ** -25 * (np.sqrt(K) / 2.4 + 4)
+
+    def far(got, want):
+        return np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want)
+    got = oc.matmul_nd_bias(gpu, a[None], b, bias)
+    assert far(got[0], exact) <= bound
+    np.testing.assert_array_equal(oc.matmul_nd_bias(gpu, a[None], b, bias), got)
+    assert far(oc.matmul_nd_bias(gpu, a[None], b, bias, z=z)[0], exact + z[0]) <= bound
+    from scipy.special import erfc
+    assert far(oc.matmul_nd_bias(gpu, a[None], b, bias, gelu=True)[0], 0.5 * exact * erfc(-exact / np.sqrt(2))) <= 2 * bound
+
+
 def test_gelu_epilogue_against_64_bits(gpu):
     """A product with the identity is its left operand, so this is the epilogue's Gelu of chosen values: to 3 units of the last
     place of its argument (the formula's last two roundings and the fits' 2e-9), infinities and NaN as 0.5 x (1 + erf) has them."""
