@@ -12,11 +12,12 @@
 //        (half-wave h takes channel c+h), i.e. nine MFMAs fed by nine
 //        contiguous filter words and nine input words at base + tap_off[j].
 //   1x1: the reduction index is the channel; addresses advance by a constant.
-// All loads are unconditional (clamped addresses; what must not contribute is
-// masked on the B side at the time of use), so the compiler can track the
+// All loads go to the lane's offset plus a scalar one, what must not contribute has bit 31 of its offset set and reads zero: no
+// vector instruction per load and none per MFMA (there were two and two; conv 3x3 64 -> 64 at 56x56 8.0 -> 7.7 us, with the
+// work behind the reduction spread over the wavefronts; ResNet-50 at batch 1 423 -> 400).  The compiler can track the
 // hardware load counter and the register ring keeps several iterations of
-// loads in flight.  Offsets are 32-bit: the dispatcher only takes these
-// kernels when every operand is below 2^31 elements.
+// loads in flight.  Offsets are 31-bit: the dispatcher only takes these
+// kernels when every operand is below 2^29 elements.
 #include "igemm_f32.h"
 
 #include <type_traits>
@@ -25,7 +26,22 @@ namespace dnnrt {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ float mask_f(float v, unsigned m) { return __uint_as_float(__float_as_uint(v) & m); }
+// Operands are read with raw buffer loads: the lane's offset and a scalar one, so a load costs no vector instruction (an fp32
+// MFMA and the vector instructions share their multipliers: they take turns).  A lane whose offset has bit 31 set reads zero.
+[[maybe_unused]] constexpr unsigned SMALL_OUT_OF_RANGE = 0x80000000u;
+#if __HIP_DEVICE_COMPILE__
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t small_rsrc(const float *base) {  // offsets below 2^31 are the caller's care
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), 0, 0x7fffffff, 0x00020000);
+}
+__device__ __forceinline__ float small_load(__amdgpu_buffer_rsrc_t rsrc, unsigned voff, unsigned soff) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)voff, (int)soff, 0));
+}
+typedef unsigned small_uintx4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float4 small_load4(__amdgpu_buffer_rsrc_t rsrc, unsigned voff, unsigned soff) {
+  const small_uintx4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff, (int)soff, 0);
+  return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+}
+#endif
 
 // The 16 accumulator registers of a lane hold rows m0 + 8 * (r >> 2) + 4 * half + (r & 3)
 // of output column n0 + l32.
@@ -34,83 +50,65 @@ __device__ __forceinline__ int acc_row(int m0, int half, int r) { return m0 + 8 
 // address arithmetic per row is then a uniform offset (scalar unit) added to one per-lane base.
 __device__ __forceinline__ constexpr int row_k(int r) { return 8 * (r >> 2) + (r & 3); }
 
-// Bias of the lane's 16 rows, requested at kernel start so that the values
-// are there when the epilogue wants them (a load per row at that point costs
-// a memory round trip each: the rows are handled under a divergent branch).
-__device__ __forceinline__ void prefetch_bias(const IgemmArgs &a, int z, int m0, int half, float (&bias_r)[16]) {
-  if (a.bias) {
-    const float *__restrict__ biasg = a.bias + (int64_t)z * a.bias_z_stride;
-    if (m0 + 32 <= a.M && (reinterpret_cast<uintptr_t>(biasg) & 15u) == 0) {
-      // whole tile inside the matrix: the lane's rows are four runs of four, one 16-byte load each
+// Of a tile's 16 accumulator registers each of the KS wavefronts finishes 16 / KS: what they need beside the sums (bias of
+// a register's row, residual of its element), requested at kernel start so that the values are there when the epilogue wants them.
+template <int KS>
+struct Finish {
+  static constexpr int N = 16 / KS;
+  float bias[N], res[N];
+};
+template <int KS>
+__device__ __forceinline__ void prefetch_finish(const IgemmArgs &a, int z, int m0, int half, int wave, int img, int pq, Finish<KS> &f) {
+  constexpr int N = Finish<KS>::N;
+  const float *__restrict__ biasg = a.bias ? a.bias + (int64_t)z * a.bias_z_stride : nullptr;
+  const float *__restrict__ Cg = a.Cin ? a.Cin + (int64_t)z * a.c_z_stride + (int64_t)img * a.y_img_stride + pq : nullptr;
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const float4 v = *reinterpret_cast<const float4 *>(biasg + m0 + 8 * g + 4 * half);
-        bias_r[4 * g] = v.x; bias_r[4 * g + 1] = v.y; bias_r[4 * g + 2] = v.z; bias_r[4 * g + 3] = v.w;
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 16; r++) bias_r[r] = biasg[min(acc_row(m0, half, r), a.M - 1)];
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < 16; r++) bias_r[r] = 0.f;
+  for (int i = 0; i < N; i++) {
+    const int row = min(acc_row(m0, half, wave * N + i), a.M - 1);
+    f.bias[i] = biasg ? biasg[row] : 0.f;
+    f.res[i] = Cg ? Cg[(int64_t)row * a.c_row_stride] : 0.f;
   }
 }
 
-// Sum the KS partial tiles in LDS, then bias / residual / activation / store by wavefront 0.
+// Sum the KS partial tiles in LDS, then bias / residual / activation / store, 16 / KS registers of the tile per wavefront (on one
+// wavefront alone the reads of the other seven's sums, and of up to sixteen parts, are a chain of 112 and 256 loads).
 // The reduction may also be split over gridDim.y workgroups.  Each of them
 // leaves its partial tile in `partials` and bumps the tile's arrival counter;
 // whoever arrives last adds the partials up in split order -- the order of
 // arrival does not matter, so the result is the same bits on every run -- and
 // finishes the tile.  Nobody waits for anybody.  The last arriver puts the
 // counter back to zero for the next kernel on the stream.
-template <int KS, bool WIDE_FIXUP>
-__device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 acc, const float (&bias_r)[16], float bias_c, float (*red)[16][64],
+template <int KS>
+__device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 acc, const Finish<KS> &f, float bias_c, float (*red)[16][64],
                                                  int wave, int lane, int m0, int img, int pq, bool col_ok, int z, unsigned tile,
                                                  float *partials, unsigned *counters) {
+  constexpr int N = 16 / KS;
   const int half = lane >> 5;
-  const bool full = m0 + 32 <= a.M;  // the whole tile lies inside the matrix (same for every lane)
-  // the residual tensor's 16 values, requested before anything is waited for
-  const int64_t ycol = (int64_t)img * a.y_img_stride + pq;
-  float res_r[16];
-  if (a.Cin) {
-    if (wave == 0) {
-      const float *__restrict__ Cg = a.Cin + (int64_t)z * a.c_z_stride;
-      if (full) {
-        const float *__restrict__ c0 = Cg + ycol + (int64_t)(m0 + 4 * half) * a.c_row_stride;
+  float v[N];
+  if constexpr (KS > 1) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) res_r[r] = c0[(int64_t)row_k(r) * a.c_row_stride];
-      } else {
+    for (int r = 0; r < 16; r++) red[wave][r][lane] = acc[r];
+    __syncthreads();
 #pragma unroll
-        for (int r = 0; r < 16; r++) res_r[r] = Cg[ycol + (int64_t)min(acc_row(m0, half, r), a.M - 1) * a.c_row_stride];
-      }
+    for (int i = 0; i < N; i++) {
+      v[i] = red[0][wave * N + i][lane];
+#pragma unroll
+      for (int w = 1; w < KS; w++) v[i] += red[w][wave * N + i][lane];
     }
   } else {
 #pragma unroll
-    for (int r = 0; r < 16; r++) res_r[r] = 0.f;
-  }
-  if (KS > 1) {
-    if (wave > 0) {
-#pragma unroll
-      for (int r = 0; r < 16; r++) red[wave - 1][r][lane] = acc[r];
-    }
-    __syncthreads();
-    if (wave > 0) return;
-#pragma unroll
-    for (int w = 0; w < KS - 1; w++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[r] += red[w][r][lane];
+    for (int i = 0; i < N; i++) v[i] = acc[i];
   }
   const int splits = (int)gridDim.y;
   if (splits > 1) {
-    float *mine = partials + ((size_t)tile * splits + blockIdx.y) * 1024;
+    float *mine = partials + ((size_t)tile * splits + blockIdx.y) * 1024 + wave * N * 64 + lane;
 #pragma unroll
-    for (int r = 0; r < 16; r++) __hip_atomic_store(&mine[r * 64 + lane], acc[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // The hand-over.  Every workgroup of a tile (1) writes its partial tile with device-scope atomic
+    for (int i = 0; i < N; i++) __hip_atomic_store(&mine[i * 64], v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // The hand-over.  Every wavefront of every workgroup of a tile (1) writes its part of the partial tile with device-scope atomic
     // stores, which go past the per-XCD L2 to the point where all XCDs agree, (2) waits until every one of
     // them is acknowledged (s_waitcnt 0: the counters of a wavefront reach zero only when its stores have been
-    // written there), (3) adds one to the tile's arrival counter with a device-scope atomic, performed at
-    // that same point.  Whoever reads splits - 1 knows that every other workgroup's step (2) is over, so its
+    // written there); behind the workgroup's barrier (3) one thread adds one to the tile's arrival counter with a device-scope
+    // atomic, performed at that same point.  Whoever reads splits - 1 knows that every other workgroup's step (2) is over, so its
     // device-scope atomic loads, issued after the counter's value has come back (the branch depends on it and
     // a wavefront issues in order), read the finished partial tiles.  Nobody waits for anybody: a workgroup
     // that is not last leaves.  What this rests on is the hardware's behaviour, stated above, not the
@@ -123,61 +121,54 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
     __builtin_amdgcn_s_waitcnt(0);  // vmcnt(0) expcnt(0) lgkmcnt(0)
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     unsigned arrived = 0;
-    if (lane == 0) arrived = __hip_atomic_fetch_add(&counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (KS > 1) {
+      __syncthreads();
+      volatile unsigned *arrived_s = reinterpret_cast<unsigned *>(&red[0][0][0]);  // the sums have been read
+      if (wave == 0 && lane == 0) *arrived_s = __hip_atomic_fetch_add(&counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      arrived = *arrived_s;
+    } else if (lane == 0) {
+      arrived = __hip_atomic_fetch_add(&counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     arrived = __builtin_amdgcn_readfirstlane(arrived);
     if (arrived != (unsigned)splits - 1) return;
-    // splits is a power of two >= 2: the partial tiles are requested four
-    // (WIDE_FIXUP: eight) at a time, a memory round trip each time, and added in split order
-    const float *all = partials + (size_t)tile * splits * 1024 + lane;
+    if (wave == 0 && lane == 0) __hip_atomic_store(&counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // splits is a power of two >= 2: the partial tiles are requested as many at a time as there are up to sixteen values, and added
+    // in split order
+    const float *all = partials + (size_t)tile * splits * 1024 + wave * N * 64 + lane;
+    constexpr int AT_ONCE = N >= 8 ? 2 : N == 4 ? 4 : 8;
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0.f;
-    auto part = [&](int y, float (&p)[16]) {
+    for (int i = 0; i < N; i++) v[i] = 0.f;
+    for (int y = 0; y < splits; y += AT_ONCE) {
+      float p[AT_ONCE][N];
 #pragma unroll
-      for (int r = 0; r < 16; r++) p[r] = __hip_atomic_load(all + (size_t)y * 1024 + r * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    if (splits == 2) {
-      float p0[16], p1[16];
-      part(0, p0); part(1, p1);
+      for (int u = 0; u < AT_ONCE; u++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[r] = (acc[r] + p0[r]) + p1[r];
-    } else if (splits == 4 || !WIDE_FIXUP) {
-      for (int y = 0; y < splits; y += 4) {
-        float p0[16], p1[16], p2[16], p3[16];
-        part(y, p0); part(y + 1, p1); part(y + 2, p2); part(y + 3, p3);
+        for (int i = 0; i < N; i++)
+          p[u][i] = __hip_atomic_load(all + (size_t)min(y + u, splits - 1) * 1024 + i * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = (((acc[r] + p0[r]) + p1[r]) + p2[r]) + p3[r];
-      }
-    } else {  // the 3x3 kernel has the registers for it anyway
-      for (int y = 0; y < splits; y += 8) {
-        float p0[16], p1[16], p2[16], p3[16], p4[16], p5[16], p6[16], p7[16];
-        part(y, p0); part(y + 1, p1); part(y + 2, p2); part(y + 3, p3);
-        part(y + 4, p4); part(y + 5, p5); part(y + 6, p6); part(y + 7, p7);
+      for (int u = 0; u < AT_ONCE; u++)
+        if (y + u < splits) {
 #pragma unroll
-        for (int r = 0; r < 16; r++)
-          acc[r] = (((((((acc[r] + p0[r]) + p1[r]) + p2[r]) + p3[r]) + p4[r]) + p5[r]) + p6[r]) + p7[r];
-      }
+          for (int i = 0; i < N; i++) v[i] += p[u][i];
+        }
     }
-    if (lane == 0) __hip_atomic_store(&counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (!col_ok) return;
-  float *__restrict__ y0 = a.Y + (int64_t)z * a.y_z_stride + ycol + (int64_t)(m0 + 4 * half) * a.y_row_stride;
-  // one copy of the store loop per activation mode, picked once (the mode is the same for every lane);
-  // only a tile that sticks out of the matrix checks its rows
-  auto store_rows = [&](auto mode_c, auto full_c) {
-    constexpr int MODE = decltype(mode_c)::value;
-    constexpr bool FULL = decltype(full_c)::value;
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      if (!FULL && acc_row(m0, half, r) >= a.M) continue;
-      float v = a.alpha * acc[r] + bias_r[r] + bias_c;
-      if (a.Cin) v += a.beta * res_r[r];
-      y0[(int64_t)row_k(r) * a.y_row_stride] = apply_act(v, MODE, a.act_coef);
-    }
-  };
+  const int row0 = acc_row(m0, half, wave * N);  // the rows of a wavefront's registers: row0 + row_k(wave * N + i) - row_k(wave * N)
+  float *__restrict__ y0 = a.Y + (int64_t)z * a.y_z_stride + (int64_t)img * a.y_img_stride + pq;
+  // one copy of the store loop per activation mode, picked once (the mode is the same for every lane)
   auto store = [&](auto mode_c) {
-    if (full) store_rows(mode_c, std::true_type{});
-    else store_rows(mode_c, std::false_type{});
+    constexpr int MODE = decltype(mode_c)::value;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int row = N <= 4 ? row0 + i : acc_row(m0, half, wave * N + i);  // four registers are four consecutive rows
+      if (row >= a.M) continue;
+      float x = a.alpha * v[i] + f.bias[i] + bias_c;
+      if (a.Cin) x += a.beta * f.res[i];
+      y0[(int64_t)row * a.y_row_stride] = apply_act(x, MODE, a.act_coef);
+    }
   };
   switch (a.act) {
     case DNNRT_ACT_RELU: store(std::integral_constant<int, DNNRT_ACT_RELU>{}); break;
@@ -191,8 +182,9 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
 template <int KS, bool AMC>
 __global__ __launch_bounds__(64 * KS) void conv3x3_f32_small_kernel(const IgemmArgs a, const int c_per_wave, float *partials,
                                                                     unsigned *counters) {
-  __shared__ float red[KS > 1 ? KS - 1 : 1][16][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, half = lane >> 5;
+  #if __HIP_DEVICE_COMPILE__
+  __shared__ float red[KS > 1 ? KS : 1][16][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, half = lane >> 5;
   // Workgroups go round-robin over the 8 XCDs (gridDim.x is a multiple of 8, so that holds for every y and
   // z as well), each with its own L2.  The XCDs are laid out as a grid of xcd_m x (8 / xcd_m) over the
   // (filter-row tile, column tile) plane and each owns one rectangle of tiles: it fetches 1 / xcd_m of the
@@ -207,89 +199,94 @@ __global__ __launch_bounds__(64 * KS) void conv3x3_f32_small_kernel(const IgemmA
   if (tm_local >= tm_per || tile_m >= tiles_m || tile_n >= tiles_n) return;
   const int tile_id = tile_m * tiles_n + tile_n;
   const int m0 = tile_m * 32, n0 = tile_n * 32, z = blockIdx.z;
-  const float *__restrict__ Ag = a.A + (int64_t)z * a.a_z_stride;
-  const float *__restrict__ Xg = a.X + (int64_t)z * a.x_z_stride;
+  const __amdgpu_buffer_rsrc_t rsrc_a = small_rsrc(a.A + (int64_t)z * a.a_z_stride), rsrc_x = small_rsrc(a.X + (int64_t)z * a.x_z_stride);
 
-  const int m = m0 + l32, mrow = m < a.M ? m : 0;
+  const int mrow = min(m0 + l32, a.M - 1);
   const int col = n0 + l32;
   const bool col_ok = col < a.Ncols;
   const int PQ = a.P * a.Q, HW = a.H * a.W, C = a.Kdim / 9;
-  float bias_r[16];
-  prefetch_bias(a, z, m0, half, bias_r);
   const float bias_c = 0.f;  // a per-column bias belongs to matrix products, which are never 3x3
   const int img = col_ok ? div_magic(col, PQ, a.magic_pq) : 0, pq = col_ok ? col - img * PQ : 0;
   const int p = div_magic(pq, a.Q, a.magic_q), q = pq - p * a.Q;
   const int ih0 = p * a.sh - a.ph, iw0 = q * a.sw - a.pw;
-  unsigned tap_off[9], tap_mask[9];
+  // Half-wave h of iteration i takes channel cbeg + 2 i + h: the lane's offsets hold h, a tap's filter word or pixel and the mask
+  // of what lies outside; the channel is in the scalar offset.
+  unsigned x_off[9];
 #pragma unroll
   for (int j = 0; j < 9; j++) {
     const int ih = ih0 + j / 3, iw = iw0 + j % 3;
     const bool ok = col_ok && (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
-    tap_off[j] = ok ? (unsigned)(ih * a.W + iw) : 0u;
-    tap_mask[j] = ok ? 0xffffffffu : 0u;
+    x_off[j] = ok ? 4u * (unsigned)((int64_t)img * a.x_img_stride + half * HW + ih * a.W + iw) : SMALL_OUT_OF_RANGE;
   }
-  const unsigned x_img = (unsigned)((int64_t)img * a.x_img_stride);
-  const unsigned a_row = (unsigned)mrow * (unsigned)a.Kdim, lda = (unsigned)a.a_ld;
+  const unsigned a_ch4 = 4u * 9u * (AMC ? (unsigned)a.a_ld : 1u), a_tap4 = 4u * (AMC ? (unsigned)a.a_ld : 1u);  // bytes between channels and taps
+  const unsigned a_off = half * a_ch4 + 4u * (AMC ? (unsigned)mrow : (unsigned)mrow * (unsigned)a.Kdim);
 
   const int cbeg = ((int)blockIdx.y * KS + wave) * c_per_wave, cend = min(C, cbeg + c_per_wave);
-  const int niter = c_per_wave >> 1;
+  const int niter = max(0, (cend - cbeg + 1) >> 1);
+  const bool odd = ((cend - cbeg) & 1) != 0;  // C is odd: the last iteration's second channel is none
 
   constexpr int DEPTH = 4;
   float ra[DEPTH][9], rb[DEPTH][9];
-  unsigned cm[DEPTH];
-  auto load_iter = [&](int i, float (&av)[9], float (&bv)[9], unsigned &cmask) {
-    const int c = cbeg + 2 * i + half;
-    const unsigned cc = (unsigned)min(c, C - 1);
-    cmask = c < cend ? 0xffffffffu : 0u;
-    const unsigned bo = x_img + cc * (unsigned)HW;
-    if (AMC) {  // filter stored [k][K_out]: 32 lanes read 32 consecutive words
-      const unsigned ao = cc * 9u * lda + (unsigned)mrow;
+  auto load_iter = [&](int i, float (&av)[9], float (&bv)[9]) {
+    const unsigned c = (unsigned)(cbeg + 2 * i), as = c * a_ch4, xs = c * (unsigned)(4 * HW);
+    if (odd && i == niter - 1) {
+      const unsigned past = (unsigned)half << 31;
 #pragma unroll
-      for (int j = 0; j < 9; j++) av[j] = Ag[ao + (unsigned)j * lda];
+      for (int j = 0; j < 9; j++) {
+        av[j] = small_load(rsrc_a, a_off | past, as + j * a_tap4);
+        bv[j] = small_load(rsrc_x, x_off[j] | past, xs);
+      }
     } else {
-      const unsigned ao = a_row + cc * 9u;
 #pragma unroll
-      for (int j = 0; j < 9; j++) av[j] = Ag[ao + j];
+      for (int j = 0; j < 9; j++) av[j] = small_load(rsrc_a, a_off, as + j * a_tap4);
+#pragma unroll
+      for (int j = 0; j < 9; j++) bv[j] = small_load(rsrc_x, x_off[j], xs);
     }
-#pragma unroll
-    for (int j = 0; j < 9; j++) bv[j] = Xg[bo + tap_off[j]];
   };
 
   floatx16 acc;
 #pragma unroll
   for (int r = 0; r < 16; r++) acc[r] = 0.f;
-#pragma unroll
-  for (int d = 0; d < DEPTH; d++) load_iter(d, ra[d], rb[d], cm[d]);
   auto mfma_iter = [&](int u) {
 #pragma unroll
-    for (int j = 0; j < 9; j++)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u][j], mask_f(rb[u][j], tap_mask[j] & cm[u]), acc, 0, 0, 0);
+    for (int j = 0; j < 9; j++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u][j], rb[u][j], acc, 0, 0, 0);
   };
   // Iteration i lives in slot i % DEPTH and is refilled with iteration
   // i + DEPTH.  Whole groups that need every refill run without a branch; the
   // last DEPTH iterations refill nothing, and the group in between asks per
   // slot.  Most batch-1 layers have exactly DEPTH iterations per wavefront:
   // everything is requested by the prologue and nothing is loaded in vain.
+  if (niter >= DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load_iter(d, ra[d], rb[d]);
+  } else {
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++)
+      if (d < niter) load_iter(d, ra[d], rb[d]);
+  }
+  Finish<KS> f;
+  prefetch_finish<KS>(a, z, m0, half, wave, img, pq, f);
   int i0 = 0;
   for (; i0 + 2 * DEPTH <= niter; i0 += DEPTH) {
 #pragma unroll
     for (int u = 0; u < DEPTH; u++) {
       mfma_iter(u);
-      load_iter(i0 + u + DEPTH, ra[u], rb[u], cm[u]);
+      load_iter(i0 + u + DEPTH, ra[u], rb[u]);
     }
   }
 #pragma unroll
   for (int u = 0; u < DEPTH; u++) {
     if (i0 + u < niter) {
       mfma_iter(u);
-      if (i0 + u + DEPTH < niter) load_iter(i0 + u + DEPTH, ra[u], rb[u], cm[u]);
+      if (i0 + u + DEPTH < niter) load_iter(i0 + u + DEPTH, ra[u], rb[u]);
     }
   }
   i0 += DEPTH;
 #pragma unroll
   for (int u = 0; u < DEPTH; u++)
     if (i0 + u < niter) mfma_iter(u);
-  reduce_and_store<KS, true>(a, acc, bias_r, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), partials, counters);
+  reduce_and_store<KS>(a, acc, f, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), partials, counters);
+#endif
 }
 
 // 1x1 geometry (convolution, possibly strided, or matrix product with A rows
@@ -297,8 +294,9 @@ __global__ __launch_bounds__(64 * KS) void conv3x3_f32_small_kernel(const IgemmA
 template <int KS, bool AMC>
 __global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmArgs a, const int k_per_wave, float *partials,
                                                                     unsigned *counters) {
-  __shared__ float red[KS > 1 ? KS - 1 : 1][16][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, half = lane >> 5;
+  #if __HIP_DEVICE_COMPILE__
+  __shared__ float red[KS > 1 ? KS : 1][16][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, half = lane >> 5;
   // Workgroups go round-robin over the 8 XCDs (gridDim.x is a multiple of 8, so that holds for every y and
   // z as well), each with its own L2.  The XCDs are laid out as a grid of xcd_m x (8 / xcd_m) over the
   // (filter-row tile, column tile) plane and each owns one rectangle of tiles: it fetches 1 / xcd_m of the
@@ -317,81 +315,89 @@ __global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmA
   // lies in one of them (the launcher makes k_per_wave divide Kdim), so it only picks its operands here.
   const int kbeg_all = ((int)blockIdx.y * KS + wave) * k_per_wave;
   const bool second = a.A2 != nullptr && kbeg_all >= a.Kdim;
-  const float *__restrict__ Ag = second ? a.A2 : a.A + (int64_t)z * a.a_z_stride;
-  const float *__restrict__ Xg = second ? a.X2 : a.X + (int64_t)z * a.x_z_stride;
+  const __amdgpu_buffer_rsrc_t rsrc_a = small_rsrc(second ? a.A2 : a.A + (int64_t)z * a.a_z_stride),
+                               rsrc_x = small_rsrc(second ? a.X2 : a.X + (int64_t)z * a.x_z_stride);
   const int Kd = second ? a.Kdim2 : a.Kdim;
 
-  const int m = m0 + l32, mrow = m < a.M ? m : 0;
+  const int mrow = min(m0 + l32, a.M - 1);
   const int col = n0 + l32;
   const bool col_ok = col < a.Ncols;
   const int PQ = a.P * a.Q, HW = second ? a.H2 * a.W2 : a.H * a.W;
-  float bias_r[16];
-  prefetch_bias(a, z, m0, half, bias_r);
-  if (a.A2 != nullptr && a.bias2 != nullptr) {  // both biases ride in the one epilogue
-#pragma unroll
-    for (int r = 0; r < 16; r++) bias_r[r] += a.bias2[min(acc_row(m0, half, r), a.M - 1)];
-  }
-  const float bias_c = load_bias_col(a, col_ok ? col : 0);  // requested up front as well
   const int img = col_ok ? div_magic(col, PQ, a.magic_pq) : 0, pq = col_ok ? col - img * PQ : 0;
   const int p = div_magic(pq, a.Q, a.magic_q), q = pq - p * a.Q;
   const unsigned x_pix = second ? (unsigned)((int64_t)img * a.x2_img_stride + (int64_t)(p * a.sh2) * a.W2 + q * a.sw2)
                                 : (unsigned)((int64_t)img * a.x_img_stride + (int64_t)(p * a.sh) * a.W + q * a.sw);
-  const unsigned a_row = (unsigned)mrow * (unsigned)Kd, lda = (unsigned)a.a_ld;
+  // Half-wave h of iteration i takes k kbeg + 8 i + 4 h .. + 3 (Kd is a multiple of 4): h in the lane's offset, the rest in the scalar one.
+  const unsigned x_k4 = 4u * (unsigned)HW, a_k4 = 4u * (AMC ? (unsigned)a.a_ld : 1u);
+  const unsigned x_off = col_ok ? 4u * x_pix + 4u * half * x_k4 : SMALL_OUT_OF_RANGE;
+  const unsigned a_off = 4u * half * a_k4 + 4u * (AMC ? (unsigned)mrow : (unsigned)mrow * (unsigned)Kd);
 
   const int kbeg = second ? kbeg_all - a.Kdim : kbeg_all, kend = min(Kd, kbeg + k_per_wave);
-  const int niter = k_per_wave >> 3;
+  const int niter = max(0, (kend - kbeg + 7) >> 3);
+  const bool odd = ((kend - kbeg) & 7) != 0;  // the last iteration's second four k are none
 
   constexpr int DEPTH = 4;
   float4 ra[DEPTH];
   float rb[DEPTH][4];
-  unsigned km[DEPTH];
-  auto load_iter = [&](int i, float4 &av, float (&bv)[4], unsigned &kmask) {
-    const int ka = kbeg + 8 * i + 4 * half;
-    const unsigned kc = (unsigned)min(ka, Kd - 4);
-    kmask = ka < kend ? 0xffffffffu : 0u;
+  auto load_iter = [&](int i, float4 &av, float (&bv)[4]) {
+    const unsigned k = (unsigned)(kbeg + 8 * i), as = k * a_k4, xs = k * x_k4;
+    const unsigned past = odd && i == niter - 1 ? (unsigned)half << 31 : 0u;
     if (AMC) {
-      const unsigned ao = kc * lda + (unsigned)mrow;
-      av.x = Ag[ao]; av.y = Ag[ao + lda]; av.z = Ag[ao + 2u * lda]; av.w = Ag[ao + 3u * lda];
+      av.x = small_load(rsrc_a, a_off | past, as); av.y = small_load(rsrc_a, a_off | past, as + a_k4);
+      av.z = small_load(rsrc_a, a_off | past, as + 2u * a_k4); av.w = small_load(rsrc_a, a_off | past, as + 3u * a_k4);
     } else {
-      av = *reinterpret_cast<const float4 *>(Ag + (a_row + kc));
+      av = small_load4(rsrc_a, a_off | past, as);
     }
-    const unsigned bo = x_pix + kc * (unsigned)HW;
 #pragma unroll
-    for (int j = 0; j < 4; j++) bv[j] = Xg[bo + (unsigned)(j * HW)];
+    for (int j = 0; j < 4; j++) bv[j] = small_load(rsrc_x, x_off | past, xs + j * x_k4);
   };
 
   floatx16 acc;
 #pragma unroll
   for (int r = 0; r < 16; r++) acc[r] = 0.f;
-#pragma unroll
-  for (int d = 0; d < DEPTH; d++) load_iter(d, ra[d], rb[d], km[d]);
   auto mfma_iter = [&](int u) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].x, mask_f(rb[u][0], km[u]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].y, mask_f(rb[u][1], km[u]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].z, mask_f(rb[u][2], km[u]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].w, mask_f(rb[u][3], km[u]), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].x, rb[u][0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].y, rb[u][1], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].z, rb[u][2], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].w, rb[u][3], acc, 0, 0, 0);
   };
   // refills as in the 3x3 kernel: branch-free groups, then one group that asks per slot, then none
+  if (niter >= DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load_iter(d, ra[d], rb[d]);
+  } else {
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++)
+      if (d < niter) load_iter(d, ra[d], rb[d]);
+  }
+  Finish<KS> f;
+  prefetch_finish<KS>(a, z, m0, half, wave, img, pq, f);
+  if (a.A2 != nullptr && a.bias2 != nullptr) {  // both biases ride in the one epilogue
+#pragma unroll
+    for (int i = 0; i < Finish<KS>::N; i++) f.bias[i] += a.bias2[min(acc_row(m0, half, wave * Finish<KS>::N + i), a.M - 1)];
+  }
+  const float bias_c = load_bias_col(a, col_ok ? col : 0);  // requested up front as well
   int i0 = 0;
   for (; i0 + 2 * DEPTH <= niter; i0 += DEPTH) {
 #pragma unroll
     for (int u = 0; u < DEPTH; u++) {
       mfma_iter(u);
-      load_iter(i0 + u + DEPTH, ra[u], rb[u], km[u]);
+      load_iter(i0 + u + DEPTH, ra[u], rb[u]);
     }
   }
 #pragma unroll
   for (int u = 0; u < DEPTH; u++) {
     if (i0 + u < niter) {
       mfma_iter(u);
-      if (i0 + u + DEPTH < niter) load_iter(i0 + u + DEPTH, ra[u], rb[u], km[u]);
+      if (i0 + u + DEPTH < niter) load_iter(i0 + u + DEPTH, ra[u], rb[u]);
     }
   }
   i0 += DEPTH;
 #pragma unroll
   for (int u = 0; u < DEPTH; u++)
     if (i0 + u < niter) mfma_iter(u);
-  reduce_and_store<KS, false>(a, acc, bias_r, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), partials, counters);
+  reduce_and_store<KS>(a, acc, f, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), partials, counters);
+#endif
 }
 
 // A fill kernel rather than hipMemsetAsync: a caller may be recording the stream into a graph.
@@ -409,18 +415,18 @@ bool launch_igemm_f32_small(const dnnrtContext *ctx, const IgemmArgs &a, int rsm
   launched = false;
   if (layout != 0 && layout != 2) return true;
   const bool amc = layout == 2;
-  // 32-bit element offsets inside the kernels
+  // byte offsets below 2^31 inside the kernels
   const int64_t a_elems = amc ? (int64_t)a.Kdim * a.a_ld : (int64_t)a.M * a.Kdim;
   const int64_t x_elems = (int64_t)((a.Ncols + a.P * a.Q - 1) / (a.P * a.Q)) * a.x_img_stride + (int64_t)a.Kdim * a.H * a.W;
-  if (a_elems >= (1ll << 31) || x_elems >= (1ll << 31)) return true;
+  if (a_elems >= (1ll << 29) || x_elems >= (1ll << 29)) return true;
   const bool is3x3 = rsmode == 3 && a.Kdim % 9 == 0 && !a.bias_col;
   const bool is1x1 = rsmode == 1 && (amc || a.a_vec4) && a.Kdim % 4 == 0 && a.Kdim >= 4;
   if (!is3x3 && !is1x1) return true;
   const bool dual = a.A2 != nullptr;
   if (dual) {
     const int64_t x2_elems = (int64_t)((a.Ncols + a.P * a.Q - 1) / (a.P * a.Q)) * a.x2_img_stride + (int64_t)a.Kdim2 * a.H2 * a.W2;
-    if (!is1x1 || a.Z != 1 || a.Kdim2 % 8 != 0 || a.Kdim % 8 != 0 || x2_elems >= (1ll << 31) || (int64_t)a.Kdim2 * a.a_ld >= (1ll << 31) ||
-        (int64_t)a.M * a.Kdim2 >= (1ll << 31))
+    if (!is1x1 || a.Z != 1 || a.Kdim2 % 8 != 0 || a.Kdim % 8 != 0 || x2_elems >= (1ll << 29) || (int64_t)a.Kdim2 * a.a_ld >= (1ll << 29) ||
+        (int64_t)a.M * a.Kdim2 >= (1ll << 29))
       return true;
   }
 
