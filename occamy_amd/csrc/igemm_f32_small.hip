@@ -179,6 +179,55 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
   }
 }
 
+// The 3x3 kernel's iterations 0 .. niter - 1: load(i, slot, last) and multiply(slot) in a ring of four slots, each loaded two
+// ahead of its multiplication; `last` says where i can be the last iteration, which may have only its first half.  A compute unit
+// accepts one of these 4-byte loads in six cycles, and an iteration has eighteen a wavefront: with all four slots requested first (most
+// batch-1 layers have four iterations a wavefront), 1.7 us passed before the first MFMA.  Two ahead are 1 us of MFMA
+// work, which covers the latency: 64 -> 64 at 56x56 7.71 -> 6.75 us, ResNet-50 at batch 1 399 -> 385.  (The 1x1 kernel's
+// iterations are 0.2 us: there all four slots stay in flight; two ahead cost MobileNetV2 2%.)  The counted waits
+// need code in which it is certain which loads have been issued, hence the groups of four without a branch and the two endings.
+template <class Load, class Multiply>
+__device__ __forceinline__ void small_pipeline(int niter, Load load, Multiply multiply) {
+  constexpr std::integral_constant<int, 0> s0{};
+  constexpr std::integral_constant<int, 1> s1{};
+  constexpr std::integral_constant<int, 2> s2{};
+  constexpr std::integral_constant<int, 3> s3{};
+  constexpr std::true_type perhaps_last{};
+  constexpr std::false_type not_last{};
+  if (niter >= 4) {
+    load(0, s0, not_last);
+    load(1, s1, not_last);
+    int i = 0;
+    for (; i + 6 <= niter; i += 4) {
+      load(i + 2, s2, not_last); multiply(s0);
+      load(i + 3, s3, not_last); multiply(s1);
+      load(i + 4, s0, not_last); multiply(s2);
+      load(i + 5, s1, perhaps_last); multiply(s3);
+    }
+    // two to five are left, the first two of them requested
+    if (i + 4 <= niter) {
+      load(i + 2, s2, not_last); multiply(s0);
+      load(i + 3, s3, perhaps_last); multiply(s1);
+      multiply(s2);
+      if (i + 5 == niter) load(i + 4, s0, perhaps_last);
+      multiply(s3);
+      if (i + 5 == niter) multiply(s0);
+    } else {
+      if (i + 3 == niter) load(i + 2, s2, perhaps_last);
+      multiply(s0);
+      multiply(s1);
+      if (i + 3 == niter) multiply(s2);
+    }
+    return;
+  }
+  if (niter > 0) load(0, s0, perhaps_last);
+  if (niter > 1) load(1, s1, perhaps_last);
+  if (niter > 2) load(2, s2, perhaps_last);
+  if (niter > 0) multiply(s0);
+  if (niter > 1) multiply(s1);
+  if (niter > 2) multiply(s2);
+}
+
 template <int KS, bool AMC>
 __global__ __launch_bounds__(64 * KS) void conv3x3_f32_small_kernel(const IgemmArgs a, const int c_per_wave, float *partials,
                                                                     unsigned *counters) {
@@ -227,64 +276,27 @@ __global__ __launch_bounds__(64 * KS) void conv3x3_f32_small_kernel(const IgemmA
 
   constexpr int DEPTH = 4;
   float ra[DEPTH][9], rb[DEPTH][9];
-  auto load_iter = [&](int i, float (&av)[9], float (&bv)[9]) {
+  auto load_iter = [&](int i, float (&av)[9], float (&bv)[9], auto last) {
     const unsigned c = (unsigned)(cbeg + 2 * i), as = c * a_ch4, xs = c * (unsigned)(4 * HW);
-    if (odd && i == niter - 1) {
-      const unsigned past = (unsigned)half << 31;
+    // only the last iteration's lanes are masked, by an instruction a load
+    const unsigned past = last && odd && i == niter - 1 ? (unsigned)half << 31 : 0u;
 #pragma unroll
-      for (int j = 0; j < 9; j++) {
-        av[j] = small_load(rsrc_a, a_off | past, as + j * a_tap4);
-        bv[j] = small_load(rsrc_x, x_off[j] | past, xs);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 9; j++) av[j] = small_load(rsrc_a, a_off, as + j * a_tap4);
-#pragma unroll
-      for (int j = 0; j < 9; j++) bv[j] = small_load(rsrc_x, x_off[j], xs);
+    for (int j = 0; j < 9; j++) {
+      av[j] = small_load(rsrc_a, last ? a_off | past : a_off, as + j * a_tap4);
+      bv[j] = small_load(rsrc_x, last ? x_off[j] | past : x_off[j], xs);
     }
   };
 
   floatx16 acc;
 #pragma unroll
   for (int r = 0; r < 16; r++) acc[r] = 0.f;
-  auto mfma_iter = [&](int u) {
-#pragma unroll
-    for (int j = 0; j < 9; j++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u][j], rb[u][j], acc, 0, 0, 0);
-  };
-  // Iteration i lives in slot i % DEPTH and is refilled with iteration
-  // i + DEPTH.  Whole groups that need every refill run without a branch; the
-  // last DEPTH iterations refill nothing, and the group in between asks per
-  // slot.  Most batch-1 layers have exactly DEPTH iterations per wavefront:
-  // everything is requested by the prologue and nothing is loaded in vain.
-  if (niter >= DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) load_iter(d, ra[d], rb[d]);
-  } else {
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++)
-      if (d < niter) load_iter(d, ra[d], rb[d]);
-  }
   Finish<KS> f;
   prefetch_finish<KS>(a, z, m0, half, wave, img, pq, f);
-  int i0 = 0;
-  for (; i0 + 2 * DEPTH <= niter; i0 += DEPTH) {
+  small_pipeline(niter, [&](int i, auto slot, auto last) { load_iter(i, ra[slot], rb[slot], last); },
+                 [&](auto slot) {
 #pragma unroll
-    for (int u = 0; u < DEPTH; u++) {
-      mfma_iter(u);
-      load_iter(i0 + u + DEPTH, ra[u], rb[u]);
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < DEPTH; u++) {
-    if (i0 + u < niter) {
-      mfma_iter(u);
-      if (i0 + u + DEPTH < niter) load_iter(i0 + u + DEPTH, ra[u], rb[u]);
-    }
-  }
-  i0 += DEPTH;
-#pragma unroll
-  for (int u = 0; u < DEPTH; u++)
-    if (i0 + u < niter) mfma_iter(u);
+                   for (int j = 0; j < 9; j++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[slot][j], rb[slot][j], acc, 0, 0, 0);
+                 });
   reduce_and_store<KS>(a, acc, f, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), partials, counters);
 #endif
 }
@@ -361,7 +373,10 @@ __global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmA
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].z, rb[u][2], acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[u].w, rb[u][3], acc, 0, 0, 0);
   };
-  // refills as in the 3x3 kernel: branch-free groups, then one group that asks per slot, then none
+  // Iteration i lives in slot i % DEPTH and is refilled with iteration i + DEPTH.  Whole groups that need every
+  // refill run without a branch; the last DEPTH iterations refill nothing, and the group in between asks per
+  // slot.  Most batch-1 layers have exactly DEPTH iterations per wavefront: everything is requested by the
+  // prologue and nothing is loaded in vain.
   if (niter >= DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; d++) load_iter(d, ra[d], rb[d]);

@@ -1654,6 +1654,26 @@ def test_conv_3x3_by_minimal_filtering(gpu, case):
         np.testing.assert_allclose(got, ref, rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("crsk", [False, True])
+@pytest.mark.parametrize("geometry", [(2, 62, 64, 128, 1), (1, 14, 13, 40, 2)], ids=["many-tiles", "split"])
+@pytest.mark.parametrize("Cc", [1, 2, 3, 5, 6, 9, 17, 24, 33, 41, 48, 57, 64, 131])
+def test_conv_3x3_small_for_every_length_of_a_wavefronts_slice(gpu, geometry, Cc, crsk):
+    """One to eight and more iterations of two channels a wavefront, the last with one channel or two, wavefronts without any:
+    every ending of the 3x3 small kernel's ring of loads.  Bound: each of the 9 C + 1 additions rounds by at most 2^-24
+    of the sum of magnitudes."""
+    import torch
+    N, H, W, K, st = geometry
+    r = rng(Cc)
+    x = r.standard_normal((N, Cc, H, W)).astype(np.float32)
+    w = (r.standard_normal((K, Cc, 3, 3)) * np.sqrt(2.0 / (9 * Cc))).astype(np.float32)
+    b = r.uniform(-0.5, 0.5, K).astype(np.float32)
+    conv64 = lambda t, f, v: torch.nn.functional.conv2d(*(torch.from_numpy(u).double() for u in (t, f, v)), stride=st, padding=1).numpy()  # noqa: E731
+    ref, magnitude = conv64(x, w, b), conv64(np.abs(x), np.abs(w), np.abs(b))
+    for _ in range(2):  # twice: the split reduction's counters must be back at zero
+        got = oc.conv(gpu, x, w, b, (1, 1), (st, st), 1, _abi.ACT_IDENTITY, crsk=crsk)
+        assert (np.abs(got - ref) <= (9 * Cc + 1) * 2.0 ** -24 * magnitude).all()
+
+
 def test_conv_3x3_by_minimal_filtering_keeps_infinities_in_their_place(gpu, cpu):
     """The transforms take differences within a 4x4 patch: an infinity, a NaN and values whose differences leave fp32's range
     must reach the results that use them and no others, as they do tap by tap."""
