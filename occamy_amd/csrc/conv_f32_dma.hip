@@ -36,8 +36,9 @@ constexpr int D32_BK = 16;
 
 // How a launch is cut: workgroups 0 .. units - 1 (a multiple of 8) are the split tiles' parts, the rest whole tiles.
 struct Dma32Plan {
-  int tiles_m, whole, rest, splits, units, steps, steps_per_split;
-  unsigned magic_tiles_m, magic_rest;
+  int tiles_m, whole, rest, splits, round, units, steps, steps_per_split;  // round: workgroups per part number
+  bool neighbours;  // how the parts go to the XCDs (xcd_tile())
+  unsigned magic_tiles_m, magic_round;
 };
 
 // s_waitcnt vmcnt(N), lgkmcnt as given (15: any); gfx9 encoding.
@@ -91,9 +92,11 @@ __global__ __launch_bounds__(256) void conv_f32_dma_kernel(const IgemmArgs a, co
   const int b = (int)blockIdx.x;
   const bool part = b < pl.units;
   if (part) {
-    split = div_magic(b, pl.rest, pl.magic_rest);
+    split = div_magic(b, pl.round, pl.magic_round);
     if (split >= pl.splits) return;
-    tile = pl.whole + (b - split * pl.rest);
+    tile = pl.neighbours ? xcd_tile(b - split * pl.round, pl.rest) : b - split * pl.round;
+    if (tile < 0) return;
+    tile += pl.whole;
     s_beg = split * pl.steps_per_split;
     s_end = min(s_end, s_beg + pl.steps_per_split);
   } else {  // consecutive tiles (the filter rows of one column range first) on one XCD: they share operands in its L2
@@ -587,7 +590,14 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
         pl.splits = s;
         pl.rest = s > 1 ? (int)rest : 0;
         pl.whole = (int)tiles - pl.rest;
-        pl.units = (int)(ceil_div((int64_t)pl.rest * s, 8) * 8);
+        // Parts of neighbouring tiles on one XCD, or every eighth tile (with the usual multiples of eight filter-row tiles:
+        // one range of filters per XCD): whichever operand is the larger is fetched once, the other by all eight L2s.  The
+        // activations count once a tap, as a tap's pass over the channels outlasts what an L2 keeps.  512 -> 512, 3x3
+        // stride 2 at 14x14, batch 32: 119 -> 84 us, 256 -> 256 at 28x28: 79 -> 72.  A tile's parts stay on one XCD
+        // and consecutive workgroups are of different tiles: the other way round layers of few tiles lost 10 to 20%.
+        pl.neighbours = (pl.rest % 8 == 0 || pl.rest >= 64) && (int64_t)a.M * a.Kdim <= images * a.x_img_stride * RS;
+        pl.round = pl.neighbours ? (int)ceil_div(pl.rest, 8) * 8 : pl.rest;
+        pl.units = (int)(ceil_div((int64_t)pl.round * s, 8) * 8);
         pl.steps = steps;
         pl.steps_per_split = per;
       }
@@ -598,7 +608,7 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
   if (launched) return true;
   if (best_shape < 0 || best + 1.5 > at_most_us) return true;
   pl.magic_tiles_m = magic_of(pl.tiles_m);
-  pl.magic_rest = magic_of(pl.rest > 0 ? pl.rest : 1);
+  pl.magic_round = magic_of(pl.round > 0 ? pl.round : 1);
   launched = true;
   switch (best_shape) {
     case 0: return launch_tile32<128, 128, 2, 2, 3, 1>(ctx, a, pl, mode, av4, bv4);

@@ -11,6 +11,13 @@
 
 namespace dnnrt {
 
+// Of `count` tiles, the one for workgroup w of those dealt round-robin to the 8 XCDs, w < count rounded up to a multiple of 8: an XCD
+// gets a run of neighbouring tiles, an eighth of them or one less, which share operands in its L2.  Negative: none.
+__device__ __forceinline__ int xcd_tile(int w, int count) {
+  const int x = w & 7, tile = ((x * count) >> 3) + (w >> 3);
+  return tile < ((x + 1) * count) >> 3 ? tile : -1;
+}
+
 struct IgemmArgs {
   const float *A;     // [M][Kdim] (k contiguous), or [Kdim][a_ld] when a_mcontig
   int64_t a_ld;       // a_mcontig: elements between consecutive k (>= M)

@@ -198,6 +198,14 @@ def test_conv_f32_direct_to_lds_tiles(gpu, cpu, case):
     np.testing.assert_array_equal(oc.conv(gpu, x, w, b, *args, _abi.ACT_RELU, crsk=True, z=z, inplace=True), gotz)
 
 
+# 168, 65 and 8 tiles in three, seven and six parts, runs of neighbouring tiles per XCD: rounds of parts that are multiples of
+# eight workgroups and one that is not; 32 tiles in eight parts with more filters than activations, every eighth tile on one XCD
+@pytest.mark.parametrize("case", [(8, 128, 41, 41, 192, 3, 2, 1), (4, 512, 28, 28, 320, 3, 2, 1), (5, 64, 57, 57, 256, 3, 2, 1),
+                                  (2, 1024, 14, 14, 1024, 3, 2, 1)], ids=lambda c: "x".join(map(str, c)))
+def test_conv_f32_split_tiles_on_their_xcd(gpu, cpu, case):
+    test_conv_f32_direct_to_lds_tiles(gpu, cpu, case)
+
+
 # channel counts around the four rows a wavefront loads at a time; sizes that fill the chip, whole tiles and split ones
 @pytest.mark.parametrize("C", [1, 2, 3, 5, 29, 30, 33, 47])
 @pytest.mark.parametrize("N,H,W,K,stride", [(3, 75, 75, 66, 1), (6, 56, 56, 64, 1), (10, 60, 60, 128, 2)])
