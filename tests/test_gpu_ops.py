@@ -1082,6 +1082,39 @@ def test_conv_f16(gpu, cpu, case, fmt):
         np.testing.assert_array_equal(conv_f16(gpu, x, w, b, (pd, pd), (st, st), 1, _abi.ACT_RELU, fmt, z=z, inplace=True), gotz)
 
 
+# N, C, H, W, K, R, S, stride, pad: one, two and three steps of 16 taps; every number of filters; images of less than 32 pixels, of
+# no multiple of 32 and of several runs of 32 a wavefront; filters that are not square, windows past every border
+@pytest.mark.parametrize("case", [(2, 3, 37, 53, 32, 3, 3, (2, 2), (1, 1)), (1, 4, 20, 19, 64, 3, 3, (1, 1), (2, 2)), (5, 3, 5, 5, 24, 3, 3, (1, 1), (1, 1)),
+                                  (2, 1, 9, 40, 16, 1, 3, (1, 2), (0, 1)), (1, 2, 33, 9, 48, 3, 2, (3, 1), (2, 1)), (1, 4, 8, 8, 32, 2, 2, (2, 2), (0, 0)),
+                                  (70, 3, 64, 96, 32, 3, 3, (2, 2), (1, 1)), (3, 3, 1, 1, 64, 3, 3, (1, 1), (1, 1))], ids=lambda c: "x".join(map(str, c[:7])))
+@pytest.mark.parametrize("activ", [_abi.ACT_IDENTITY, _abi.ACT_RELU])
+def test_conv_f16_first_layers(gpu, cpu, case, activ):
+    """Against 64-bit sums: the fp32 additions, at most 2^-24 of the sum of magnitudes each, and one rounding to fp16 (two with a
+    residual operand); infinities and NaN only where a window holds them."""
+    import torch
+    N, C, H, W, K, R, S, st, pd = case
+    r = rng(N + H + W + K)
+    x = r.standard_normal((N, C, H, W)).astype(np.float16)
+    w = (r.standard_normal((K, C, R, S)) * np.sqrt(2.0 / (C * R * S))).astype(np.float16)
+    b = r.uniform(-0.3, 0.3, K).astype(np.float16)
+    conv64 = lambda t, f, v: torch.nn.functional.conv2d(*(torch.from_numpy(u).double() for u in (t, f, v)), stride=st, padding=pd).numpy()  # noqa: E731
+    act = (lambda t: np.maximum(t, 0)) if activ == _abi.ACT_RELU else (lambda t: t)
+    ref, magnitude = conv64(x, w, b), conv64(np.abs(x), np.abs(w), np.abs(b))
+    exact = (C * R * S + 2) * 2.0 ** -24 * magnitude
+    got = conv_f16(gpu, x, w, b, pd, st, 1, activ, _abi.NCHW_TO_NHWC).astype(np.float64)
+    assert (np.abs(got - act(ref)) <= exact + 2.0 ** -11 * (np.abs(ref) + exact) + 2.0 ** -25).all()
+    z = r.standard_normal(ref.shape).astype(np.float16)
+    got = conv_f16(gpu, x, w, b, pd, st, 1, activ, _abi.NCHW_TO_NHWC, z=z)
+    twice = exact + 2.0 ** -11 * (np.abs(ref) + exact) + 2.0 ** -25
+    assert (np.abs(got - act(ref + z)) <= twice + 2.0 ** -11 * (np.abs(ref + z) + twice) + 2.0 ** -25).all()
+    x[0, C - 1, H // 2, W // 3] = np.nan
+    x[N - 1, 0, H - 1, W - 1] = -np.inf
+    got, ref = conv_f16(gpu, x, w, b, pd, st, 1, _abi.ACT_IDENTITY, _abi.NCHW_TO_NHWC), oc.conv(cpu, x, w, b, pd, st, 1, _abi.ACT_IDENTITY)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    np.testing.assert_array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    assert np.isfinite(got[np.isfinite(ref)]).all()
+
+
 @pytest.mark.parametrize("case", [(2, 32, 14, 14, 32, 3, 1, 1, 32), (1, 96, 28, 28, 96, 3, 2, 1, 96), (2, 6, 7, 7, 12, 3, 1, 1, 6),
                                   (1, 16, 10, 10, 32, 3, 1, 1, 4), (2, 128, 9, 9, 128, 1, 1, 0, 2), (3, 144, 13, 9, 144, 3, 2, 1, 144),
                                   (1, 960, 7, 7, 960, 3, 1, 1, 960), (2, 24, 9, 9, 24, 5, 1, 2, 24), (1, 12, 6, 6, 12, 3, 1, 1, 12)],
