@@ -684,6 +684,15 @@ def test_attention(gpu, cpu):
                                oc.attention_packed(cpu, qkv, 4, 0.125).astype(np.float32), rtol=2e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("L", [1, 5, 63, 64, 65, 200])
+def test_every_lane_counts_once_in_sums_and_maxima_over_a_wavefront(gpu, L):
+    """Rows with one element of weight: L * mean is exactly it wherever it lies, and a soft-max over -300 and one 0 is one-hot."""
+    x = 2.0 ** 20 * np.eye(L, dtype=np.float32) + np.float32(1)
+    np.testing.assert_array_equal(oc.reduce_mean(gpu, x.reshape(L, L), (L, 1)), np.full((L, 1), np.float32(2 ** 20 + L) / np.float32(L)))
+    hot = np.where(np.eye(L, dtype=bool), 0, -300).astype(np.float32)
+    np.testing.assert_array_equal(oc.softmax(gpu, hot, 1), np.eye(L, dtype=np.float32))
+
+
 @pytest.mark.parametrize("case", [(1, 384, 384, 12, 64), (2, 31, 257, 3, 64), (1, 70, 129, 2, 32), (1, 64, 160, 5, 32), (1, 45, 513, 2, 128),
                                   (1, 1, 1, 1, 64), (3, 33, 32, 2, 64), (1, 600, 600, 16, 64)], ids=str)
 def test_attention_f16_blocks_and_wavefronts(gpu, cpu, case):
