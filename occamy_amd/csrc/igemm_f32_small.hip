@@ -179,39 +179,36 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
   }
 }
 
-// The 3x3 kernel's iterations 0 .. niter - 1: load(i, slot, last) and multiply(slot) in a ring of four slots, each loaded two
+// The 3x3 kernel's iterations 0 .. niter - 1: load(i, slot, last) and multiply(slot) in a ring of three slots, each loaded two
 // ahead of its multiplication; `last` says where i can be the last iteration, which may have only its first half.  A compute unit
-// accepts one of these 4-byte loads in six cycles, and an iteration has eighteen a wavefront: with all four slots requested first (most
-// batch-1 layers have four iterations a wavefront), 1.7 us passed before the first MFMA.  Two ahead are 1 us of MFMA
-// work, which covers the latency: 64 -> 64 at 56x56 7.71 -> 6.75 us, ResNet-50 at batch 1 399 -> 385.  (The 1x1 kernel's
-// iterations are 0.2 us: there all four slots stay in flight; two ahead cost MobileNetV2 2%.)  The counted waits
-// need code in which it is certain which loads have been issued, hence the groups of four without a branch and the two endings.
+// accepts one of these 4-byte loads in six cycles, and an iteration has eighteen a wavefront: with four requested first (most batch-1
+// layers have no more a wavefront), 1.7 us passed before the first MFMA.  Two ahead are 1 us of MFMA
+// work, which covers the latency: 64 -> 64 at 56x56 7.71 -> 6.75 us, ResNet-50 at batch 1 399 -> 385; and with three slots for four two
+// workgroups of eight wavefronts fit a compute unit: 6.5 and 379, 128 -> 128 at 28x28, batch 4, 17.3 -> 15.6.  (The 1x1 kernel's
+// iterations are 0.2 us: there four slots stay in flight; two ahead cost MobileNetV2 2%.)  The counted waits
+// need code in which it is certain which loads have been issued, hence the groups of three without a branch and the endings.
 template <class Load, class Multiply>
 __device__ __forceinline__ void small_pipeline(int niter, Load load, Multiply multiply) {
   constexpr std::integral_constant<int, 0> s0{};
   constexpr std::integral_constant<int, 1> s1{};
   constexpr std::integral_constant<int, 2> s2{};
-  constexpr std::integral_constant<int, 3> s3{};
   constexpr std::true_type perhaps_last{};
   constexpr std::false_type not_last{};
-  if (niter >= 4) {
+  if (niter >= 3) {
     load(0, s0, not_last);
     load(1, s1, not_last);
     int i = 0;
-    for (; i + 6 <= niter; i += 4) {
+    for (; i + 5 <= niter; i += 3) {
       load(i + 2, s2, not_last); multiply(s0);
-      load(i + 3, s3, not_last); multiply(s1);
-      load(i + 4, s0, not_last); multiply(s2);
-      load(i + 5, s1, perhaps_last); multiply(s3);
+      load(i + 3, s0, not_last); multiply(s1);
+      load(i + 4, s1, perhaps_last); multiply(s2);
     }
-    // two to five are left, the first two of them requested
-    if (i + 4 <= niter) {
+    // two to four are left, the first two of them requested
+    if (i + 4 == niter) {
       load(i + 2, s2, not_last); multiply(s0);
-      load(i + 3, s3, perhaps_last); multiply(s1);
+      load(i + 3, s0, perhaps_last); multiply(s1);
       multiply(s2);
-      if (i + 5 == niter) load(i + 4, s0, perhaps_last);
-      multiply(s3);
-      if (i + 5 == niter) multiply(s0);
+      multiply(s0);
     } else {
       if (i + 3 == niter) load(i + 2, s2, perhaps_last);
       multiply(s0);
@@ -222,14 +219,12 @@ __device__ __forceinline__ void small_pipeline(int niter, Load load, Multiply mu
   }
   if (niter > 0) load(0, s0, perhaps_last);
   if (niter > 1) load(1, s1, perhaps_last);
-  if (niter > 2) load(2, s2, perhaps_last);
   if (niter > 0) multiply(s0);
   if (niter > 1) multiply(s1);
-  if (niter > 2) multiply(s2);
 }
 
 template <int KS, bool AMC>
-__global__ __launch_bounds__(64 * KS) void conv3x3_f32_small_kernel(const IgemmArgs a, const int c_per_wave, float *partials,
+__global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS >= 2 ? 4 : 3))) void conv3x3_f32_small_kernel(const IgemmArgs a, const int c_per_wave, float *partials,
                                                                     unsigned *counters) {
   #if __HIP_DEVICE_COMPILE__
   __shared__ float red[KS > 1 ? KS : 1][16][64];
@@ -274,7 +269,7 @@ __global__ __launch_bounds__(64 * KS) void conv3x3_f32_small_kernel(const IgemmA
   const int niter = max(0, (cend - cbeg + 1) >> 1);
   const bool odd = ((cend - cbeg) & 1) != 0;  // C is odd: the last iteration's second channel is none
 
-  constexpr int DEPTH = 4;
+  constexpr int DEPTH = 3;
   float ra[DEPTH][9], rb[DEPTH][9];
   auto load_iter = [&](int i, float (&av)[9], float (&bv)[9], auto last) {
     const unsigned c = (unsigned)(cbeg + 2 * i), as = c * a_ch4, xs = c * (unsigned)(4 * HW);
