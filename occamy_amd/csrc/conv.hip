@@ -607,7 +607,7 @@ void *dnnrtConvBiasAddConvBiasActiv(dnnrtHandle_t handle, const void *X, const i
     a.magic_rs = dnnrt::magic_of(1); a.magic_s = dnnrt::magic_of(1);
     const auto wgs64 = dnnrt::ceil_div(a.M, 64) * dnnrt::ceil_div(a.Ncols, 64);
     bool launched = false;
-    if (!dnnrt::launch_conv_f32_dma(handle, a, wgs64 < handle->num_cu ? dnnrt::small_f32_estimate_us(a) : 1e30, launched)) return nullptr;
+    if (!dnnrt::launch_conv_f32_dma(handle, a, wgs64 < handle->num_cu ? dnnrt::small_f32_estimate_us(handle->num_cu, a) : 1e30, launched)) return nullptr;
     if (launched) return Y;
     if (wgs64 < handle->num_cu) {  // where a convolution of its own would take the small kernels as well
       if (!dnnrt::launch_igemm_f32_small(handle, a, 1, crsk ? 2 : 0, launched)) return nullptr;

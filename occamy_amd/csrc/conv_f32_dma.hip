@@ -578,11 +578,17 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
       const int unit = bm * bn <= 4096 ? 2 : 1;  // 16-k steps per ring stage: a part starts on a stage
       const int per = (int)ceil_div(ceil_div(steps, s), unit) * unit;
       if (ceil_div(steps, per) != s) continue;
-      const int64_t parts = ceil_div(rest * s, ctx->num_cu);  // of a split tile, on the busiest compute unit
+      // Parts of neighbouring tiles on one XCD, or every eighth tile (with the usual multiples of eight filter-row tiles:
+      // one range of filters per XCD): whichever operand is the larger is fetched once, the other by all eight L2s.  The
+      // activations count once a tap, as a tap's pass over the channels outlasts what an L2 keeps.  512 -> 512, 3x3
+      // stride 2 at 14x14, batch 32: 119 -> 84 us, 256 -> 256 at 28x28: 79 -> 72.  A tile's parts stay on one XCD
+      // and consecutive workgroups are of different tiles: the other way round layers of few tiles lost 10 to 20%.
+      const bool neighbours = (rest % 8 == 0 || rest >= 64) && (int64_t)a.M * a.Kdim <= images * a.x_img_stride * RS;
+      const int64_t parts = neighbours ? ceil_div(ceil_div(rest, 8) * s, ceil_div(ctx->num_cu, 8)) : ceil_div(rest * s, ctx->num_cu);  // of a split tile, on the busiest compute unit
       const double load = (double)rounds * steps + (double)parts * per;
       double cost = load * (rounds + parts > 1 ? shapes[i].tm : shapes[i].t1) + fixed;
       if (rounds + parts > 1 && cost < fixed + shapes[i].t1 * per) cost = fixed + shapes[i].t1 * per;
-      if (s > 1) cost += 3.0 + s * (bm * bn / 4096.0) * 0.3;
+      if (s > 1) cost += (rounds > 0 ? 2.5 : 3.0) + s * (bm * bn / 4096.0) * 0.3;  // partly behind the whole tiles
       if (best_shape < 0 || cost < best) {
         best = cost;
         best_shape = i;
@@ -590,12 +596,7 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
         pl.splits = s;
         pl.rest = s > 1 ? (int)rest : 0;
         pl.whole = (int)tiles - pl.rest;
-        // Parts of neighbouring tiles on one XCD, or every eighth tile (with the usual multiples of eight filter-row tiles:
-        // one range of filters per XCD): whichever operand is the larger is fetched once, the other by all eight L2s.  The
-        // activations count once a tap, as a tap's pass over the channels outlasts what an L2 keeps.  512 -> 512, 3x3
-        // stride 2 at 14x14, batch 32: 119 -> 84 us, 256 -> 256 at 28x28: 79 -> 72.  A tile's parts stay on one XCD
-        // and consecutive workgroups are of different tiles: the other way round layers of few tiles lost 10 to 20%.
-        pl.neighbours = (pl.rest % 8 == 0 || pl.rest >= 64) && (int64_t)a.M * a.Kdim <= images * a.x_img_stride * RS;
+        pl.neighbours = s > 1 && neighbours;
         pl.round = pl.neighbours ? (int)ceil_div(pl.rest, 8) * 8 : pl.rest;
         pl.units = (int)(ceil_div((int64_t)pl.round * s, 8) * 8);
         pl.steps = steps;
@@ -604,9 +605,9 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
     }
   }
   // 3x3 layers with stride 1: by Winograd's method where that is estimated to be faster
-  if (!launch_conv_f32_winograd(ctx, args, best_shape < 0 || best + 1.5 > at_most_us ? at_most_us - 1.5 : best, launched)) return false;
+  if (!launch_conv_f32_winograd(ctx, args, best_shape < 0 || best > at_most_us ? at_most_us : best, launched)) return false;
   if (launched) return true;
-  if (best_shape < 0 || best + 1.5 > at_most_us) return true;
+  if (best_shape < 0 || best > at_most_us) return true;
   pl.magic_tiles_m = magic_of(pl.tiles_m);
   pl.magic_round = magic_of(pl.round > 0 ? pl.round : 1);
   launched = true;

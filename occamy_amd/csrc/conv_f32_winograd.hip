@@ -451,7 +451,7 @@ bool launch_conv_f32_winograd(const dnnrtContext *ctx, const IgemmArgs &args, do
   const int64_t tiles = pl.tiles_m * ceil_div(pl.n_tiles, W32_BT);
   if (tiles > (1 << 28)) return true;
   // Estimated time in microseconds: a stage takes a compute unit 0.62 whether one or two workgroups share it, a workgroup's
-  // start and end 9 with the launch and 2.3 for every further one in a row, a split tile's hand-over 2.5 and 0.7 per part (measured on layers
+  // start and end 9 with the launch and 2.3 for every further one in a row, a split tile's hand-over 3.1 and 0.7 per part, a lone workgroup's stores to rows of odd length 1.4 (measured on layers
   // of 0.8 .. 26 GFLOP, 64 to 1320 tiles, within 12 %).  As in conv_f32_dma.hip the tiles left over after the last full round are split.
   const int64_t rounds = tiles / ctx->num_cu, rest = tiles - rounds * ctx->num_cu;
   double best = 0;
@@ -460,7 +460,7 @@ bool launch_conv_f32_winograd(const dnnrtContext *ctx, const IgemmArgs &args, do
     const int per = (int)ceil_div(pl.stages, s);
     if (ceil_div(pl.stages, per) != s) continue;
     const int64_t parts = ceil_div(rest * s, ctx->num_cu);
-    const double cost = 9.0 + 0.62 * ((double)rounds * pl.stages + (double)parts * per) + 2.3 * (double)(rounds + parts - 1) + (s > 1 ? 2.5 + 0.7 * s : 0.0);
+    const double cost = 9.0 + 0.62 * ((double)rounds * pl.stages + (double)parts * per) + 2.3 * (double)(rounds + parts - 1) + (s > 1 ? 3.1 + 0.7 * s : 0.0) + (a.Q % 2 && rounds + parts == 1 ? 1.4 : 0.0);
     if (!pl.splits || cost < best) {
       best = cost;
       pl.splits = s;

@@ -83,15 +83,34 @@ bool launch_conv3x3_f32_tiled(const dnnrtContext *ctx, const IgemmArgs &a, int l
 bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &a, double at_most_us, bool &launched);
 // 3x3 convolutions with stride 1 and C,R,S,K filters by Winograd's method (conv_f32_winograd.hip), likewise.
 bool launch_conv_f32_winograd(const dnnrtContext *ctx, const IgemmArgs &a, double at_most_us, bool &launched);
-// What the small-problem kernels take for a convolution, estimated in microseconds: single launches of 0.1 .. 2 GFLOP
-// (counting whole 32x32 tiles) measure 5 + 18 per GFLOP for 3x3 filters, 5 + 15.5 for 1x1, 60 and more per GFLOP on the
-// general kernel.  0 below a quarter of a GFLOP: there either way is launch and latency, and inside a network, with its
-// operands further away, the small kernels have the shorter chain (56x56 layers of a ResNet-50 at batch 1: 8.1 against 8.6).
-inline double small_f32_estimate_us(const IgemmArgs &a) {
-  const double gflop = 2e-9 * 1024 * (double)ceil_div(a.M, 32) * (double)ceil_div(a.Ncols, 32) * (a.Kdim + (a.A2 ? a.Kdim2 : 0));
+// How the small kernels (igemm_f32_small.hip) cut the reduction of `tiles` 32x32 tiles: over ks wavefronts of a workgroup, until the
+// chip has eight wavefronts per compute unit, and over `splits` workgroups, until it has one workgroup per compute unit.
+inline void small_f32_cut(int num_cu, int64_t tiles, int red_len, int min_slice, int &ks, int &splits) {
+  ks = splits = 1;
+  while (ks < 8 && tiles * ks < (int64_t)num_cu * 8 && ceil_div(red_len, ks * 2) >= min_slice) ks *= 2;
+  while (splits < 16 && tiles * splits * 2 <= num_cu && ceil_div(red_len, ks * splits * 2) >= min_slice) splits *= 2;
+}
+constexpr int SMALL_3X3_MIN_SLICE = 4;  // channels worth a wavefront
+// What the small-problem kernels take for a convolution, estimated in microseconds.  3x3 filters: 4.3, 1.36 times the MFMA time
+// of the workgroups in a row on the busiest compute unit, 0.7 for each but the first, a split's hand-over 1.6 and 0.12 per part
+// (46 layers of 0.1 to 11 GFLOP, batch 1 to 8: all within 10%).  Inside a network, operands and above all filters further away, the
+// tiles with their deeper rings lose less: hence 9% and 0.08 per megabyte of filter on top (1024 -> 1024 at 7x7, batch 2, 27.7 against
+// 29.0 alone, in YOLO v1 1 to 3 more).  1x1: single launches of 0.1 .. 2 GFLOP (counting whole 32x32
+// tiles) measure 5 + 15.5 per GFLOP, general kernel 60 and more per GFLOP; 0 below a quarter of a GFLOP: there either way is
+// launch and latency, and inside a network, with its operands further away, the small kernels have the shorter chain.
+inline double small_f32_estimate_us(int num_cu, const IgemmArgs &a) {
+  const int64_t tiles = ceil_div(a.M, 32) * ceil_div(a.Ncols, 32);
+  if (a.R == 3 && a.S == 3) {
+    int ks, splits;
+    small_f32_cut(num_cu, tiles * a.Z, a.Kdim / 9, SMALL_3X3_MIN_SLICE, ks, splits);
+    const double in_a_row = (double)ceil_div(tiles * a.Z * splits, num_cu), mfma_us = (double)a.Kdim / splits / 300.0;
+    const double alone = 4.3 + 1.36 * in_a_row * mfma_us + 0.7 * (in_a_row - 1) + (splits > 1 ? 1.6 + 0.12 * splits : 0.0);
+    return 1.09 * alone + 8e-8 * 4.0 * a.M * a.Kdim;
+  }
+  const double gflop = 2e-9 * 1024 * (double)tiles * (a.Kdim + (a.A2 ? a.Kdim2 : 0));
   const bool pointwise = a.R == 1 && a.S == 1 && a.ph == 0 && a.pw == 0;
-  if (gflop < 0.25 && (pointwise || (a.R == 3 && a.S == 3))) return 0;
-  return 5.0 + (pointwise ? 15.5 : a.R == 3 && a.S == 3 ? 18.0 : 60.0) * gflop;
+  if (gflop < 0.25 && pointwise) return 0;
+  return 5.0 + (pointwise ? 15.5 : 60.0) * gflop;
 }
 // Row-major products (gemm_f32_waves.hip); `launched` says whether it applied.
 bool launch_gemm_f32_waves(const dnnrtContext *ctx, const IgemmArgs &a, bool &launched);

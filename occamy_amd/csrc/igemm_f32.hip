@@ -302,7 +302,7 @@ bool launch_igemm_f32(const dnnrtContext *ctx, const IgemmArgs &args) {
   const bool fills_chip = ceil_div(a.M, 64) * ceil_div(a.Ncols, 64) * a.Z >= ctx->num_cu;
   if (layout == 2) {  // C,R,S,K filters: always where 64x64 tiles fill the chip, below that where it beats the small kernels
     bool launched = false;
-    if (!launch_conv_f32_dma(ctx, a, fills_chip ? 1e30 : small_f32_estimate_us(a), launched)) return false;
+    if (!launch_conv_f32_dma(ctx, a, fills_chip ? 1e30 : small_f32_estimate_us(ctx->num_cu, a), launched)) return false;
     if (launched) return true;
   }
   if (rsmode == 3) {  // the 3x3 specialisation takes the problems the tiles below would get

@@ -443,27 +443,22 @@ bool launch_igemm_f32_small(const dnnrtContext *ctx, const IgemmArgs &a, int rsm
   const int64_t tiles64 = ceil_div(a.M, 32) * ceil_div(a.Ncols, 32);
   if (tiles64 > INT32_MAX) return true;
   const int tiles = (int)tiles64;
-  const int64_t want_waves = (int64_t)ctx->num_cu * 8;
   const int red_len = is3x3 ? a.Kdim / 9 : a.Kdim + (dual ? a.Kdim2 : 0);   // channels
   // reduction slice worth a wavefront; 1x1 problems of at most 32 tiles (the last stages of a MobileNetV2 at batch 1)
   // go down to 16 channels: 0.264 -> 0.260 ms per inference there, with more tiles it costs more than it gives
-  const int min_slice = is3x3 ? 4 : (tiles <= 32 ? 16 : 32);
-  int ks = 1;
-  while (ks < 8 && (int64_t)tiles * a.Z * ks < want_waves && ceil_div(red_len, ks * 2) >= min_slice) ks *= 2;
-  // Still far from filling the chip (deep layers at batch 1: a few dozen tiles
-  // over a reduction of thousands): split the reduction over workgroups too.
-  int splits = 1;
-  while (splits < 16 && (int64_t)tiles * a.Z * splits * 2 <= ctx->num_cu &&
-         ceil_div(red_len, ks * splits * 2) >= min_slice) {
-    if ((int64_t)tiles * a.Z * splits * 2 * 4096 > ctx->splitk_partial_bytes || (int64_t)tiles * a.Z > ctx->splitk_max_tiles) {
-      if (!ctx->splitk_shared) break;  // a handle's own scratch: a shallower split is as good
+  const int min_slice = is3x3 ? SMALL_3X3_MIN_SLICE : (tiles <= 32 ? 16 : 32);
+  int ks, splits;
+  small_f32_cut(ctx->num_cu, (int64_t)tiles * a.Z, red_len, min_slice, ks, splits);
+  if (splits > 1 && ((int64_t)tiles * a.Z * splits * 4096 > ctx->splitk_partial_bytes || (int64_t)tiles * a.Z > ctx->splitk_max_tiles)) {
+    if (ctx->splitk_shared) {
       set_error("igemm_f32(small): the split reduction of this problem needs %lld bytes of scratch and %lld counters, "
                 "the static scratch holds %lld and %d",
-                (long long)tiles * a.Z * splits * 2 * 4096, (long long)tiles * a.Z, (long long)ctx->splitk_partial_bytes,
+                (long long)tiles * a.Z * splits * 4096, (long long)tiles * a.Z, (long long)ctx->splitk_partial_bytes,
                 ctx->splitk_max_tiles);
       return false;
     }
-    splits *= 2;
+    // a handle's own scratch: a shallower split is as good
+    while (splits > 1 && ((int64_t)tiles * a.Z * splits * 4096 > ctx->splitk_partial_bytes || (int64_t)tiles * a.Z > ctx->splitk_max_tiles)) splits /= 2;
   }
   int k_per_wave_1x1 = (int)(ceil_div(ceil_div(red_len, ks * splits), 8) * 8);
   if (dual) {
