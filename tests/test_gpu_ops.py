@@ -684,6 +684,16 @@ def test_attention(gpu, cpu):
                                oc.attention_packed(cpu, qkv, 4, 0.125).astype(np.float32), rtol=2e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16, np.int64])
+@pytest.mark.parametrize("dims,perm", [((2, 3, 2, 2, 5, w), (0, 1, 4, 2, 5, 3)) for w in (1, 2, 3, 4, 6, 8, 234)] +
+                         [((2, 12), (1, 0)), ((2, 3, 12), (2, 1, 0)), ((5, 2, 8), (0, 2, 1)), ((2, 5, 8), (1, 2, 0)), ((3, 2, 7, 4), (0, 2, 3, 1))], ids=str)
+def test_transpose_rows_in_pairs(gpu, dims, perm, dtype):
+    """The last result dim two strided elements, the one before it the input's last: pixel shuffles by two and plain
+    transposes of two rows, of widths and strides the wide loads take and do not."""
+    x = rng(len(dims)).integers(-999, 999, dims).astype(dtype)
+    np.testing.assert_array_equal(oc.transpose(gpu, x, perm), x.transpose(perm))
+
+
 @pytest.mark.parametrize("L", [1, 5, 63, 64, 65, 200])
 def test_every_lane_counts_once_in_sums_and_maxima_over_a_wavefront(gpu, L):
     """Rows with one element of weight: L * mean is exactly it wherever it lies, and a soft-max over -300 and one 0 is one-hot."""
