@@ -275,6 +275,124 @@ __global__ __launch_bounds__(256) void conv_f32_narrow_kernel(
     }
 }
 
+// The same for 3x3 filters with stride 1, four pixels in a column per thread: 18 loads a channel for the four instead of 36, and a
+// filter value read once for the four; the four wavefronts of a patch take a quarter of the channels each.  A patch is 2^q_log2
+// pixels wide, 64 where the image is: patches of 16 halve every cache line, and with neighbours on different XCDs each half
+// came from memory by itself.  64 -> 3 at 360x468, behind the layer that wrote its input: a pixel per thread in patches of 16 x 16
+// 32.6 us, four pixels per thread 33.9, wide patches 23.4, timestamps included; bound by its loads and FMAs, about evenly.
+template <int K>
+__global__ __launch_bounds__(256) void conv3x3_f32_narrow_kernel(const float *__restrict__ X, const float *__restrict__ Wt, const float *__restrict__ bias,
+                                                                 const float *Zr, float *Y, int C, int H, int W, int P, int Q, int ph, int pw,
+                                                                 int act, float act_coef, int w_k, int w_tap, int tiles, int q_log2) {
+#if __HIP_DEVICE_COMPILE__
+  extern __shared__ float wl[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = xcd_tile((int)blockIdx.x, tiles);
+  if (tile < 0) return;
+  const int tiles_q = (Q + (1 << q_log2) - 1) >> q_log2, p_log2 = 8 - q_log2, tiles_p = (P + (1 << p_log2) - 1) >> p_log2;
+  const int tq = tile % tiles_q, tp = (tile / tiles_q) % tiles_p, n = tile / (tiles_q * tiles_p);
+  const int p0 = (tp << p_log2) + 4 * (lane >> q_log2), q = (tq << q_log2) + (lane & ((1 << q_log2) - 1));
+  const int HW = H * W;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(X) + (int64_t)n * C * HW, 0, 4 * C * HW, 0x00020000);
+  unsigned off[6][3];  // bit 31: outside the image, past the end of the buffer, reads zero
+#pragma unroll
+  for (int r = 0; r < 6; r++)
+#pragma unroll
+    for (int s = 0; s < 3; s++) {
+      const int ih = p0 - ph + r, iw = q - pw + s;
+      off[r][s] = (unsigned)ih < (unsigned)H && (unsigned)iw < (unsigned)W ? 4u * (unsigned)(ih * W + iw) : 0x80000000u;
+    }
+  struct Taps { float v[6][3]; };
+  const int per = (C + 3) >> 2, c_end = min(C, (wave + 1) * per);
+  auto fetch = [&](int c) {  // channels past the end re-read the last one and are not used
+    Taps t;
+#pragma unroll
+    for (int r = 0; r < 6; r++)
+#pragma unroll
+      for (int s = 0; s < 3; s++)
+        t.v[r][s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)off[r][s], 4 * min(c, C - 1) * HW, 0));
+    return t;
+  };
+  float acc[4][K];
+#pragma unroll
+  for (int o = 0; o < 4; o++)
+#pragma unroll
+    for (int k = 0; k < K; k++) acc[o][k] = 0.f;
+  auto use = [&](const Taps &t, int c) {
+    const float4 *w = reinterpret_cast<const float4 *>(wl) + c * 9;
+#pragma unroll
+    for (int s = 0; s < 3; s++)
+#pragma unroll
+      for (int tr = 0; tr < 3; tr++) {
+        const float4 f4 = w[tr * 3 + s];
+        const float f[4] = {f4.x, f4.y, f4.z, f4.w};
+#pragma unroll
+        for (int o = 0; o < 4; o++)
+#pragma unroll
+          for (int k = 0; k < K; k++) acc[o][k] = fmaf(t.v[o + tr][s], f[k], acc[o][k]);
+      }
+  };
+  auto lds_barrier = []() {  // for LDS accesses only: the loads stay in flight
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  int c = wave * per;
+  // The filters to LDS, [c][tap][4]: eight loads requested before the first is stored, or each is a round trip.
+  for (int i0 = threadIdx.x; i0 < C * 9 * K; i0 += 256 * 8) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int i = min(i0 + 256 * u, C * 9 * K - 1), ct = i / K;  // ct = c * 9 + tap
+      v[u] = Wt[(int64_t)(i - ct * K) * w_k + (int64_t)ct * w_tap];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int i = min(i0 + 256 * u, C * 9 * K - 1), ct = i / K;
+      wl[4 * ct + i - ct * K] = v[u];
+    }
+  }
+  // Four channels in flight; the barriers keep the loads in the order in which they are waited for.
+#define ORDERED __builtin_amdgcn_sched_barrier(0)
+  Taps t0 = fetch(c); ORDERED;
+  Taps t1 = fetch(c + 1); ORDERED;
+  Taps t2 = fetch(c + 2); ORDERED;
+  Taps t3 = fetch(c + 3); ORDERED;
+  lds_barrier();
+  for (; c < c_end; c += 4) {
+    use(t0, c); ORDERED;
+    t0 = fetch(c + 4); ORDERED;
+    if (c + 1 < c_end) use(t1, c + 1);
+    ORDERED; t1 = fetch(c + 5); ORDERED;
+    if (c + 2 < c_end) use(t2, c + 2);
+    ORDERED; t2 = fetch(c + 6); ORDERED;
+    if (c + 3 < c_end) use(t3, c + 3);
+    ORDERED; t3 = fetch(c + 7); ORDERED;
+  }
+#undef ORDERED
+  __syncthreads();  // the filters have been read: their place takes the wavefronts' sums
+#pragma unroll
+  for (int o = 0; o < 4; o++)
+#pragma unroll
+    for (int k = 0; k < K; k++) wl[((wave * 4 + o) * K + k) * 64 + lane] = acc[o][k];
+  __syncthreads();
+  const int p = p0 + wave;  // a wavefront ends one row of each four
+  if (p >= P || q >= Q) return;
+  const int64_t PQ = (int64_t)P * Q, pix = (int64_t)p * Q + q;
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    float r = 0.f;
+#pragma unroll
+    for (int v = 0; v < 4; v++) r += wl[((v * 4 + wave) * K + k) * 64 + lane];
+    const int64_t o = ((int64_t)n * K + k) * PQ + pix;
+    if (bias) r += bias[k];
+    if (Zr) r += Zr[o];
+    Y[o] = apply_act(r, act, act_coef);
+  }
+#endif
+}
+
 // 3 -> 64 channels, 7x7, stride 2, pad 3: the shape conv_f32_stem.hip is written for.
 static bool stem_f32_shape(const ConvShape &s) {
   return s.group == 1 && s.C == 3 && s.K == 64 && s.R == 7 && s.S == 7 && s.sh == 2 && s.sw == 2 && s.ph == 3 && s.pw == 3;
@@ -324,7 +442,16 @@ static void *conv_f32_nchw(const dnnrtContext *ctx, const ConvShape &s, const fl
     dim3 grid((unsigned)blocks), block(256);
     const size_t lds = (size_t)s.C * s.R * s.S * 4 * sizeof(float);
     const int w_k = crsk ? 1 : s.C * s.R * s.S, w_tap = crsk ? s.K : 1;
-    if (s.R == 3)
+    const int q_log2 = s.Q > 32 ? 6 : s.Q > 16 ? 5 : 4;
+    const int64_t tiles = (int64_t)s.N * ceil_div(s.P, 256 >> q_log2) * ceil_div(s.Q, 1 << q_log2);
+    if (s.R == 3 && s.sh == 1 && s.sw == 1 && (int64_t)s.C * s.H * s.W < (1ll << 29) && tiles < (1 << 28)) {
+      grid = dim3((unsigned)(ceil_div(tiles, 8) * 8));
+#define NARROW(K_)                                                                                                                    \
+  case K_: hipLaunchKernelGGL((conv3x3_f32_narrow_kernel<K_>), grid, block, std::max<size_t>(lds, 4096 * K_), ctx->stream, X, Wt, bias, Z, Y, s.C, \
+                              s.H, s.W, s.P, s.Q, s.ph, s.pw, act, ctx->act_coef, w_k, w_tap, (int)tiles, q_log2); break
+      switch (s.K) { NARROW(1); NARROW(2); NARROW(3); default: NARROW(4); }
+#undef NARROW
+    } else if (s.R == 3)
       hipLaunchKernelGGL((conv_f32_narrow_kernel<4, 3, 3>), grid, block, lds, ctx->stream, X, Wt, bias, Z, Y, s.C, s.H, s.W, s.K,
                          s.P, s.Q, s.ph, s.pw, s.sh, s.sw, act, ctx->act_coef, w_k, w_tap);
     else

@@ -1734,6 +1734,28 @@ def test_conv_3x3_small_for_every_length_of_a_wavefronts_slice(gpu, geometry, Cc
         assert (np.abs(got - ref) <= (9 * Cc + 1) * 2.0 ** -24 * magnitude).all()
 
 
+# N, C, H, W, K, pad: patches cut by every border, fewer channels than wavefronts and odd numbers of them, every number of filters
+@pytest.mark.parametrize("case", [(1, 1, 1, 1, 1, 1), (2, 2, 17, 15, 2, 1), (1, 3, 16, 33, 3, 0), (2, 7, 20, 18, 4, 2), (1, 64, 90, 117, 3, 1), (3, 13, 5, 70, 1, 1)],
+                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("crsk", [False, True])
+def test_conv_f32_3x3_with_at_most_four_filters(gpu, cpu, case, crsk):
+    """Bound: each of the 9 C + 2 additions rounds by at most 2^-24 of the sum of magnitudes; a NaN stays in its windows."""
+    import torch
+    N, Cc, H, W, K, pad = case
+    r = rng(sum(case))
+    x = r.standard_normal((N, Cc, H, W)).astype(np.float32)
+    w = (r.standard_normal((K, Cc, 3, 3)) * np.sqrt(2.0 / (9 * Cc))).astype(np.float32)
+    b = r.uniform(-0.5, 0.5, K).astype(np.float32)
+    conv64 = lambda t, f, v: torch.nn.functional.conv2d(*(torch.from_numpy(u).double() for u in (t, f, v)), padding=pad).numpy()  # noqa: E731
+    ref, magnitude = conv64(x, w, b), conv64(np.abs(x), np.abs(w), np.abs(b))
+    z = r.standard_normal(ref.shape).astype(np.float32)
+    got = oc.conv(gpu, x, w, b, (pad, pad), (1, 1), 1, _abi.ACT_RELU, crsk=crsk, z=z, inplace=True)
+    assert (np.abs(got - np.maximum(ref + z, 0)) <= (9 * Cc + 2) * 2.0 ** -24 * (magnitude + np.abs(z))).all()
+    x[N - 1, Cc - 1, H // 2, W // 2] = np.nan
+    got, ref = oc.conv(gpu, x, w, b, (pad, pad), (1, 1), 1, _abi.ACT_IDENTITY, crsk=crsk), oc.conv(cpu, x, w, b, (pad, pad), (1, 1), 1, _abi.ACT_IDENTITY)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+
+
 def test_conv_3x3_by_minimal_filtering_keeps_infinities_in_their_place(gpu, cpu):
     """The transforms take differences within a 4x4 patch: an infinity, a NaN and values whose differences leave fp32's range
     must reach the results that use them and no others, as they do tap by tap."""
