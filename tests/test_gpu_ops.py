@@ -1288,6 +1288,42 @@ def test_first_layer_fp32_alone_and_with_its_max_pool(gpu, cpu, case, crsk, acti
     np.testing.assert_array_equal(got, gpu.get(Y2))
 
 
+# batches of many tiles, where workgroups walk down columns of tiles: one walk a column and several, walks that end in a
+# partial step, one-row and one-column edges, images of one step
+@pytest.mark.parametrize("case", [(32, 224, 224), (9, 130, 97), (40, 21, 230), (130, 8, 8), (3, 300, 300), (2, 448, 448)], ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("pool", [False, True])
+def test_first_layer_fp32_in_walks(gpu, case, pool):
+    """Against 64-bit sums: 148 additions, each rounding by at most 2^-24 of the sum of magnitudes (a maximum adds none); a NaN
+    reaches the windows that hold it and no others."""
+    import torch
+    N, H, W = case
+    g = torch.Generator().manual_seed(H)
+    x, w = torch.randn(N, 3, H, W, generator=g), torch.randn(64, 3, 7, 7, generator=g) * (2.0 / 147) ** 0.5
+    b = torch.rand(64, generator=g) * 0.6 - 0.5
+    x[N // 2, 1, H // 2, W // 3] = float("nan")
+    X, Wt, B = gpu.put(x.numpy()), gpu.put(w.numpy()), gpu.put(b.numpy())
+    P, Q = (H - 1) // 2 + 1, (W - 1) // 2 + 1
+    shape = (N, 64, (P - 1) // 2 + 1, (Q - 1) // 2 + 1) if pool else (N, 64, P, Q)
+    Y = gpu.empty(shape, np.float32)
+    if pool:
+        gpu.ops.conv_bias_activ_max_pool(gpu.ptr(X), x.shape, gpu.ptr(Wt), w.shape, gpu.ptr(B), (3, 3), (2, 2), _abi.ACT_IDENTITY,
+                                         (3, 3), (1, 1, 1, 1), (2, 2), gpu.ptr(Y), shape, dtype=_abi.F32)
+    else:
+        gpu.ops.conv_bias_activ(gpu.ptr(X), x.shape, gpu.ptr(Wt), w.shape, gpu.ptr(B), (3, 3), (2, 2), _abi.ACT_IDENTITY, gpu.ptr(Y))
+    gpu.sync()
+    got = torch.from_numpy(gpu.get(Y))
+    for n in sorted({0, N // 2, N - 1}):
+        ref = torch.nn.functional.conv2d(x[n:n + 1].double(), w.double(), b.double(), stride=2, padding=3)
+        bound = 148 * 2.0 ** -24 * torch.nn.functional.conv2d(x[n:n + 1].nan_to_num().abs().double(), w.abs().double(), b.abs().double(), stride=2, padding=3)
+        if pool:
+            nan = torch.nn.functional.max_pool2d(ref.isnan().float(), 3, 2, 1) > 0
+            ref, bound = torch.nn.functional.max_pool2d(ref.nan_to_num(nan=-1e30), 3, 2, 1), torch.nn.functional.max_pool2d(bound, 3, 2, 1)
+            ref[nan] = float("nan")
+        assert (got[n].isnan() == ref[0].isnan()).all()
+        ok = ~ref[0].isnan()
+        assert ((got[n] - ref[0]).abs()[ok] <= bound[0][ok]).all()
+
+
 def test_first_layer_fp32_with_its_max_pool_refuses_other_shapes(gpu):
     r = rng(4)
     x = r.standard_normal((1, 3, 32, 32)).astype(np.float32)
