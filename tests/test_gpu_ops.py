@@ -694,6 +694,23 @@ def test_transpose_rows_in_pairs(gpu, dims, perm, dtype):
     np.testing.assert_array_equal(oc.transpose(gpu, x, perm), x.transpose(perm))
 
 
+@pytest.mark.parametrize("case", [(9, 4, 10), (32, 2048, 1000), (33, 20, 31), (64, 1280, 70), (100, 512, 513), (11, 2052, 1)], ids=str)
+def test_matmul2d_f32_rows_of_the_right_operand(gpu, case):
+    """Batches of dozens against a right operand with its reduction in a row: ragged in both directions, split reductions and
+    none, every kind of C.  Bound: K + 3 roundings of at most 2^-24 of the sum of magnitudes."""
+    M, K, N = case
+    r = rng(sum(case))
+    a, b = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((N, K)).astype(np.float32)
+    c, row = r.standard_normal((M, N)).astype(np.float32), r.standard_normal(N).astype(np.float32)
+    ab, mag = a.astype(np.float64) @ b.T.astype(np.float64), np.abs(a).astype(np.float64) @ np.abs(b).T.astype(np.float64)
+    check = lambda got, ref, m: np.testing.assert_array_less(np.abs(got - ref), (K + 3) * 2.0 ** -24 * m + 1e-30)  # noqa: E731
+    for _ in range(2):  # twice: the split reduction's counters must be back at zero
+        check(oc.matmul2d(gpu, a, b, transB=1), ab, mag)
+        check(oc.matmul2d(gpu, a, b, c, 0.5, 2.0, transB=1), 0.5 * ab + 2.0 * c, 0.5 * mag + 2 * np.abs(c))
+        check(oc.matmul2d_row(gpu, a, b, row, transB=1), ab + row, mag + np.abs(row))
+        check(oc.matmul2d_row(gpu, a, b, row, 1.0, 0.25, transB=1), ab + 0.25 * row, mag + np.abs(row))
+
+
 @pytest.mark.parametrize("L", [1, 5, 63, 64, 65, 200])
 def test_every_lane_counts_once_in_sums_and_maxima_over_a_wavefront(gpu, L):
     """Rows with one element of weight: L * mean is exactly it wherever it lies, and a soft-max over -300 and one 0 is one-hot."""
