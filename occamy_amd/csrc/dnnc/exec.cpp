@@ -533,6 +533,12 @@ bool Session::place_constants(std::vector<UploadChunk> &chunks) const {
         if (c.first < 0) c.first = at;
         c.last = std::max(c.last, at);
       }
+      // A copy that is not made (the alias_copies pass) names the constant's own bytes as its result: they are read
+      // until the result's last reader, as live_slots has it for everything but constants.
+      if (op->result && !op->operands.empty()) {
+        const auto it = item_of.find(op->operands.back());
+        if (it != item_of.end()) item_of[op->result] = it->second;
+      }
       n++;
     }
   }
