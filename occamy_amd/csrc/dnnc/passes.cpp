@@ -274,7 +274,9 @@ void alias_copies(Program &p) {
 // at batch 64 the last convolution of a ResNet-50 first-stage block reads 129 MB and writes 103 MB, and with a
 // separate output what it leaves in the memory-side cache is no longer the whole tensor the next layer reads.
 // Not done when the residual's buffer is also the convolution's input, or is used (a reader of anything written
-// there, a copy to the host) after the call.  The reference
+// there, a copy to the host) after the call, or holds what the host sent (a constant or an argument behind a copy that
+// alias_copies took away: a resident session uploads constants once, and a run in place reads arguments at the caller's
+// address).  The reference
 // has no such pattern (src/Transform/DNN/mallocPoolOpt.cpp places every result in a slot of its own).
 void inplace_residual(Program &p) {
   std::vector<Op *> closers;
@@ -298,6 +300,7 @@ void inplace_residual(Program &p) {
     for (const auto &u : zbuf->uses) {  // direct users of the buffer: whoever wrote it (the residual's producer last), copies, the dealloc
       if (u.first == m || u.first->kind == OP_DEALLOC) continue;
       if (p.order(u.first) > at) ok = false;
+      if (u.first->kind == OP_MEMCPY && u.first->mode == 1 && u.second == 0) ok = false;  // sent by the host
       const bool writes = u.first->kind != OP_MEMCPY && !u.first->operands.empty() && u.first->operands.back() == zbuf;
       if (writes && u.first->result)
         for (const auto &r : u.first->result->uses)  // readers of what was written there

@@ -347,6 +347,34 @@ def test_ssd_resnet50_program():
         np.testing.assert_allclose(y, x, rtol=1e-4, atol=1e-4 * float(np.abs(x).max()))
 
 
+@pytest.mark.parametrize("residual", ["constant", "argument"])
+@pytest.mark.parametrize("flags", [dict(), dict(compact_pool=True)])
+def test_inplace_residual_leaves_what_the_host_sent(residual, flags):
+    """A residual that is a reshaped constant or argument, the reshape not being made: the sum does not go over the
+    constant, which a resident session uploads once, nor over the argument, which a run in place reads at the caller's."""
+    rng = np.random.default_rng(12)
+    g = compiler.Graph()
+    values = [rng.standard_normal(s).astype(np.float32) for s in ((1, 4, 8, 8), (4, 64))]
+    x = g.input("x", values[0].shape)
+    sent = g.input("z", values[1].shape) if residual == "argument" else g.constant(values[1])
+    z = g.node("Reshape", [sent, g.constant(np.array([1, 4, 8, 8], np.int64))])
+    conv = lambda y: g.node("Conv", [y, g.constant((rng.standard_normal((4, 4, 3, 3)) / 5).astype(np.float32)),  # noqa: E731
+                                     g.constant(rng.standard_normal(4).astype(np.float32))], kernel_shape=[3, 3], pads=[1] * 4, strides=[1, 1], group=1)
+    y = g.node("Relu", [g.node("Add", [conv(x), z])])
+    g.output(g.node("Relu", [conv(y)]))
+    inputs = values if residual == "argument" else values[:1]
+    want = graph_eval.evaluate(g, inputs)[0]
+    p = g.compile(fusion=True, fuse_residual=True, alias_copies=True, inplace_residual=True, **flags)
+    call, = [line for line in p.text.splitlines() if "conv-bias-add" in line]
+    operands = call.split("dnn.")[1].split("{")[0].replace(",", " ").split()[1:]
+    assert [line.split()[1:3] for line in p.text.splitlines() if line.startswith("dnn.memcpy " + operands[-1] + ",")] == []
+    for mode in (compiler.MODE_OCCAMY, compiler.MODE_RESIDENT):
+        s = p.session(mode, runtime_library=ORACLE_PATH)
+        for _ in range(3):
+            np.testing.assert_allclose(s.run(*inputs)[0], want, rtol=1e-4, atol=1e-5)
+        s.close()
+
+
 def test_compact_pool_changes_nothing():
     """Offsets from the planner that knows every lifetime: the same bits from the oracle, per inference with a
     poisoned pool and resident, for ResNet-50 with every fusion, MobileNetV2, BERT and YOLOv1."""
