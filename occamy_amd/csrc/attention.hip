@@ -369,21 +369,13 @@ __global__ __launch_bounds__(64 * NW) void attention_f16_kernel(const _Float16 *
   }
 }
 
-// More than 64 KiB of dynamic LDS must be asked for once per kernel.
-template <typename F>
-static void raise_lds(F *kernel, size_t lds, bool &raised) {
-  if (raised) return;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  raised = true;
-}
-
 template <int DH>
 static void launch_attention(const dnnrtContext *ctx, const float *Q, const float *K, const float *V, float *Y, int B,
                              int Sq, int Sk, int H, int ld_in, float scale) {
   constexpr int ROW = DH + 4;
   const size_t lds = (size_t)((ATT_QB + 2 * ATT_KB) * ROW + 8 * 32) * sizeof(float);
-  static bool raised = false;
-  raise_lds(&attention_kernel<DH>, lds, raised);
+  static LdsRaised raised;
+  (void)raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&attention_kernel<DH>), (int)lds);  // refused: the launch says so
   hipLaunchKernelGGL((attention_kernel<DH>), dim3((unsigned)ceil_div(Sq, ATT_QB), (unsigned)H, (unsigned)B), dim3(256),
                      lds, ctx->stream, Q, K, V, Y, Sq, Sk, ld_in, H * DH, scale);
 }
@@ -393,8 +385,8 @@ static void launch_attention_f16(const dnnrtContext *ctx, const __half *Q, const
                                  int Sq, int Sk, int H, int ld_in, float scale) {
   const size_t lds = (size_t)NW * 32 * (DH + 4 + 2) * sizeof(float);  // the partial results; the V tiles lie under them
   static_assert((DH + 8) * 2 <= (DH + 4) * 4, "V tiles fit");
-  static bool raised = false;
-  raise_lds(&attention_f16_kernel<DH, NW, WIDE>, lds, raised);
+  static LdsRaised raised;
+  (void)raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&attention_f16_kernel<DH, NW, WIDE>), (int)lds);
   hipLaunchKernelGGL((attention_f16_kernel<DH, NW, WIDE>), dim3((unsigned)ceil_div(Sq, 32), (unsigned)H, (unsigned)B), dim3(64 * NW), lds, ctx->stream,
                      (const _Float16 *)Q, (const _Float16 *)K, (const _Float16 *)V, (_Float16 *)Y, Sq, Sk, ld_in, H * DH, scale);
 }

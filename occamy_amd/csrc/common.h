@@ -9,6 +9,7 @@
 #include <stdio.h>
 
 #include "../../include/dnnrt.h"
+#include "lds_limit.h"
 
 struct dnnrtContext {
   hipStream_t stream;  // kernels of this handle are launched here

@@ -417,14 +417,10 @@ bool block_f16_applies(const dnnrtContext *ctx, const dnnrtExecBlock &k) {
 
 template <int S, int KC, int GM>
 static bool launch_one(const dnnrtContext *ctx, dim3 grid, dim3 threads, size_t lds, const BlockF16Args &a) {
-  static bool raised[16] = {};
-  if (ctx->device < 0 || ctx->device >= 16) { set_error("inverted residual block (fp16): device ordinal %d", ctx->device); return false; }
-  if (!raised[ctx->device]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&conv_f16_block_kernel<S, KC, GM>), hipFuncAttributeMaxDynamicSharedMemorySize, BLOCK_LDS) != hipSuccess) {
-      set_error("inverted residual block (fp16): cannot reserve %d bytes of LDS", BLOCK_LDS);
-      return false;
-    }
-    raised[ctx->device] = true;
+  static LdsRaised raised;
+  if (!raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&conv_f16_block_kernel<S, KC, GM>), BLOCK_LDS)) {
+    set_error("inverted residual block (fp16): cannot reserve %d bytes of LDS", BLOCK_LDS);
+    return false;
   }
   hipLaunchKernelGGL((conv_f16_block_kernel<S, KC, GM>), grid, threads, lds, ctx->stream, a);
   return true;

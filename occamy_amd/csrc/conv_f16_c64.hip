@@ -280,15 +280,10 @@ bool launch_conv_f16_c64(const dnnrtContext *ctx, const ConvF16Args &a) {
   int patch_px = (int)ceil_div(4 * (a.W + 2), 8) * 8;
   while (c64_lds_bytes(patch_px, a.W) - 64 * 2 - patch_px * 128 < 36 * 1024) patch_px += 8;
   const int smem = c64_lds_bytes(patch_px, a.W);
-  static bool raised[16] = {};
-  if (ctx->device < 0 || ctx->device >= 16) { set_error("conv(fp16): device ordinal %d", ctx->device); return false; }
-  if (!raised[ctx->device]) {  // more than 64 KiB of LDS has to be asked for, once per device (the largest any width needs)
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&conv3x3_f16_c64_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            c64_lds_bytes(256, 62)) != hipSuccess) {
-      set_error("conv(fp16): cannot reserve %d bytes of LDS", c64_lds_bytes(256, 62));
-      return false;
-    }
-    raised[ctx->device] = true;
+  static LdsRaised raised;  // the largest that any width needs
+  if (!raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&conv3x3_f16_c64_kernel), c64_lds_bytes(256, 62))) {
+    set_error("conv(fp16): cannot reserve %d bytes of LDS", c64_lds_bytes(256, 62));
+    return false;
   }
   hipLaunchKernelGGL(conv3x3_f16_c64_kernel, dim3((unsigned)workers, (unsigned)tiles_m), dim3(256), (size_t)smem, ctx->stream, am,
                      tiles_n, tiles_per_image, magic_of(tiles_per_image), patch_px);

@@ -422,19 +422,13 @@ __global__ __launch_bounds__(64 * WM * WN) void conv_f16_dma_kernel(const ConvF1
 #endif
 }
 
-// More than 64 KiB of LDS per workgroup has to be asked for, once per kernel and device.
 template <int BM, int BN, int WM, int WN, int NS, bool MASKED, bool DUAL = false>
 static bool launch_dma_masked(const dnnrtContext *ctx, const ConvF16Args &a, unsigned grid, int tiles) {
   constexpr int SMEM = NS * (BM + BN) * 128;
-  static bool raised[16] = {};
-  if (ctx->device < 0 || ctx->device >= 16) { set_error("conv(fp16): device ordinal %d", ctx->device); return false; }
-  if (!raised[ctx->device]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&conv_f16_dma_kernel<BM, BN, WM, WN, NS, MASKED, DUAL>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) {
-      set_error("conv(fp16): cannot reserve %d bytes of LDS", SMEM);
-      return false;
-    }
-    raised[ctx->device] = true;
+  static LdsRaised raised;
+  if (!raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&conv_f16_dma_kernel<BM, BN, WM, WN, NS, MASKED, DUAL>), SMEM)) {
+    set_error("conv(fp16): cannot reserve %d bytes of LDS", SMEM);
+    return false;
   }
   hipLaunchKernelGGL((conv_f16_dma_kernel<BM, BN, WM, WN, NS, MASKED, DUAL>), dim3(grid), dim3(64 * WM * WN), SMEM, ctx->stream, a, tiles);
   return true;

@@ -423,15 +423,10 @@ static bool launch_patch(const dnnrtContext *ctx, const ConvF16Args &a, bool onl
   const int64_t NPQ = (int64_t)a.N * a.P * a.Q;
   const int64_t tiles = ceil_div(a.K, BM) * ceil_div(NPQ, BN);
   if (tiles + 8 > INT32_MAX) { set_error("conv(fp16): too many tiles"); return false; }
-  static bool raised[16] = {};
-  if (ctx->device < 0 || ctx->device >= 16) { set_error("conv(fp16): device ordinal %d", ctx->device); return false; }
-  if (!raised[ctx->device]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&conv3x3_f16_patch_kernel<BM, BN, WM, WN, KG, PCAP, NS>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) {
-      set_error("conv(fp16): cannot reserve %d bytes of LDS", SMEM);
-      return false;
-    }
-    raised[ctx->device] = true;
+  static LdsRaised raised;
+  if (!raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&conv3x3_f16_patch_kernel<BM, BN, WM, WN, KG, PCAP, NS>), SMEM)) {
+    set_error("conv(fp16): cannot reserve %d bytes of LDS", SMEM);
+    return false;
   }
   ConvF16Args am = a;
   am.magic_pw = magic_of(a.W + 2);

@@ -479,14 +479,10 @@ bool launch_conv_f32_winograd(const dnnrtContext *ctx, const IgemmArgs &args, do
   launched = true;
   const unsigned grid = (unsigned)(pl.units + ceil_div(pl.whole, 8) * 8);
   const auto kernel = av4 ? conv_f32_winograd_kernel<4> : conv_f32_winograd_kernel<1>;
-  static bool raised[16][2] = {};  // more than 64 KiB of LDS has to be asked for, once per kernel and device
-  if (ctx->device < 0 || ctx->device >= 16) { set_error("conv(fp32, winograd): device ordinal %d", ctx->device); return false; }
-  if (!raised[ctx->device][av4]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, W32_SMEM) != hipSuccess) {
-      set_error("conv(fp32, winograd): cannot reserve %d bytes of LDS", W32_SMEM);
-      return false;
-    }
-    raised[ctx->device][av4] = true;
+  static LdsRaised raised[2];
+  if (!raise_lds(raised[av4], ctx->device, reinterpret_cast<const void *>(kernel), W32_SMEM)) {
+    set_error("conv(fp32, winograd): cannot reserve %d bytes of LDS", W32_SMEM);
+    return false;
   }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), W32_SMEM, ctx->stream, a, pl, ctx->splitk_partials, ctx->splitk_counters);
   const hipError_t e = hipGetLastError();

@@ -354,15 +354,12 @@ static bool launch_gd(const dnnrtContext *ctx, const GemmF16Args &g, int Z, int 
   const int64_t tiles = ceil_div(g.M, FM) * ceil_div(g.N, FN);
   const bool kc = g.b_sk == 1;
   if (SMEM > 64 * 1024) {
-    static bool raised[16] = {};  // more than 64 KiB of LDS has to be asked for, once per kernel and device
-    if (ctx->device < 0 || ctx->device >= 16) { set_error("matmul(fp16): device ordinal %d", ctx->device); return false; }
-    if (!raised[ctx->device]) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_f16_dma_kernel<FN, FM, WN, WM, NS, true>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess ||
-          hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_f16_dma_kernel<FN, FM, WN, WM, NS, false>), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM) != hipSuccess) {
-        set_error("matmul(fp16): cannot reserve %d bytes of LDS", SMEM);
-        return false;
-      }
-      raised[ctx->device] = true;
+    static LdsRaised raised[2];
+    const void *kernel = kc ? reinterpret_cast<const void *>(&gemm_f16_dma_kernel<FN, FM, WN, WM, NS, true>)
+                            : reinterpret_cast<const void *>(&gemm_f16_dma_kernel<FN, FM, WN, WM, NS, false>);
+    if (!raise_lds(raised[kc], ctx->device, kernel, SMEM)) {
+      set_error("matmul(fp16): cannot reserve %d bytes of LDS", SMEM);
+      return false;
     }
   }
   const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8), (unsigned)splits, (unsigned)Z), block(64 * WN * WM);
