@@ -356,38 +356,69 @@ __global__ __launch_bounds__(256, 2) void conv_f32_winograd_kernel(const IgemmAr
     x = x < 0.f ? below : x;
     return x > ceiling ? ceiling : x;
   };
-  // What is not finite here is computed again, tap by tap: differences of infinities, and sums that left fp32's range,
-  // are none of the convolution's, and they spread over a tile.
-  auto direct = [&](int row, int q) -> float {
-    float s = 0.f;
-    const float *w = a.A + row, *x = a.X + img * a.x_img_stride;
-    for (int r = 0; r < 3; r++)
-      for (int u = 0; u < 3; u++) {
-        const int ih = p_out - a.ph + r, iw = q - a.pw + u;
-        if ((unsigned)ih >= (unsigned)a.H || (unsigned)iw >= (unsigned)a.W) continue;
-#pragma unroll 4
-        for (int c = 0; c < C; c++) s = fmaf(w[(int64_t)(c * 9 + r * 3 + u) * a.a_ld], x[(int64_t)c * HW + ih * a.W + iw], s);
-      }
-    return s;
-  };
-  unsigned top = 0;
+  // What is not finite here is computed again, tap by tap: differences of infinities, and sums that left fp32's range, are
+  // none of the convolution's, and they spread over a tile.  The wavefront takes their pixels one by one, sixteen lanes to a
+  // channel, a lane for each filter; finite results keep their bits, and once every sum is a NaN nothing more is read.
+  // 1024 -> 324 channels at 38x38, three images, 184 us: with one NaN 198, an image of NaN 396, one infinity 1020.  (A lane
+  // to a channel, 64 lines an instruction: 232, 833, 8870.  Every result of such a wavefront by its own lane: 28 ms each.)
+  unsigned wrong[2] = {0, 0};  // bit i: filter row0 + i of pixel j
 #pragma unroll
   for (int i = 0; i < 16; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) top = max(top, __builtin_bit_cast(unsigned, v[i][j]) & 0x7fffffffu);
-  if (__any(top >= 0x7f800000u)) {
+    for (int j = 0; j < 2; j++)
+      if ((__builtin_bit_cast(unsigned, v[i][j]) & 0x7fffffffu) >= 0x7f800000u && (j ? ok1 : ok0) && row0 + i < a.M) wrong[j] |= 1u << i;
+  if (__any((wrong[0] | wrong[1]) != 0)) {
+    // in this wavefront's own rows of what it read above, behind the word of the hand-over: [pixel][filter][lane]
+    float *there = reinterpret_cast<float *>(smem + W32_TILE * 2 + 16 * wave * W32_BT * 8) + lane;
+    constexpr int PIXEL = W32_TILE * 2 / 4;
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) there[j * PIXEL + 64 * i] = v[i][j];
 #pragma unroll 1
-    for (int i = 0; i < 16; i++) {
-      if (row0 + i >= a.M) break;
+    for (int j = 0; j < 2; j++) {
+      const unsigned mine = j ? wrong[1] : wrong[0];
 #pragma unroll 1
-      for (int j = 0; j < 2; j++) {
-        if (!(j ? ok1 : ok0)) continue;
-        float x = direct(row0 + i, q_out + j) + (a.bias ? a.bias[row0 + i] : 0.f);
-        if (a.Cin) x += a.Cin[at + j + (int64_t)(row0 + i) * a.c_row_stride];
-        a.Y[at + j + (int64_t)(row0 + i) * a.y_row_stride] = apply_act(x, a.act, a.act_coef);
+      for (uint64_t pixels = __ballot(mine != 0); pixels; pixels &= pixels - 1) {
+        const int l = __builtin_ctzll(pixels);
+        const int ih0 = __builtin_amdgcn_readlane(p_out, l) - a.ph, iw0 = __builtin_amdgcn_readlane(q_out, l) + j - a.pw;
+        const bool wanted = ((unsigned)__builtin_amdgcn_readlane((int)mine, l) >> (lane & 15)) & 1;
+        const float *x = a.X + __builtin_amdgcn_readlane(img, l) * a.x_img_stride, *w = a.A + min(row0 + (lane & 15), a.M - 1);
+        float s = 0.f, sum = 0.f;
+#pragma unroll 1
+        for (int c0 = 0; c0 < C; c0 += 8) {
+          float xs[2][9], ws[2][9];
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            const int64_t c = min(c0 + 4 * u + (lane >> 4), C - 1);
+#pragma unroll
+            for (int k = 0; k < 9; k++) {
+              xs[u][k] = x[c * HW + min(max(ih0 + k / 3, 0), a.H - 1) * a.W + min(max(iw0 + k % 3, 0), a.W - 1)];
+              ws[u][k] = w[(c * 9 + k) * a.a_ld];
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int k = 0; k < 9; k++) {
+              const bool in = (unsigned)(ih0 + k / 3) < (unsigned)a.H && (unsigned)(iw0 + k % 3) < (unsigned)a.W && c0 + 4 * u < C;
+              s = in ? fmaf(ws[u][k], xs[u][k], s) : s;  // what is outside the image is no 0 to be multiplied
+            }
+          sum = s + __shfl_xor(s, 16);
+          sum += __shfl_xor(sum, 32);
+          if (__all(!wanted || __builtin_isnan(sum))) break;
+        }
+        for (unsigned rows = (unsigned)__builtin_amdgcn_readlane((int)mine, l); rows; rows &= rows - 1) {
+          const int i = __builtin_ctz(rows);
+          const float of_i = __shfl(sum, i);
+          if (lane == l) there[j * PIXEL + 64 * i] = of_i;
+        }
       }
     }
-    return;
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) v[i][j] = there[j * PIXEL + 64 * i];
   }
   const bool full = row0 + 16 <= a.M, pairs = __all(!ok0 || ok1);  // every lane's two pixels are in the image
   float *__restrict__ Y = a.Y + at + (int64_t)row0 * a.y_row_stride;

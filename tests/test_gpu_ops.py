@@ -1831,3 +1831,44 @@ def test_conv_3x3_by_minimal_filtering_keeps_infinities_in_their_place(gpu, cpu)
     np.testing.assert_allclose(got[ok], ref[ok], rtol=RTOL, atol=ATOL)
     far = np.isfinite(ref[3]) & (np.abs(ref[3]) > 1e30)
     np.testing.assert_allclose(got[3][far], ref[3][far], rtol=RTOL)
+
+
+@pytest.mark.parametrize("case", [(7, 64, 56, 56, 64), (11, 64, 56, 56, 64), (3, 512, 19, 19, 486), (2, 512, 28, 28, 256)], ids=["whole", "rest-split", "odd-rows", "split"])
+def test_conv_3x3_by_minimal_filtering_recomputes_only_what_is_not_finite(gpu, case):
+    """A NaN or an infinity reaches the results whose windows hold it, and of the finite results only those of the same 2x2
+    tiles may change a bit; with a whole image of NaN, the other images keep theirs."""
+    import torch
+    N, Cc, H, W, K = case
+    r = rng(Cc)
+    x = np.maximum(r.standard_normal((N, Cc, H, W)), 0).astype(np.float32)
+    w = (r.standard_normal((K, Cc, 3, 3)) * np.sqrt(2.0 / (9 * Cc))).astype(np.float32)
+    w[2, 0] = w[2, Cc - 1] = 0
+    b = r.uniform(-0.5, 0.5, K).astype(np.float32)
+    run = lambda t, f=w: oc.conv(gpu, t, f, b, (1, 1), (1, 1), 1, _abi.ACT_IDENTITY, crsk=True)  # noqa: E731
+    conv64 = lambda t, f=w: torch.nn.functional.conv2d(*(torch.from_numpy(u).double() for u in (t, f, b)), padding=1).numpy()  # noqa: E731
+    plain = run(x)
+    for value in (np.nan, np.inf):
+        y = x.copy()
+        y[1, Cc - 1, 10, 7] = value
+        y[0, 0, 0, 0] = value
+        got, ref = run(y), conv64(y)
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+        np.testing.assert_array_equal(np.isposinf(got), np.isposinf(ref))
+        np.testing.assert_array_equal(np.isneginf(got), np.isneginf(ref))
+        tiles = np.zeros((N, 1, H, W), bool)
+        tiles[1, :, 8:12, 6:10] = True  # the tiles whose patches hold row 10, column 7
+        tiles[0, :, 0:2, 0:2] = True
+        tiles = np.broadcast_to(tiles, plain.shape)
+        np.testing.assert_array_equal(got[~tiles], plain[~tiles])
+        ok = np.isfinite(ref)
+        np.testing.assert_allclose(got[ok], ref[ok], rtol=RTOL, atol=ATOL)
+    y = x.copy()
+    y[1] = np.nan
+    got = run(y)
+    assert np.isnan(got[1]).all()
+    np.testing.assert_array_equal(np.delete(got, 1, 0), np.delete(plain, 1, 0))
+    f = w.copy()
+    f[3, 5, 1, 1] = np.nan
+    got = run(x, f)
+    assert np.isnan(got[:, 3]).all()
+    np.testing.assert_array_equal(np.delete(got, 3, 1), np.delete(plain, 3, 1))
