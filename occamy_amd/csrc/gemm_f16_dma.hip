@@ -46,7 +46,9 @@ __device__ __forceinline__ void gd_barrier() {
 #if __HIP_DEVICE_COMPILE__
 // ds_read_b64_tr_b16 at LDS address `at` + OFFSET.  By hand: ahead of the builtin the compiler waits for every load into LDS
 // that is still on its way (vmcnt 0), and so for the whole ring.  It knows nothing of this read either: the value is there
-// behind the next wait for lgkmcnt, and gd_arrived() ties it to that place.
+// behind the next wait for lgkmcnt, and gd_arrived() ties its uses to that place.  Nothing keeps the compiler from copying or
+// spilling the register in between; that it does not, along every branch, is looked up in its output by
+// tests/test_untracked_reads.py, which is to be run again with another compiler.
 template <int OFFSET>
 __device__ __forceinline__ gd_short4 gd_read_tr(unsigned at) {
   gd_short4 v;
@@ -192,10 +194,14 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
     constexpr int S = decltype(set_c)::value;
     constexpr bool FULL = decltype(full_c)::value;
     // the next step has landed, NS - 2 behind it may still be on their way; this one's operands are here
-    if (FULL) gd_wait<(NS - 2) * L, 0>();
-    else if (NS > 3 && ahead > 2) gd_wait<(NS > 3 ? 2 : 0) * L, 0>();
-    else if (NS > 2 && ahead > 1) gd_wait<(NS > 2 ? 1 : 0) * L, 0>();
-    else gd_wait<0, 0>();
+    if (FULL) {
+      gd_wait<(NS - 2) * L, 0>();
+    } else {
+      gd_wait<63, 0>();  // whatever the branches below
+      if (NS > 3 && ahead > 2) gd_wait<(NS > 3 ? 2 : 0) * L>();
+      else if (NS > 2 && ahead > 1) gd_wait<(NS > 2 ? 1 : 0) * L>();
+      else gd_wait<0>();
+    }
     if constexpr (!B_KC) {
 #pragma unroll
       for (int sub = 0; sub < 4; sub++)
@@ -246,6 +252,10 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
       step_body(set1, std::false_type{}, ahead - 1);
     }
     if (ahead == 0) step_body(set0, std::false_type{}, 0);
+  }
+  if constexpr (!B_KC) {
+    gd_wait<63, 0>();  // no read is on its way, whatever the branches above: the registers are free
+    __builtin_amdgcn_sched_barrier(0);
   }
   gd_barrier();  // nobody reads the operand stages any more
 

@@ -44,7 +44,9 @@ __device__ __forceinline__ void gw_wait_lgkm() {
 #if __HIP_DEVICE_COMPILE__
 // ds_read_b64_tr_b16 at LDS address `at` + OFFSET.  By hand: ahead of the builtin the compiler waits for every load into LDS
 // that is still on its way (vmcnt 0), and so for the whole ring.  It knows nothing of this read either: the value is there
-// behind the next wait for lgkmcnt, and gw_arrived() ties it to that place.
+// behind the next wait for lgkmcnt, and gw_arrived() ties its uses to that place.  Nothing keeps the compiler from copying or
+// spilling the register in between; that it does not, along every branch, is looked up in its output by
+// tests/test_untracked_reads.py, which is to be run again with another compiler.
 template <int OFFSET>
 __device__ __forceinline__ gw_short4 gw_read_tr(unsigned at) {
   gw_short4 v;
@@ -235,6 +237,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
       step(c1, ahead - 1);
     }
     if (ahead == 0) step(c0, 0);
+  }
+  if constexpr (!B_KC) {
+    gw_wait_lgkm();  // no read is on its way, whatever the branches above: the registers are free
+    __builtin_amdgcn_sched_barrier(0);
   }
 
   // ---- the four wavefronts' sums meet in LDS: [m][n] in fp32, 16-byte chunk c of row m at c ^ (m & 15) ----
