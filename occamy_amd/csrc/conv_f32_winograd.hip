@@ -361,13 +361,18 @@ __global__ __launch_bounds__(256, 2) void conv_f32_winograd_kernel(const IgemmAr
   // channel, a lane for each filter; finite results keep their bits, and once every sum is a NaN nothing more is read.
   // 1024 -> 324 channels at 38x38, three images, 184 us: with one NaN 198, an image of NaN 396, one infinity 1020.  (A lane
   // to a channel, 64 lines an instruction: 232, 833, 8870.  Every result of such a wavefront by its own lane: 28 ms each.)
-  unsigned wrong[2] = {0, 0};  // bit i: filter row0 + i of pixel j
+  unsigned top = 0;
 #pragma unroll
   for (int i = 0; i < 16; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++)
-      if ((__builtin_bit_cast(unsigned, v[i][j]) & 0x7fffffffu) >= 0x7f800000u && (j ? ok1 : ok0) && row0 + i < a.M) wrong[j] |= 1u << i;
-  if (__any((wrong[0] | wrong[1]) != 0)) {
+    for (int j = 0; j < 2; j++) top = max(top, __builtin_bit_cast(unsigned, v[i][j]) & 0x7fffffffu);
+  if (__any(top >= 0x7f800000u)) {
+    unsigned wrong[2] = {0, 0};  // bit i: filter row0 + i of pixel j
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        if (!(__builtin_fabsf(v[i][j]) < __builtin_inff()) && (j ? ok1 : ok0) && row0 + i < a.M) wrong[j] |= 1u << i;
     // in this wavefront's own rows of what it read above, behind the word of the hand-over: [pixel][filter][lane]
     float *there = reinterpret_cast<float *>(smem + W32_TILE * 2 + 16 * wave * W32_BT * 8) + lane;
     constexpr int PIXEL = W32_TILE * 2 / 4;
