@@ -82,6 +82,10 @@ typedef struct {
                              before it places anything (largest tensor first, lowest free offset) instead of the
                              reference's first fit in program order; the pool is then usually the bytes alive at
                              once.  dnncProgramPoolBytes is that pool, not the reference's maxAllocByte (default 0) */
+  int32_t direct_convolutions; /* no reference flag: fp32 convolutions get DNNRT_CONV_ALGO_DIRECT as their `algo` operand
+                             (include/dnnrt.h): no minimal filtering, for activations that are mostly zero or whose
+                             values differ by many orders of magnitude (default 0: only those whose filters
+                             are mostly zero get it) */
 } dnncOptions;
 /* the graph must outlive the program: constants are not copied again */
 dnncProgram *dnncCompile(dnncGraph *g, const dnncOptions *opt);

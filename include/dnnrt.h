@@ -84,8 +84,8 @@ enum { DNNRT_REDUCE_AVG = 5 };
 /* memcpy kinds (src/Dialect/DNN/DNN.td:61-83). */
 enum { DNNRT_H2D = 1, DNNRT_D2H = 2, DNNRT_D2D = 3 };
 
-/* `algo` operand of the convolution calls: BASE + a variant id of dnnrtListConvTiles */
-enum { DNNRT_CONV_ALGO_BASE = 1000 };
+/* `algo` operand of the convolution calls: BASE + a variant id of dnnrtListConvTiles (fp16), or DIRECT (fp32) */
+enum { DNNRT_CONV_ALGO_BASE = 1000, DNNRT_CONV_ALGO_DIRECT = 2000 };
 
 /* ---- handle / stream ------------------------------------------------- */
 
@@ -202,9 +202,17 @@ int32_t dnnrtHostFree(void *ptr);
  * (src/Conversion/ONNXToDNN/ONNXToDNNCommonCUDA.cu:57-111, Ops/cudnn/Conv.cpp:82-83).
  * Here DNNRT_CONV_ALGO_BASE + id names the fp16 channels-last variant `id` of
  * dnnrtListConvTiles: the call uses it where it can run the problem, and the
- * automatic choice otherwise, as for every other value of `algo` (cuDNN's
+ * automatic choice otherwise, as for every other value of `algo` but one (cuDNN's
  * numbers name nothing here).  Every variant gives results to the same
- * tolerance; a handle's dnnrtSetConvTile goes first. */
+ * tolerance; a handle's dnnrtSetConvTile goes first.
+ * DNNRT_CONV_ALGO_DIRECT: fp32 results are sums of the products of input and
+ * filter values themselves, each within (9 C + 1) 2^-24 of the sum of their
+ * magnitudes for a 3x3 filter over C channels.  The automatic choice computes
+ * large 3x3 convolutions with stride 1 by minimal filtering instead, whose
+ * operands are rounded sums over a 4x4 patch and over the filter's nine values:
+ * the error against exact sums is smaller in the 2-norm for dense values (0.7 to
+ * 0.8), but larger for activations or filters that are nearly all zero (1.2 to 1.6
+ * times), and a result is only as exact as the largest values of its patch allow. */
 void *dnnrtConv(dnnrtHandle_t handle, const void *X, const int64_t *dimX,
                 const void *W, const int64_t *dimW, void *workspace,
                 int64_t workspaceBytes, int64_t algo, int64_t group,

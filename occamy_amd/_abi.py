@@ -91,6 +91,7 @@ OP_ADD, OP_MUL, OP_SQRT = 0, 1, 4
 REDUCE_AVG = 5
 H2D, D2H, D2D = 1, 2, 3
 CONV_ALGO_BASE = 1000
+CONV_ALGO_DIRECT = 2000
 
 
 def bind(cdll):

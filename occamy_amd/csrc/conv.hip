@@ -399,7 +399,7 @@ static bool stem_f32_shape(const ConvShape &s) {
 }
 
 static void *conv_f32_nchw(const dnnrtContext *ctx, const ConvShape &s, const float *X,
-                           const float *Wt, const float *bias, const float *Z, int act, float *Y) {
+                           const float *Wt, const float *bias, const float *Z, int act, float *Y, bool direct_sums) {
   // Filter storage: K,C,R,S (the reference's) or C,R,S,K (k_out contiguous),
   // which lets 32 lanes that own 32 consecutive output channels read one
   // contiguous 128-byte line per reduction element.
@@ -487,6 +487,7 @@ static void *conv_f32_nchw(const dnnrtContext *ctx, const ConvShape &s, const fl
   a.b_kcontig = false; a.a_mcontig = crsk;
   a.a_vec4 = !crsk && (a.Kdim % 4 == 0) && aligned16(Wt);
   a.b_vec4 = false;
+  a.direct_sums = direct_sums;
   if (!launch_igemm_f32(ctx, a)) return nullptr;
   return Y;
 }
@@ -494,6 +495,7 @@ static void *conv_f32_nchw(const dnnrtContext *ctx, const ConvShape &s, const fl
 // The `algo` operand of the convolution calls: DNNRT_CONV_ALGO_BASE + id asks for the fp16 channels-last variant
 // `id` of dnnrtListConvTiles where that variant can run the problem (else, and for every other value, the
 // automatic choice).  Values below the base are cuDNN's algorithm numbers, which name nothing here.
+// DNNRT_CONV_ALGO_DIRECT keeps fp32 calls off minimal filtering.
 static int variant_of_algo(int64_t algo) {
   if (algo <= DNNRT_CONV_ALGO_BASE || algo >= DNNRT_CONV_ALGO_BASE + 1000) return 0;
   const int id = (int)(algo - DNNRT_CONV_ALGO_BASE);
@@ -514,7 +516,8 @@ static void *conv_dispatch(const char *who, dnnrtHandle_t h, const void *X, cons
   if (!parse_conv(who, dX, dW, group, pads, strides, s)) return nullptr;
   if (dtype == DNNRT_F32) {
     if (h->format != DNNRT_NCHW) DNNRT_FAIL("%s: fp32 tensors are NCHW only", who);
-    return conv_f32_nchw(h, s, (const float *)X, (const float *)W, (const float *)B, (const float *)Z, act, (float *)Y);
+    return conv_f32_nchw(h, s, (const float *)X, (const float *)W, (const float *)B, (const float *)Z, act, (float *)Y,
+                         algo == DNNRT_CONV_ALGO_DIRECT);
   }
   if (dtype == DNNRT_F16) {
     ConvF16Args a{};

@@ -604,8 +604,8 @@ bool launch_conv_f32_dma(const dnnrtContext *ctx, const IgemmArgs &args, double 
       }
     }
   }
-  // 3x3 layers with stride 1: by Winograd's method where that is estimated to be faster
-  if (!launch_conv_f32_winograd(ctx, args, best_shape < 0 || best > at_most_us ? at_most_us : best, launched)) return false;
+  // 3x3 layers with stride 1: by Winograd's method where that is estimated to be faster and the caller has not asked for direct sums
+  if (!a.direct_sums && !launch_conv_f32_winograd(ctx, args, best_shape < 0 || best > at_most_us ? at_most_us : best, launched)) return false;
   if (launched) return true;
   if (best_shape < 0 || best > at_most_us) return true;
   pl.magic_tiles_m = magic_of(pl.tiles_m);

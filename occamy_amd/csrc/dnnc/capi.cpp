@@ -130,6 +130,7 @@ dnncProgram *dnncCompile(dnncGraph *g, const dnncOptions *opt) {
   func_args_to_device(p);
   erase_dummy_constants(p);
   p.channels_last_requested = opt->channels_last != 0;
+  p.direct_convolutions = opt->direct_convolutions != 0;
   if (opt->fusion) fuse_conv_bias_activ(p);
   if (opt->fusion && opt->fuse_activations) fuse_conv_activations(p);
   if (opt->fusion && opt->fuse_matmul_bias) fuse_matmul_bias(p);

@@ -148,6 +148,7 @@ class Session {
   float cur_act_coef = 0.f;   // what the handle's activation coefficient was last set to
   std::map<std::string, bool> crsk_const;  // constants re-laid C,R,S,K on the host
   std::vector<char> filter_crsk;           // value id -> its device copy is C,R,S,K
+  std::set<std::string> sparse_const;      // 3x3 filters that are mostly zeros
   void *pool = nullptr, *weights = nullptr, *graph = nullptr;
   // Recorded graphs of other argument / result addresses than the current ones (runs in place hold the caller's
   // addresses in the graph): a caller that alternates between a few sets of buffers gets its graph back instead

@@ -57,6 +57,7 @@ struct IgemmArgs {
   bool a_mcontig;     // A stored [Kdim][M]: GEMM with transA
   bool a_vec4;        // A rows may be read as aligned float4
   bool b_vec4;        // (b_kcontig) B rows may be read as aligned float4
+  bool direct_sums;   // the products summed are those of A and B themselves (DNNRT_CONV_ALGO_DIRECT)
 };
 
 // The per-column bias of a lane's column, or 0 without one.  The load is

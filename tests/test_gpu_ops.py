@@ -1735,10 +1735,10 @@ def test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, re
 
 @pytest.mark.parametrize("case", [
     # N, C, H, W, K, pad, residual, activation: sizes at which the launcher picks the tiles of conv_f32_winograd.hip
-    (11, 64, 56, 56, 64, 1, False, _abi.ACT_RELU),          # 270 tiles: 14 left over, one stage of four channels per part
+    (22, 64, 56, 56, 64, 1, False, _abi.ACT_RELU),          # 539 tiles: 27 left over, in parts of four stages of four channels
     (6, 48, 75, 77, 100, 1, True, _abi.ACT_LEAKY_RELU),     # odd image, filters off the 64 grid
     (3, 512, 19, 19, 486, 1, False, _abi.ACT_IDENTITY),     # filter rows off the 16-byte grid
-    (2, 128, 64, 63, 128, 0, True, _abi.ACT_RELU),          # two stages per part, no padding
+    (4, 128, 64, 63, 128, 0, True, _abi.ACT_RELU),          # no padding
     (1, 256, 50, 51, 256, 2, False, _abi.ACT_CLIPPED_RELU),
     (2, 512, 28, 28, 256, 1, True, _abi.ACT_RELU),
 ])
@@ -1765,6 +1765,63 @@ def test_conv_3x3_by_minimal_filtering(gpu, case):
         got = oc.conv(gpu, x, w, b, (pad, pad), (1, 1), 1, activ, crsk=True, z=z, coef=coef, inplace=residual)
         assert np.linalg.norm(got - ref) <= bound * np.linalg.norm(ref)
         np.testing.assert_allclose(got, ref, rtol=RTOL, atol=ATOL)
+    direct = oc.conv(gpu, x, w, b, (pad, pad), (1, 1), 1, activ, crsk=True, z=z, coef=coef, inplace=residual, algo=_abi.CONV_ALGO_DIRECT)
+    assert (got != direct).any()  # the kernel under test is the one that ran
+    np.testing.assert_allclose(direct, ref, rtol=RTOL, atol=ATOL)
+
+
+def _minimal_filtering_magnitudes(x, w, pad):
+    """F(2x2, 3x3) with every value and every coefficient replaced by its magnitude, in 64 bits."""
+    import torch
+    G = torch.tensor([[1, 0, 0], [.5, .5, .5], [.5, .5, .5], [0, 0, 1]], dtype=torch.float64)
+    B = torch.tensor([[1, 0, 1, 0], [0, 1, 1, 0], [0, 1, 1, 0], [0, 1, 0, 1]], dtype=torch.float64)
+    A = torch.tensor([[1, 1, 1, 0], [0, 1, 1, 1]], dtype=torch.float64)
+    N, Cc, H, W = x.shape
+    K, P, Q = w.shape[0], H + 2 * pad - 2, W + 2 * pad - 2
+    th, tw = (P + 1) // 2, (Q + 1) // 2
+    d = torch.zeros((N, Cc, 2 * th + 2, 2 * tw + 2), dtype=torch.float64)
+    d[:, :, pad:pad + H, pad:pad + W] = torch.from_numpy(np.abs(x)).double()[:, :, :2 * th + 2 - pad, :2 * tw + 2 - pad]
+    V = torch.matmul(torch.matmul(B, d.unfold(2, 4, 2).unfold(3, 4, 2)), B.T).permute(4, 5, 1, 0, 2, 3).reshape(4, 4, Cc, -1)
+    U = torch.matmul(torch.matmul(G, torch.from_numpy(np.abs(w)).double()), G.T)
+    M = torch.stack([torch.stack([U[:, :, i, j] @ V[i, j] for j in range(4)], -1) for i in range(4)], -2)  # [K][tiles][4][4]
+    Y = torch.matmul(torch.matmul(A, M), A.T).reshape(K, N, th, tw, 2, 2).permute(1, 0, 2, 4, 3, 5).reshape(N, K, 2 * th, 2 * tw)
+    return Y[:, :, :P, :Q].numpy()
+
+
+@pytest.mark.parametrize("values", ["dense", "sparse", "pruned", "both", "uneven"])
+@pytest.mark.parametrize("case", [(3, 512, 19, 19, 486, 1), (2, 256, 56, 55, 256, 1), (4, 128, 64, 63, 128, 0)], ids=["512", "256", "128"])
+def test_conv_3x3_of_sparse_and_uneven_values(gpu, case, values):
+    """What the two ways of a 3x3 convolution promise for any values.  Direct sums: each of the 9 C + 1 additions rounds by at
+    most 2^-24 of the sum of magnitudes.  Minimal filtering: a patch value has passed two roundings and a filter value
+    four when they are multiplied, C products are added, four more additions and up to sixteen parts lead back, and one
+    adds the bias: C + 27 roundings of the magnitudes' own minimal filtering, which know the patch and not the window.  With
+    values that differ by orders of magnitude within a patch the first bound does not hold for the second way."""
+    import torch
+    N, Cc, H, W, K, pad = case
+    r = rng(Cc)
+    x = np.maximum(r.standard_normal((N, Cc, H, W)), 0)
+    w = r.standard_normal((K, Cc, 3, 3)) * np.sqrt(2.0 / (9 * Cc))
+    b = r.uniform(-0.01, 0.01, K).astype(np.float32)
+    if values in ("sparse", "both"):
+        x = np.abs(r.standard_normal(x.shape)) * (r.random(x.shape) < 0.05)
+    if values in ("pruned", "both"):
+        w *= r.random(w.shape) < 0.1
+    if values == "uneven":  # the centre tap alone, pixels over eight decades
+        x = np.abs(r.standard_normal(x.shape)) * 10.0 ** r.uniform(-4, 4, (N, 1, H, W))
+        w *= np.pad(np.ones((1, 1)), 1)
+    x, w = x.astype(np.float32), w.astype(np.float32)
+    conv64 = lambda t, f, v: torch.nn.functional.conv2d(*(torch.from_numpy(u).double() for u in (t, f, v)), padding=pad).numpy()  # noqa: E731
+    ref, magnitude = conv64(x, w, b), conv64(np.abs(x), np.abs(w), np.abs(b))
+    default, direct = (oc.conv(gpu, x, w, b, (pad, pad), (1, 1), 1, _abi.ACT_IDENTITY, crsk=True, algo=a) for a in (1, _abi.CONV_ALGO_DIRECT))
+    assert (np.abs(direct - ref) <= (9 * Cc + 1) * 2.0 ** -24 * magnitude).all()
+    bound = (Cc + 27) * 2.0 ** -24 * (_minimal_filtering_magnitudes(x, w, pad) + np.abs(b)[:, None, None])
+    assert (np.abs(default - ref) <= bound).all()
+    assert (default != direct).any()
+    if values == "uneven":
+        assert (np.abs(default - ref) > (9 * Cc + 1) * 2.0 ** -24 * magnitude).any()
+    error = [np.linalg.norm(v - ref) for v in (default, direct)]
+    # measured: dense 0.7 to 0.8, sparse 1.1 to 1.3, pruned 1.4 to 1.6, both 2.1 to 2.4, uneven 1.3 to 1.5
+    assert error[0] <= {"dense": 1.0, "sparse": 1.6, "pruned": 2.0, "both": 3.0, "uneven": 2.0}[values] * error[1]
 
 
 @pytest.mark.parametrize("crsk", [False, True])
@@ -1814,8 +1871,10 @@ def test_conv_3x3_by_minimal_filtering_keeps_infinities_in_their_place(gpu, cpu)
     must reach the results that use them and no others, as they do tap by tap."""
     r = rng(9)
     x = r.standard_normal((6, 48, 75, 77)).astype(np.float32)
-    w = (r.standard_normal((64, 48, 3, 3)) * 0.1).astype(np.float32)
-    b = r.uniform(-0.5, 0.5, 64).astype(np.float32)
+    w = (r.standard_normal((100, 48, 3, 3)) * 0.1).astype(np.float32)
+    b = r.uniform(-0.5, 0.5, 100).astype(np.float32)
+    plain = [oc.conv(gpu, x, w, b, (1, 1), (1, 1), 1, _abi.ACT_IDENTITY, crsk=True, algo=a) for a in (1, _abi.CONV_ALGO_DIRECT)]
+    assert (plain[0] != plain[1]).any()  # the kernel under test is the one that ran
     x[0, 3, 10, 20] = np.inf
     x[1, 5, 0, 0] = -np.inf
     x[2, 7, 74, 76] = np.nan
@@ -1833,7 +1892,7 @@ def test_conv_3x3_by_minimal_filtering_keeps_infinities_in_their_place(gpu, cpu)
     np.testing.assert_allclose(got[3][far], ref[3][far], rtol=RTOL)
 
 
-@pytest.mark.parametrize("case", [(7, 64, 56, 56, 64), (11, 64, 56, 56, 64), (3, 512, 19, 19, 486), (2, 512, 28, 28, 256)], ids=["whole", "rest-split", "odd-rows", "split"])
+@pytest.mark.parametrize("case", [(7, 64, 56, 56, 64), (22, 64, 56, 56, 64), (3, 512, 19, 19, 486), (2, 512, 28, 28, 256)], ids=["whole", "rest-split", "odd-rows", "split"])
 def test_conv_3x3_by_minimal_filtering_recomputes_only_what_is_not_finite(gpu, case):
     """A NaN or an infinity reaches the results whose windows hold it, and of the finite results only those of the same 2x2
     tiles may change a bit; with a whole image of NaN, the other images keep theirs."""
@@ -1847,6 +1906,7 @@ def test_conv_3x3_by_minimal_filtering_recomputes_only_what_is_not_finite(gpu, c
     run = lambda t, f=w: oc.conv(gpu, t, f, b, (1, 1), (1, 1), 1, _abi.ACT_IDENTITY, crsk=True)  # noqa: E731
     conv64 = lambda t, f=w: torch.nn.functional.conv2d(*(torch.from_numpy(u).double() for u in (t, f, b)), padding=1).numpy()  # noqa: E731
     plain = run(x)
+    assert (plain != oc.conv(gpu, x, w, b, (1, 1), (1, 1), 1, _abi.ACT_IDENTITY, crsk=True, algo=_abi.CONV_ALGO_DIRECT)).any()
     for value in (np.nan, np.inf):
         y = x.copy()
         y[1, Cc - 1, 10, 7] = value
