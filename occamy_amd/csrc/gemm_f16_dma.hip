@@ -14,8 +14,8 @@
 // no longer wait for the whole ring, gd_read_tr), and reductions split over workgroups where tiles are few (partial tiles through the handle's scratch,
 // the last to arrive adds them in split order; nobody waits).  128x128 tiles on eight wavefronts take the products of
 // thousands of rows (4096 cubed: 650 TFLOP/s, 333 us on 64x64 tiles, 212 on these).
-// Against gemm_f16.hip's kernel, which keeps what is not aligned (K x N -> us before, now): 384 rows, 768 x 2304 19.4 -> 7.2,
-// 768 x 768 15.9 -> 7.3, 768 x 3072 + GELU 24.7 -> 9.7, 3072 x 768 26.7 -> 11.5; 2048 rows, 768 x 2304 20.4.  Products of at most a tile per
+// Against gemm_f16.hip's kernel, which keeps what is not aligned (K x N -> us before, now): 384 rows, 768 x 2304 19.4 -> 7.0,
+// 768 x 768 15.9 -> 7.0, 768 x 3072 + GELU 24.7 -> 9.1, 3072 x 768 26.7 -> 11.2; 2048 rows, 768 x 2304 18.2.  Products of at most a tile per
 // compute unit go to gemm_f16_waves.hip.
 #include "gemm_f16.h"
 

@@ -9,8 +9,8 @@
 //
 // Time of a workgroup, 384 x 768 x 2304 (us): set-up 0.5, first data 1.0, six stages 2.5, sums 0.6, epilogue and code fetched on the way 1.0.
 // Rings of four stages gained in the loop what they lost waiting for the first data; 96 rows per tile cost 1.2 more per
-// launch and never paid.  K x N, us against gemm_f16_dma.hip (before its reads were put right, after, here): 384 rows, 768 x 2304
-// 8.0, 7.2, 6.9; 768 x 768 7.9, 7.3, 6.2; 3072 x 768 12.1, 11.8, 10.1; 128 rows, 768 x 3072 + GELU 9.8, 7.8, 7.7; 16 rows, 768 x 768 6.7, 6.7, 5.7.
+// launch and never paid.  K x N, us on gemm_f16_dma.hip -> here, back to back on one card: 384 rows, 768 x 2304 7.0 -> 6.6;
+// 768 x 768 7.0 -> 6.2; 3072 x 768 11.2 -> 10.1; 128 rows, 768 x 3072 + GELU 7.1 -> 6.8; 16 rows, 768 x 768 6.4 -> 5.6.
 #include "gemm_f16.h"
 
 #include <type_traits>
