@@ -373,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void conv_f32_winograd_kernel(const IgemmAr
   for (int i = 0; i < 16; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++) top = max(top, __builtin_bit_cast(unsigned, v[i][j]) & 0x7fffffffu);
-  if (__any(top >= 0x7f800000u)) {
+  if (__builtin_expect(__any(top >= 0x7f800000u), 0)) {
     unsigned wrong[2] = {0, 0};  // bit i: filter row0 + i of pixel j
 #pragma unroll
     for (int i = 0; i < 16; i++)
