@@ -408,7 +408,7 @@ bool launch_gemm_f16_dma(const dnnrtContext *ctx, const GemmF16Args &args, int Z
   }
   // The kernel whose wavefronts share the reduction: a stage of 32 k takes each of the four 0.43, what comes before and after
   // them 0.3 more than here, a split's hand-over 2.3 and 0.25 per part.  One workgroup per compute unit: with two it is the
-  // slower one (384 x 768 x 3072 9.7 us here, 10.3 there).
+  // slower one (384 x 768 x 3072 by 6 %).
   const int stages = (int)ceil_div(g.K, 32);
   const int64_t tiles = ceil_div(g.M, 64) * ceil_div(g.N, 64) * Z;
   int waves_splits = 0;
