@@ -11,6 +11,12 @@
 #include "../../include/dnnrt.h"
 #include "lds_limit.h"
 
+// A cut of an fp32 inverted residual block (conv_f32_block.hip) and the sizes it was found for.
+struct dnnrtBlockCut {
+  int64_t sizes[11];
+  int nb, qw, waves, splits;
+};
+
 struct dnnrtContext {
   hipStream_t stream;  // kernels of this handle are launched here
   int format;          // DNNRT_NCHW / DNNRT_NHWC / DNNRT_NCHW_TO_NHWC
@@ -31,6 +37,9 @@ struct dnnrtContext {
   // split would have to shrink to fit instead of shrinking it.
   bool splitk_shared;
   bool scratch_is_static;  // the two buffers are the library's static array (held by one handle per device), not allocations
+  // The cuts found last, a ring: a search takes 20 to 60 us, as long as several launches.  A handle is used by one thread at a time.
+  mutable dnnrtBlockCut block_cuts[32];
+  mutable unsigned block_cuts_found;
   int f16_tile;        // dnnrtSetConvTile: 0 = pick the fp16 convolution variant by problem size, otherwise one of F16_TILE_IDS
 };
 

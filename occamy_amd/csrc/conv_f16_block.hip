@@ -32,6 +32,9 @@
 
 namespace dnnrt {
 
+bool block_f32_applies(const dnnrtContext *ctx, const dnnrtExecBlock &k);  // conv_f32_block.hip
+bool launch_block_f32(const dnnrtContext *ctx, const dnnrtExecBlock &k);
+
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -457,7 +460,7 @@ bool launch_block_f16(const dnnrtContext *ctx, const dnnrtExecBlock &k) {
 extern "C" {
 
 int32_t dnnrtExecBlockApplies(dnnrtHandle_t handle, const dnnrtExecBlock *block) {
-  return handle && block && dnnrt::block_f16_applies(handle, *block) ? 1 : 0;
+  return handle && block && (block->dtype == DNNRT_F32 ? dnnrt::block_f32_applies(handle, *block) : dnnrt::block_f16_applies(handle, *block)) ? 1 : 0;
 }
 
 void dnnrtExecBlockFilter(void *dst, const void *src, int64_t rows, int64_t cols) {
@@ -474,7 +477,7 @@ int32_t dnnrtExecRunBlock(dnnrtHandle_t handle, const dnnrtExecBlock *block) {
     dnnrt::set_error("dnnrtExecRunBlock: bad arguments");
     return 1;
   }
-  return dnnrt::launch_block_f16(handle, *block) ? 0 : 1;
+  return (block->dtype == DNNRT_F32 ? dnnrt::launch_block_f32(handle, *block) : dnnrt::launch_block_f16(handle, *block)) ? 0 : 1;
 }
 
 }  // extern "C"

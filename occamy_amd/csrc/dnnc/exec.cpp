@@ -49,6 +49,7 @@ bool load_runtime(const std::string &path, RuntimeApi &rt, std::string &err) {
   *(void **)(&rt.dnnrtExecBlockApplies) = dlsym(rt.dl, "dnnrtExecBlockApplies");
   *(void **)(&rt.dnnrtExecRunBlock) = dlsym(rt.dl, "dnnrtExecRunBlock");
   *(void **)(&rt.dnnrtExecBlockFilter) = dlsym(rt.dl, "dnnrtExecBlockFilter");
+  *(void **)(&rt.dnnrtExecBlockFilterF32) = dlsym(rt.dl, "dnnrtExecBlockFilterF32");
   return true;
 }
 #undef LOAD
@@ -267,7 +268,7 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
       if (f == block_filters.end()) continue;
       uint8_t *host = (uint8_t *)ptr[(size_t)op->operands[1]->id];
       const std::vector<uint8_t> rows(host, host + op->bytes);
-      rt.dnnrtExecBlockFilter(host, rows.data(), f->second.first, f->second.second);
+      block_filter(f->first)(host, rows.data(), f->second.first, f->second.second);
       if (rt.dnnrtMemcpy(ptr[(size_t)op->operands[0]->id], host, op->bytes, 1, stream)) { err = rt_error("dnnrtMemcpy(constant)"); return false; }
     }
     if (!block_filters.empty() && rt.dnnrtSync(handle)) { err = rt_error("dnnrtSync"); return false; }
@@ -397,7 +398,7 @@ const Value *Session::buffer_of(const Value *v) const {
 // gets bytes that are free from here to its last reader: those of the two wide tensors that are not stored any more, as
 // a rule.  Nothing else moves.
 void Session::plan_blocks() {
-  if (host_backend || !rt.dnnrtExecBlockApplies || !rt.dnnrtExecRunBlock || !rt.dnnrtExecBlockFilter) return;
+  if (host_backend || !rt.dnnrtExecBlockApplies || !rt.dnnrtExecRunBlock || !rt.dnnrtExecBlockFilter || !rt.dnnrtExecBlockFilterF32) return;
   std::vector<const Op *> ops;
   std::map<const Op *, int> number;
   for (const Op *op : prog->ops)
@@ -438,6 +439,10 @@ void Session::plan_blocks() {
     bool read_later = true;  // by operations that launch something
     for (const auto &u : pr->result->uses) read_later = read_later && is_compute(u.first->kind) && launches(u.first) && !elided.count(u.first);
     if (!read_later) continue;
+    // fp32 filters come C,R,S,K
+    bool layouts = true;
+    for (const Op *op : {ex, dw, pr}) layouts = layouts && (!op || prog->channels_last || filter_crsk[(size_t)op->operands[1]->id]);
+    if (!layouts) continue;
     Block b{ex, dw, pr, (int)i, -1};
     dnnrtExecBlock k;
     fill_block(b, k);
@@ -706,7 +711,7 @@ bool Session::plan_uploads(const std::vector<UploadChunk> &chunks, std::string &
       void *at = (char *)upload_host + host + in;
       const void *from = ptr[(size_t)copy->operands[1]->id];
       const auto f = block_filters.find(copy->operands[0]);
-      if (f != block_filters.end()) rt.dnnrtExecBlockFilter(at, from, f->second.first, f->second.second);
+      if (f != block_filters.end()) block_filter(f->first)(at, from, f->second.first, f->second.second);
       else std::memcpy(at, from, (size_t)item.bytes);
       moved[(size_t)copy->operands[1]->id] = at;
       upload_slots.push_back({(size_t)copy->operands[0]->id, k.off + in});

@@ -83,6 +83,7 @@ struct RuntimeApi {
   decltype(&::dnnrtExecBlockApplies) dnnrtExecBlockApplies = nullptr;
   decltype(&::dnnrtExecRunBlock) dnnrtExecRunBlock = nullptr;
   decltype(&::dnnrtExecBlockFilter) dnnrtExecBlockFilter = nullptr;
+  decltype(&::dnnrtExecBlockFilterF32) dnnrtExecBlockFilterF32 = nullptr;
 };
 
 bool load_runtime(const std::string &path, RuntimeApi &rt, std::string &err);
@@ -187,6 +188,7 @@ class Session {
   bool tunable(const Op *op) const;
   void fill_block(const Block &b, dnnrtExecBlock &k) const;
   std::map<const Value *, std::pair<int64_t, int64_t>> block_filters;  // device tensors uploaded in the block call's layout; rows, columns
+  decltype(&::dnnrtExecBlockFilter) block_filter(const Value *filter) const { return filter->dtype == F16 ? rt.dnnrtExecBlockFilter : rt.dnnrtExecBlockFilterF32; }
   void plan_blocks();
   std::map<const Value *, Range> live_slots() const;
   // Per-inference mode on the GPU runtime: the constants as they go to the device on a second stream, ahead of the

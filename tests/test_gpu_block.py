@@ -202,3 +202,28 @@ def test_profile_knows_copies_that_are_not_launched():
     assert elided and all(ops[i][0] in ("dnn.flatten", "dnn.reshape", "dnn.squeeze", "dnn.unsqueeze") for i in elided)
     assert all((m > 0) == (o[4] == i) for i, (m, o) in enumerate(zip(ms, ops)))
     s.close()
+
+
+@pytest.mark.parametrize("batch,height,width,stride,pads", [(1, 56, 57, 1, (1, 1)), (3, 31, 30, 2, (2, 1)), (4, 60, 5, 1, (2, 1)), (1, 28, 28, 1, (3, 3))], ids=str)
+def test_fp32_blocks_in_programs(batch, height, width, stride, pads):
+    """fp32 programs with a block in one launch (and one with a padding that it does not take), per inference and resident, against
+    the oracle; every mode and a replay the same bits."""
+    import torch
+    flags = dict(FLAGS, channels_last=False)
+    build = lambda: small_net(batch, height, width, stride, pads, dtype=np.float32)  # noqa: E731
+    ref, _ = run(build, ORACLE_PATH, fusion=True)
+    g, inputs = build()
+    p = g.compile(**flags)
+    s = p.session(compiler.MODE_RESIDENT)
+    assert any(o[1] == "inverted_block" for o in s.compute_ops()) == (max(pads) <= 2)
+    out = s.run(*inputs)[0]
+    np.testing.assert_allclose(out, ref[0], rtol=1e-4, atol=1e-5 * float(np.abs(ref[0]).max()))
+    x, y = torch.from_numpy(inputs[0]).cuda(), torch.empty(out.shape, device="cuda")
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        s.run_device([x.data_ptr()], [y.data_ptr()])
+        s.sync()
+        np.testing.assert_array_equal(y.cpu().numpy(), out)
+    s.close()
+    np.testing.assert_array_equal(run(build, mode=compiler.MODE_OCCAMY, **flags)[0][0], out)

@@ -1733,6 +1733,82 @@ def test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, re
     np.testing.assert_allclose(got.numpy(), want.numpy(), rtol=4e-3, atol=8e-3)
 
 
+@pytest.mark.parametrize("n,cin,h,w,ch,cout,stride,pads,expand,residual,acts", [
+    (1, 8, 5, 7, 16, 8, 1, (1, 1), True, False, (3, 3, 5)),      # less than a tile, one group of hidden channels
+    (1, 16, 33, 17, 96, 24, 2, (1, 1), True, False, (3, 3, 5)),  # ragged tiles, half a block of output channels
+    (1, 24, 28, 29, 144, 24, 1, (1, 1), True, True, (3, 3, 3)),  # the hidden channels over workgroups, residual
+    (16, 32, 30, 31, 192, 32, 1, (2, 0), True, True, (1, 3, 1)),  # many tiles
+    (1, 64, 14, 14, 384, 64, 1, (1, 1), True, True, (3, 3, 5)),
+    (3, 40, 11, 10, 208, 72, 2, (0, 2), True, False, (5, 1, 5)),  # a last chunk of one step in four
+    (24, 96, 13, 14, 288, 96, 1, (1, 1), True, False, (3, 3, 5)),
+    (1, 96, 7, 9, 576, 160, 2, (1, 1), True, False, (3, 3, 5)),
+    (1, 160, 7, 7, 960, 328, 1, (1, 1), True, False, (3, 3, 5)),  # output channels over three workgroups, the last with one block
+    (40, 160, 7, 6, 480, 160, 1, (1, 1), True, True, (3, 3, 5)),
+    (2, 120, 9, 2, 112, 16, 1, (1, 2), True, False, (3, 3, 5)),  # an image narrower than a square's window
+    (1, 32, 30, 31, 32, 16, 1, (1, 1), False, False, (0, 3, 5)),  # no expansion
+    (5, 48, 13, 12, 48, 24, 2, (1, 1), False, False, (0, 1, 5)),
+])
+def test_inverted_residual_block_fp32(n, cin, h, w, ch, cout, stride, pads, expand, residual, acts):
+    """The fp32 block call against 64 bits: every result within the bound that its three sums' lengths and magnitudes give, and
+    the same bits in a second call (the parts' counters are back at zero)."""
+    import torch
+    import torch.nn.functional as F
+    g = torch.Generator().manual_seed(n * 1000 + cin + h)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    x, w1, b1 = rnd(n, cin, h, w), rnd(ch, cin) * (2 / cin) ** 0.5, rnd(ch) * 0.5
+    wd, bd, w3, b3 = rnd(ch, 1, 3, 3) * 0.4, rnd(ch) * 0.5, rnd(cout, ch) * (1 / ch) ** 0.5, rnd(cout) * 0.5
+    act = lambda t, mode: t if mode == 5 else t.clamp(0, 6) if mode == 3 else t.clamp(min=0)  # noqa: E731
+    u, d = 2.0 ** -24, lambda t: t.double()  # noqa: E731
+    t, err = d(x), torch.zeros_like(d(x))
+    if expand:
+        k = d(w1)[:, :, None, None]
+        err = (cin + 2) * u * (F.conv2d(t.abs(), k.abs()) + d(b1).abs()[:, None, None])
+        t = act(F.conv2d(t, k, d(b1)), acts[0])
+    k, mag = d(wd), t.abs()
+    err = F.conv2d(err, k.abs(), None, stride, pads, groups=ch) + 11 * u * (F.conv2d(mag, k.abs(), None, stride, pads, groups=ch) + d(bd).abs()[:, None, None])
+    t = act(F.conv2d(t, k, d(bd), stride, pads, groups=ch), acts[1])
+    k, mag = d(w3)[:, :, None, None], t.abs()
+    err = F.conv2d(err, k.abs()) + (ch + 4) * u * (F.conv2d(mag, k.abs()) + d(b3).abs()[:, None, None])
+    want = F.conv2d(t, k, d(b3))
+    p, q = want.shape[2:]
+    z = rnd(n, cout, p, q) if residual else None
+    if residual:
+        want, err = want + d(z), err + 2 * u * (want.abs() + d(z).abs())
+    want = act(want, acts[2])
+
+    lib = C.CDLL(_abi.RUNTIME_PATH)
+    handle = C.c_void_p()
+    assert lib.dnnrtCreate(C.byref(handle)) == 0
+    lib.dnnrtExecBlockFilterF32.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64]
+
+    def blocked(m):
+        out, crsk = torch.empty_like(m), m.t().contiguous()
+        lib.dnnrtExecBlockFilterF32(out.data_ptr(), crsk.data_ptr(), m.shape[0], m.shape[1])
+        return out.cuda()
+    keep = dict(x=x.cuda(), w1=blocked(w1) if expand else None, b1=b1.cuda() if expand else None, wd=wd.reshape(ch, 9).t().contiguous().cuda(), bd=bd.cuda(),
+                w3=blocked(w3), b3=b3.cuda(), z=None if z is None else z.cuda(), y=torch.full((n, cout, p, q), float("nan"), device="cuda"))
+    k = ExecBlock(n=n, cin=cin, h=h, w=w, ch=ch, r=3, s=3, stride=stride, pad_h=pads[0], pad_w=pads[1], p=p, q=q, cout=cout, act1=acts[0], actd=acts[1],
+                  act=acts[2], coef1=6.0, coefd=6.0, coef=6.0, expand=int(expand), dtype=_abi.F32, format=_abi.NCHW, **{m: v.data_ptr() for m, v in keep.items() if v is not None})
+    torch.cuda.synchronize()
+    lib.dnnrtLastError.restype = C.c_char_p
+    got = []
+    for _ in range(2):
+        assert lib.dnnrtExecRunBlock(handle, C.byref(k)) == 0, lib.dnnrtLastError()
+        torch.cuda.synchronize()
+        got.append(keep["y"].cpu())
+        keep["y"].fill_(float("nan"))
+        torch.cuda.synchronize()
+    assert torch.equal(*got)
+    worst = ((got[0].double() - want).abs() / err).max()
+    assert worst <= 1, worst
+    for bad in (dict(cin=cin + 4), dict(ch=ch + 8), dict(cout=cout + 4), dict(format=_abi.NHWC), dict(q=q + 1), dict(pad_h=3), dict(actd=6)):  # not run: refused
+        other = ExecBlock.from_buffer_copy(k)
+        for name, value in bad.items():
+            setattr(other, name, value)
+        assert not lib.dnnrtExecBlockApplies(handle, C.byref(other)) and lib.dnnrtExecRunBlock(handle, C.byref(other)) != 0, bad
+    lib.dnnrtDestroy(handle)
+
+
 @pytest.mark.parametrize("case", [
     # N, C, H, W, K, pad, residual, activation: sizes at which the launcher picks the tiles of conv_f32_winograd.hip
     (22, 64, 56, 56, 64, 1, False, _abi.ACT_RELU),          # 539 tiles: 27 left over, in parts of four stages of four channels
