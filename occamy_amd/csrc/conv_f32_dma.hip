@@ -22,6 +22,7 @@
 // 256 -> 64 1x1 there 110 -> 34; 256 -> 256 3x3 at 38x38, 3 images 111 -> 51 (100); 256 -> 512 3x3 at 56x56, 2 images
 // 201 -> 117 (126); 1024 -> 1024 3x3 at 7x7, 2 images 42 -> 32.  ResNet-50 at 32 images 4.92 -> 2.7 ms.
 #include "igemm_f32.h"
+#include "partials.h"
 
 #include <type_traits>
 
@@ -388,14 +389,17 @@ __global__ __launch_bounds__(256) void conv_f32_dma_kernel(const IgemmArgs a, co
   if (part && pl.splits > 1) {
     constexpr int TILE = BM * BN;
     const int rt = tile - pl.whole;
-    float *mine = partials + ((size_t)rt * pl.splits + split) * TILE + tid;
+    const __amdgpu_buffer_rsrc_t parts = part_rsrc(partials);
+    const unsigned mine = 16u * (unsigned)tid, first_part = (unsigned)(rt * pl.splits) * (4u * TILE);  // [four registers][thread]
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
       for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++)
-          __hip_atomic_store(&mine[((i * TN + j) * 16 + r) * 256], acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int g = 0; g < 4; g++) {
+          const floatx16 &o = acc[i][j];
+          part_store(parts, mine + 4096 * ((i * TN + j) * 4 + g), first_part + (unsigned)split * (4u * TILE), part_floatx4{o[4 * g], o[4 * g + 1], o[4 * g + 2], o[4 * g + 3]});
+        }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -404,25 +408,26 @@ __global__ __launch_bounds__(256) void conv_f32_dma_kernel(const IgemmArgs a, co
     __syncthreads();
     if (*arrived_s != (unsigned)pl.splits - 1) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    const float *all = partials + (size_t)rt * pl.splits * TILE + tid;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
       for (int j = 0; j < TN; j++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-    for (int y = 0; y < pl.splits; y++) {
+    constexpr int AT_ONCE = 4 / (TM * TN);  // no more registers than the reduction leaves free
+    for (int y = 0; y < pl.splits; y += AT_ONCE) {  // so many parts in flight, added in split order
+      part_floatx4 p[AT_ONCE][TM * TN * 4];
 #pragma unroll
-      for (int i = 0; i < TM; i++)
+      for (int u = 0; u < AT_ONCE; u++)
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-          float p[16];
+        for (int g = 0; g < TM * TN * 4; g++)
+          p[u][g] = part_load<part_floatx4>(parts, y + u < pl.splits ? mine + 4096 * g : PART_NONE, first_part + (unsigned)min(y + u, pl.splits - 1) * (4u * TILE));
 #pragma unroll
-          for (int r = 0; r < 16; r++)
-            p[r] = __hip_atomic_load(&all[(size_t)y * TILE + ((i * TN + j) * 16 + r) * 256], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int u = 0; u < AT_ONCE; u++)
 #pragma unroll
-          for (int r = 0; r < 16; r++) acc[i][j][r] += p[r];
-        }
+        for (int g = 0; g < TM * TN * 4; g++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[g / 4 / TN][g / 4 % TN][4 * (g & 3) + e] += p[u][g][e];
     }
     if (tid == 0) __hip_atomic_store(&counters[rt], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }

@@ -27,6 +27,7 @@
 // are all zero need not be zero.  The caller has the choice (DNNRT_CONV_ALGO_DIRECT); the executor makes it where a filter is
 // mostly zero.
 #include "igemm_f32.h"
+#include "partials.h"
 
 #include <type_traits>
 
@@ -318,11 +319,11 @@ __global__ __launch_bounds__(256, 2) void conv_f32_winograd_kernel(const IgemmAr
   // ---- a split tile: the hand-over of the other fp32 kernels (igemm_f32_small.hip states what it rests on) ----
   if (part && pl.splits > 1) {
     const int rt = tile - pl.whole;
-    float *mine = partials + ((size_t)rt * pl.splits + split) * W32_TILE + tid;
+    const __amdgpu_buffer_rsrc_t parts = part_rsrc(partials);
+    const unsigned mine = 16u * (unsigned)tid, first_part = (unsigned)(rt * pl.splits) * (4u * W32_TILE);  // [two filters][thread]
 #pragma unroll
-    for (int i = 0; i < 16; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++) __hip_atomic_store(&mine[(2 * i + j) * 256], v[i][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = 0; i < 16; i += 2)
+      part_store(parts, mine + 2048 * i, first_part + (unsigned)split * (4u * W32_TILE), part_floatx4{v[i][0], v[i][1], v[i + 1][0], v[i + 1][1]});
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -333,19 +334,19 @@ __global__ __launch_bounds__(256, 2) void conv_f32_winograd_kernel(const IgemmAr
     if (*arrived_s != (unsigned)pl.splits - 1) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     if (tid == 0) __hip_atomic_store(&counters[rt], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const float *all = partials + (size_t)rt * pl.splits * W32_TILE + tid;
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i][0] = v[i][1] = 0.f;
     for (int y = 0; y < pl.splits; y += 4) {  // four partial tiles in flight, added in split order
-      float p[4][32];
+      part_floatx4 p[4][8];
 #pragma unroll
       for (int u = 0; u < 4; u++)
 #pragma unroll
-        for (int i = 0; i < 32; i++) p[u][i] = __hip_atomic_load(all + (size_t)min(y + u, pl.splits - 1) * W32_TILE + i * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int i = 0; i < 8; i++)
+          p[u][i] = part_load<part_floatx4>(parts, y + u < pl.splits ? mine + 4096 * i : PART_NONE, first_part + (unsigned)min(y + u, pl.splits - 1) * (4u * W32_TILE));
 #pragma unroll
       for (int u = 0; u < 4; u++)
 #pragma unroll
-        for (int i = 0; i < 32; i++) v[i >> 1][i & 1] += y + u < pl.splits ? p[u][i] : 0.f;
+        for (int i = 0; i < 32; i++) v[i >> 1][i & 1] += p[u][i >> 2][i & 3];
     }
   }
 

@@ -18,6 +18,7 @@
 // 768 x 768 15.9 -> 7.0, 768 x 3072 + GELU 24.7 -> 9.1, 3072 x 768 26.7 -> 11.2; 2048 rows, 768 x 2304 18.2.  Products of at most a tile per
 // compute unit go to gemm_f16_waves.hip.
 #include "gemm_f16.h"
+#include "partials.h"
 
 #include <type_traits>
 
@@ -265,13 +266,16 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
     constexpr int TILE = FN * FM;
     volatile unsigned *arrived = reinterpret_cast<unsigned *>(smem);
     const unsigned t = (unsigned)z * (unsigned)tiles + (unsigned)tile;
-    float *mine = a.partials + ((size_t)t * splits + blockIdx.y) * TILE + tid;
+    const __amdgpu_buffer_rsrc_t parts = part_rsrc(a.partials);
+    const unsigned mine = 16u * (unsigned)tid, first_part = t * (unsigned)splits * (4u * TILE);  // [four registers][thread]
 #pragma unroll
     for (int i = 0; i < TN; i++)
 #pragma unroll
       for (int j = 0; j < TM; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) __hip_atomic_store(&mine[((i * TM + j) * 16 + r) * NT], acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int g = 0; g < 4; g++)
+          part_store(parts, mine + 16 * NT * ((i * TM + j) * 4 + g), first_part + blockIdx.y * (4u * TILE),
+                     part_floatx4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]});
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -280,7 +284,6 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
     __syncthreads();
     if (*arrived != (unsigned)splits - 1) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    const float *all = a.partials + (size_t)t * splits * TILE + tid;
 #pragma unroll
     for (int i = 0; i < TN; i++)
 #pragma unroll
@@ -292,18 +295,16 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
       for (int i = 0; i < TN; i++)
 #pragma unroll
         for (int j = 0; j < TM; j++) {
-          float p[4][16];
+          part_floatx4 p[4][4];
 #pragma unroll
           for (int y = 0; y < 4; y++)
 #pragma unroll
-            for (int r = 0; r < 16; r++)
-              p[y][r] = __hip_atomic_load(&all[(size_t)min(y0 + y, splits - 1) * TILE + ((i * TM + j) * 16 + r) * NT], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int g = 0; g < 4; g++)
+              p[y][g] = part_load<part_floatx4>(parts, y0 + y < splits ? mine + 16 * NT * ((i * TM + j) * 4 + g) : PART_NONE, first_part + (unsigned)min(y0 + y, splits - 1) * (4u * TILE));
 #pragma unroll
           for (int y = 0; y < 4; y++)
-            if (y0 + y < splits) {
 #pragma unroll
-              for (int r = 0; r < 16; r++) acc[i][j][r] += p[y][r];
-            }
+            for (int r = 0; r < 16; r++) acc[i][j][r] += p[y][r >> 2][r & 3];
         }
     }
     if (tid == 0) __hip_atomic_store(&a.counters[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

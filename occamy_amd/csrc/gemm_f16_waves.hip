@@ -12,6 +12,7 @@
 // launch and never paid.  K x N, us on gemm_f16_dma.hip -> here, back to back on one card: 384 rows, 768 x 2304 7.0 -> 6.6;
 // 768 x 768 7.0 -> 6.2; 3072 x 768 11.2 -> 10.1; 128 rows, 768 x 3072 + GELU 7.1 -> 6.8; 16 rows, 768 x 768 6.4 -> 5.6.
 #include "gemm_f16.h"
+#include "partials.h"
 
 #include <type_traits>
 
@@ -274,9 +275,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
   const int splits = (int)gridDim.y;
   if (splits > 1) {
     const unsigned t = (unsigned)z * (unsigned)tiles + (unsigned)tile;
-    float *mine = a.partials + ((size_t)t * splits + blockIdx.y) * (FM * 64) + tid;
+    const __amdgpu_buffer_rsrc_t parts = part_rsrc(a.partials);
+    const unsigned mine = 16u * (unsigned)tid, first_part = t * (unsigned)splits * (FM * 256u);
 #pragma unroll
-    for (int e = 0; e < E; e++) __hip_atomic_store(&mine[e * 256], v[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int e = 0; e < E; e += 4) part_store(parts, mine + 1024 * e, first_part + blockIdx.y * (FM * 256u), part_floatx4{v[e], v[e + 1], v[e + 2], v[e + 3]});
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -287,21 +289,19 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
     if (*arrived != (unsigned)splits - 1) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     if (tid == 0) __hip_atomic_store(&a.counters[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const float *all = a.partials + (size_t)t * splits * (FM * 64) + tid;
 #pragma unroll
     for (int e = 0; e < E; e++) v[e] = 0.f;
     for (int y0 = 0; y0 < splits; y0 += 4) {  // four parts requested at a time, added in split order
-      float p[4][E];
+      part_floatx4 p[4][E / 4];
 #pragma unroll
       for (int y = 0; y < 4; y++)
 #pragma unroll
-        for (int e = 0; e < E; e++) p[y][e] = __hip_atomic_load(&all[(size_t)min(y0 + y, splits - 1) * (FM * 64) + e * 256], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int e = 0; e < E; e += 4)
+          p[y][e / 4] = part_load<part_floatx4>(parts, y0 + y < splits ? mine + 1024 * e : PART_NONE, first_part + (unsigned)min(y0 + y, splits - 1) * (FM * 256u));
 #pragma unroll
       for (int y = 0; y < 4; y++)
-        if (y0 + y < splits) {
 #pragma unroll
-          for (int e = 0; e < E; e++) v[e] += p[y][e];
-        }
+        for (int e = 0; e < E; e++) v[e] += p[y][e / 4][e % 4];
     }
   }
 

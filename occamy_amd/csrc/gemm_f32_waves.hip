@@ -13,6 +13,7 @@
 // 768 x 2304 12.7 -> 11.3, 768 x 3072 15.1 -> 13.8, 3072 x 768 16.0 -> 14.7; 384 rows 20.5 -> 16.6, 32.9 -> 24.4, 26.3 -> 22.7; 4096
 // rows (the big-tile kernel of igemm_f32.hip before) 224 -> 133, 234 -> 174, 166 -> 158.
 #include "igemm_f32.h"
+#include "partials.h"
 
 #include <type_traits>
 
@@ -205,9 +206,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const IgemmArgs 
   const int splits = pl.splits;
   if (part && splits > 1) {
     const int rt = tile - pl.whole;
-    float *mine = partials + ((size_t)rt * splits + split) * 4096 + tid;
+    const __amdgpu_buffer_rsrc_t parts = part_rsrc(partials);
+    const unsigned mine = 16u * (unsigned)tid, first_part = (unsigned)(rt * splits) * 16384u;
 #pragma unroll
-    for (int e = 0; e < 16; e++) __hip_atomic_store(&mine[e * 256], v[e >> 2][e & 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int o = 0; o < 4; o++) part_store(parts, mine + 4096 * o, first_part + 16384u * (unsigned)split, v[o]);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -218,21 +220,19 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const IgemmArgs 
     if (*arrived != (unsigned)splits - 1) return;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     if (tid == 0) __hip_atomic_store(&counters[rt], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const float *all = partials + (size_t)rt * splits * 4096 + tid;
 #pragma unroll
     for (int o = 0; o < 4; o++) v[o] = floatx4{0.f, 0.f, 0.f, 0.f};
     for (int y0 = 0; y0 < splits; y0 += 4) {  // four parts requested at a time, added in split order
-      float p[4][16];
+      part_floatx4 p[4][4];
 #pragma unroll
       for (int y = 0; y < 4; y++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) p[y][e] = __hip_atomic_load(&all[(size_t)min(y0 + y, splits - 1) * 4096 + e * 256], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int o = 0; o < 4; o++)
+          p[y][o] = part_load<part_floatx4>(parts, y0 + y < splits ? mine + 4096 * o : PART_NONE, first_part + 16384u * (unsigned)min(y0 + y, splits - 1));
 #pragma unroll
       for (int y = 0; y < 4; y++)
-        if (y0 + y < splits) {
 #pragma unroll
-          for (int e = 0; e < 16; e++) v[e >> 2][e & 3] += p[y][e];
-        }
+        for (int o = 0; o < 4; o++) v[o] += p[y][o];
     }
   }
 

@@ -19,6 +19,7 @@
 // loads in flight.  Offsets are 31-bit: the dispatcher only takes these
 // kernels when every operand is below 2^29 elements.
 #include "igemm_f32.h"
+#include "partials.h"
 
 #include <type_traits>
 
@@ -101,15 +102,25 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
   }
   const int splits = (int)gridDim.y;
   if (splits > 1) {
-    float *mine = partials + ((size_t)tile * splits + blockIdx.y) * 1024 + wave * N * 64 + lane;
+#if __HIP_DEVICE_COMPILE__
+    // a partial tile: [wavefront][vector of its registers][lane]
+    typedef std::conditional_t<N == 2, part_floatx2, part_floatx4> vec_t;
+    constexpr int E = N == 2 ? 2 : 4, VECS = N / E;
+    const __amdgpu_buffer_rsrc_t parts = part_rsrc(partials);
+    const unsigned mine = (unsigned)(wave * N * 256 + lane * 4 * E), first_part = tile * (unsigned)splits * 4096u;
 #pragma unroll
-    for (int i = 0; i < N; i++) __hip_atomic_store(&mine[i * 64], v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // The hand-over.  Every wavefront of every workgroup of a tile (1) writes its part of the partial tile with device-scope atomic
+    for (int i = 0; i < VECS; i++) {
+      vec_t o;
+#pragma unroll
+      for (int e = 0; e < E; e++) o[e] = v[E * i + e];
+      part_store(parts, mine + 256 * E * i, first_part + 4096u * blockIdx.y, o);
+    }
+    // The hand-over.  Every wavefront of every workgroup of a tile (1) writes its part of the partial tile with device-scope
     // stores, which go past the per-XCD L2 to the point where all XCDs agree, (2) waits until every one of
     // them is acknowledged (s_waitcnt 0: the counters of a wavefront reach zero only when its stores have been
     // written there); behind the workgroup's barrier (3) one thread adds one to the tile's arrival counter with a device-scope
     // atomic, performed at that same point.  Whoever reads splits - 1 knows that every other workgroup's step (2) is over, so its
-    // device-scope atomic loads, issued after the counter's value has come back (the branch depends on it and
+    // device-scope loads, issued after the counter's value has come back (the branch depends on it and
     // a wavefront issues in order), read the finished partial tiles.  Nobody waits for anybody: a workgroup
     // that is not last leaves.  What this rests on is the hardware's behaviour, stated above, not the
     // language's memory model, which would ask for a release on (3) and an acquire in the reader; on this
@@ -134,26 +145,27 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
     arrived = __builtin_amdgcn_readfirstlane(arrived);
     if (arrived != (unsigned)splits - 1) return;
     if (wave == 0 && lane == 0) __hip_atomic_store(&counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // splits is a power of two >= 2: the partial tiles are requested as many at a time as there are up to sixteen values, and added
-    // in split order
-    const float *all = partials + (size_t)tile * splits * 1024 + wave * N * 64 + lane;
-    constexpr int AT_ONCE = N >= 8 ? 2 : N == 4 ? 4 : 8;
+    // the partial tiles are requested as many at a time as there are up to 32 values, and added in split order
 #pragma unroll
     for (int i = 0; i < N; i++) v[i] = 0.f;
-    for (int y = 0; y < splits; y += AT_ONCE) {
-      float p[AT_ONCE][N];
+    auto add_parts = [&](int y, auto at_once_c) {
+      constexpr int AT_ONCE = decltype(at_once_c)::value;
+      vec_t p[AT_ONCE][VECS];
 #pragma unroll
       for (int u = 0; u < AT_ONCE; u++)
 #pragma unroll
-        for (int i = 0; i < N; i++)
-          p[u][i] = __hip_atomic_load(all + (size_t)min(y + u, splits - 1) * 1024 + i * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int i = 0; i < VECS; i++)
+          p[u][i] = part_load<vec_t>(parts, y + u < splits ? mine + 256 * E * i : PART_NONE, first_part + 4096u * (unsigned)min(y + u, splits - 1));
 #pragma unroll
       for (int u = 0; u < AT_ONCE; u++)
-        if (y + u < splits) {
 #pragma unroll
-          for (int i = 0; i < N; i++) v[i] += p[u][i];
-        }
-    }
+        for (int i = 0; i < N; i++) v[i] += p[u][i / E][i % E];
+    };
+    constexpr int MOST = N <= 2 ? 16 : N == 4 ? 8 : N == 8 ? 4 : 2;
+    if (MOST > 4 && splits <= 4) add_parts(0, std::integral_constant<int, 4>{});
+    else
+      for (int y = 0; y < splits; y += MOST) add_parts(y, std::integral_constant<int, MOST>{});
+#endif
   }
   if (!col_ok) return;
   const int row0 = acc_row(m0, half, wave * N);  // the rows of a wavefront's registers: row0 + row_k(wave * N + i) - row_k(wave * N)
