@@ -834,6 +834,12 @@ def test_matmul_f32_shared_reduction(gpu, case):
     assert far(oc.matmul_nd_bias(gpu, a[None], b, bias, gelu=True)[0], 0.5 * exact * erfc(-exact / np.sqrt(2))) <= 2 * bound
 
 
+# where tiles of 32 rows are taken: rows and columns off them, one to three stages a wavefront, whole and split tiles side by side
+@pytest.mark.parametrize("case", [(128, 768, 2304), (97, 784, 3076), (100, 3088, 772), (161, 752, 2180), (130, 160, 12292), (520, 16, 16404)], ids=str)
+def test_matmul_f32_shared_reduction_of_few_rows(gpu, case):
+    test_matmul_f32_shared_reduction(gpu, case)
+
+
 def test_gelu_epilogue_against_64_bits(gpu):
     """A product with the identity is its left operand, so this is the epilogue's Gelu of chosen values: to 3 units of the last
     place of its argument (the formula's last two roundings and the fits' 2e-9), infinities and NaN as 0.5 x (1 + erf) has them."""
