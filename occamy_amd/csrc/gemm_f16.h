@@ -26,7 +26,7 @@ bool launch_gemm_f16_dma(const dnnrtContext *ctx, const GemmF16Args &g, int Z, b
 
 // ... and on tiles whose four wavefronts share the reduction (gemm_f16_waves.hip); launch_gemm_f16_dma, its caller, has checked
 // the forms.
-bool launch_gemm_f16_waves(const dnnrtContext *ctx, const GemmF16Args &g, int Z, int splits);
+bool launch_gemm_f16_waves(const dnnrtContext *ctx, const GemmF16Args &g, int Z, int rows, int splits);
 
 // Out[z][M,N] = alpha * op(A[z]) op(B[z]) + beta * C[z]; strides in elements,
 // 0 = operand shared by every z.

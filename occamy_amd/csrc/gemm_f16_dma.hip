@@ -20,6 +20,7 @@
 #include "gemm_f16.h"
 #include "partials.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace dnnrt {
@@ -407,22 +408,24 @@ bool launch_gemm_f16_dma(const dnnrtContext *ctx, const GemmF16Args &args, int Z
       if (best < 0 || cost < best_cost) { best = i; best_cost = cost; best_splits = s; g.steps_per_split = per; }
     }
   }
-  // The kernel whose wavefronts share the reduction: a stage of 32 k takes each of the four 0.43, what comes before and after
-  // them 0.3 more than here, a split's hand-over 2.3 and 0.25 per part.  One workgroup per compute unit: with two it is the
-  // slower one (384 x 768 x 3072 by 6 %).
+  // The kernel whose wavefronts share the reduction: a stage of 32 k takes each of the four 0.43, with tiles of 32 rows 0.36, what
+  // comes before and after them 0.3 more than here, a split's hand-over 2.3 and 0.25 per part (0.13).  One workgroup per compute
+  // unit of the XCD that gets the most tiles: with two it is the slower one (384 x 768 x 3072 by 6 %).
   const int stages = (int)ceil_div(g.K, 32);
-  const int64_t tiles = ceil_div(g.M, 64) * ceil_div(g.N, 64) * Z;
-  int waves_splits = 0;
-  for (int s = 1; s <= 16 && s <= stages && tiles * s <= ctx->num_cu; s++) {
-    if (s > 1 && (ctx->splitk_shared || tiles > ctx->splitk_max_tiles || tiles * s * 16384 > ctx->splitk_partial_bytes)) break;
-    const int per = (int)ceil_div(stages, s);
-    if (ceil_div(stages, per) != s) continue;
-    const double cost = 0.3 + 0.43 * (double)ceil_div(per, 4) + (s > 1 ? 2.3 + 0.25 * s : 0);
-    if (best < 0 || cost < best_cost) { best = 2; best_cost = cost; waves_splits = s; }
+  int waves_splits = 0, waves_rows = 0;
+  for (int rows = 64; rows >= 32; rows -= 32) {
+    const int64_t tiles = ceil_div(g.M, rows) * ceil_div(g.N, 64) * Z;
+    for (int s = 1; s <= 16 && s <= stages && ceil_div(tiles, 8) * s <= std::max(ctx->num_cu / 8, 1); s++) {
+      if (s > 1 && (ctx->splitk_shared || tiles > ctx->splitk_max_tiles || tiles * s * rows * 256 > ctx->splitk_partial_bytes)) break;
+      const int per = (int)ceil_div(stages, s);
+      if (ceil_div(stages, per) != s) continue;
+      const double cost = 0.3 + (rows == 64 ? 0.43 : 0.36) * (double)ceil_div(per, 4) + (s > 1 ? 2.3 + rows / 256.0 * s : 0);
+      if (best < 0 || cost < best_cost) { best = 2; best_cost = cost; waves_splits = s; waves_rows = rows; }
+    }
   }
   if (best < 0) return true;
   launched = true;
-  if (waves_splits) return launch_gemm_f16_waves(ctx, g, Z, waves_splits);
+  if (waves_splits) return launch_gemm_f16_waves(ctx, g, Z, waves_rows, waves_splits);
   switch (best) {
     case 0: return launch_gd<64, 64, 2, 2, 4>(ctx, g, Z, best_splits);
     default: return launch_gd<128, 128, 2, 4, 4>(ctx, g, Z, best_splits);

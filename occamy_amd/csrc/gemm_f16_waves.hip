@@ -2,15 +2,17 @@
 // GELU behind them (the forms of gemm_f16_dma.hip).
 //
 // What bounds such a product is a chain of latencies, and in gemm_f16_dma.hip most of it is the loop: a barrier, LDS reads and
-// their round trip per 64 k, every operand read by two wavefronts.  Here each of the four wavefronts owns the whole 64x64 tile
-// for a quarter of the reduction: a ring of two stages of 32 k that nobody else touches, so no barrier, every operand read
-// once, 16 MFMAs per stage and wavefront from 12 reads; the four sums meet in LDS at the end, where each lane gets eight
+// their round trip per 64 k, every operand read by two wavefronts.  Here each of the four wavefronts owns the whole tile, 64 columns
+// and 64 or 32 rows, for a quarter of the reduction: a ring of two or three stages of 32 k that nobody else touches, so no
+// barrier, every operand read once, 16 MFMAs per stage and wavefront from 12 reads; the four sums meet in LDS at the end, where each lane gets eight
 // neighbouring columns of two rows, bias and residual having been requested before the first load.
 //
 // Time of a workgroup, 384 x 768 x 2304 (us): set-up 0.5, first data 1.0, six stages 2.5, sums 0.6, epilogue and code fetched on the way 1.0.
 // Rings of four stages gained in the loop what they lost waiting for the first data; 96 rows per tile cost 1.2 more per
-// launch and never paid.  K x N, us on gemm_f16_dma.hip -> here, back to back on one card: 384 rows, 768 x 2304 7.0 -> 6.6;
-// 768 x 768 7.0 -> 6.2; 3072 x 768 11.2 -> 10.1; 128 rows, 768 x 3072 + GELU 7.1 -> 6.8; 16 rows, 768 x 768 6.4 -> 5.6.
+// launch and never paid.  32 rows are taken where they spare a split reduction its hand-over, or make one of it with half the
+// bytes (us, 64 rows alone and with 32): 384 rows, 768 x 768 6.4 -> 5.2; 128 rows, 768 x 2304 6.7 -> 5.3, 768 x 3072 7.1 -> 5.6,
+// 3072 x 768 9.3 -> 7.9; 16 rows 6.0 -> 5.0, 6.2 -> 5.5, 8.4 -> 6.8; BERT at 384 tokens 564 -> 548.  K x N, us on gemm_f16_dma.hip
+// -> here with 64 rows, back to back on one card: 384 rows, 768 x 2304 7.0 -> 6.6; 3072 x 768 11.2 -> 10.1.
 #include "gemm_f16.h"
 #include "partials.h"
 
@@ -27,7 +29,9 @@ typedef __attribute__((address_space(3))) void *gw_lds;
 
 [[maybe_unused]] constexpr unsigned GW_OUT_OF_RANGE = 0x80000000u;  // above every num_records used here: reads as zeros
 constexpr int GW_BK = 32;                      // k of a stage
-[[maybe_unused]] constexpr int GW_NS = 2;      // stages of a wavefront's ring
+constexpr int gw_ring(int tm) { return tm == 2 ? 2 : 3; }                       // stages of a wavefront's ring
+constexpr int gw_stage(int tm) { return (64 + 32 * tm) * GW_BK * 2; }            // bytes of a stage
+constexpr int gw_wave(int tm) { return tm == 2 ? 64 * 64 * 4 : 3 * gw_stage(1); }  // a wavefront's LDS: its ring and, later, its sums
 
 template <int N>
 __device__ __forceinline__ void gw_wait_vmcnt() {  // LDS accesses stay on their side of it
@@ -60,13 +64,13 @@ __device__ __forceinline__ void gw_arrived(T &v) {
   asm volatile("" : "+v"(v));
 }
 
-// Tiles of 64 columns n and 64 rows m; B_KC: B stored [N,K].
-template <bool B_KC>
+// Tiles of 64 columns n and 32 TM rows m; B_KC: B stored [N,K].
+template <bool B_KC, int TM>
 __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Args a, const int tiles) {
 #if __HIP_DEVICE_COMPILE__
-  constexpr int NS = GW_NS, TM = 2, FM = 32 * TM, STAGE = (64 + FM) * GW_BK * 2, WAVE_LDS = FM * 64 * 4;
+  constexpr int NS = gw_ring(TM), FM = 32 * TM, STAGE = gw_stage(TM), WAVE_LDS = gw_wave(TM);
   constexpr int M_L = FM / 16, L = 4 + M_L;  // loads of a stage
-  static_assert(NS * STAGE <= WAVE_LDS, "a wavefront's ring and, later, its sums");
+  static_assert(NS * STAGE <= WAVE_LDS && FM * 64 * 4 <= WAVE_LDS, "a wavefront's ring and, later, its sums");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
 
   const int per_xcd = (tiles + 7) >> 3;  // consecutive tiles (all rows m of one column range) on one XCD share B in its L2
@@ -196,6 +200,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
   };
   constexpr std::integral_constant<int, 0> c0{};
   constexpr std::integral_constant<int, 1> c1{};
+  auto landed = [&](int behind) {  // the oldest stage in flight has landed, up to NS - 1 behind it may still be on their way
+    if (behind >= NS - 1) gw_wait_vmcnt<(NS - 1) * L>();
+    else if (NS > 2 && behind == 1) gw_wait_vmcnt<L>();
+    else gw_wait_vmcnt<0>();
+  };
   // One stage, its operands in set S or on their way there; `ahead` follow it.
   auto step = [&](auto set_c, int ahead) {
     constexpr int S = decltype(set_c)::value;
@@ -214,8 +223,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
     multiply(set_c, c0);
     __builtin_amdgcn_sched_barrier(0);
     if (ahead > 0) {
-      if (ahead > 1) gw_wait_vmcnt<L>();  // the next stage has landed, the one behind it may still be on its way
-      else gw_wait_vmcnt<0>();
+      landed(ahead - 1);
       read_stage(std::integral_constant<int, 1 - S>{});
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -223,13 +231,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
     __builtin_amdgcn_sched_barrier(0);
   };
   if (nk > 0) {
-    issue_stage();
-    if (nk > 1) {
-      issue_stage();
-      gw_wait_vmcnt<L>();
-    } else {
-      gw_wait_vmcnt<0>();
-    }
+#pragma unroll
+    for (int i = 0; i < NS; i++)
+      if (i < nk) issue_stage();
+    landed(nk - 1);
     read_stage(c0);
     int ahead = nk - 1;
 #pragma unroll 1
@@ -326,19 +331,33 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
 #endif
 }
 
-bool launch_gemm_f16_waves(const dnnrtContext *ctx, const GemmF16Args &args, int Z, int splits) {
+template <bool B_KC, int TM>
+static bool launch_one(const dnnrtContext *ctx, const GemmF16Args &g, const dim3 &grid, int tiles) {
+  constexpr int SMEM = 4 * gw_wave(TM);
+  if constexpr (SMEM > 64 * 1024) {
+    static LdsRaised raised;
+    if (!raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&gemm_f16_waves_kernel<B_KC, TM>), SMEM)) {
+      set_error("matmul(fp16): cannot reserve %d bytes of LDS", SMEM);
+      return false;
+    }
+  }
+  hipLaunchKernelGGL((gemm_f16_waves_kernel<B_KC, TM>), grid, dim3(256), SMEM, ctx->stream, g, tiles);
+  return true;
+}
+
+bool launch_gemm_f16_waves(const dnnrtContext *ctx, const GemmF16Args &args, int Z, int rows, int splits) {
   GemmF16Args g = args;
-  const int tiles = (int)(ceil_div(g.M, 64) * ceil_div(g.N, 64)), stages = (int)ceil_div(g.K, GW_BK);
+  const int tiles = (int)(ceil_div(g.M, rows) * ceil_div(g.N, 64)), stages = (int)ceil_div(g.K, GW_BK);
   g.steps_per_split = (int)ceil_div(stages, splits);
   splits = (int)ceil_div(stages, g.steps_per_split);  // no empty split: every arrival carries a partial tile
-  if (splits > 1 && ((int64_t)tiles * Z * splits * 16384 > ctx->splitk_partial_bytes || (int64_t)tiles * Z > ctx->splitk_max_tiles)) {
+  if (splits > 1 && ((int64_t)tiles * Z * splits * rows * 256 > ctx->splitk_partial_bytes || (int64_t)tiles * Z > ctx->splitk_max_tiles)) {
     set_error("matmul(fp16): %d parts of %d tiles do not fit the reduction scratch", splits, tiles);
     return false;
   }
   const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8), (unsigned)splits, (unsigned)Z);
-  constexpr int SMEM = 4 * 64 * 64 * 4;
-  if (g.b_sk == 1) hipLaunchKernelGGL((gemm_f16_waves_kernel<true>), grid, dim3(256), SMEM, ctx->stream, g, tiles);
-  else hipLaunchKernelGGL((gemm_f16_waves_kernel<false>), grid, dim3(256), SMEM, ctx->stream, g, tiles);
+  const bool done = g.b_sk == 1 ? (rows == 64 ? launch_one<true, 2>(ctx, g, grid, tiles) : launch_one<true, 1>(ctx, g, grid, tiles))
+                                : (rows == 64 ? launch_one<false, 2>(ctx, g, grid, tiles) : launch_one<false, 1>(ctx, g, grid, tiles));
+  if (!done) return false;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("matmul(fp16): launch failed: %s", hipGetErrorString(e)); return false; }
   return true;

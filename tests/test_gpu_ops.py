@@ -811,6 +811,13 @@ def test_matmul_f16_shared_reduction(gpu, case, trans_b):
     np.testing.assert_allclose(got, exact, rtol=2.0 ** -11, atol=2.0 ** -16)
 
 
+# both heights of its tiles: rows off them, whole and split reductions, a partial last stage, one to four of its wavefronts without any
+@pytest.mark.parametrize("case", [(384, 768, 2304), (383, 808, 2312), (385, 776, 776), (200, 3080, 776), (33, 768, 3080), (31, 1032, 64), (97, 72, 8200)], ids=str)
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_matmul_f16_shared_reduction_heights(gpu, case, trans_b):
+    test_matmul_f16_shared_reduction(gpu, case, trans_b)
+
+
 # rows and columns off the tiles, one stage of 16 k (three wavefronts without any), a few, odd and even counts, whole tiles
 # beside split ones, a handful of split tiles
 @pytest.mark.parametrize("case", [(4100, 16, 3104), (1030, 48, 4100), (300, 336, 2052), (161, 1296, 1000), (384, 768, 3072), (128, 3072, 768), (65, 6160, 132)], ids=str)
