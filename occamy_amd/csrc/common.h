@@ -11,7 +11,7 @@
 #include "../../include/dnnrt.h"
 #include "lds_limit.h"
 
-// A cut of an fp32 inverted residual block (conv_f32_block.hip) and the sizes it was found for.
+// A cut of an inverted residual block (conv_f16_block.hip, conv_f32_block.hip) and the sizes it was found for.
 struct dnnrtBlockCut {
   int64_t sizes[11];
   int nb, qw, waves, splits;

@@ -18,22 +18,44 @@
 // are read in blocks of 32 rows and 8 columns (512 contiguous bytes), the order the executor uploads them in: rows of the
 // plain matrix would cost a cache line per lane and load, and took longer than everything else.
 //
-// What bounds it: vector instructions and LDS accesses about evenly where tiles are many, at three wavefronts per SIMD; where
-// they are few, a launch's own 8 us and the 3.5 to 5 us of a round.
+// Where the tiles are few the hidden channels are also cut over workgroups (gridDim.z): partial sums through the handle's
+// scratch, the last to arrive adds them in order.
 //
-// Measured against the three calls at batch 64 (us): 16 -> 96 -> 24 channels, 112x112 stride 2: 104 -> 54; 24 -> 144 -> 24 at
-// 56x56: 85 -> 48; 24 -> 144 -> 32 stride 2: 52 -> 30; 32 -> 192 -> 32 at 28x28: 34 -> 17; 64 -> 384 -> 64 at 14x14: 34 -> 15.5;
-// 96 -> 576 -> 96: 38 -> 22.5; 32 -> 16 behind a depthwise layer at 112x112, no expansion: 49 -> 36.5.  MobileNetV2 0.77 -> 0.50 ms.
-// 160 -> 960 -> 160 at 7x7 was slower (64 workgroups, 34 against 30) and is left to the three calls.
+// What bounds it: where tiles are many, vector instructions (24 -> 144 -> 24 at 56x56, three wavefronts per SIMD: a round of 7500
+// cycles is 650 of them a wavefront, the depthwise sums 288) or, with stride 2, the LDS of a tile's slabs, which leaves one and
+// a half wavefronts per SIMD; where they are few, the chain of a launch: 3500 cycles until the patch is there, 2500 for the
+// filters, 5000 to 8000 a round, 3000 for the result, 6000 to 11000 for a hand-over (160 -> 960 -> 160 at 7x7, batch 64, four parts).
+//
+// Measured against the three calls at batch 64 (us): 16 -> 96 -> 24 channels, 112x112 stride 2: 104 -> 55; 24 -> 144 -> 24 at
+// 56x56: 85 -> 42; 24 -> 144 -> 32 stride 2: 52 -> 29; 32 -> 192 -> 32 at 28x28: 34 -> 17; 64 -> 384 -> 64 at 14x14: 34 -> 15.5;
+// 96 -> 576 -> 96: 38 -> 22; 32 -> 16 behind a depthwise layer at 112x112, no expansion: 49 -> 37; 160 -> 960 -> 160 at 7x7 30 -> 20.3
+// (30.5 uncut).  MobileNetV2, whole channels and cut: batch 1 249 -> 213, 4 296 -> 243, 8 315 -> 255, 16 358 -> 283, 32 378 -> 350,
+// 64 510 -> 482.
 #include "conv_f16.h"
 #include "dnnrt_exec.h"
+#include "partials.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace dnnrt {
 
 bool block_f32_applies(const dnnrtContext *ctx, const dnnrtExecBlock &k);  // conv_f32_block.hip
 bool launch_block_f32(const dnnrtContext *ctx, const dnnrtExecBlock &k);
+
+// The handle's ring of cuts, for both types.
+const dnnrtBlockCut *find_block_cut(const dnnrtContext *ctx, const int64_t (&sizes)[11]) {
+  constexpr unsigned KEPT = sizeof(ctx->block_cuts) / sizeof(ctx->block_cuts[0]);
+  for (unsigned i = 0; i < std::min(ctx->block_cuts_found, KEPT); i++)
+    if (std::equal(sizes, sizes + 11, ctx->block_cuts[i].sizes)) return &ctx->block_cuts[i];
+  return nullptr;
+}
+void keep_block_cut(const dnnrtContext *ctx, const int64_t (&sizes)[11], dnnrtBlockCut cut) {
+  constexpr unsigned KEPT = sizeof(ctx->block_cuts) / sizeof(ctx->block_cuts[0]);
+  std::copy(sizes, sizes + 11, cut.sizes);
+  ctx->block_cuts[ctx->block_cuts_found % KEPT] = cut;
+  ctx->block_cuts_found = ctx->block_cuts_found + 1 < 2 * KEPT ? ctx->block_cuts_found + 1 : KEPT;  // stays past KEPT once it is there
+}
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
@@ -47,6 +69,7 @@ struct BlockF16Args {
   int TH, TW, QH, QW, PH, PW;      // tile, its 2 x 2 squares, its patch
   int xs_bytes, slab_bytes, xrow;  // LDS: input patch, a wavefront's slab; bytes of an input pixel
   int tiles_w, tiles_hw, tiles, per_xcd, blocks_y;  // blocks_y: blocks of 32 output channels per workgroup
+  int per_split, part_px;          // groups of 32 hidden channels of a part (gridDim.z of them); pixels of a partial tile
   unsigned magic_tiles_w, magic_tiles_hw, magic_qw, magic_c8;
   unsigned lo1, hi1, lod, hid;  // the inner activations as clamps, twice in a word
   float lo, hi;
@@ -80,13 +103,15 @@ __device__ __forceinline__ void lds_barrier() {
 // S: the depthwise stride.  KC: steps of 16 input channels (0: no expansion, X holds the hidden channels).  GM: most
 // wavefronts of a workgroup.
 template <int S, int KC, int GM>
-__global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2 ? 3 : 2))) void conv_f16_block_kernel(const BlockF16Args a) {
+__global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2 ? 3 : 2))) void conv_f16_block_kernel(const BlockF16Args a, float *partials,
+                                                                                                                       unsigned *counters) {
   constexpr bool EXPAND = KC > 0;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = (int)(blockDim.x >> 6);
   char *Xs = smem, *slabs = smem + a.xs_bytes, *mine = slabs + wave * a.slab_bytes;
-  const int groups = (a.Ch + 31) >> 5;
+  // this workgroup's groups of 32 hidden channels: from group0 on
+  const int group0 = (int)blockIdx.z * a.per_split, groups = min(a.per_split, ((a.Ch + 31) >> 5) - group0);
   float *B1 = reinterpret_cast<float *>(slabs + G * a.slab_bytes), *Bd = B1 + 32 * groups;  // the inner biases, padded to the last group's end
   _Float16 *Wd = reinterpret_cast<_Float16 *>(Bd + 32 * groups);  // the depthwise filters, [channel][tap]
 
@@ -112,7 +137,9 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
   // The input patch, the depthwise filters and the inner biases to LDS: everything is requested before anything is stored
   // (as loops of load and store, four to six times the latency of memory before the first product).
   {
-    const auto x_rsrc = rsrc_of(Xn, a.H * a.W * a.Cin), wd_rsrc = rsrc_of(a.Wd, 9 * a.Ch), b1_rsrc = rsrc_of(a.b1, a.Ch), bd_rsrc = rsrc_of(a.bd, a.Ch);
+    const int from = 32 * group0;
+    const auto x_rsrc = rsrc_of(Xn, a.H * a.W * a.Cin), wd_rsrc = rsrc_of(a.Wd + 9 * from, 9 * (a.Ch - from));
+    const auto b1_rsrc = rsrc_of(a.b1 ? a.b1 + from : nullptr, a.Ch - from), bd_rsrc = rsrc_of(a.bd ? a.bd + from : nullptr, a.Ch - from);
     constexpr int XU = EXPAND ? 6 : 0, WU = 3, BU = 3;
     const int c8n = a.Cin >> 3, x_units = EXPAND ? NP * c8n : 0, w_units = 36 * groups, b_units = 32 * groups, step = 64 * G;
     for (int x0 = tid, w0 = tid, b0 = tid; x0 < x_units || w0 < w_units || b0 < b_units; x0 += XU * step, w0 += WU * step, b0 += BU * step) {
@@ -165,7 +192,7 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
 #pragma unroll
       for (int k = 0; k < KC; k++) wa[k] = load_rows(w1_rsrc, a.Ch, a.Cin, g, 16 * k + 8 * half);
   };
-  load_expand(min(wave, groups - 1));
+  load_expand(group0 + min(wave, groups - 1));
 
   // projection: a wavefront's block of 32 output channels; its 32 pixels of the tile, or all 64 where the wavefronts do not
   // suffice for twice the blocks
@@ -174,7 +201,7 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
   const int pm = pairs ? wave >> 1 : wave, ppx = pairs ? 32 * (wave & 1) : 0;
   floatx16 acc[2];
   {
-    const auto b3_rsrc = rsrc_of(a.b3, a.Cout);
+    const auto b3_rsrc = rsrc_of(blockIdx.z == 0 ? a.b3 : nullptr, a.Cout);  // in the first part's sums
 #pragma unroll
     for (int gq = 0; gq < 4; gq++) {
       const half4 v = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(b3_rsrc, 2 * (32 * (mfirst + pm) + 8 * gq + 4 * half), 0, 0));
@@ -185,14 +212,14 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
   __syncthreads();
 
   for (int first = 0; first < groups; first += G) {
-    const int g = first + wave, ch = 32 * g;
+    const int g = first + wave, ch = 32 * (group0 + g), own = 32 * g;  // hidden channels; theirs among the workgroup's
     half8 wp[2 * GM];  // the projection's filter for this round, requested well ahead where registers allow
     auto load_project = [&]() {
 #pragma unroll
       for (int q = 0; q < GM; q++)
 #pragma unroll
         for (int k = 0; k < 2; k++) {
-          const int c = 32 * (first + q) + 16 * k + 8 * half;
+          const int c = 32 * (group0 + first + q) + 16 * k + 8 * half;
           wp[2 * q + k] = load_rows(w3_rsrc, a.Cout, a.Ch, mfirst + min(pm, mblocks - 1), q < G ? c : a.Ch);
         }
     };
@@ -205,7 +232,7 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
         floatx16 bias;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-          const float4 v = *reinterpret_cast<const float4 *>(B1 + ch + 8 * q + 4 * half);
+          const float4 v = *reinterpret_cast<const float4 *>(B1 + own + 8 * q + 4 * half);
           bias[4 * q] = v.x; bias[4 * q + 1] = v.y; bias[4 * q + 2] = v.z; bias[4 * q + 3] = v.w;
         }
         for (int p = 0; p < NP; p += 32) {
@@ -228,7 +255,7 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
             if (px < NP) *reinterpret_cast<uint2 *>(mine + at * SLAB_PX + 16 * q + 8 * half) = o;
           }
         }
-        load_expand(min(g + G, groups - 1));
+        load_expand(group0 + min(g + G, groups - 1));
       } else {
         for (int u = lane; u < NP * 4; u += 64) {
           const int px = u >> 2, q = u & 3, r = row_of(px), c = ch + 8 * q;
@@ -241,11 +268,11 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
       constexpr int WIN = 3 + S;  // rows and columns of input under a square
       half8 w[9];  // filter e of the eight, tap t: value 9 e + t
 #pragma unroll
-      for (int i = 0; i < 9; i++) w[i] = *reinterpret_cast<const half8 *>(Wd + (ch + 8 * cg) * 9 + 8 * i);
+      for (int i = 0; i < 9; i++) w[i] = *reinterpret_cast<const half8 *>(Wd + (own + 8 * cg) * 9 + 8 * i);
       float sum[4][8];
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        const float bv = Bd[ch + 8 * cg + e];
+        const float bv = Bd[own + 8 * cg + e];
 #pragma unroll
         for (int o = 0; o < 4; o++) sum[o][e] = bv;
       }
@@ -299,14 +326,73 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
     if (first + G < groups) lds_barrier();
   }
 
+  auto place = [&](int px, int &p, int &q) -> bool {  // the tile's pixel px in the image
+    const int sq = px >> 2, py = div_magic(sq, a.QW, a.magic_qw);
+    p = p0 + 2 * py + (px >> 1 & 1);
+    q = q0 + 2 * (sq - py * a.QW) + (px & 1);
+    return py < a.QH && p < a.P && q < a.Q;
+  };
+  // ---- hidden channels cut over workgroups: partial sums through the handle's scratch (igemm_f32_small.hip states what the
+  // hand-over rests on), [block of channels][four of them][pixel]; the last to arrive adds the parts in order and goes on
+#if __HIP_DEVICE_COMPILE__
+  if (const int parts = (int)gridDim.z; parts > 1) {
+    const __amdgpu_buffer_rsrc_t rsrc = part_rsrc(partials);
+    const unsigned slot = blockIdx.y * (unsigned)a.tiles + (unsigned)tile, part_bytes = (unsigned)a.blocks_y * 128u * (unsigned)a.part_px;
+    const int across = min(a.TW, a.Q);
+    unsigned at[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      int p, q;
+      const bool ok = place(ppx + 32 * t + l32, p, q) && pm < mblocks && (t == 0 || !pairs);
+      at[t] = ok ? 16u * (unsigned)((pm * 8 + half) * a.part_px + (p - p0) * across + q - q0) : PART_NONE;
+    }
+    const unsigned step = 32u * (unsigned)a.part_px;  // from four channels of a lane to the next
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int gq = 0; gq < 4; gq++)
+        if (t == 0 || !pairs)
+          part_store(rsrc, at[t], (slot * parts + blockIdx.z) * part_bytes + gq * step, part_floatx4{acc[t][4 * gq], acc[t][4 * gq + 1], acc[t][4 * gq + 2], acc[t][4 * gq + 3]});
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();
+    volatile unsigned *arrived = reinterpret_cast<unsigned *>(smem);
+    if (tid == 0) *arrived = __hip_atomic_fetch_add(&counters[slot], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*arrived != (unsigned)parts - 1) return;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    if (tid == 0) __hip_atomic_store(&counters[slot], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[t][r] = 0.f;
+    for (int y = 0; y < parts; y += 2) {  // two parts in flight
+      part_floatx4 v[2][2][4];
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int gq = 0; gq < 4; gq++)
+            v[u][t][gq] = part_load<part_floatx4>(rsrc, y + u < parts ? at[t] : PART_NONE, (slot * parts + (unsigned)min(y + u, parts - 1)) * part_bytes + gq * step);
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[t][r] += v[u][t][r >> 2][r & 3];
+    }
+  }
+#endif
+
   // ---- residual, activation: the lane's pixel, four consecutive channels per access ------------------------------
   if (pm >= mblocks) return;
 #pragma unroll
   for (int t = 0; t < 2; t++) {
     if (t == 1 && pairs) break;
-    const int px = ppx + 32 * t + l32, sq = px >> 2, py = div_magic(sq, a.QW, a.magic_qw);
-    const int p = p0 + 2 * py + (px >> 1 & 1), q = q0 + 2 * (sq - py * a.QW) + (px & 1);
-    if (py >= a.QH || p >= a.P || q >= a.Q) continue;
+    int p, q;
+    if (!place(ppx + 32 * t + l32, p, q)) continue;
     const int c0y = 32 * (mfirst + pm) + 4 * half;
     const int64_t at = (((int64_t)n * a.P + p) * a.Q + q) * a.Cout + c0y;
     half4 z[4] = {};
@@ -345,7 +431,8 @@ constexpr int BLOCK_PER_GROUP = 2 * 32 * 4 + 32 * 9 * 2;  // biases and depthwis
 
 // grid_y, G: workgroups per tile, wavefronts per workgroup
 // `faster`: refuse what the separate calls do sooner.
-static bool plan_block_f16(int num_cu, const dnnrtExecBlock &k, bool faster, BlockF16Args &a, int &kc, int &grid_y, int &G) {
+static bool plan_block_f16(const dnnrtContext *ctx, const dnnrtExecBlock &k, bool faster, BlockF16Args &a, int &kc, int &grid_y, int &G, int &parts) {
+  const int num_cu = ctx->num_cu;
   if (k.dtype != DNNRT_F16 || k.format != DNNRT_NHWC || k.r != 3 || k.s != 3 || (k.stride != 1 && k.stride != 2) || k.cin % 8 || k.ch % 8 || k.cout % 8) return false;
   if (!k.expand && k.cin != k.ch) return false;
   // Every tile's patch must hold a row and a column of the image (the kernel divides by their number, and with none it would
@@ -359,7 +446,7 @@ static bool plan_block_f16(int num_cu, const dnnrtExecBlock &k, bool faster, Blo
   a.lo = k.act == DNNRT_ACT_IDENTITY ? -__builtin_inff() : 0.f;
   a.hi = k.act == DNNRT_ACT_CLIPPED_RELU ? k.coef : __builtin_inff();
   const int steps = (int)ceil_div(k.cin, 16);
-  kc = !k.expand ? 0 : steps <= 1 ? 1 : steps <= 2 ? 2 : steps <= 4 ? 4 : steps <= 6 ? 6 : -1;
+  kc = !k.expand ? 0 : steps <= 1 ? 1 : steps <= 2 ? 2 : steps <= 4 ? 4 : steps <= 6 ? 6 : steps <= 10 ? 10 : -1;
   if (kc < 0) return false;
   a.N = (int)k.n; a.H = (int)k.h; a.W = (int)k.w; a.Cin = (int)k.cin; a.Ch = (int)k.ch; a.P = (int)k.p; a.Q = (int)k.q; a.Cout = (int)k.cout;
   a.ph = (int)k.pad_h; a.pw = (int)k.pad_w;
@@ -369,40 +456,58 @@ static bool plan_block_f16(int num_cu, const dnnrtExecBlock &k, bool faster, Blo
   a.blocks_y = (int)ceil_div(mall, grid_y);
   const int most = kc <= 2 ? 4 : 8;  // wavefronts, the kernel's GM
   if (a.blocks_y > most) return false;
-  // Tile and wavefronts by estimated time: vector instructions, with the lanes and wavefronts that idle counted as busy,
-  // and what a launch and a round wait for (fitted at batch 64: 14x14, 64 -> 384 -> 64 channels 15.5 us, 96 -> 576 22).
-  double best = 0;
-  for (int qw = 1; qw <= 16 && (qw == 1 || 2 * (qw - 1) < a.Q); qw++) {
+  // Tile, wavefronts and parts by estimated time, fitted to 6300 cuts of MobileNetV2's twelve kinds of blocks at batch 1, 4, 16, 32
+  // and 64, 6 .. 60 us, within 8 % on the whole; the cut it picks takes 3 % more than the best of them on average.  What counts
+  // is what a round waits for, less what it computes.
+  auto cut = [&](int qw, int g, int n_parts, BlockF16Args &o) -> double {  // microseconds; 0: cannot be
     const int qh = std::min(16 / qw, (a.P + 1) / 2), tw = 2 * qw, th = 2 * qh;
     const int pw = (tw - 1) * (int)k.stride + 3, ph = (th - 1) * (int)k.stride + 3, np = pw * ph;
     const int xs = (int)ceil_div(np, 32) * 32 * a.xrow, slab = std::max(np, 64) * SLAB_PX;
-    const double tiles = (double)a.N * (double)ceil_div(a.P, th) * (double)ceil_div(a.Q, tw) * grid_y;
-    const int in = std::min(ph, a.H) * std::min(pw, a.W);
-    for (int g = a.blocks_y; g <= most; g++) {
-      if (g > a.blocks_y && g > groups) break;
-      const int lds = xs + g * slab + BLOCK_PER_GROUP * groups;
-      if (lds > BLOCK_LDS) break;
-      const double rounds = (double)ceil_div(groups, g);
-      const double per_round = 450 + (k.expand ? 75.0 + 10 * kc : 20.0) * (double)ceil_div(in, 32) + 60;
-      const int per_cu = std::min(160 * 1024 / lds, (kc <= 2 ? 12 : 8) / g);  // two or three wavefronts per SIMD
-      if (per_cu < 1) continue;
-      // what a compute unit has at a time, and how long that takes: four SIMDs, each busy at least a round's latency
-      const double at_once = std::min((double)per_cu, std::max(1.0, tiles / num_cu));
-      const double waves = at_once * g / 4;
-      const double cost = (rounds * std::max(waves, 2.0) * per_round + 1000) * std::max(1.0, tiles / (at_once * num_cu));
-      const double us = 8 + 4 * 1.3 / 2400 * cost + (kc > 4 ? 0.35 * (kc - 4) * rounds : 0.0) * std::max(1.0, tiles / (at_once * num_cu));
-      if (best == 0 || us < best) {
-        best = us;
-        a.TH = th; a.TW = tw; a.QH = qh; a.QW = qw; a.PH = ph; a.PW = pw; a.xs_bytes = xs; a.slab_bytes = slab; G = g;
-      }
-    }
+    const int per = (int)ceil_div(groups, n_parts);
+    if (ceil_div(groups, per) != n_parts) return 0;
+    const int lds = xs + g * slab + BLOCK_PER_GROUP * per;
+    if (lds > BLOCK_LDS) return 0;
+    const double tiles = (double)a.N * (double)ceil_div(a.P, th) * (double)ceil_div(a.Q, tw) * grid_y, units = tiles * n_parts;
+    const int in = std::min(ph, a.H) * std::min(pw, a.W), part_px = std::min(th, a.P) * std::min(tw, a.Q);
+    const double part_bytes = a.blocks_y * 128.0 * part_px;
+    if (n_parts > 1 && (ctx->splitk_shared || tiles > ctx->splitk_max_tiles || units * part_bytes > (double)ctx->splitk_partial_bytes)) return 0;
+    const double rounds = (double)ceil_div(per, g);
+    const double per_round = (k.stride == 1 ? 520.0 : 1880.0) + 28.0 * kc * (double)ceil_div(in, 32);  // cycles of a wavefront beside others
+    const int per_cu = std::min(160 * 1024 / lds, (kc <= 2 ? 12 : 8) / g);  // two or three wavefronts per SIMD
+    if (per_cu < 1) return 0;
+    // what a compute unit has at a time, and how long that takes
+    const double at_once = std::min((double)per_cu, std::max(1.0, units / num_cu));
+    const double turns = std::max(1.0, units / (at_once * num_cu)), turn = rounds * (per_round * at_once * g / 4 + 7560 + 72.0 * kc * g) + 6290;
+    o.TH = th; o.TW = tw; o.QH = qh; o.QW = qw; o.PH = ph; o.PW = pw; o.xs_bytes = xs; o.slab_bytes = slab; o.per_split = per; o.part_px = part_px;
+    return 0.95 + 0.43 * a.blocks_y + turn * (turns + 0.81 * (std::ceil(turns) - turns)) / 2300 + (n_parts > 1 ? 2.7 + n_parts * part_bytes / 4.4e4 : 0.0);
+  };
+  const int64_t sizes[11] = {k.n, k.cin, k.h, k.w, k.ch, k.cout, k.stride, k.pad_h, k.pad_w, k.expand + 2 * k.dtype, ctx->splitk_partial_bytes};
+  double best = 0;
+  if (const dnnrtBlockCut *f = find_block_cut(ctx, sizes)) {
+    best = cut(f->qw, f->waves, f->splits, a);
+    G = f->waves;
+    parts = f->splits;
   }
-  if (best == 0) return false;
-  // What the separate calls take, in microseconds: a launch each, and their bytes and products at the rates they reach.
+  if (best == 0) {
+    BlockF16Args t = a;
+    int best_qw = 0;
+    for (int qw = 1; qw <= 16 && (qw == 1 || 2 * (qw - 1) < a.Q); qw++)
+      for (int g = std::max(a.blocks_y, k.expand ? 2 : 1); g <= most && (g == a.blocks_y || g <= std::max(groups, 2)); g++)
+        for (int n = 1; n <= groups && n <= 32; n++) {
+          const double us = cut(qw, g, n, t);
+          if (us > 0 && (best == 0 || us < best)) { best = us; best_qw = qw; G = g; parts = n; }
+          if ((double)a.N * (double)(ceil_div(a.P, 2 * std::min(16 / qw, (a.P + 1) / 2)) * ceil_div(a.Q, 2 * qw)) * grid_y * n >= 2.0 * num_cu) break;  // enough of them
+        }
+    if (best == 0) return false;
+    cut(best_qw, G, parts, a);
+    keep_block_cut(ctx, sizes, dnnrtBlockCut{{}, 0, best_qw, G, parts});
+  }
+  // What the separate calls take inside a network, in microseconds (MobileNetV2's at batch 1, 8, 16 and 32, within a fifth): a
+  // launch each, their megabytes, and the projection's long reduction on few tiles (up to 64 pixels have a kernel of their own).
   const double in_px = (double)a.N * a.H * a.W, out_px = (double)a.N * a.P * a.Q;
-  const double us1 = k.expand ? std::max(4.5, 2 + in_px * (a.Cin + a.Ch) * 2 / 2.8e6 + 2 * in_px * a.Cin * a.Ch / 150e6) : 0;
-  const double usd = std::max(4.5, 2 + (in_px + out_px) * a.Ch * 2 / 2.8e6);
-  const double us3 = std::max(4.5, 2 + out_px * (a.Ch + a.Cout) * 2 / 2.8e6 + 2 * out_px * a.Ch * a.Cout / 150e6);
+  const double mb1 = in_px * (a.Cin + a.Ch) * 2e-6, mbd = (in_px + out_px) * a.Ch * 2e-6, mb3 = out_px * (a.Ch + a.Cout) * 2e-6;
+  const double us1 = k.expand ? 3.8 + std::min(1.2, 2 * mb1) + 0.55 * mb1 : 0, usd = 4.8 + 0.35 * mbd;
+  const double us3 = 3.6 + (out_px <= 64 ? 0.0015 : 0.0055) * a.Ch + 0.2 * mb3;
   if (faster && best > 0.95 * (us1 + usd + us3)) return false;
   a.tiles_w = (int)ceil_div(a.Q, a.TW);
   a.tiles_hw = a.tiles_w * (int)ceil_div(a.P, a.TH);
@@ -414,8 +519,8 @@ static bool plan_block_f16(int num_cu, const dnnrtExecBlock &k, bool faster, Blo
 
 bool block_f16_applies(const dnnrtContext *ctx, const dnnrtExecBlock &k) {
   BlockF16Args a{};
-  int kc, gy, g;
-  return plan_block_f16(ctx->num_cu, k, true, a, kc, gy, g);
+  int kc, gy, g, parts;
+  return plan_block_f16(ctx, k, true, a, kc, gy, g, parts);
 }
 
 template <int S, int KC, int GM>
@@ -425,34 +530,38 @@ static bool launch_one(const dnnrtContext *ctx, dim3 grid, dim3 threads, size_t 
     set_error("inverted residual block (fp16): cannot reserve %d bytes of LDS", BLOCK_LDS);
     return false;
   }
-  hipLaunchKernelGGL((conv_f16_block_kernel<S, KC, GM>), grid, threads, lds, ctx->stream, a);
+  hipLaunchKernelGGL((conv_f16_block_kernel<S, KC, GM>), grid, threads, lds, ctx->stream, a, ctx->splitk_partials, ctx->splitk_counters);
   return true;
 }
 
-bool launch_block_f16(const dnnrtContext *ctx, const dnnrtExecBlock &k) {
-  BlockF16Args a{};
-  int kc, gy, g;
-  if (!plan_block_f16(ctx->num_cu, k, false, a, kc, gy, g)) { set_error("inverted residual block (fp16): not a shape this kernel takes"); return false; }
+static bool launch_cut(const dnnrtContext *ctx, const dnnrtExecBlock &k, BlockF16Args &a, int kc, int gy, int g, int parts) {
   a.X = static_cast<const _Float16 *>(k.x); a.W1 = static_cast<const _Float16 *>(k.w1); a.b1 = static_cast<const _Float16 *>(k.b1);
   a.Wd = static_cast<const _Float16 *>(k.wd); a.bd = static_cast<const _Float16 *>(k.bd);
   a.W3 = static_cast<const _Float16 *>(k.w3); a.b3 = static_cast<const _Float16 *>(k.b3);
   a.Z = static_cast<const _Float16 *>(k.z); a.Y = static_cast<_Float16 *>(k.y);
   for (const void *q : {k.x, k.w1, k.b1, k.wd, k.bd, k.w3, k.b3, k.z, (const void *)k.y})
     if (!aligned16(q)) { set_error("inverted residual block (fp16): an operand is not 16-byte aligned"); return false; }
-  const dim3 grid((unsigned)(8 * a.per_xcd), (unsigned)gy), threads(64 * (unsigned)g);
-  const size_t lds = (size_t)a.xs_bytes + (size_t)g * (size_t)a.slab_bytes + BLOCK_PER_GROUP * (size_t)ceil_div(a.Ch, 32);
+  const dim3 grid((unsigned)(8 * a.per_xcd), (unsigned)gy, (unsigned)parts), threads(64 * (unsigned)g);
+  const size_t lds = (size_t)a.xs_bytes + (size_t)g * (size_t)a.slab_bytes + BLOCK_PER_GROUP * (size_t)a.per_split;
 #define BLOCK(S, KC) if (!launch_one<S, KC, KC <= 2 ? 4 : 8>(ctx, grid, threads, lds, a)) return false
   if (k.stride == 1) switch (kc) {
     case 0: BLOCK(1, 0); break; case 1: BLOCK(1, 1); break; case 2: BLOCK(1, 2); break;
-    case 4: BLOCK(1, 4); break; default: BLOCK(1, 6); break;
+    case 4: BLOCK(1, 4); break; case 6: BLOCK(1, 6); break; default: BLOCK(1, 10); break;
   } else switch (kc) {
     case 0: BLOCK(2, 0); break; case 1: BLOCK(2, 1); break; case 2: BLOCK(2, 2); break;
-    case 4: BLOCK(2, 4); break; default: BLOCK(2, 6); break;
+    case 4: BLOCK(2, 4); break; case 6: BLOCK(2, 6); break; default: BLOCK(2, 10); break;
   }
 #undef BLOCK
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("inverted residual block (fp16): launch failed: %s", hipGetErrorString(e)); return false; }
   return true;
+}
+
+bool launch_block_f16(const dnnrtContext *ctx, const dnnrtExecBlock &k) {
+  BlockF16Args a{};
+  int kc, gy, g, parts;
+  if (!plan_block_f16(ctx, k, false, a, kc, gy, g, parts)) { set_error("inverted residual block (fp16): not a shape this kernel takes"); return false; }
+  return launch_cut(ctx, k, a, kc, gy, g, parts);
 }
 
 }  // namespace dnnrt

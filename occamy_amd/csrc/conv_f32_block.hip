@@ -448,6 +448,9 @@ static double block_f32_us(int num_cu, const dnnrtExecBlock &k, const BlockF32Ar
   return 3.15 + turn * (turns + 0.57 * (std::ceil(turns) - turns)) / 2300 + (a.splits > 1 ? 1.7 : 0.0);
 }
 
+const dnnrtBlockCut *find_block_cut(const dnnrtContext *ctx, const int64_t (&sizes)[11]);  // conv_f16_block.hip
+void keep_block_cut(const dnnrtContext *ctx, const int64_t (&sizes)[11], dnnrtBlockCut cut);
+
 // `faster`: refuse what the separate calls do sooner.
 static bool plan_block_f32(const dnnrtContext *ctx, const dnnrtExecBlock &k, bool faster, BlockF32Args &a, BlockF32Cut &c) {
   if (k.dtype != DNNRT_F32 || k.format != DNNRT_NCHW || k.r != 3 || k.s != 3 || (k.stride != 1 && k.stride != 2)) return false;
@@ -458,13 +461,10 @@ static bool plan_block_f32(const dnnrtContext *ctx, const dnnrtExecBlock &k, boo
   const int64_t lim = 1ll << 28;  // elements of an image and of a filter: byte offsets below 2^31, what lies past an end included
   if (k.h * k.w > lim || k.p * k.q > lim || k.h * k.w * (k.cin + 16) > lim || k.p * k.q * (k.cout + 16) > lim || k.n > lim) return false;
   if ((k.expand && !clamp_of(k.act1, k.coef1, a.lo1, a.hi1)) || !clamp_of(k.actd, k.coefd, a.lod, a.hid) || !clamp_of(k.act, k.coef, a.lo, a.hi)) return false;
-  const int64_t sizes[11] = {k.n, k.cin, k.h, k.w, k.ch, k.cout, k.stride, k.pad_h, k.pad_w, k.expand, ctx->splitk_partial_bytes};
-  constexpr unsigned KEPT = sizeof(ctx->block_cuts) / sizeof(ctx->block_cuts[0]);
+  const int64_t sizes[11] = {k.n, k.cin, k.h, k.w, k.ch, k.cout, k.stride, k.pad_h, k.pad_w, k.expand + 2 * k.dtype, ctx->splitk_partial_bytes};
   double best = 0;
-  for (unsigned i = 0; i < std::min(ctx->block_cuts_found, KEPT) && best == 0; i++) {
-    const dnnrtBlockCut &f = ctx->block_cuts[i];
-    if (std::equal(sizes, sizes + 11, f.sizes) && cut_block_f32(ctx, k, f.nb, f.qw, f.waves, f.splits, a, c)) best = block_f32_us(ctx->num_cu, k, a, c);
-  }
+  if (const dnnrtBlockCut *f = find_block_cut(ctx, sizes))
+    if (cut_block_f32(ctx, k, f->nb, f->qw, f->waves, f->splits, a, c)) best = block_f32_us(ctx->num_cu, k, a, c);
   if (best == 0) {
     BlockF32Args t = a;
     BlockF32Cut u{};
@@ -478,10 +478,7 @@ static bool plan_block_f32(const dnnrtContext *ctx, const dnnrtExecBlock &k, boo
             if (t.units >= 4 * ctx->num_cu) break;  // enough of them without cutting the channels further
           }
     if (best == 0) return false;
-    dnnrtBlockCut &f = ctx->block_cuts[ctx->block_cuts_found % KEPT];
-    ctx->block_cuts_found = ctx->block_cuts_found + 1 < 2 * KEPT ? ctx->block_cuts_found + 1 : KEPT;  // stays past KEPT once it is there
-    std::copy(sizes, sizes + 11, f.sizes);
-    f.nb = c.nb; f.qw = a.QW; f.waves = c.G; f.splits = a.splits;
+    keep_block_cut(ctx, sizes, dnnrtBlockCut{{}, c.nb, a.QW, c.G, a.splits});
   }
   // What the separate calls take, in microseconds; inside a network, whose other kernels had the caches, 15 % longer.
   const double in_px = (double)k.n * k.h * k.w, out_px = (double)k.n * k.p * k.q;

@@ -227,3 +227,19 @@ def test_fp32_blocks_in_programs(batch, height, width, stride, pads):
         np.testing.assert_array_equal(y.cpu().numpy(), out)
     s.close()
     np.testing.assert_array_equal(run(build, mode=compiler.MODE_OCCAMY, **flags)[0][0], out)
+
+
+@pytest.mark.parametrize("batch,side,sizes", [(1, 14, dict(cin=96, hidden=576, cout=96)), (2, 7, dict(cin=160, hidden=960, cout=160))], ids=str)
+def test_fp16_blocks_in_parts_in_programs(batch, side, sizes):
+    """Few tiles, so the hidden channels of a block go to several workgroups: close to the oracle, and the same bits run after run
+    (the parts are added in order, and their counters are back at zero)."""
+    build = lambda: small_net(batch, side, side, 1, (1, 1), **sizes)  # noqa: E731
+    ref, _ = run(lambda: as_fp32_graph(*build()), ORACLE_PATH, fusion=True)
+    g, inputs = build()
+    s = g.compile(**FLAGS).session(compiler.MODE_RESIDENT)
+    assert any(o[1] == "inverted_block" for o in s.compute_ops())
+    out = s.run(*inputs)[0]
+    close16(out, ref[0])
+    for _ in range(4):
+        np.testing.assert_array_equal(s.run(*inputs)[0], out)
+    s.close()

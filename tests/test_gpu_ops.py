@@ -1746,6 +1746,19 @@ def test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, re
     np.testing.assert_allclose(got.numpy(), want.numpy(), rtol=4e-3, atol=8e-3)
 
 
+@pytest.mark.parametrize("n,cin,h,w,ch,cout,stride,expand,residual", [
+    (1, 160, 7, 7, 960, 160, 1, True, True),     # ten steps of input channels, parts of the hidden ones
+    (40, 136, 7, 6, 840, 160, 1, True, False),   # a last step and a last group that are not full
+    (2, 160, 7, 7, 960, 320, 1, True, False),    # output channels over two workgroups, each with parts
+    (1, 96, 14, 13, 576, 96, 1, True, True),
+    (1, 32, 9, 11, 200, 24, 2, True, False),     # seven groups in parts of unequal size
+    (3, 192, 8, 8, 192, 16, 1, False, False),    # parts without an expansion
+])
+def test_inverted_residual_block_fp16_in_parts(n, cin, h, w, ch, cout, stride, expand, residual):
+    """The hidden channels cut over workgroups."""
+    test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, residual)
+
+
 @pytest.mark.parametrize("n,cin,h,w,ch,cout,stride,pads,expand,residual,acts", [
     (1, 8, 5, 7, 16, 8, 1, (1, 1), True, False, (3, 3, 5)),      # less than a tile, one group of hidden channels
     (1, 16, 33, 17, 96, 24, 2, (1, 1), True, False, (3, 3, 5)),  # ragged tiles, half a block of output channels
