@@ -229,7 +229,7 @@ def test_fp32_blocks_in_programs(batch, height, width, stride, pads):
     np.testing.assert_array_equal(run(build, mode=compiler.MODE_OCCAMY, **flags)[0][0], out)
 
 
-@pytest.mark.parametrize("batch,side,sizes", [(1, 14, dict(cin=96, hidden=576, cout=96)), (2, 7, dict(cin=160, hidden=960, cout=160))], ids=str)
+@pytest.mark.parametrize("batch,side,sizes", [(1, 14, dict(cin=96, hidden=576, cout=96)), (10, 7, dict(cin=160, hidden=960, cout=160))], ids=str)
 def test_fp16_blocks_in_parts_in_programs(batch, side, sizes):
     """Few tiles, so the hidden channels of a block go to several workgroups: close to the oracle, and the same bits run after run
     (the parts are added in order, and their counters are back at zero)."""
