@@ -75,11 +75,12 @@ static std::mutex g_scratch_mutex;
 }  // namespace dnnrt
 
 namespace dnnrt {
-// Host (pinned) to device.  The link bounds it: 32 workgroups with 16 bytes per thread in flight move 9 MB in 168 us
-// (56 GB/s; 8 workgroups 366, 1024 of them 201), and leave the other compute units to the kernels beside it.  A copy
-// through the DMA engine takes as long for large sizes and 7 to 20 us more in a stream that also runs kernels:
-// 256 KB 7.4 us against 14.2, 64 KB 3.7 against 10.8, alone.
-constexpr int UPLOAD_WORKGROUPS = 32;
+// Host (pinned) to device.  The link bounds it: 24 workgroups with 16 bytes per thread in flight move 9 MB in 169 us
+// (56 GB/s; 8 workgroups 366, 16 of them 186, 32 168, 1024 201), and leave the other compute units to the kernels beside
+// it.  The executor has two copies under way: with 24 workgroups each, a ResNet-50 with its 102 MB of constants takes
+// 2.42 ms, with 16 2.47, with 32 2.47 and with 48 2.57.  A copy through the DMA engine takes as long for large sizes and
+// 7 to 20 us more in a stream that also runs kernels: 256 KB 7.2 us against 14.2, 64 KB 3.7 against 10.8, alone.
+constexpr int UPLOAD_WORKGROUPS = 24;
 __global__ __launch_bounds__(256) void upload_kernel(uint4 *dst, const uint4 *src, int64_t n16, int tail) {
   const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x;
   for (int64_t i = first; i < n16; i += UPLOAD_WORKGROUPS * 256) dst[i] = src[i];

@@ -78,7 +78,7 @@ Session::~Session() {
   for (void *p : host_in) rt.dnnrtHostFree(p);
   if (handle) rt.dnnrtDestroy(handle);
   if (stream) rt.dnnrtStreamDestroy(stream);
-  if (upload_stream) rt.dnnrtStreamDestroy(upload_stream);
+  for (dnnrtStream_t s : upload_stream) if (s) rt.dnnrtStreamDestroy(s);
 }
 
 std::string Session::rt_error(const char *what) const {
@@ -114,6 +114,24 @@ static void permute_kcrs_to_crsk(const uint8_t *src, uint8_t *dst, const Shape &
 
 static bool is_compute(OpKind k) { return k >= OP_CONVFWD && k < OP_RETURN; }
 
+// The operations' stream and, where constants may be uploaded ahead, those of the uploads.  These three have to be on
+// hardware queues of their own: on a shared one, copies wait for the kernels in front of them and kernels for copies.  HIP
+// gives a process four queues, makes one at each of the first streams, and then puts each new stream on one that has the
+// fewest, which can be the one that the stream before it has just made: with one or two more streams in the process a
+// ResNet-50 took 2.61 or 2.75 ms instead of 2.42.  Streams that are dropped again make all four first; of three streams
+// created then in a row no two are on one queue (2.41 to 2.44 ms with 0 to 5 other sessions).
+bool Session::create_streams(std::string &err) {
+  dnnrtStream_t first[4] = {nullptr, nullptr, nullptr, nullptr};
+  const bool ahead = mode == MODE_OCCAMY && !host_backend;
+  bool ok = true;
+  for (dnnrtStream_t &s : first) ok = ok && (!ahead || !rt.dnnrtStreamCreate(&s));
+  ok = ok && !rt.dnnrtStreamCreate(&stream);
+  for (dnnrtStream_t &s : upload_stream) ok = ok && (!ahead || !rt.dnnrtStreamCreate(&s));
+  if (!ok) err = rt_error("dnnrtStreamCreate");
+  for (dnnrtStream_t s : first) if (s) rt.dnnrtStreamDestroy(s);
+  return ok;
+}
+
 bool Session::init(const Program *p,const std::string &runtime_path, int mode_, std::string &err) {
   prog = p;
   mode = mode_;
@@ -122,7 +140,7 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
   host_backend = rt.dnnrtIsHostBackend() != 0;
   if (prog->channels_last && host_backend) { err = "channels-last programs need the GPU runtime"; return false; }
   if (rt.dnnrtCreate(&handle)) { err = rt_error("dnnrtCreate"); return false; }
-  if (rt.dnnrtStreamCreate(&stream)) { err = rt_error("dnnrtStreamCreate"); return false; }
+  if (!create_streams(err)) return false;
   if (rt.dnnrtSetStream(handle, stream)) { err = rt_error("dnnrtSetStream"); return false; }
   ptr.assign(prog->value_store.size(), nullptr);
 
@@ -520,13 +538,17 @@ void Session::plan_blocks() {
 // Issued in program order on one stream, a constant waits for the operation in front of its reader (that operation's
 // filter lies where this one goes), the reader waits for the copy, and the link idles during every kernel and the
 // hand-overs between engines around it: 3.56 ms for a ResNet-50 whose 102 MB take 1.85 at the link's 55 GB/s.  The plan
-// gives every constant its own place in the pool instead, the one whose bytes come free earliest on the whole, and a
-// second stream copies them in program order, each part as soon as the operations that used its bytes are done.  The
+// gives every constant its own place in the pool instead, the one whose bytes come free earliest on the whole, and
+// streams of their own copy them in program order, each part as soon as the operations that used its bytes are done.  The
 // pool stays the planned one to the byte, activations stay where the planner put them, and every constant still crosses
 // the link in every inference.  Small constants that follow each other travel together (a copy costs 3.5 us beside its
 // bytes, a wait of one stream for the other 15); the first chunks are small so that the first operations start early.
 // (128 KB, 1.5 MB: within 2 %.)  ResNet-50 3.51 -> 2.56 ms, of which the link 1.85; MobileNetV2 1.52 -> 0.87.
-static constexpr int64_t UPLOAD_PART_BYTES = 512 << 10;
+// The chunks go to two streams in turn: on one stream the link idles from the last bytes of a copy over its completion and
+// the event behind it to the first bytes of the next, some 5 us at each of ResNet-50's 80 copies; now the next one is under
+// way, and a part whose bytes are in use holds back only every other chunk.  2.59 -> 2.42 ms, MobileNetV2 0.95 -> 0.82.
+// (Parts of 512 KB: 1 % more; chunks of 2 MB: as now.)
+static constexpr int64_t UPLOAD_PART_BYTES = 1 << 20;
 bool Session::place_constants(std::vector<UploadChunk> &chunks) const {
   std::vector<UploadItem> items;
   std::map<const Value *, size_t> item_of;
@@ -700,10 +722,9 @@ bool Session::plan_uploads(const std::vector<UploadChunk> &chunks, std::string &
   for (const UploadChunk &k : chunks) total += align_up(k.bytes, 256);
   if (!total) return true;
   if (rt.dnnrtHostAlloc(&upload_host, total)) { err = rt_error("dnnrtHostAlloc(constants)"); return false; }
-  if (rt.dnnrtStreamCreate(&upload_stream)) { err = rt_error("dnnrtStreamCreate"); return false; }
   int64_t host = 0;
   std::map<size_t, void *> moved;
-  int waited = 0;
+  int on = 0;
   for (const UploadChunk &k : chunks) {
     int64_t in = 0;
     for (const UploadItem &item : k.items) {
@@ -719,13 +740,11 @@ bool Session::plan_uploads(const std::vector<UploadChunk> &chunks, std::string &
     }
     for (size_t i = 0; i < k.parts.size(); i++) {
       const UploadPart &q = k.parts[i];
-      uploads.push_back({host + q.lo - k.off, q.lo, q.hi - q.lo, k.first, k.last, q.after, nullptr});
+      uploads.push_back({host + q.lo - k.off, q.lo, q.hi - q.lo, k.first, k.last, q.after, on, nullptr});
       if (i + 1 == k.parts.size() && rt.dnnrtExecFenceCreate(&uploads.back().landed)) { err = rt_error("dnnrtExecFenceCreate"); return false; }
-      if (q.after > waited) {
-        waited = q.after;
-        if (rt.dnnrtExecFenceCreate(&op_done[waited])) { err = rt_error("dnnrtExecFenceCreate"); return false; }
-      }
+      if (q.after > 0 && !op_done[q.after] && rt.dnnrtExecFenceCreate(&op_done[q.after])) { err = rt_error("dnnrtExecFenceCreate"); return false; }
     }
+    on ^= 1;
     host += align_up(k.bytes, 256);
   }
   for (const auto &m : moved) ptr[m.first] = m.second;
@@ -985,7 +1004,7 @@ bool Session::fill_dead(const std::vector<Range> &held, int n, void *base) const
 bool Session::run_uploading(const void *const *inputs, void *const *outputs, std::string &err) {
   void *run_pool = nullptr;
   size_t next = 0, landed = 0;  // the next upload to issue; those that the compute stream has waited for
-  int n = 0, waited = 0;
+  int n = 0, waited[2] = {0, 0};
   std::vector<Range> held;
   if (debug_fill >= 0) {
     held = moved_results;
@@ -997,12 +1016,12 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
   auto pump = [&]() -> bool {
     for (; next < uploads.size() && uploads[next].after <= n; next++) {
       const Upload &u = uploads[next];
-      if (u.after > waited) {
-        waited = u.after;
-        if (rt.dnnrtExecStreamWait(upload_stream, op_done[u.after])) return fail("dnnrtExecStreamWait");
+      if (u.after > waited[u.on]) {
+        waited[u.on] = u.after;
+        if (rt.dnnrtExecStreamWait(upload_stream[u.on], op_done[u.after])) return fail("dnnrtExecStreamWait");
       }
-      if (rt.dnnrtExecUpload((char *)run_pool + u.dev_off, (char *)upload_host + u.host_off, u.bytes, upload_stream)) return fail("dnnrtExecUpload(constants)");
-      if (u.landed && rt.dnnrtEventRecord(u.landed, upload_stream)) return fail("dnnrtEventRecord");
+      if (rt.dnnrtExecUpload((char *)run_pool + u.dev_off, (char *)upload_host + u.host_off, u.bytes, upload_stream[u.on])) return fail("dnnrtExecUpload(constants)");
+      if (u.landed && rt.dnnrtEventRecord(u.landed, upload_stream[u.on])) return fail("dnnrtEventRecord");
     }
     return true;
   };
@@ -1042,12 +1061,11 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
       default: break;
     }
     if (!pump()) return false;
-    size_t need = landed;
-    while (need < uploads.size() && uploads[need].first <= n) need++;  // whole chunks: the last of their parts has the event
-    if (need > landed) {
-      landed = need;
-      if (rt.dnnrtExecStreamWait(stream, uploads[need - 1].landed)) return fail("dnnrtExecStreamWait");
-    }
+    void *last_landed[2] = {nullptr, nullptr};
+    for (; landed < uploads.size() && uploads[landed].first <= n; landed++)  // whole chunks: the last of their parts has the event
+      last_landed[uploads[landed].on] = uploads[landed].landed;
+    for (void *event : last_landed)
+      if (event && rt.dnnrtExecStreamWait(stream, event)) return fail("dnnrtExecStreamWait");
     if (!issue(op, err)) return false;
     if (debug_fill >= 0 && !fill_dead(held, n, run_pool)) return fail("dnnrtMemFill");
     n++;

@@ -191,24 +191,26 @@ class Session {
   decltype(&::dnnrtExecBlockFilter) block_filter(const Value *filter) const { return filter->dtype == F16 ? rt.dnnrtExecBlockFilter : rt.dnnrtExecBlockFilterF32; }
   void plan_blocks();
   std::map<const Value *, Range> live_slots() const;
-  // Per-inference mode on the GPU runtime: the constants as they go to the device on a second stream, ahead of the
-  // operations that read them (plan_uploads).  Compute operations are counted in program order.
+  // Per-inference mode on the GPU runtime: the constants as they go to the device on two streams of their own, ahead of
+  // the operations that read them (plan_uploads).  Compute operations are counted in program order.
   struct Upload {
     int64_t host_off, dev_off, bytes;  // in upload_host, in the pool
     int first, last;                   // the first and the last operation that read it
     int after;                         // these bytes of the pool are free once this many operations are done
+    int on;                            // which of the two streams
     void *landed;                      // recorded behind the copy; null where the next entry completes the same constants
   };
   std::vector<Upload> uploads;
   std::vector<std::pair<size_t, int64_t>> upload_slots;  // value id of a constant's device tensor, its offset in the pool
   std::map<int, void *> op_done;                         // recorded when that many operations are issued
   void *upload_host = nullptr;
-  dnnrtStream_t upload_stream = nullptr;
+  dnnrtStream_t upload_stream[2] = {nullptr, nullptr};
   // Constants that travel together, side by side in the pool; `parts` have places that come free at different times.
   struct UploadItem { const Op *copy; int64_t bytes; int first, last; };
   struct UploadPart { int64_t lo, hi; int after; };
   struct UploadChunk { std::vector<UploadItem> items; int64_t bytes, off; int first, last; std::vector<UploadPart> parts; };
   bool place_constants(std::vector<UploadChunk> &chunks) const;
+  bool create_streams(std::string &err);
   bool plan_uploads(const std::vector<UploadChunk> &chunks, std::string &err);
   bool fill_dead(const std::vector<Range> &held, int n, void *base) const;
   bool run_uploading(const void *const *inputs, void *const *outputs, std::string &err);

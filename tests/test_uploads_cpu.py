@@ -82,3 +82,76 @@ def test_a_constant_read_through_copies_that_are_not_made_stays_until_its_last_r
             np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-4)
     assert uploads() > before  # the plan under test is the one that ran
     s.close()
+
+
+LATE_SHIM = r"""
+#define dnnrtIsHostBackend dnnrt_oracle_is_host_backend
+#define dnnrtStreamCreate dnnrt_oracle_stream_create
+#define dnnrtSetStream dnnrt_oracle_set_stream
+#define dnnrtEventRecord dnnrt_oracle_event_record
+#define dnnrtEventDestroy dnnrt_oracle_event_destroy
+#include "%(oracle)s"
+#undef dnnrtIsHostBackend
+#undef dnnrtStreamCreate
+#undef dnnrtSetStream
+#undef dnnrtEventRecord
+#undef dnnrtEventDestroy
+enum { QUEUED = 4096 };
+static struct { void *dst; const void *src; int64_t bytes; } queue[8][QUEUED];
+static int streams, queued[8], done[8];
+static dnnrtStream_t computing;
+struct Mark { int at, upto; };
+static int most_streams;
+int used_streams(void) { return most_streams; }
+int32_t dnnrtIsHostBackend(void) { return 0; }
+int32_t dnnrtStreamCreate(dnnrtStream_t *s) { *s = (dnnrtStream_t)(intptr_t)(1 + streams++ %% 7); return 0; }
+int32_t dnnrtSetStream(dnnrtHandle_t h, dnnrtStream_t s) { (void)h; computing = s; return 0; }
+static void run_upto(int s, int n) {
+  for (; done[s] < n; done[s]++) memcpy(queue[s][done[s] %% QUEUED].dst, queue[s][done[s] %% QUEUED].src, (size_t)queue[s][done[s] %% QUEUED].bytes);
+}
+int32_t dnnrtExecFenceCreate(void **event) { *event = calloc(1, sizeof(struct Mark)); return 0; }
+int32_t dnnrtEventRecord(void *event, dnnrtStream_t s) { *(struct Mark *)event = (struct Mark){(int)(intptr_t)s, queued[(intptr_t)s]}; return 0; }
+int32_t dnnrtEventDestroy(void *event) { free(event); return 0; }
+int32_t dnnrtExecStreamWait(dnnrtStream_t s, void *event) {
+  const struct Mark *m = event;
+  if (s == computing) run_upto(m->at, m->upto);
+  return 0;
+}
+int32_t dnnrtExecUpload(void *dst, const void *src, int64_t bytes, dnnrtStream_t stream) {
+  const int s = (int)(intptr_t)stream;
+  if (stream == computing) { memcpy(dst, src, (size_t)bytes); return 0; }
+  queue[s][queued[s] %% QUEUED].dst = dst;
+  queue[s][queued[s] %% QUEUED].src = src;
+  queue[s][queued[s]++ %% QUEUED].bytes = bytes;
+  int n = 0;
+  for (int i = 0; i < 8; i++) n += queued[i] > 0;
+  if (n > most_streams) most_streams = n;
+  return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("flags", [dict(), dict(alias_copies=True, compact_pool=True)])
+def test_a_constant_is_there_when_its_stream_is_as_late_as_the_waits_allow(tmp_path, flags):
+    """Every copy is made only when the operations' stream waits for an event behind it on that copy's stream."""
+    if not shutil.which("gcc"):
+        pytest.skip("no host compiler")
+    (tmp_path / "runtime.c").write_text(LATE_SHIM % {"oracle": os.path.join(ROOT, "oracle", "dnnrt_oracle.c")})
+    runtime = str(tmp_path / "runtime.so")
+    subprocess.check_call(["gcc", "-O1", "-fPIC", "-shared", "-std=gnu11", "-ffp-contract=off", "-fopenmp", "-I", os.path.join(ROOT, "oracle"),
+                           "-o", runtime, str(tmp_path / "runtime.c"), "-lm"])
+    r = np.random.default_rng(5)
+    g = compiler.Graph()
+    h = g.input("x", (16, 512))
+    for rows, cols in [(512, 64), (64, 640), (640, 768), (768, 48), (48, 512), (512, 512)]:
+        h = g.node("MatMul", [h, g.constant((r.standard_normal((rows, cols)) / rows ** 0.5).astype(np.float32))])
+        h = g.node("Relu", [g.node("Add", [h, g.constant(r.standard_normal((1, cols)).astype(np.float32))])])
+    g.output(h)
+    inputs = [r.standard_normal((16, 512)).astype(np.float32)]
+    want = graph_eval.evaluate(g, inputs)
+    s = g.compile(**flags).session(compiler.MODE_OCCAMY, runtime_library=runtime)
+    for _ in range(3):
+        for got, ref in zip(s.run(*inputs), want):
+            np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-4)
+    assert C.CDLL(runtime).used_streams() == 2
+    s.close()
