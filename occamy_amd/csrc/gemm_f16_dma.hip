@@ -63,10 +63,14 @@ __device__ __forceinline__ void gd_arrived(T &v) {
   asm volatile("" : "+v"(v));
 }
 
-// FN x FM: columns n and rows m of a workgroup's tile, over WN x WM wavefronts; NS ring stages; B_KC: B stored [N,K].
+// FN x FM: columns n and rows m of a workgroup's tile, over WN x WM wavefronts; NS ring stages; B_KC: B stored [N,K].  What the
+// ring's first loads need stands in front of the struct and is in registers when a wavefront starts; the rest comes 0.45 us later.
 template <int FN, int FM, int WN, int WM, int NS, bool B_KC>
-__global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF16Args a, const int tiles) {
+__global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const __half *A, const __half *B, int64_t az, int64_t bz, int M, int N, int K, int tiles,
+                                                                     unsigned magic_tiles_m, int steps_per_split, const GemmF16Args args, int splits) {
 #if __HIP_DEVICE_COMPILE__
+  GemmF16Args a = args;
+  a.M = M; a.N = N; a.K = K; a.steps_per_split = steps_per_split;
   constexpr int NW = WN * WM, NT = 64 * NW, TN = FN / WN / 32, TM = FM / WM / 32;
   constexpr int STAGE = (FN + FM) * 128;
   constexpr int N_L = FN / 8 / NW, M_L = FM / 8 / NW, L = N_L + M_L;  // loads per wavefront and step
@@ -83,11 +87,11 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
   const int wn0 = (wave / WM) * (FN / WN), wm0 = (wave % WM) * (FM / WM);
-  const int tiles_m = (a.M + FM - 1) / FM, tile_n = tile / tiles_m, tile_m = tile - tile_n * tiles_m;
+  const int tiles_m = (a.M + FM - 1) / FM, tile_n = div_magic(tile, tiles_m, magic_tiles_m), tile_m = tile - tile_n * tiles_m;
   const int n0 = tile_n * FN, m0 = tile_m * FM, z = blockIdx.z;
 
-  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(a.A) + (int64_t)z * a.az, 0, 2 * a.M * a.K, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(a.B) + (int64_t)z * a.bz, 0, 2 * a.K * a.N, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(A) + (int64_t)z * az, 0, 2 * a.M * a.K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(B) + (int64_t)z * bz, 0, 2 * a.K * a.N, 0x00020000);
 
   // ---- loader constants: byte offset of this lane's chunk, and the k of the step it belongs to ----
   unsigned m_off[M_L], n_off[N_L];
@@ -137,19 +141,6 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
     for (int j = 0; j < TM; j++)
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-  // bias of this lane's columns, older than every ring load (the counted waits below rest on that)
-  gd_half4 bias4[TN][4];
-#pragma unroll
-  for (int i = 0; i < TN; i++)
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-      const int n = n0 + wn0 + i * 32 + 8 * g + 4 * half;
-      const gd_half4 zero = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
-      bias4[i][g] = a.bias ? *reinterpret_cast<const gd_half4 *>(reinterpret_cast<const _Float16 *>(a.bias) + (n < a.N ? n : 0)) : zero;
-    }
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-
   // ---- operand fetch --------------------------------------------------------
   const unsigned ld_m0 = (unsigned)((FN + wm0 + l32) * 128 + ((half ^ ((l32 >> 1) & 7)) * 16));
   [[maybe_unused]] const unsigned ld_n0 = (unsigned)((wn0 + l32) * 128 + ((half ^ ((l32 >> 1) & 7)) * 16));
@@ -229,12 +220,29 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
         for (int j = 0; j < TM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fn[S][sub][i], fm[S][sub][j], acc[i][j], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
-  const int nk = s_end - s_beg;
-  {
-    const int pre = nk < NS ? nk : NS;
+  const int nk = s_end - s_beg, pre = nk < NS ? nk : NS;
 #pragma unroll
-    for (int q = 0; q < NS; q++)
-      if (q < pre) issue_loads();
+  for (int q = 0; q < NS; q++)
+    if (q < pre) issue_loads();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  // The other arguments, all at once: read where they are used, each is waited for there.
+  asm volatile("" : "+s"(a.bias), "+s"(a.C), "+s"(a.c_sm), "+s"(a.cz), "+s"(a.yz), "+s"(a.Out), "+s"(a.alpha), "+s"(a.beta), "+s"(a.act), "+s"(a.act_coef),
+               "+s"(a.partials), "+s"(a.counters), "+s"(splits));
+  // Bias of this lane's columns, behind the ring's first loads: the counted waits are for the loads of the ring alone, these make the
+  // first of them stricter.
+  gd_half4 bias4[TN][4];
+#pragma unroll
+  for (int i = 0; i < TN; i++)
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const int n = n0 + wn0 + i * 32 + 8 * g + 4 * half;
+      const gd_half4 zero = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
+      bias4[i][g] = a.bias ? *reinterpret_cast<const gd_half4 *>(reinterpret_cast<const _Float16 *>(a.bias) + (n < a.N ? n : 0)) : zero;
+    }
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  {
     if (pre == 1) gd_wait<0>();
     else if (pre == 2) gd_wait<L>();
     else if (pre == 3) gd_wait<(NS > 2 ? 2 : 0) * L>();
@@ -262,7 +270,6 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f16_dma_kernel(const GemmF1
   gd_barrier();  // nobody reads the operand stages any more
 
   // ---- a split reduction: the hand-over of the fp32 kernels (igemm_f32_small.hip states what it rests on) ----
-  const int splits = (int)gridDim.y;
   if (splits > 1) {
     constexpr int TILE = FN * FM;
     volatile unsigned *arrived = reinterpret_cast<unsigned *>(smem);
@@ -375,8 +382,11 @@ static bool launch_gd(const dnnrtContext *ctx, const GemmF16Args &g, int Z, int 
     }
   }
   const dim3 grid((unsigned)(ceil_div(tiles, 8) * 8), (unsigned)splits, (unsigned)Z), block(64 * WN * WM);
-  if (kc) hipLaunchKernelGGL((gemm_f16_dma_kernel<FN, FM, WN, WM, NS, true>), grid, block, SMEM, ctx->stream, g, (int)tiles);
-  else hipLaunchKernelGGL((gemm_f16_dma_kernel<FN, FM, WN, WM, NS, false>), grid, block, SMEM, ctx->stream, g, (int)tiles);
+  const unsigned magic = magic_of((int)ceil_div(g.M, FM));
+  if (kc) hipLaunchKernelGGL((gemm_f16_dma_kernel<FN, FM, WN, WM, NS, true>), grid, block, SMEM, ctx->stream, g.A, g.B, g.az, g.bz, g.M, g.N, g.K, (int)tiles, magic,
+                             g.steps_per_split, g, (int)grid.y);
+  else hipLaunchKernelGGL((gemm_f16_dma_kernel<FN, FM, WN, WM, NS, false>), grid, block, SMEM, ctx->stream, g.A, g.B, g.az, g.bz, g.M, g.N, g.K, (int)tiles, magic,
+                             g.steps_per_split, g, (int)grid.y);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("matmul(fp16): launch failed: %s", hipGetErrorString(e)); return false; }
   return true;

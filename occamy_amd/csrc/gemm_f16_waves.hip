@@ -64,10 +64,14 @@ __device__ __forceinline__ void gw_arrived(T &v) {
   asm volatile("" : "+v"(v));
 }
 
-// Tiles of 64 columns n and 32 TM rows m; B_KC: B stored [N,K].
+// Tiles of 64 columns n and 32 TM rows m; B_KC: B stored [N,K].  The arguments in front of the struct are in registers when a
+// wavefront starts: all that the ring's first loads need, so that nothing waits for the rest, which comes 0.45 us later.
 template <bool B_KC, int TM>
-__global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Args a, const int tiles) {
+__global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const __half *A, const __half *B, int64_t az, int64_t bz, int M, int N, int K, int tiles,
+                                                                unsigned magic_tiles_m, int steps_per_split, const GemmF16Args args, int splits) {
 #if __HIP_DEVICE_COMPILE__
+  GemmF16Args a = args;
+  a.M = M; a.N = N; a.K = K; a.steps_per_split = steps_per_split;
   constexpr int NS = gw_ring(TM), FM = 32 * TM, STAGE = gw_stage(TM), WAVE_LDS = gw_wave(TM);
   constexpr int M_L = FM / 16, L = 4 + M_L;  // loads of a stage
   static_assert(NS * STAGE <= WAVE_LDS && FM * 64 * 4 <= WAVE_LDS, "a wavefront's ring and, later, its sums");
@@ -78,7 +82,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
   if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= tiles) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
-  const int tiles_m = (a.M + FM - 1) / FM, tile_n = tile / tiles_m, tile_m = tile - tile_n * tiles_m;
+  const int tiles_m = (a.M + FM - 1) / FM, tile_n = div_magic(tile, tiles_m, magic_tiles_m), tile_m = tile - tile_n * tiles_m;
   const int n0 = tile_n * 64, m0 = tile_m * FM, z = blockIdx.z;
   char *ring = smem + wave * WAVE_LDS;
 
@@ -87,24 +91,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
   const int s_beg = (int)blockIdx.y * a.steps_per_split, s_end = min(stages, s_beg + a.steps_per_split);
   const int per_wave = (s_end - s_beg + 3) >> 2, my_beg = s_beg + wave * per_wave, nk = max(0, min(per_wave, s_end - my_beg));
 
-  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(a.A) + (int64_t)z * a.az, 0, 2 * a.M * a.K, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(a.B) + (int64_t)z * a.bz, 0, 2 * a.K * a.N, 0x00020000);
-
-  // What the lane finishes: eight columns out_n .. + 7 of the rows out_m + 32 o.  Bias and residual are requested first of all.
-  const int out_m = m0 + (tid >> 3), out_n = n0 + 8 * (tid & 7);
-  const gw_half4 zero4 = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
-  gw_half4 bias4[2] = {zero4, zero4}, c4[TM][2];
-  if (a.bias) {
-#pragma unroll
-    for (int q = 0; q < 2; q++) bias4[q] = *reinterpret_cast<const gw_half4 *>(reinterpret_cast<const _Float16 *>(a.bias) + min(out_n + 4 * q, a.N - 4));
-  }
-  if (a.C) {
-    const _Float16 *Cg = reinterpret_cast<const _Float16 *>(a.C) + (int64_t)z * a.cz;
-#pragma unroll
-    for (int o = 0; o < TM; o++)
-#pragma unroll
-      for (int q = 0; q < 2; q++) c4[o][q] = *reinterpret_cast<const gw_half4 *>(Cg + (int64_t)min(out_m + 32 * o, a.M - 1) * a.c_sm + min(out_n + 4 * q, a.N - 4));
-  }
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(A) + (int64_t)z * az, 0, 2 * a.M * a.K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(B) + (int64_t)z * bz, 0, 2 * a.K * a.N, 0x00020000);
 
   // ---- loader constants: byte offset of this lane's chunk, and the k of the stage it belongs to ----
   // k-contiguous rows: 64 bytes a row, 16-byte chunk c of row r at c ^ ((r >> 2) & 3); sixteen rows per instruction
@@ -186,7 +174,30 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
     for (int j = 0; j < TM; j++)
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-  // The counted waits below assume that bias and residual are older than every ring load.
+#pragma unroll
+  for (int i = 0; i < NS; i++)
+    if (i < nk) issue_stage();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  // The other arguments, all at once: read where they are used, each is waited for there.
+  asm volatile("" : "+s"(a.bias), "+s"(a.C), "+s"(a.c_sm), "+s"(a.cz), "+s"(a.yz), "+s"(a.Out), "+s"(a.alpha), "+s"(a.beta), "+s"(a.act), "+s"(a.act_coef),
+               "+s"(a.partials), "+s"(a.counters), "+s"(splits));
+  // What the lane finishes: eight columns out_n .. + 7 of the rows out_m + 32 o.  Bias and residual are requested behind
+  // the ring's first loads; the counted waits below are for the loads of the ring alone, these make the first of them stricter.
+  const int out_m = m0 + (tid >> 3), out_n = n0 + 8 * (tid & 7);
+  const gw_half4 zero4 = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
+  gw_half4 bias4[2] = {zero4, zero4}, c4[TM][2];
+  if (a.bias) {
+#pragma unroll
+    for (int q = 0; q < 2; q++) bias4[q] = *reinterpret_cast<const gw_half4 *>(reinterpret_cast<const _Float16 *>(a.bias) + min(out_n + 4 * q, a.N - 4));
+  }
+  if (a.C) {
+    const _Float16 *Cg = reinterpret_cast<const _Float16 *>(a.C) + (int64_t)z * a.cz;
+#pragma unroll
+    for (int o = 0; o < TM; o++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) c4[o][q] = *reinterpret_cast<const gw_half4 *>(Cg + (int64_t)min(out_m + 32 * o, a.M - 1) * a.c_sm + min(out_n + 4 * q, a.N - 4));
+  }
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 
@@ -231,9 +242,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
     __builtin_amdgcn_sched_barrier(0);
   };
   if (nk > 0) {
-#pragma unroll
-    for (int i = 0; i < NS; i++)
-      if (i < nk) issue_stage();
     landed(nk - 1);
     read_stage(c0);
     int ahead = nk - 1;
@@ -277,7 +285,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const GemmF16Arg
     }
 
   // ---- a split reduction: the hand-over of the fp32 kernels (igemm_f32_small.hip states what it rests on) ----
-  const int splits = (int)gridDim.y;
   if (splits > 1) {
     const unsigned t = (unsigned)z * (unsigned)tiles + (unsigned)tile;
     const __amdgpu_buffer_rsrc_t parts = part_rsrc(a.partials);
@@ -341,7 +348,8 @@ static bool launch_one(const dnnrtContext *ctx, const GemmF16Args &g, const dim3
       return false;
     }
   }
-  hipLaunchKernelGGL((gemm_f16_waves_kernel<B_KC, TM>), grid, dim3(256), SMEM, ctx->stream, g, tiles);
+  hipLaunchKernelGGL((gemm_f16_waves_kernel<B_KC, TM>), grid, dim3(256), SMEM, ctx->stream, g.A, g.B, g.az, g.bz, g.M, g.N, g.K, tiles,
+                     magic_of((int)ceil_div(g.M, 32 * TM)), g.steps_per_split, g, (int)grid.y);
   return true;
 }
 

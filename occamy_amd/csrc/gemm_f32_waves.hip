@@ -45,10 +45,16 @@ __device__ __forceinline__ void f32w_wait() {  // s_waitcnt vmcnt(N) lgkmcnt(LGK
   asm volatile("" ::: "memory");
 }
 
-// TM: blocks of 32 rows of a tile.
+// TM: blocks of 32 rows of a tile.  The arguments in front of the structs are in registers when a wavefront starts: all that the
+// ring's first loads need, so that nothing waits for the rest, which comes 0.45 us later.  (They are in `args` and `plan` too.)
 template <int TM>
-__global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const IgemmArgs a, const Waves32Plan pl, float *partials, unsigned *counters) {
+__global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const float *A, const float *X, int M, int Kdim, int Ncols, int units, int rest, int whole,
+                                                                int stages_per_split, int tiles_m, unsigned magic_round, unsigned magic_tiles_m,
+                                                                const IgemmArgs args, const Waves32Plan plan, float *partials, unsigned *counters) {
 #if __HIP_DEVICE_COMPILE__
+  IgemmArgs a = args;
+  a.A = A; a.X = X; a.M = M; a.Kdim = Kdim; a.Ncols = Ncols;
+  const Waves32Plan pl = {tiles_m, whole, rest, 0, units, stages_per_split, magic_tiles_m, magic_round};
   constexpr int L = 4 + 2 * TM;  // loads of a stage
   constexpr int STAGE = f32w_stage(TM), WAVE = f32w_wave(TM), NS = WAVE / STAGE, TILE = 64 * 32 * TM;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -78,15 +84,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const IgemmArgs 
 
   // ---- this wavefront's stages ----------------------------------------------
   const int per_wave = (s_end - s_beg + 3) >> 2, my_beg = s_beg + wave * per_wave, nk = max(0, min(per_wave, s_end - my_beg));
-
-  // What the lane finishes: columns out_n .. + 3 of the rows out_m + 16 o.  Bias and residual are requested first of all.
-  const int out_m = m0 + (tid >> 4), out_n = n0 + 4 * (tid & 15), out_nc = min(out_n, a.Ncols - 4);
-  floatx4 bias = {0.f, 0.f, 0.f, 0.f}, res[2 * TM];
-  if (a.bias_col) bias = *reinterpret_cast<const float4u *>(a.bias_col + out_nc);
-  if (a.Cin) {
-#pragma unroll
-    for (int o = 0; o < 2 * TM; o++) res[o] = *reinterpret_cast<const float4u *>(a.Cin + (int64_t)min(out_m + 16 * o, a.M - 1) * a.c_row_stride + out_nc);
-  }
 
   // ---- loaders: byte offsets of this lane -----------------------------------
   // A: 64 bytes a row, 16-byte chunk c of row r at c ^ ((r >> 2) & 3), sixteen rows per instruction; B: as in memory, four k
@@ -144,7 +141,24 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const IgemmArgs 
 #pragma unroll
         for (int i = 0; i < SUMS - 1; i++) more[i][u][j][r] = 0.f;
       }
-  // The counted waits below assume that bias and residual are older than every ring load.
+#pragma unroll
+  for (int i = 0; i < NS; i++)
+    if (i < nk) issue_stage();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  // The other arguments, all at once: read where they are used, each is waited for there.
+  int splits = plan.splits;
+  asm volatile("" : "+s"(a.bias_col), "+s"(a.Cin), "+s"(a.c_row_stride), "+s"(a.Y), "+s"(a.y_row_stride), "+s"(a.alpha), "+s"(a.beta), "+s"(a.act),
+               "+s"(a.act_coef), "+s"(splits), "+s"(partials), "+s"(counters));
+  // What the lane finishes: columns out_n .. + 3 of the rows out_m + 16 o.  Bias and residual are requested behind the ring's
+  // first loads; the counted waits below are for the loads of the ring alone, these make the first of them stricter.
+  const int out_m = m0 + (tid >> 4), out_n = n0 + 4 * (tid & 15), out_nc = min(out_n, a.Ncols - 4);
+  floatx4 bias = {0.f, 0.f, 0.f, 0.f}, res[2 * TM];
+  if (a.bias_col) bias = *reinterpret_cast<const float4u *>(a.bias_col + out_nc);
+  if (a.Cin) {
+#pragma unroll
+    for (int o = 0; o < 2 * TM; o++) res[o] = *reinterpret_cast<const float4u *>(a.Cin + (int64_t)min(out_m + 16 * o, a.M - 1) * a.c_row_stride + out_nc);
+  }
   asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 
@@ -186,9 +200,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const IgemmArgs 
     __builtin_amdgcn_sched_barrier(0);
   };
   if (nk > 0) {
-#pragma unroll
-    for (int i = 0; i < NS; i++)
-      if (i < nk) issue_stage();
     landed(nk - 1);
     read_stage(c0);
     int ahead = nk - 1;
@@ -228,7 +239,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const IgemmArgs 
   }
 
   // ---- a split reduction: the hand-over that igemm_f32_small.hip describes ----
-  const int splits = pl.splits;
   if (part && splits > 1) {
     const int rt = tile - pl.whole;
     const __amdgpu_buffer_rsrc_t parts = part_rsrc(partials);
@@ -336,7 +346,8 @@ bool launch_gemm_f32_waves(const dnnrtContext *ctx, const IgemmArgs &a, bool &la
     set_error("gemm_f32(waves): cannot reserve %d bytes of LDS", lds);
     return false;
   }
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), (size_t)lds, ctx->stream, a, pl, ctx->splitk_partials, ctx->splitk_counters);
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), (size_t)lds, ctx->stream, a.A, a.X, a.M, a.Kdim, a.Ncols, pl.units, pl.rest, pl.whole,
+                     pl.stages_per_split, pl.tiles_m, pl.magic_round, pl.magic_tiles_m, a, pl, ctx->splitk_partials, ctx->splitk_counters);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("gemm_f32(waves): launch failed: %s", hipGetErrorString(e)); return false; }
   launched = true;
