@@ -81,7 +81,7 @@ __device__ __forceinline__ void prefetch_finish(const IgemmArgs &a, int z, int m
 // counter back to zero for the next kernel on the stream.
 template <int KS>
 __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 acc, const Finish<KS> &f, float bias_c, float (*red)[16][64],
-                                                 int wave, int lane, int m0, int img, int pq, bool col_ok, int z, unsigned tile,
+                                                 int wave, int lane, int m0, int img, int pq, bool col_ok, int z, unsigned tile, int splits,
                                                  float *partials, unsigned *counters) {
   constexpr int N = 16 / KS;
   const int half = lane >> 5;
@@ -100,7 +100,6 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
 #pragma unroll
     for (int i = 0; i < N; i++) v[i] = acc[i];
   }
-  const int splits = (int)gridDim.y;
   if (splits > 1) {
 #if __HIP_DEVICE_COMPILE__
     // a partial tile: [wavefront][vector of its registers][lane]
@@ -199,8 +198,8 @@ __device__ __forceinline__ void reduce_and_store(const IgemmArgs &a, floatx16 ac
 // workgroups of eight wavefronts fit a compute unit: 6.5 and 379, 128 -> 128 at 28x28, batch 4, 17.3 -> 15.6.  (The 1x1 kernel's
 // iterations are 0.2 us: there four slots stay in flight; two ahead cost MobileNetV2 2%.)  The counted waits
 // need code in which it is certain which loads have been issued, hence the groups of three without a branch and the endings.
-template <class Load, class Multiply>
-__device__ __forceinline__ void small_pipeline(int niter, Load load, Multiply multiply) {
+template <class Load, class Multiply, class Then>
+__device__ __forceinline__ void small_pipeline(int niter, Load load, Multiply multiply, Then then) {
   constexpr std::integral_constant<int, 0> s0{};
   constexpr std::integral_constant<int, 1> s1{};
   constexpr std::integral_constant<int, 2> s2{};
@@ -209,6 +208,7 @@ __device__ __forceinline__ void small_pipeline(int niter, Load load, Multiply mu
   if (niter >= 3) {
     load(0, s0, not_last);
     load(1, s1, not_last);
+    then();
     int i = 0;
     for (; i + 5 <= niter; i += 3) {
       load(i + 2, s2, not_last); multiply(s0);
@@ -231,14 +231,52 @@ __device__ __forceinline__ void small_pipeline(int niter, Load load, Multiply mu
   }
   if (niter > 0) load(0, s0, perhaps_last);
   if (niter > 1) load(1, s1, perhaps_last);
+  then();
   if (niter > 0) multiply(s0);
   if (niter > 1) multiply(s1);
 }
 
-template <int KS, bool AMC>
-__global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS >= 2 ? 4 : 3))) void conv3x3_f32_small_kernel(const IgemmArgs a, const int c_per_wave, float *partials,
-                                                                    unsigned *counters) {
+// The arguments in front of the struct are in registers when a wavefront starts.  PLAIN: they are all that the loads need (one
+// image size in and out, stride 1, one z, images side by side, one reduction), and nothing waits for the rest, which comes 0.45 us
+// later; otherwise only the struct and per_wave are read.  per_wave: the slice of the reduction a wavefront takes, times 4, and log2 of the
+// XCD grid's columns.
+template <bool PLAIN>
+__device__ __forceinline__ IgemmArgs small_args(const float *A, const float *X, int M, int Ncols, int Kdim, int a_ld, int H, int W, int RS, unsigned per_wave,
+                                                unsigned magic_tn_per, unsigned magic_pq, const IgemmArgs &args) {
+  IgemmArgs a = args;
+  if constexpr (PLAIN) {
+    a.A = A; a.X = X; a.M = M; a.Ncols = Ncols; a.Kdim = Kdim; a.a_ld = a_ld;
+    a.H = a.P = H; a.W = a.Q = W; a.sh = a.sw = 1;
+    a.ph = a.pw = RS == 9 ? 1 : 0;
+    a.x_img_stride = (int64_t)(Kdim / RS) * (H * W);
+    a.xcd_n_log2 = (int)(per_wave & 3);
+    a.tm_per = ((M + 31) / 32 + (8 >> a.xcd_n_log2) - 1) >> (3 - a.xcd_n_log2);
+    a.tn_per = ((Ncols + 31) / 32 + (1 << a.xcd_n_log2) - 1) >> a.xcd_n_log2;
+    a.magic_tn_per = magic_tn_per;
+    a.magic_pq = magic_pq;
+    a.A2 = nullptr;
+    a.a_z_stride = a.x_z_stride = 0;
+  } else {  // all at once: read where they are first used, they come in several rounds
+    asm volatile("" ::"s"(a.A), "s"(a.X), "s"(a.M), "s"(a.Ncols), "s"(a.Kdim), "s"(a.a_ld), "s"(a.H), "s"(a.W), "s"(a.P), "s"(a.Q), "s"(a.sh), "s"(a.sw),
+                 "s"(a.x_img_stride), "s"(a.a_z_stride), "s"(a.x_z_stride), "s"(a.xcd_n_log2), "s"(a.tm_per), "s"(a.tn_per), "s"(a.magic_tn_per), "s"(a.magic_pq),
+                 "s"(a.magic_q), "s"(a.A2), "s"(a.bias), "s"(a.Cin));
+    if (RS == 1) asm volatile("" ::"s"(a.X2), "s"(a.Kdim2), "s"(a.H2), "s"(a.W2), "s"(a.sh2), "s"(a.sw2), "s"(a.x2_img_stride), "s"(a.bias2));
+  }
+  return a;
+}
+// What the end of the kernel needs, requested at once: read where it is used, each is waited for there.
+#define SMALL_LATE_ARGS()                                                                                                                  \
+  asm volatile("" : "+s"(a.bias), "+s"(a.bias_col), "+s"(a.Cin), "+s"(a.c_row_stride), "+s"(a.Y), "+s"(a.y_row_stride), "+s"(a.y_img_stride), "+s"(a.alpha), \
+               "+s"(a.beta), "+s"(a.act), "+s"(a.act_coef), "+s"(splits), "+s"(partials), "+s"(counters))
+
+template <int KS, bool AMC, bool PLAIN>
+__global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS >= 2 ? 4 : 3))) void conv3x3_f32_small_kernel(
+    const float *A, const float *X, int M, int Ncols, int Kdim, int a_ld, int H, int W, unsigned per_wave, unsigned magic_tn_per, unsigned magic_pq,
+    unsigned magic_q, const IgemmArgs args, int splits, float *partials, unsigned *counters) {
   #if __HIP_DEVICE_COMPILE__
+  IgemmArgs a = small_args<PLAIN>(A, X, M, Ncols, Kdim, a_ld, H, W, 9, per_wave, magic_tn_per, magic_pq, args);
+  if constexpr (PLAIN) a.magic_q = magic_q;
+  const int c_per_wave = (int)(per_wave >> 2);
   __shared__ float red[KS > 1 ? KS : 1][16][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, half = lane >> 5;
   // Workgroups go round-robin over the 8 XCDs (gridDim.x is a multiple of 8, so that holds for every y and
@@ -254,7 +292,7 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS >= 2
   const int tile_n = (xcd & ((1 << a.xcd_n_log2) - 1)) * tn_per + (in_xcd - tm_local * tn_per);
   if (tm_local >= tm_per || tile_m >= tiles_m || tile_n >= tiles_n) return;
   const int tile_id = tile_m * tiles_n + tile_n;
-  const int m0 = tile_m * 32, n0 = tile_n * 32, z = blockIdx.z;
+  const int m0 = tile_m * 32, n0 = tile_n * 32, z = PLAIN ? 0 : blockIdx.z;
   const __amdgpu_buffer_rsrc_t rsrc_a = small_rsrc(a.A + (int64_t)z * a.a_z_stride), rsrc_x = small_rsrc(a.X + (int64_t)z * a.x_z_stride);
 
   const int mrow = min(m0 + l32, a.M - 1);
@@ -298,22 +336,28 @@ __global__ __launch_bounds__(64 * KS) __attribute__((amdgpu_waves_per_eu(KS >= 2
 #pragma unroll
   for (int r = 0; r < 16; r++) acc[r] = 0.f;
   Finish<KS> f;
-  prefetch_finish<KS>(a, z, m0, half, wave, img, pq, f);
   small_pipeline(niter, [&](int i, auto slot, auto last) { load_iter(i, ra[slot], rb[slot], last); },
                  [&](auto slot) {
 #pragma unroll
                    for (int j = 0; j < 9; j++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[slot][j], rb[slot][j], acc, 0, 0, 0);
+                 },
+                 [&]() {
+                   if constexpr (PLAIN) SMALL_LATE_ARGS();
+                   prefetch_finish<KS>(a, z, m0, half, wave, img, pq, f);
                  });
-  reduce_and_store<KS>(a, acc, f, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), partials, counters);
+  reduce_and_store<KS>(a, acc, f, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), splits, partials, counters);
 #endif
 }
 
 // 1x1 geometry (convolution, possibly strided, or matrix product with A rows
 // k-contiguous and B columns contiguous); Kdim % 4 == 0, A rows 16-byte aligned.
-template <int KS, bool AMC>
-__global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmArgs a, const int k_per_wave, float *partials,
-                                                                    unsigned *counters) {
+template <int KS, bool AMC, bool PLAIN>
+__global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const float *A, const float *X, int M, int Ncols, int Kdim, int a_ld, int pixels,
+                                                                    unsigned per_wave, unsigned magic_tn_per, unsigned magic_pq, const IgemmArgs args,
+                                                                    int splits, float *partials, unsigned *counters) {
   #if __HIP_DEVICE_COMPILE__
+  IgemmArgs a = small_args<PLAIN>(A, X, M, Ncols, Kdim, a_ld, 1, pixels, 1, per_wave, magic_tn_per, magic_pq, args);
+  const int k_per_wave = (int)(per_wave >> 2);
   __shared__ float red[KS > 1 ? KS : 1][16][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, half = lane >> 5;
   // Workgroups go round-robin over the 8 XCDs (gridDim.x is a multiple of 8, so that holds for every y and
@@ -329,7 +373,7 @@ __global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmA
   const int tile_n = (xcd & ((1 << a.xcd_n_log2) - 1)) * tn_per + (in_xcd - tm_local * tn_per);
   if (tm_local >= tm_per || tile_m >= tiles_m || tile_n >= tiles_n) return;
   const int tile_id = tile_m * tiles_n + tile_n;
-  const int m0 = tile_m * 32, n0 = tile_n * 32, z = blockIdx.z;
+  const int m0 = tile_m * 32, n0 = tile_n * 32, z = PLAIN ? 0 : blockIdx.z;
   // With a second convolution (a.A2) the reduction is the first's followed by the second's; a wavefront's slice
   // lies in one of them (the launcher makes k_per_wave divide Kdim), so it only picks its operands here.
   const int kbeg_all = ((int)blockIdx.y * KS + wave) * k_per_wave;
@@ -343,7 +387,7 @@ __global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmA
   const bool col_ok = col < a.Ncols;
   const int PQ = a.P * a.Q, HW = second ? a.H2 * a.W2 : a.H * a.W;
   const int img = col_ok ? div_magic(col, PQ, a.magic_pq) : 0, pq = col_ok ? col - img * PQ : 0;
-  const int p = div_magic(pq, a.Q, a.magic_q), q = pq - p * a.Q;
+  const int p = PLAIN ? 0 : div_magic(pq, a.Q, a.magic_q), q = pq - p * a.Q;
   const unsigned x_pix = second ? (unsigned)((int64_t)img * a.x2_img_stride + (int64_t)(p * a.sh2) * a.W2 + q * a.sw2)
                                 : (unsigned)((int64_t)img * a.x_img_stride + (int64_t)(p * a.sh) * a.W + q * a.sw);
   // Half-wave h of iteration i takes k kbeg + 8 i + 4 h .. + 3 (Kd is a multiple of 4): h in the lane's offset, the rest in the scalar one.
@@ -392,6 +436,7 @@ __global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmA
     for (int d = 0; d < DEPTH; d++)
       if (d < niter) load_iter(d, ra[d], rb[d]);
   }
+  if constexpr (PLAIN) SMALL_LATE_ARGS();
   Finish<KS> f;
   prefetch_finish<KS>(a, z, m0, half, wave, img, pq, f);
   if (a.A2 != nullptr && a.bias2 != nullptr) {  // both biases ride in the one epilogue
@@ -418,7 +463,7 @@ __global__ __launch_bounds__(64 * KS) void conv1x1_f32_small_kernel(const IgemmA
 #pragma unroll
   for (int u = 0; u < DEPTH; u++)
     if (i0 + u < niter) mfma_iter(u);
-  reduce_and_store<KS>(a, acc, f, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), partials, counters);
+  reduce_and_store<KS>(a, acc, f, bias_c, red, wave, lane, m0, img, pq, col_ok, z, (unsigned)(z * tiles + tile_id), splits, partials, counters);
 #endif
 }
 
@@ -511,25 +556,36 @@ bool launch_igemm_f32_small(const dnnrtContext *ctx, const IgemmArgs &a, int rsm
   }
   dim3 grid((unsigned)slots, splits, a.Z);
   if (ctx->splitk_shared && splits > 1) clear_split_counters(ctx, tiles * a.Z);
-#define LAUNCH_KS2(KERNEL, AMC_, ARG)                                                                  \
-  switch (ks) {                                                                                          \
-    case 1: hipLaunchKernelGGL((KERNEL<1, AMC_>), grid, dim3(64), 0, ctx->stream, am, ARG, ctx->splitk_partials, ctx->splitk_counters); break;  \
-    case 2: hipLaunchKernelGGL((KERNEL<2, AMC_>), grid, dim3(128), 0, ctx->stream, am, ARG, ctx->splitk_partials, ctx->splitk_counters); break; \
-    case 4: hipLaunchKernelGGL((KERNEL<4, AMC_>), grid, dim3(256), 0, ctx->stream, am, ARG, ctx->splitk_partials, ctx->splitk_counters); break; \
-    default: hipLaunchKernelGGL((KERNEL<8, AMC_>), grid, dim3(512), 0, ctx->stream, am, ARG, ctx->splitk_partials, ctx->splitk_counters); break; \
+  const int per_wave = is3x3 ? (int)(ceil_div(ceil_div(red_len, ks * splits), 2) * 2) : k_per_wave_1x1;
+  const unsigned per_wave_xn = 4u * (unsigned)per_wave + (unsigned)am.xcd_n_log2;
+  const bool one_image = a.Ncols <= a.P * a.Q;  // of the images' distance nothing is read
+  const bool plain = a.Z == 1 && !dual && a.sh == 1 && a.sw == 1 && a.P == a.H && a.Q == a.W && a.ph == (is3x3 ? 1 : 0) && a.pw == a.ph &&
+                     (one_image || a.x_img_stride == (int64_t)(a.Kdim / (is3x3 ? 9 : 1)) * a.H * a.W);
+#define LAUNCH_3X3(KS_, AMC_, PLAIN_)                                                                                                          \
+  hipLaunchKernelGGL((conv3x3_f32_small_kernel<KS_, AMC_, PLAIN_>), grid, dim3(64 * KS_), 0, ctx->stream, a.A, a.X, a.M, a.Ncols, a.Kdim,       \
+                     (int)a.a_ld, a.H, a.W, per_wave_xn, am.magic_tn_per, am.magic_pq, am.magic_q, am, splits, ctx->splitk_partials, ctx->splitk_counters)
+#define LAUNCH_1X1(KS_, AMC_, PLAIN_)                                                                                                          \
+  hipLaunchKernelGGL((conv1x1_f32_small_kernel<KS_, AMC_, PLAIN_>), grid, dim3(64 * KS_), 0, ctx->stream, a.A, a.X, a.M, a.Ncols, a.Kdim,       \
+                     (int)a.a_ld, a.H * a.W, per_wave_xn, am.magic_tn_per, am.magic_pq, am, splits, ctx->splitk_partials, ctx->splitk_counters)
+#define LAUNCH_KS(WHICH, AMC_, PLAIN_)          \
+  switch (ks) {                                 \
+    case 1: WHICH(1, AMC_, PLAIN_); break;      \
+    case 2: WHICH(2, AMC_, PLAIN_); break;      \
+    case 4: WHICH(4, AMC_, PLAIN_); break;      \
+    default: WHICH(8, AMC_, PLAIN_); break;     \
   }
-#define LAUNCH_KS(KERNEL, ARG)                                                                         \
-  do {                                                                                                 \
-    if (amc) { LAUNCH_KS2(KERNEL, true, ARG) } else { LAUNCH_KS2(KERNEL, false, ARG) }                 \
+#define LAUNCH_AMC(WHICH, PLAIN_)                                                            \
+  do {                                                                                       \
+    if (amc) { LAUNCH_KS(WHICH, true, PLAIN_) } else { LAUNCH_KS(WHICH, false, PLAIN_) }     \
   } while (0)
-  if (is3x3) {
-    const int c_per_wave = (int)(ceil_div(ceil_div(red_len, ks * splits), 2) * 2);
-    LAUNCH_KS(conv3x3_f32_small_kernel, c_per_wave);
-  } else {
-    LAUNCH_KS(conv1x1_f32_small_kernel, k_per_wave_1x1);
-  }
+  if (is3x3 && plain) LAUNCH_AMC(LAUNCH_3X3, true);
+  else if (is3x3) LAUNCH_AMC(LAUNCH_3X3, false);
+  else if (plain) LAUNCH_AMC(LAUNCH_1X1, true);
+  else LAUNCH_AMC(LAUNCH_1X1, false);
+#undef LAUNCH_AMC
 #undef LAUNCH_KS
-#undef LAUNCH_KS2
+#undef LAUNCH_1X1
+#undef LAUNCH_3X3
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("igemm_f32(small): launch failed: %s", hipGetErrorString(e)); return false; }
   launched = true;

@@ -1946,6 +1946,28 @@ def test_conv_3x3_small_for_every_length_of_a_wavefronts_slice(gpu, geometry, Cc
         assert (np.abs(got - ref) <= (9 * Cc + 1) * 2.0 ** -24 * magnitude).all()
 
 
+# N, C, H, W, K, filter side, stride, pad, groups: on either side of the line between the kernels that know one image size, stride 1 and one
+# group, and those that take any; one image and several, tiles that end within an image, slices that end the reduction early
+@pytest.mark.parametrize("case", [(1, 40, 9, 13, 36, 1, 1, 0, 1), (3, 40, 9, 13, 36, 1, 1, 0, 1), (2, 72, 7, 5, 68, 1, 2, 0, 1), (2, 64, 6, 11, 48, 1, 1, 0, 2), (1, 256, 14, 14, 64, 1, 1, 0, 1),
+                                  (1, 12, 9, 13, 36, 3, 1, 1, 1), (3, 12, 9, 13, 36, 3, 1, 1, 1), (2, 12, 9, 13, 36, 3, 1, 0, 1), (2, 12, 8, 13, 36, 3, 1, 2, 1),
+                                  (1, 24, 9, 10, 40, 3, 2, 1, 1), (2, 16, 6, 11, 48, 3, 1, 1, 2), (1, 96, 14, 14, 64, 3, 1, 1, 1)], ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("crsk", [False, True])
+def test_conv_f32_small_of_one_image_size_and_others(gpu, case, crsk):
+    """Bound: each of the C R S + 2 additions rounds by at most 2^-24 of the sum of magnitudes."""
+    import torch
+    N, Cc, H, W, K, R, st, pad, g = case
+    r = rng(sum(case))
+    x = r.standard_normal((N, Cc, H, W)).astype(np.float32)
+    w = (r.standard_normal((K, Cc // g, R, R)) * np.sqrt(2.0 / (R * R * Cc))).astype(np.float32)
+    b = r.uniform(-0.5, 0.5, K).astype(np.float32)
+    conv64 = lambda t, f, v: torch.nn.functional.conv2d(*(torch.from_numpy(u).double() for u in (t, f, v)), stride=st, padding=pad, groups=g).numpy()  # noqa: E731
+    ref, magnitude = conv64(x, w, b), conv64(np.abs(x), np.abs(w), np.abs(b))
+    z = r.standard_normal(ref.shape).astype(np.float32)
+    for _ in range(2):  # twice: the split reduction's counters must be back at zero
+        got = oc.conv(gpu, x, w, b, (pad, pad), (st, st), g, _abi.ACT_RELU, crsk=crsk, z=z)
+        assert (np.abs(got - np.maximum(ref + z, 0)) <= (Cc // g * R * R + 2) * 2.0 ** -24 * (magnitude + np.abs(z))).all()
+
+
 # N, C, H, W, K, pad: patches cut by every border, fewer channels than wavefronts and odd numbers of them, every number of filters
 @pytest.mark.parametrize("case", [(1, 1, 1, 1, 1, 1), (2, 2, 17, 15, 2, 1), (1, 3, 16, 33, 3, 0), (2, 7, 20, 18, 4, 2), (1, 64, 90, 117, 3, 1), (3, 13, 5, 70, 1, 1)],
                          ids=lambda c: "x".join(map(str, c)))
