@@ -82,6 +82,15 @@ __global__ __launch_bounds__(256) void conv_f32_dma_kernel(const IgemmArgs a, co
   static_assert(A_RPI <= 4 && B_RPI <= 4, "an instruction's rows belong to one wavefront");
   constexpr int L = 4 * A_IPR / A_RPI + 4 * B_IPR / B_RPI;  // loads per wavefront and step
   extern __shared__ __attribute__((aligned(1024))) char smem[];
+  // The arguments, all at once: read where they are first used, they came in four rounds in front of the first load and in more at
+  // the end, a fraction of a microsecond each.
+  asm volatile("" ::"s"(pl.tiles_m), "s"(pl.whole), "s"(pl.rest), "s"(pl.splits), "s"(pl.round), "s"(pl.units), "s"(pl.steps), "s"(pl.steps_per_split),
+               "s"((int)pl.neighbours), "s"(pl.magic_tiles_m), "s"(pl.magic_round), "s"(a.A), "s"(a.X), "s"(a.a_ld), "s"(a.M), "s"(a.Kdim), "s"(a.Ncols),
+               "s"(a.H), "s"(a.W), "s"(a.P), "s"(a.Q), "s"(a.sh), "s"(a.sw), "s"(a.x_img_stride), "s"(a.magic_pq), "s"(a.magic_q), "s"(a.bias));
+  asm volatile("" ::"s"(a.Y), "s"(a.Cin), "s"(a.y_img_stride), "s"(a.y_row_stride), "s"(a.c_row_stride), "s"(a.act), "s"(a.act_coef), "s"(partials),
+               "s"(counters));
+  if constexpr (MODE != D32_POINTWISE) asm volatile("" ::"s"(a.R), "s"(a.S), "s"(a.ph), "s"(a.pw));
+  if constexpr (DUAL) asm volatile("" ::"s"(a.A2), "s"(a.X2), "s"(a.bias2), "s"(a.Kdim2), "s"(a.H2), "s"(a.W2), "s"(a.sh2), "s"(a.sw2), "s"(a.x2_img_stride));
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

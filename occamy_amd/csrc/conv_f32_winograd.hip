@@ -66,6 +66,12 @@ template <int AV>
 __global__ __launch_bounds__(256, 2) void conv_f32_winograd_kernel(const IgemmArgs a, const Wino32Plan pl, float *partials, unsigned *counters) {
 #if __HIP_DEVICE_COMPILE__
   extern __shared__ __attribute__((aligned(1024))) char smem[];
+  // the arguments, all at once, as in conv_f32_dma.hip
+  asm volatile("" ::"s"(pl.tiles_m), "s"(pl.whole), "s"(pl.rest), "s"(pl.splits), "s"(pl.units), "s"(pl.stages), "s"(pl.stages_per_split), "s"(pl.th), "s"(pl.tw),
+               "s"(pl.n_tiles), "s"(pl.magic_tiles_m), "s"(pl.magic_rest), "s"(pl.magic_thw), "s"(pl.magic_tw), "s"(a.A), "s"(a.X), "s"(a.a_ld), "s"(a.M),
+               "s"(a.Kdim), "s"(a.Ncols), "s"(a.H), "s"(a.W), "s"(a.P), "s"(a.Q), "s"(a.ph), "s"(a.pw), "s"(a.x_img_stride), "s"(a.magic_pq), "s"(a.bias));
+  asm volatile("" ::"s"(a.Y), "s"(a.Cin), "s"(a.y_img_stride), "s"(a.y_row_stride), "s"(a.c_row_stride), "s"(a.act), "s"(a.act_coef), "s"(partials),
+               "s"(counters));
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
