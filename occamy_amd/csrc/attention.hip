@@ -7,7 +7,7 @@
 // CUDAMatmulNdFunc, the scaling Mul, CUDASoftmaxFunc, CUDAMatmulNdFunc, Transpose
 // + Reshape back -- twelve launches and eleven round trips through memory.
 //
-// fp32: one workgroup = 32 queries of one head; its four wavefronts split every block
+// fp32, many workgroups (attention_few_kernel takes the others): one workgroup = 32 queries of one head; its four wavefronts split every block
 // of 128 keys (32 each).  Scores are computed transposed (keys x queries) so
 // that a lane owns one query: the soft-max statistics are per lane, and the
 // exponentiated scores already sit in the register layout the second product
@@ -19,6 +19,7 @@
 namespace dnnrt {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 att_half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 att_half4 __attribute__((ext_vector_type(4)));
 typedef short att_short4 __attribute__((ext_vector_type(4)));
@@ -192,6 +193,150 @@ __global__ __launch_bounds__(256) void attention_kernel(const float *__restrict_
     }
     store4(Yg + (int64_t)(q0 + q) * ld + c4 * 4, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
   }
+}
+
+// fp32, few workgroups: 16 queries of one head.  Its NW wavefronts take every NW-th block of 32 keys, each on its own, with its own
+// running maximum and sum, and no barrier until the partial results meet.  All operands go straight from global memory into the shape of
+// v_mfma_f32_16x16x4f32: a lane has the quarter (lane / 16) of the head dimension of its query and its keys, and of V the four
+// keys of its quarter, whose probabilities are in its registers.  The next block's keys are requested behind the scores, its values
+// behind the second product.
+// Bound by the chain of one block: loads, half the 32-query kernel's MFMAs, exponentials, the meeting in LDS.  Back to back, against that
+// kernel (us): 12 heads of 64, 128 tokens 7.0 -> 5.6, 32 tokens 7.1 -> 4.5, 256 tokens 11.0 -> 8.3, 16 queries over 512 keys 18.3 -> 11.2;
+// 8 heads of 128, 128 tokens 10.5 -> 8.5.  Error against 64 bits 0.88 to 1.0 of that kernel's.  A BERT-base over 128 tokens 664 -> 641.
+template <typename F>
+__device__ __forceinline__ float over_quarters(float v, F f) {  // f of the four lanes that hold a query's keys, in all
+#if __HIP_DEVICE_COMPILE__
+  const auto rows = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  v = f(__builtin_bit_cast(float, (unsigned)rows[0]), __builtin_bit_cast(float, (unsigned)rows[1]));
+#endif
+  return over_halves(v, f);
+}
+
+template <int DH, int NW>
+__global__ __launch_bounds__(64 * NW) void attention_few_kernel(const float *__restrict__ Q, const float *__restrict__ K, const float *__restrict__ V,
+                                                                float *__restrict__ Y, int Sq, int Sk, int ld_in, int ld, float scale) {
+#if __HIP_DEVICE_COMPILE__
+  constexpr int T = DH / 16, ROW = DH + 4;
+  __shared__ __attribute__((aligned(16))) float red[NW * 16 * ROW];
+  __shared__ float mx[NW * 16], sm[NW * 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, quarter = lane >> 4;
+  const int q0 = blockIdx.x * 16, head = blockIdx.y, b = blockIdx.z;
+  const float *Qg = Q + (int64_t)b * Sq * ld_in + head * DH + quarter * (DH / 4);
+  const float *Kg = K + (int64_t)b * Sk * ld_in + head * DH + quarter * (DH / 4);
+  const float *Vg = V + (int64_t)b * Sk * ld_in + head * DH + l16;
+  float4 qf[T], kf[2][T];
+  float vf[2][4][T];
+  auto fetch_keys = [&](int k0) {  // rows past the end repeat the last key, masked below
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int j = 0; j < T; j++) kf[u][j] = load4(Kg + (int64_t)min(k0 + 16 * u + l16, Sk - 1) * ld_in + 4 * j);
+  };
+  auto fetch_values = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int t = 0; t < T; t++) vf[u][r][t] = Vg[(int64_t)min(k0 + 16 * u + 4 * quarter + r, Sk - 1) * ld_in + 16 * t];
+  };
+#pragma unroll
+  for (int j = 0; j < T; j++) qf[j] = load4(Qg + (int64_t)min(q0 + l16, Sq - 1) * ld_in + 4 * j);
+  floatx4 o[T];
+#pragma unroll
+  for (int t = 0; t < T; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[t][r] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  int k0 = 32 * wave;
+  if (k0 < Sk) { fetch_keys(k0); fetch_values(k0); }
+  for (; k0 < Sk; k0 += 32 * NW) {
+    floatx4 s[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) s[u][r] = 0.f;
+#pragma unroll
+    for (int j = 0; j < T; j++) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][j].x, qf[j].x, s[u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < 2; u++) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][j].y, qf[j].y, s[u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < 2; u++) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][j].z, qf[j].z, s[u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < 2; u++) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][j].w, qf[j].w, s[u], 0, 0, 0);
+    }
+    const bool more = k0 + 32 * NW < Sk, last = k0 + 32 > Sk;
+    if (more) fetch_keys(k0 + 32 * NW);
+    // register r of s[u]: key k0 + 16 u + 4 quarter + r, query l16
+    float m_new = m_run;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const bool in = !last || k0 + 16 * u + 4 * quarter + r < Sk;
+        s[u][r] = in ? s[u][r] * scale : -INFINITY;
+        m_new = fmaxf(m_new, s[u][r]);
+      }
+    m_new = over_quarters(m_new, [](float x, float y) { return fmaxf(x, y); });
+    const float from = m_new == -INFINITY ? 0.f : m_new;  // this wavefront's keys alone may all have no weight
+    const float alpha = expf(m_run - from);               // 0 on the first block
+    float lsum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) { s[u][r] = expf(s[u][r] - from); lsum += s[u][r]; }
+    l_run = l_run * alpha + lsum;  // this lane's keys; the quarters and wavefronts are added at the end
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) o[t][r] *= alpha;
+    if (last) {  // past the end the probability is zero, which times a repeated infinity would be NaN
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+          for (int t = 0; t < T; t++) vf[u][r][t] = k0 + 16 * u + 4 * quarter + r < Sk ? vf[u][r][t] : 0.f;
+    }
+    // O^T[d][query] += V^T[d][key] P^T[key][query]: step (u, r) takes, in lane quarter h, key 16 u + 4 h + r
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int t = 0; t < T; t++) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][r][t], s[u][r], o[t], 0, 0, 0);
+    if (more) fetch_values(k0 + 32 * NW);
+  }
+  // the wavefronts' results: [NW][16 queries][ROW], their maxima and sums
+  l_run = over_quarters(l_run, [](float x, float y) { return x + y; });
+  if (quarter == 0) { mx[wave * 16 + l16] = m_run; sm[wave * 16 + l16] = l_run; }
+#pragma unroll
+  for (int t = 0; t < T; t++)
+    store4(red + (wave * 16 + l16) * ROW + 16 * t + 4 * quarter, make_float4(o[t][0], o[t][1], o[t][2], o[t][3]));
+  __syncthreads();
+  float *Yg = Y + (int64_t)b * Sq * ld + head * DH;
+  for (int i = tid; i < 16 * (DH / 4); i += 64 * NW) {
+    const int q = i / (DH / 4), c = i - q * (DH / 4);
+    if (q0 + q >= Sq) continue;
+    float m = mx[q];
+#pragma unroll
+    for (int w = 1; w < NW; w++) m = fmaxf(m, mx[w * 16 + q]);
+    float sum = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float f = expf(mx[w * 16 + q] - m);  // 0 for a wavefront that had no keys
+      const float4 p = load4(red + (w * 16 + q) * ROW + 4 * c);
+      sum += f * sm[w * 16 + q];
+      acc.x += f * p.x; acc.y += f * p.y; acc.z += f * p.z; acc.w += f * p.w;
+    }
+    const float inv = 1.0f / sum;
+    store4(Yg + (int64_t)(q0 + q) * ld + 4 * c, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
+  }
+#endif
 }
 
 // exp(d) of a score below its maximum, d <= 0 or NaN, as 2^(d log2 e) with what the product rounds away put back to first order: half
@@ -372,6 +517,15 @@ __global__ __launch_bounds__(64 * NW) void attention_f16_kernel(const _Float16 *
 template <int DH>
 static void launch_attention(const dnnrtContext *ctx, const float *Q, const float *K, const float *V, float *Y, int B,
                              int Sq, int Sk, int H, int ld_in, float scale) {
+  // While 16 queries a workgroup are no more than one per compute unit; beyond, the 32-query kernel reads K and V half as often: 384
+  // tokens, 12 heads 16.0 here, 15.2 there; 4 x 128 tokens 8.8, 7.3 (one long sequence, 1024 tokens, 48.5 and 54.9, is the exception).
+  if (ceil_div(Sq, 16) * H * B <= (int64_t)ctx->num_cu) {
+    constexpr int MORE = DH <= 64 ? 8 : 4;
+    const dim3 grid((unsigned)ceil_div(Sq, 16), (unsigned)H, (unsigned)B);
+    if (Sk > 128) hipLaunchKernelGGL((attention_few_kernel<DH, MORE>), grid, dim3(64 * MORE), 0, ctx->stream, Q, K, V, Y, Sq, Sk, ld_in, H * DH, scale);
+    else hipLaunchKernelGGL((attention_few_kernel<DH, 4>), grid, dim3(256), 0, ctx->stream, Q, K, V, Y, Sq, Sk, ld_in, H * DH, scale);
+    return;
+  }
   constexpr int ROW = DH + 4;
   const size_t lds = (size_t)((ATT_QB + 2 * ATT_KB) * ROW + 8 * 32) * sizeof(float);
   static LdsRaised raised;

@@ -720,6 +720,31 @@ def test_every_lane_counts_once_in_sums_and_maxima_over_a_wavefront(gpu, L):
     np.testing.assert_array_equal(oc.softmax(gpu, hot, 1), np.eye(L, dtype=np.float32))
 
 
+# B, queries, keys, heads, head size: on either side of 16 queries, of a block of 32 keys, of one round of four and of eight wavefronts, of
+# the number of workgroups from which 32 queries are taken at a time; wavefronts without keys
+@pytest.mark.parametrize("case", [(1, 1, 1, 1, 32), (1, 15, 31, 2, 64), (2, 16, 33, 3, 128), (1, 17, 96, 2, 64), (1, 33, 127, 4, 32), (1, 128, 128, 12, 64), (3, 20, 129, 2, 64),
+                                  (1, 50, 255, 3, 128), (1, 64, 257, 12, 64), (2, 31, 300, 2, 32), (1, 8, 700, 1, 64), (1, 337, 40, 12, 64), (1, 320, 40, 13, 64)], ids=str)
+def test_attention_f32_of_few_queries(gpu, case):
+    """Against 64 bits.  Bound: a score's product of DH terms rounds by at most (DH + 2) 2^-24 of the terms' magnitudes; a probability
+    changes by as much, relative, with its sum's, and the two sums over the keys round by 2^-24 a term."""
+    B, Sq, Sk, H, D = case
+    r = rng(sum(case))
+    q, k, v = (r.standard_normal((B, n, H * D)).astype(np.float32) for n in (Sq, Sk, Sk))
+    scale = 1.0 / np.sqrt(D)
+    split = lambda t: t.astype(np.float64).reshape(B, -1, H, D).transpose(0, 2, 1, 3)  # noqa: E731
+    q6, k6, v6 = split(q), split(k), split(v)
+    s = scale * (q6 @ k6.transpose(0, 1, 3, 2))
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    u = 2.0 ** -24
+    e = (D + 2) * u * (scale * (np.abs(q6) @ np.abs(k6).transpose(0, 1, 3, 2))).max(-1, keepdims=True) + 2 * u * (s.max(-1, keepdims=True) - s).max(-1, keepdims=True)
+    merge = lambda t: t.transpose(0, 2, 1, 3).reshape(B, Sq, H * D)  # noqa: E731
+    want, bound = merge(p @ v6), merge((4 * e + (2 * Sk + 12) * u) * (p @ np.abs(v6)))
+    got = oc.attention(gpu, q, k, v, H, scale)
+    assert (np.abs(got - want) <= bound).all()
+    np.testing.assert_array_equal(oc.attention(gpu, q, k, v, H, scale), got)
+
+
 @pytest.mark.parametrize("case", [(1, 384, 384, 12, 64), (2, 31, 257, 3, 64), (1, 70, 129, 2, 32), (1, 64, 160, 5, 32), (1, 45, 513, 2, 128),
                                   (1, 1, 1, 1, 64), (3, 33, 32, 2, 64), (1, 600, 600, 16, 64)], ids=str)
 def test_attention_f16_blocks_and_wavefronts(gpu, cpu, case):
