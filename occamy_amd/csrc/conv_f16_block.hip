@@ -108,7 +108,8 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
   constexpr bool EXPAND = KC > 0;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 #if __HIP_DEVICE_COMPILE__
-  // What the first loads need of the arguments, all at once: read where they are first used, each round is a fraction of a microsecond.
+  // What the first loads need of the arguments, all at once: read where they are first used, each round is a fraction of a microsecond
+  // (MobileNetV2 at batch 64 456.8 -> 455.8 us).
   asm volatile("" ::"s"(a.X), "s"(a.H), "s"(a.W), "s"(a.Cin), "s"(a.Ch), "s"(a.ph), "s"(a.pw), "s"(a.TH), "s"(a.TW), "s"(a.PH), "s"(a.PW), "s"(a.xs_bytes),
                "s"(a.slab_bytes), "s"(a.tiles_w), "s"(a.tiles_hw), "s"(a.tiles), "s"(a.per_xcd), "s"(a.per_split), "s"(a.magic_tiles_w), "s"(a.magic_tiles_hw),
                "s"(a.magic_c8), "s"((int)blockDim.x));

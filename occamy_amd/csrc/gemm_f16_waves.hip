@@ -65,7 +65,8 @@ __device__ __forceinline__ void gw_arrived(T &v) {
 }
 
 // Tiles of 64 columns n and 32 TM rows m; B_KC: B stored [N,K].  The arguments in front of the struct are in registers when a
-// wavefront starts: all that the ring's first loads need, so that nothing waits for the rest, which comes 0.45 us later.
+// wavefront starts: all that the ring's first loads need, so that nothing waits for the rest, which comes 0.45 us later
+// (a BERT-base over 384 tokens, 48 of its 88 launches here and in gemm_f16_dma.hip, 541 -> 530 us).
 template <bool B_KC, int TM>
 __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const __half *A, const __half *B, int64_t az, int64_t bz, int M, int N, int K, int tiles,
                                                                 unsigned magic_tiles_m, int steps_per_split, const GemmF16Args args, int splits) {

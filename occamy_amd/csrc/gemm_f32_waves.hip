@@ -46,7 +46,8 @@ __device__ __forceinline__ void f32w_wait() {  // s_waitcnt vmcnt(N) lgkmcnt(LGK
 }
 
 // TM: blocks of 32 rows of a tile.  The arguments in front of the structs are in registers when a wavefront starts: all that the
-// ring's first loads need, so that nothing waits for the rest, which comes 0.45 us later.  (They are in `args` and `plan` too.)
+// ring's first loads need, so that nothing waits for the rest, which comes 0.45 us later
+// (a BERT-base over 128 tokens, 36 of its 88 launches here and 12 in the small 1x1 kernel, 702 -> 663 us).  They are in the structs too.
 template <int TM>
 __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const float *A, const float *X, int M, int Kdim, int Ncols, int units, int rest, int whole,
                                                                 int stages_per_split, int tiles_m, unsigned magic_round, unsigned magic_tiles_m,
