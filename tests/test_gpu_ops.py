@@ -511,6 +511,23 @@ def test_layernorm(gpu, cpu):
                                    rtol=2e-2, atol=2e-2)
 
 
+# one lane's group of four to eight wavefronts a row, a last group short of the wavefront and of the row; few rows, and more than share the chip that way
+@pytest.mark.parametrize("L", [4, 252, 256, 260, 508, 768, 1028, 1536, 1540, 2044, 2048])
+@pytest.mark.parametrize("rows", [1, 130, 400])
+def test_layernorm_of_few_rows(gpu, rows, L):
+    """Against 64 bits.  Bound: the sums over a row are trees of at most 17 additions, so the mean is within 20 2^-24 of the mean magnitude,
+    and the deviations, their mean square, root, quotient and the last two operations round a few times each."""
+    r = rng(rows + L)
+    x = (r.standard_normal((rows, L)) * 3 + 1).astype(np.float32)
+    g, b = r.standard_normal(L).astype(np.float32), r.standard_normal(L).astype(np.float32)
+    x6, u = x.astype(np.float64), 2.0 ** -24
+    d = x6 - x6.mean(-1, keepdims=True)
+    inv = 1 / np.sqrt((d * d).mean(-1, keepdims=True) + 1e-5)
+    mean_error = 20 * u * np.abs(x6).mean(-1, keepdims=True)
+    bound = inv * np.abs(g) * (2 * mean_error + np.abs(d) * (28 * u + 2 * mean_error * inv)) + 4 * u * np.abs(b)
+    assert (np.abs(oc.layernorm(gpu, x, g, b, 1e-5) - (d * inv * g + b)) <= bound).all()
+
+
 # ---- pooling ---------------------------------------------------------------------------
 
 def test_pooling(gpu, cpu):
