@@ -30,7 +30,9 @@ typedef __attribute__((address_space(3))) void *lds_ptr;
 [[maybe_unused]] constexpr unsigned F32W_OUT_OF_RANGE = 0x80000000u;  // above every num_records used here: reads as zeros
 constexpr int F32W_BK = 16;                     // k of a stage
 constexpr int f32w_stage(int tm) { return (64 + 32 * tm) * F32W_BK * 4; }             // its bytes: 64 columns n and 32 tm rows m
-constexpr int f32w_wave(int tm) { return (tm == 2 ? 2 : 3) * f32w_stage(tm); }  // a wavefront's ring of two or three stages; later its sums
+// A wavefront's ring of two stages; later its sums.  With tiles of 32 rows a third stage costs where the weights come from HBM (340 MB in a
+// fp32 BERT-base, 128 tokens: 627 us with two, 634 with three, 656 with four, 676 with five) and gives nothing where they do not.
+constexpr int f32w_wave(int tm) { return 2 * f32w_stage(tm); }
 
 // How a launch is cut: workgroups 0 .. units - 1 (a multiple of 8) are the split tiles' parts, the rest whole tiles.
 struct Waves32Plan {
@@ -180,10 +182,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_waves_kernel(const float *A, 
   };
   constexpr std::integral_constant<int, 0> c0{};
   constexpr std::integral_constant<int, 1> c1{};
-  auto landed = [&](int behind) {  // the oldest stage in flight has landed, up to NS - 1 behind it may still be on their way
-    if (behind >= NS - 1) f32w_wait<(NS - 1) * L>();
-    else if (NS > 3 && behind == 2) f32w_wait<2 * L>();
-    else if (NS > 2 && behind == 1) f32w_wait<L>();
+  auto landed = [&](int behind) {  // the oldest stage in flight has landed, one behind it may still be on its way
+    if (behind >= 1) f32w_wait<L>();
     else f32w_wait<0>();
   };
   auto step = [&](auto set_c, int ahead) {  // one stage, its operands in set S or on their way there; `ahead` follow it
@@ -342,11 +342,7 @@ bool launch_gemm_f32_waves(const dnnrtContext *ctx, const IgemmArgs &a, bool &la
   const unsigned grid = (unsigned)(pl.units + ceil_div(pl.whole, 8) * 8);
   const auto kernel = tm == 2 ? gemm_f32_waves_kernel<2> : gemm_f32_waves_kernel<1>;
   const int lds = 4 * f32w_wave(tm);
-  static LdsRaised raised[2];
-  if (lds > 64 * 1024 && !raise_lds(raised[tm - 1], ctx->device, reinterpret_cast<const void *>(kernel), lds)) {
-    set_error("gemm_f32(waves): cannot reserve %d bytes of LDS", lds);
-    return false;
-  }
+  static_assert(4 * f32w_wave(2) <= 64 * 1024, "no more LDS than a kernel gets without asking");
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), (size_t)lds, ctx->stream, a.A, a.X, a.M, a.Kdim, a.Ncols, pl.units, pl.rest, pl.whole,
                      pl.stages_per_split, pl.tiles_m, pl.magic_round, pl.magic_tiles_m, a, pl, ctx->splitk_partials, ctx->splitk_counters);
   hipError_t e = hipGetLastError();
