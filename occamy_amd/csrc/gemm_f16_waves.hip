@@ -87,10 +87,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const __half *A,
   const int n0 = tile_n * 64, m0 = tile_m * FM, z = blockIdx.z;
   char *ring = smem + wave * WAVE_LDS;
 
-  // ---- this wavefront's stages ----------------------------------------------
+  // ---- this wavefront's stages: every fourth, so that the four read neighbouring rows of B and the same lines of the operands' k-contiguous rows
+  // at a time (a quarter each in a run: BERT-base over 384 tokens 526 -> 511 us) ----
   const int stages = (a.K + GW_BK - 1) / GW_BK;
   const int s_beg = (int)blockIdx.y * a.steps_per_split, s_end = min(stages, s_beg + a.steps_per_split);
-  const int per_wave = (s_end - s_beg + 3) >> 2, my_beg = s_beg + wave * per_wave, nk = max(0, min(per_wave, s_end - my_beg));
+  const int my_beg = s_beg + wave, nk = max(0, (s_end - my_beg + 3) >> 2);
 
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(A) + (int64_t)z * az, 0, 2 * a.M * a.K, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half *>(B) + (int64_t)z * bz, 0, 2 * a.K * a.N, 0x00020000);
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_waves_kernel(const __half *A,
 #pragma unroll
     for (int i = 0; i < M_L; i++)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (gw_lds)(Ms + 1024 * i), 16, m_past ? GW_OUT_OF_RANGE : m_off[i], 2 * l_k, 0, 0);
-    l_k += GW_BK;
+    l_k += 4 * GW_BK;
     l_slot = l_slot + 1 == NS ? 0 : l_slot + 1;
   };
 
