@@ -1000,7 +1000,7 @@ bool Session::fill_dead(const std::vector<Range> &held, int n, void *base) const
   return true;
 }
 
-// The per-inference sequence with the constants uploaded on a stream of their own (plan_uploads).
+// The per-inference sequence with the constants uploaded on two streams of their own (plan_uploads).
 bool Session::run_uploading(const void *const *inputs, void *const *outputs, std::string &err) {
   void *run_pool = nullptr;
   size_t next = 0, landed = 0;  // the next upload to issue; those that the compute stream has waited for
@@ -1076,10 +1076,11 @@ bool Session::run_uploading(const void *const *inputs, void *const *outputs, std
   for (size_t i = 0; i < prog->args.size(); i++) ptr[(size_t)prog->args[i]->id] = host_in[i];
   for (const Op *op : prog->ops) {
     if (one(op)) continue;
-    // both streams have to be done with the pool before it goes
-    for (size_t i = 0; i < next; i++)
-      if (uploads[i].landed) rt.dnnrtExecStreamWait(stream, uploads[i].landed);
-    rt.dnnrtSync(handle);
+    // All three streams have to be done with the pool before it goes: a copy that no event stands behind yet, too.
+    for (dnnrtStream_t s : {upload_stream[0], upload_stream[1], stream}) {
+      rt.dnnrtSetStream(handle, s);
+      rt.dnnrtSync(handle);
+    }
     if (run_pool) rt.dnnrtDealloc(run_pool);
     return false;
   }

@@ -155,3 +155,74 @@ def test_a_constant_is_there_when_its_stream_is_as_late_as_the_waits_allow(tmp_p
             np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-4)
     assert C.CDLL(runtime).used_streams() == 2
     s.close()
+
+
+FAILING_SHIM = r"""
+#define dnnrtSync late_sync
+#define dnnrtDealloc late_dealloc
+#define dnnrtMemPoolInit late_pool_init
+#define dnnrtExecUpload late_upload
+""" + LATE_SHIM.replace("(void)h; computing = s;", "(void)h; current = s; if (!computing) computing = s;").replace("static dnnrtStream_t computing;", "static dnnrtStream_t computing, current;") + r"""
+#undef dnnrtSync
+#undef dnnrtDealloc
+#undef dnnrtMemPoolInit
+#undef dnnrtExecUpload
+static int uploads_left = -1, early;
+static char *pool_lo, *pool_hi;
+void fail_at(int uploads) { uploads_left = uploads; }
+int copies_into_a_pool_that_is_gone(void) { return early; }
+int32_t dnnrtSync(dnnrtHandle_t h) { (void)h; run_upto((int)(intptr_t)current, queued[(intptr_t)current]); return 0; }
+int32_t dnnrtMemPoolInit(void **pool, int64_t bytes) {
+  const int32_t r = late_pool_init(pool, bytes);
+  pool_lo = *pool;
+  pool_hi = pool_lo + bytes;
+  return r;
+}
+int32_t dnnrtDealloc(void *p) {
+  for (int s = 0; s < 8 && p == pool_lo; s++)
+    for (; done[s] < queued[s]; done[s]++) {
+      char *dst = queue[s][done[s] %% QUEUED].dst;
+      early += dst >= pool_lo && dst < pool_hi;
+    }
+  return late_dealloc(p);
+}
+int32_t dnnrtExecUpload(void *dst, const void *src, int64_t bytes, dnnrtStream_t stream) {
+  if (uploads_left >= 0 && uploads_left-- == 0) return 1;
+  return late_upload(dst, src, bytes, stream);
+}
+"""
+
+
+def test_a_run_that_fails_waits_for_the_copies_on_their_way_into_its_pool(tmp_path):
+    """Whichever copy fails: also one whose constant is partly on its way already, without an event behind that."""
+    if not shutil.which("gcc"):
+        pytest.skip("no host compiler")
+    (tmp_path / "runtime.c").write_text(FAILING_SHIM % {"oracle": os.path.join(ROOT, "oracle", "dnnrt_oracle.c")})
+    runtime = str(tmp_path / "runtime.so")
+    subprocess.check_call(["gcc", "-O1", "-fPIC", "-shared", "-std=gnu11", "-ffp-contract=off", "-fopenmp", "-I", os.path.join(ROOT, "oracle"),
+                           "-o", runtime, str(tmp_path / "runtime.c"), "-lm"])
+    r = np.random.default_rng(6)
+    g = compiler.Graph()
+    h = g.input("x", (4, 512))
+    # a filter, the next of twice its size and more: half of that one's bytes are free at once, half behind the first
+    for rows, cols in [(512, 768), (768, 1024), (1024, 256), (256, 2048), (2048, 256)]:
+        h = g.node("Relu", [g.node("MatMul", [h, g.constant((r.standard_normal((rows, cols)) / rows ** 0.5).astype(np.float32))])])
+    g.output(h)
+    inputs = [r.standard_normal((4, 512)).astype(np.float32)]
+    want = graph_eval.evaluate(g, inputs)
+    s = g.compile().session(compiler.MODE_OCCAMY, runtime_library=runtime)
+    lib = C.CDLL(runtime)
+    for uploads in range(100):
+        lib.fail_at(uploads)
+        try:
+            got = s.run(*inputs)
+        except RuntimeError:
+            assert lib.copies_into_a_pool_that_is_gone() == 0, uploads
+            continue
+        break
+    assert 7 <= uploads < 100  # the input's, five filters and a part more
+    lib.fail_at(-1)
+    for _ in range(2):
+        np.testing.assert_allclose(got[0], want[0], rtol=1e-4, atol=1e-4)
+        got = s.run(*inputs)
+    s.close()
