@@ -226,3 +226,100 @@ def test_a_run_that_fails_waits_for_the_copies_on_their_way_into_its_pool(tmp_pa
         np.testing.assert_allclose(got[0], want[0], rtol=1e-4, atol=1e-4)
         got = s.run(*inputs)
     s.close()
+
+
+ORDER_SHIM = r"""
+#define dnnrtIsHostBackend dnnrt_oracle_is_host_backend
+#define dnnrtStreamCreate dnnrt_oracle_stream_create
+#define dnnrtSetStream dnnrt_oracle_set_stream
+#define dnnrtEventRecord dnnrt_oracle_event_record
+#define dnnrtEventDestroy dnnrt_oracle_event_destroy
+#define dnnrtMemPoolInit dnnrt_oracle_pool_init
+#define dnnrtActive dnnrt_oracle_active
+#define dnnrtMatmulNd dnnrt_oracle_matmul_nd
+#include "%(oracle)s"
+#undef dnnrtIsHostBackend
+#undef dnnrtStreamCreate
+#undef dnnrtSetStream
+#undef dnnrtEventRecord
+#undef dnnrtEventDestroy
+#undef dnnrtMemPoolInit
+#undef dnnrtActive
+#undef dnnrtMatmulNd
+enum { MOST = 4096 };
+static struct { const char *lo, *hi; int op; } used[MOST];  /* bytes that operations read or write, in the order of issue */
+static int n_used, ops, streams, behind[8], too_early, in_place_of[8];
+static dnnrtStream_t computing;
+int uploads_too_early(void) { return too_early; }
+int uploads_over_used_bytes(int which) { int n = 0; for (int i = 0; i < 8; i++) if (in_place_of[i] && which-- == 0) n = in_place_of[i]; return n; }
+static void uses(const void *p, const int64_t *dim, int rank) {
+  int64_t bytes = 4;
+  for (int i = 0; i < rank; i++) bytes *= dim[i];
+  used[n_used].lo = p;
+  used[n_used].hi = (const char *)p + bytes;
+  used[n_used++].op = ops;
+}
+int32_t dnnrtIsHostBackend(void) { return 0; }
+int32_t dnnrtStreamCreate(dnnrtStream_t *s) { *s = (dnnrtStream_t)(intptr_t)(1 + streams++ %% 7); return 0; }
+int32_t dnnrtSetStream(dnnrtHandle_t h, dnnrtStream_t s) { (void)h; computing = s; return 0; }
+int32_t dnnrtMemPoolInit(void **pool, int64_t bytes) { n_used = ops = 0; memset(behind, 0, sizeof behind); return dnnrt_oracle_pool_init(pool, bytes); }
+void *dnnrtActive(dnnrtHandle_t h, const void *X, const int64_t *dimX, int32_t mode, void *Y, int32_t dtype) {
+  uses(X, dimX, 4); uses(Y, dimX, 4); ops++;
+  return dnnrt_oracle_active(h, X, dimX, mode, Y, dtype);
+}
+void *dnnrtMatmulNd(dnnrtHandle_t h, const void *A, const int64_t *dimA, int32_t rankA, const void *B, const int64_t *dimB, int32_t rankB, void *Y,
+                    const int64_t *dimY, int32_t rankY, int32_t dtype) {
+  uses(A, dimA, rankA); uses(B, dimB, rankB); uses(Y, dimY, rankY); ops++;
+  return dnnrt_oracle_matmul_nd(h, A, dimA, rankA, B, dimB, rankB, Y, dimY, rankY, dtype);
+}
+struct Mark { dnnrtStream_t at; int ops; };
+int32_t dnnrtExecFenceCreate(void **event) { *event = calloc(1, sizeof(struct Mark)); return 0; }
+int32_t dnnrtEventRecord(void *event, dnnrtStream_t s) { *(struct Mark *)event = (struct Mark){s, ops}; return 0; }
+int32_t dnnrtEventDestroy(void *event) { free(event); return 0; }
+int32_t dnnrtExecStreamWait(dnnrtStream_t s, void *event) {
+  const struct Mark *m = event;
+  if (s != computing && m->at == computing && m->ops > behind[(intptr_t)s]) behind[(intptr_t)s] = m->ops;
+  return 0;
+}
+int32_t dnnrtExecUpload(void *dst, const void *src, int64_t bytes, dnnrtStream_t stream) {
+  const int64_t dim[1] = {(bytes + 3) / 4};
+  if (stream == computing) { uses(dst, dim, 1); ops++; }
+  else {
+    int over = 0;
+    for (int i = 0; i < n_used; i++)
+      if (used[i].lo < (char *)dst + bytes && (char *)dst < used[i].hi) { over = 1; too_early += used[i].op >= behind[(intptr_t)stream]; }
+    in_place_of[(intptr_t)stream] += over;
+  }
+  memcpy(dst, src, (size_t)bytes);
+  return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("flags", [dict(), dict(alias_copies=True, compact_pool=True)])
+def test_each_upload_stream_waits_for_whoever_used_the_bytes_it_writes(tmp_path, flags):
+    """Every copy's own stream is behind all operations issued so far that read or write its bytes: that the other stream is does not
+    count."""
+    if not shutil.which("gcc"):
+        pytest.skip("no host compiler")
+    (tmp_path / "runtime.c").write_text(ORDER_SHIM % {"oracle": os.path.join(ROOT, "oracle", "dnnrt_oracle.c")})
+    runtime = str(tmp_path / "runtime.so")
+    subprocess.check_call(["gcc", "-O1", "-fPIC", "-shared", "-std=gnu11", "-ffp-contract=off", "-fopenmp", "-I", os.path.join(ROOT, "oracle"),
+                           "-o", runtime, str(tmp_path / "runtime.c"), "-lm"])
+    r = np.random.default_rng(7)
+    g = compiler.Graph()
+    h = g.input("x", (16, 512))
+    # large filters over bytes of those before them, small ones beside them
+    for rows, cols in [(512, 640), (640, 768), (768, 320), (320, 128), (128, 1024), (1024, 512), (512, 64), (64, 896), (896, 1024), (1024, 512)]:
+        h = g.node("Relu", [g.node("MatMul", [h, g.constant((r.standard_normal((rows, cols)) / rows ** 0.5).astype(np.float32))])])
+    g.output(h)
+    inputs = [r.standard_normal((16, 512)).astype(np.float32)]
+    want = graph_eval.evaluate(g, inputs)
+    s = g.compile(**flags).session(compiler.MODE_OCCAMY, runtime_library=runtime)
+    lib = C.CDLL(runtime)
+    for _ in range(2):
+        for got, ref in zip(s.run(*inputs), want):
+            np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-4)
+    assert lib.uploads_too_early() == 0
+    assert lib.uploads_over_used_bytes(0) > 0 and lib.uploads_over_used_bytes(1) > 0  # both streams had somebody to wait for
+    s.close()
