@@ -114,21 +114,21 @@ static void permute_kcrs_to_crsk(const uint8_t *src, uint8_t *dst, const Shape &
 
 static bool is_compute(OpKind k) { return k >= OP_CONVFWD && k < OP_RETURN; }
 
-// The operations' stream and, where constants may be uploaded ahead, those of the uploads.  These three have to be on
+// The operations' stream and, where constants are uploaded ahead, those of the uploads.  These three have to be on
 // hardware queues of their own: on a shared one, copies wait for the kernels in front of them and kernels for copies.  HIP
 // gives a process four queues, makes one at each of the first streams, and then puts each new stream on one that has the
 // fewest, which can be the one that the stream before it has just made: with one or two more streams in the process a
 // ResNet-50 took 2.61 or 2.75 ms instead of 2.42.  Streams that are dropped again make all four first; of three streams
 // created then in a row no two are on one queue (2.41 to 2.44 ms with 0 to 5 other sessions).
-bool Session::create_streams(std::string &err) {
+bool Session::create_streams(bool uploading, std::string &err) {
   dnnrtStream_t first[4] = {nullptr, nullptr, nullptr, nullptr};
-  const bool ahead = mode == MODE_OCCAMY && !host_backend;
   bool ok = true;
-  for (dnnrtStream_t &s : first) ok = ok && (!ahead || !rt.dnnrtStreamCreate(&s));
+  for (dnnrtStream_t &s : first) ok = ok && (!uploading || !rt.dnnrtStreamCreate(&s));
   ok = ok && !rt.dnnrtStreamCreate(&stream);
-  for (dnnrtStream_t &s : upload_stream) ok = ok && (!ahead || !rt.dnnrtStreamCreate(&s));
+  for (dnnrtStream_t &s : upload_stream) ok = ok && (!uploading || !rt.dnnrtStreamCreate(&s));
   if (!ok) err = rt_error("dnnrtStreamCreate");
   for (dnnrtStream_t s : first) if (s) rt.dnnrtStreamDestroy(s);
+  if (ok && rt.dnnrtSetStream(handle, stream)) { err = rt_error("dnnrtSetStream"); ok = false; }
   return ok;
 }
 
@@ -140,8 +140,7 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
   host_backend = rt.dnnrtIsHostBackend() != 0;
   if (prog->channels_last && host_backend) { err = "channels-last programs need the GPU runtime"; return false; }
   if (rt.dnnrtCreate(&handle)) { err = rt_error("dnnrtCreate"); return false; }
-  if (!create_streams(err)) return false;
-  if (rt.dnnrtSetStream(handle, stream)) { err = rt_error("dnnrtSetStream"); return false; }
+  if (mode == MODE_RESIDENT && !create_streams(false, err)) return false;
   ptr.assign(prog->value_store.size(), nullptr);
 
   // Which constants are convolution filters and nothing else.  They are
@@ -292,6 +291,7 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
     if (!block_filters.empty() && rt.dnnrtSync(handle)) { err = rt_error("dnnrtSync"); return false; }
     return true;
   }
+  if (!create_streams(placed && !chunks.empty(), err)) return false;
   return !placed || plan_uploads(chunks, err);
 }
 

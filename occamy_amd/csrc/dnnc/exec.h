@@ -210,7 +210,7 @@ class Session {
   struct UploadPart { int64_t lo, hi; int after; };
   struct UploadChunk { std::vector<UploadItem> items; int64_t bytes, off; int first, last; std::vector<UploadPart> parts; };
   bool place_constants(std::vector<UploadChunk> &chunks) const;
-  bool create_streams(std::string &err);
+  bool create_streams(bool uploading, std::string &err);
   bool plan_uploads(const std::vector<UploadChunk> &chunks, std::string &err);
   bool fill_dead(const std::vector<Range> &held, int n, void *base) const;
   bool run_uploading(const void *const *inputs, void *const *outputs, std::string &err);

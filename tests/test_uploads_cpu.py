@@ -323,3 +323,31 @@ def test_each_upload_stream_waits_for_whoever_used_the_bytes_it_writes(tmp_path,
     assert lib.uploads_too_early() == 0
     assert lib.uploads_over_used_bytes(0) > 0 and lib.uploads_over_used_bytes(1) > 0  # both streams had somebody to wait for
     s.close()
+
+
+@pytest.mark.parametrize("mode", [compiler.MODE_OCCAMY, compiler.MODE_RESIDENT])
+@pytest.mark.parametrize("filters", [0, 2])
+def test_streams_for_uploads_are_made_where_something_is_uploaded(tmp_path, filters, mode):
+    if not shutil.which("gcc"):
+        pytest.skip("no host compiler")
+    shim = "#define dnnrtStreamCreate dnnrt_oracle_stream_create\n" + SHIM + """#undef dnnrtStreamCreate
+static int streams;
+int streams_made(void) { return streams; }
+int32_t dnnrtStreamCreate(dnnrtStream_t *s) { streams++; return dnnrt_oracle_stream_create(s); }
+"""
+    (tmp_path / "runtime.c").write_text(shim % {"oracle": os.path.join(ROOT, "oracle", "dnnrt_oracle.c")})
+    runtime = str(tmp_path / "runtime.so")
+    subprocess.check_call(["gcc", "-O1", "-fPIC", "-shared", "-std=c11", "-ffp-contract=off", "-fopenmp", "-I", os.path.join(ROOT, "oracle"),
+                           "-o", runtime, str(tmp_path / "runtime.c"), "-lm"])
+    r = np.random.default_rng(8)
+    g = compiler.Graph()
+    h = g.input("x", (16, 16))
+    for _ in range(filters):
+        h = g.node("MatMul", [h, g.constant(r.standard_normal((16, 16)).astype(np.float32))])
+    g.output(g.node("Relu", [h]))
+    inputs = [r.standard_normal((16, 16)).astype(np.float32)]
+    s = g.compile().session(mode, runtime_library=runtime)
+    np.testing.assert_allclose(s.run(*inputs)[0], graph_eval.evaluate(g, inputs)[0], rtol=1e-4, atol=1e-4)
+    made = C.CDLL(runtime).streams_made()
+    assert made > 2 if filters and mode == compiler.MODE_OCCAMY else made == 1
+    s.close()
