@@ -266,12 +266,13 @@ bool Session::init(const Program *p,const std::string &runtime_path, int mode_, 
   // ahead; in the reference's order a block's first filter is gone when the block runs.
   const bool ahead = !host_backend && rt.dnnrtExecFenceCreate && rt.dnnrtExecStreamWait && rt.dnnrtExecUpload;
   std::vector<UploadChunk> chunks;
-  bool placed = ahead && (mode == MODE_OCCAMY || !blocks.empty()) && place_constants(chunks);
-  if (!placed && !blocks.empty()) {
-    blocks.clear();
-    block_of.clear();
-    moved_results.clear();
-    placed = ahead && mode == MODE_OCCAMY && place_constants(chunks);
+  auto place = [&]() { return ahead && (mode == MODE_OCCAMY || !blocks.empty()) && place_constants(chunks); };
+  bool placed = place();
+  // The filters of a block lie in the pool at once: where that is too much, the block that takes the most goes.
+  while (!placed && !blocks.empty()) {
+    drop_block(tightest_block());
+    place_block_results();
+    placed = place();
   }
   for (const Block &b : blocks)
     for (const Op *op : {b.expand, b.project})
@@ -469,8 +470,42 @@ void Session::plan_blocks() {
       if (op) block_of[op] = (int)blocks.size();
     blocks.push_back(b);
   }
-  // Results that would meet the block's input or residual get a place of their own.  One that cannot takes its block out,
-  // and as the other places rest on what is not stored, the search starts again.
+  place_block_results();
+}
+
+void Session::drop_block(size_t q) {
+  blocks.erase(blocks.begin() + (long)q);
+  block_of.clear();
+  for (size_t i = 0; i < blocks.size(); i++)
+    for (const Op *op : {blocks[i].expand, blocks[i].dw, blocks[i].project})
+      if (op) block_of[op] = (int)i;
+}
+
+// The block during which tensors and the constants it reads take the most bytes together.
+size_t Session::tightest_block() const {
+  std::vector<Range> held = moved_results;
+  for (const auto &l : live_slots()) held.push_back(l.second);
+  size_t tightest = 0;
+  int64_t most = -1;
+  for (size_t q = 0; q < blocks.size(); q++) {
+    int64_t bytes = 0;
+    for (const Range &r : held)
+      if (r.first <= blocks[q].at && r.last >= blocks[q].at) bytes += r.hi - r.lo;
+    for (const Op *op : {blocks[q].expand, blocks[q].dw, blocks[q].project})
+      for (size_t i = 1; op && i <= 2; i++)
+        for (const auto &u : op->operands[i]->uses)
+          if (u.first->kind == OP_MEMCPY && u.first->mode == 1 && u.second == 0) bytes += u.first->bytes;
+    if (bytes > most) { most = bytes; tightest = q; }
+  }
+  return tightest;
+}
+
+// Results that would meet the block's input or residual get a place of their own.  One that cannot takes its block out,
+// and as the other places rest on what is not stored, the search starts again.
+void Session::place_block_results() {
+  std::map<const Op *, int> number;
+  for (const Op *op : prog->ops)
+    if (is_compute(op->kind)) { const int n = (int)number.size(); number[op] = n; }
   for (bool again = true; again;) {
     again = false;
     moved_results.clear();
@@ -522,11 +557,7 @@ void Session::plan_blocks() {
         moved_results.push_back(r);
         moved[b.project->result] = r;
       } else {
-        blocks.erase(blocks.begin() + (long)q);
-        block_of.clear();
-        for (size_t i = 0; i < blocks.size(); i++)
-          for (const Op *op : {blocks[i].expand, blocks[i].dw, blocks[i].project})
-            if (op) block_of[op] = (int)i;
+        drop_block(q);
         again = true;
       }
     }

@@ -190,6 +190,9 @@ class Session {
   std::map<const Value *, std::pair<int64_t, int64_t>> block_filters;  // device tensors uploaded in the block call's layout; rows, columns
   decltype(&::dnnrtExecBlockFilter) block_filter(const Value *filter) const { return filter->dtype == F16 ? rt.dnnrtExecBlockFilter : rt.dnnrtExecBlockFilterF32; }
   void plan_blocks();
+  void place_block_results();
+  void drop_block(size_t q);
+  size_t tightest_block() const;
   std::map<const Value *, Range> live_slots() const;
   // Per-inference mode on the GPU runtime: the constants as they go to the device on two streams of their own, ahead of
   // the operations that read them (plan_uploads).  Compute operations are counted in program order.
