@@ -101,24 +101,18 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // S: the depthwise stride.  KC: steps of 16 input channels (0: no expansion, X holds the hidden channels).  GM: most
-// wavefronts of a workgroup.
-template <int S, int KC, int GM>
+// wavefronts of a workgroup.  PARTS: the hidden channels are cut over workgroups; kernels of whole channels go without the hand-over, whose
+// operands cost them scalar registers (MobileNetV2 at batch 64: 470 us with it in every kernel, 464 without).
+template <int S, int KC, int GM, bool PARTS>
 __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2 ? 3 : 2))) void conv_f16_block_kernel(const BlockF16Args a, float *partials,
                                                                                                                        unsigned *counters) {
   constexpr bool EXPAND = KC > 0;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-#if __HIP_DEVICE_COMPILE__
-  // What the first loads need of the arguments, all at once: read where they are first used, each round is a fraction of a microsecond
-  // (MobileNetV2 at batch 64 456.8 -> 455.8 us).
-  asm volatile("" ::"s"(a.X), "s"(a.H), "s"(a.W), "s"(a.Cin), "s"(a.Ch), "s"(a.ph), "s"(a.pw), "s"(a.TH), "s"(a.TW), "s"(a.PH), "s"(a.PW), "s"(a.xs_bytes),
-               "s"(a.slab_bytes), "s"(a.tiles_w), "s"(a.tiles_hw), "s"(a.tiles), "s"(a.per_xcd), "s"(a.per_split), "s"(a.magic_tiles_w), "s"(a.magic_tiles_hw),
-               "s"(a.magic_c8), "s"((int)blockDim.x));
-#endif
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), G = (int)(blockDim.x >> 6);
   char *Xs = smem, *slabs = smem + a.xs_bytes, *mine = slabs + wave * a.slab_bytes;
   // this workgroup's groups of 32 hidden channels: from group0 on
-  const int group0 = (int)blockIdx.z * a.per_split, groups = min(a.per_split, ((a.Ch + 31) >> 5) - group0);
+  const int group0 = PARTS ? (int)blockIdx.z * a.per_split : 0, groups = min(a.per_split, ((a.Ch + 31) >> 5) - group0);
   float *B1 = reinterpret_cast<float *>(slabs + G * a.slab_bytes), *Bd = B1 + 32 * groups;  // the inner biases, padded to the last group's end
   _Float16 *Wd = reinterpret_cast<_Float16 *>(Bd + 32 * groups);  // the depthwise filters, [channel][tap]
 
@@ -208,7 +202,7 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
   const int pm = pairs ? wave >> 1 : wave, ppx = pairs ? 32 * (wave & 1) : 0;
   floatx16 acc[2];
   {
-    const auto b3_rsrc = rsrc_of(blockIdx.z == 0 ? a.b3 : nullptr, a.Cout);  // in the first part's sums
+    const auto b3_rsrc = rsrc_of(!PARTS || blockIdx.z == 0 ? a.b3 : nullptr, a.Cout);  // in the first part's sums
 #pragma unroll
     for (int gq = 0; gq < 4; gq++) {
       const half4 v = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(b3_rsrc, 2 * (32 * (mfirst + pm) + 8 * gq + 4 * half), 0, 0));
@@ -220,17 +214,20 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
 
   for (int first = 0; first < groups; first += G) {
     const int g = first + wave, ch = 32 * (group0 + g), own = 32 * g;  // hidden channels; theirs among the workgroup's
-    half8 wp[2 * GM];  // the projection's filter for this round, requested well ahead where registers allow
-    auto load_project = [&]() {
+    // The projection's filter for this round: half of it is requested well ahead where there are registers for that (all of it took more than
+    // there are, and scratch memory; 7x7 blocks of 160 channels, which have none to spare: with half ahead as fast).
+    constexpr int EARLY = KC <= 2 || KC > 8 ? 0 : GM / 2;
+    half8 wp[2 * GM];
+    auto load_project = [&](int from, int to) {
 #pragma unroll
       for (int q = 0; q < GM; q++)
 #pragma unroll
         for (int k = 0; k < 2; k++) {
           const int c = 32 * (group0 + first + q) + 16 * k + 8 * half;
-          wp[2 * q + k] = load_rows(w3_rsrc, a.Cout, a.Ch, mfirst + min(pm, mblocks - 1), q < G ? c : a.Ch);
+          if (q >= from && q < to) wp[2 * q + k] = load_rows(w3_rsrc, a.Cout, a.Ch, mfirst + min(pm, mblocks - 1), q < G ? c : a.Ch);
         }
     };
-    if constexpr (KC > 2) load_project();
+    load_project(0, EARLY);
     if (g < groups) {
       if (border)
         for (int u = lane; u < a.PH * a.PW * (SLAB_PX / 16); u += 64) *reinterpret_cast<half8 *>(mine + 16 * u) = zero8;
@@ -313,7 +310,7 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
         *reinterpret_cast<uint4 *>(mine + (4 * (lane >> 2) + o) * SLAB_PX + 16 * cg) = ch + 8 * cg < a.Ch ? d : make_uint4(0, 0, 0, 0);
       }
     }
-    if constexpr (KC <= 2) load_project();
+    load_project(EARLY, GM);
     lds_barrier();
 
     // ---- project ------------------------------------------------------------------
@@ -342,7 +339,8 @@ __global__ __launch_bounds__(64 * GM) __attribute__((amdgpu_waves_per_eu(KC <= 2
   // ---- hidden channels cut over workgroups: partial sums through the handle's scratch (igemm_f32_small.hip states what the
   // hand-over rests on), [block of channels][four of them][pixel]; the last to arrive adds the parts in order and goes on
 #if __HIP_DEVICE_COMPILE__
-  if (const int parts = (int)gridDim.z; parts > 1) {
+  if constexpr (PARTS) {
+    const int parts = (int)gridDim.z;
     const __amdgpu_buffer_rsrc_t rsrc = part_rsrc(partials);
     const unsigned slot = blockIdx.y * (unsigned)a.tiles + (unsigned)tile, part_bytes = (unsigned)a.blocks_y * 128u * (unsigned)a.part_px;
     const int across = min(a.TW, a.Q);
@@ -530,14 +528,14 @@ bool block_f16_applies(const dnnrtContext *ctx, const dnnrtExecBlock &k) {
   return plan_block_f16(ctx, k, true, a, kc, gy, g, parts);
 }
 
-template <int S, int KC, int GM>
+template <int S, int KC, int GM, bool PARTS>
 static bool launch_one(const dnnrtContext *ctx, dim3 grid, dim3 threads, size_t lds, const BlockF16Args &a) {
   static LdsRaised raised;
-  if (!raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&conv_f16_block_kernel<S, KC, GM>), BLOCK_LDS)) {
+  if (!raise_lds(raised, ctx->device, reinterpret_cast<const void *>(&conv_f16_block_kernel<S, KC, GM, PARTS>), BLOCK_LDS)) {
     set_error("inverted residual block (fp16): cannot reserve %d bytes of LDS", BLOCK_LDS);
     return false;
   }
-  hipLaunchKernelGGL((conv_f16_block_kernel<S, KC, GM>), grid, threads, lds, ctx->stream, a, ctx->splitk_partials, ctx->splitk_counters);
+  hipLaunchKernelGGL((conv_f16_block_kernel<S, KC, GM, PARTS>), grid, threads, lds, ctx->stream, a, ctx->splitk_partials, ctx->splitk_counters);
   return true;
 }
 
@@ -550,7 +548,10 @@ static bool launch_cut(const dnnrtContext *ctx, const dnnrtExecBlock &k, BlockF1
     if (!aligned16(q)) { set_error("inverted residual block (fp16): an operand is not 16-byte aligned"); return false; }
   const dim3 grid((unsigned)(8 * a.per_xcd), (unsigned)gy, (unsigned)parts), threads(64 * (unsigned)g);
   const size_t lds = (size_t)a.xs_bytes + (size_t)g * (size_t)a.slab_bytes + BLOCK_PER_GROUP * (size_t)a.per_split;
-#define BLOCK(S, KC) if (!launch_one<S, KC, KC <= 2 ? 4 : 8>(ctx, grid, threads, lds, a)) return false
+#define BLOCK(S, KC)                                                                        \
+  if (!(parts > 1 ? launch_one<S, KC, KC <= 2 ? 4 : 8, true>(ctx, grid, threads, lds, a)    \
+                  : launch_one<S, KC, KC <= 2 ? 4 : 8, false>(ctx, grid, threads, lds, a))) \
+  return false
   if (k.stride == 1) switch (kc) {
     case 0: BLOCK(1, 0); break; case 1: BLOCK(1, 1); break; case 2: BLOCK(1, 2); break;
     case 4: BLOCK(1, 4); break; case 6: BLOCK(1, 6); break; default: BLOCK(1, 10); break;
