@@ -72,6 +72,10 @@ __device__ __forceinline__ void lds_barrier32() {
 constexpr int block32_xs(int s, int nb) { return s == 1 ? 72 : nb == 1 ? 136 : 200; }
 constexpr int block32_ss(int s, int nb) { return s == 1 ? (nb == 1 ? 52 : 84) : nb == 1 ? 100 : 164; }
 constexpr int block32_kg(int kc) { return kc <= 8 ? 2 : 8; }  // k-steps of a chunk
+// Floats from the patch on that a workgroup's LDS holds at least: an expansion reads its chunks ahead through all of the template's k-steps, also
+// where the block has fewer, and up to 15 pixels past a channel's end.  What lies there is read and not used.  (Reads that stop with the
+// block's own steps took 191 us for a MobileNetV2 at batch 1 instead of 188.5.)
+constexpr int block32_reach(int kc, int xs) { return kc > 0 ? 4 * kc * xs + 15 : 0; }
 constexpr int block32_s2(int nb) { return nb == 1 ? 24 : 40; }  // between those of the depthwise results, as the patch's
 
 template <int S, int KC, int MB, int NB>
@@ -215,7 +219,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KC <= 8 ? 4
 #pragma unroll
         for (int u = 0; u < BLOCKS; u++) e[u] = bias;
         const float *xp = Xs + 2 * l4 * XS + p + l16;
-        // a chunk's pixels are read while the chunk before is multiplied; what lies behind the last is not used
+        // a chunk's pixels are read while the chunk before is multiplied; what lies behind the last (block32_reach) is not used
         float x[2][KG][BLOCKS];
         auto read = [&](int k0, float (&to)[KG][BLOCKS]) {
 #pragma unroll
@@ -432,7 +436,7 @@ static bool cut_block_f32(const dnnrtContext *ctx, const dnnrtExecBlock &k, int 
   a.tiles = (int)tiles;
   a.units = (int)units;
   if (splits > 1 && (ctx->splitk_shared || tiles * ranges > ctx->splitk_max_tiles || units * c.mb * nb * 1024 > ctx->splitk_partial_bytes)) return false;
-  c.lds = std::max((4 * a.kc * xs + G * 16 * (ss + block32_s2(nb))) * 4, G * std::min(mall, c.mb) * nb * 1024);
+  c.lds = std::max({(4 * a.kc * xs + G * 16 * (ss + block32_s2(nb))) * 4, block32_reach(c.kc, xs) * 4, G * std::min(mall, c.mb) * nb * 1024});
   if (c.lds > BLOCK32_LDS) return false;
   a.magic_tiles = magic_of(a.tiles); a.magic_splits = magic_of(a.splits);
   a.magic_tiles_w = magic_of(a.tiles_w); a.magic_tiles_hw = magic_of(a.tiles_hw); a.magic_qw = magic_of(a.QW);
