@@ -762,6 +762,35 @@ def test_attention_f32_of_few_queries(gpu, case):
     np.testing.assert_array_equal(oc.attention(gpu, q, k, v, H, scale), got)
 
 
+# B, queries, keys, heads, head size, blocks of 32 keys without weight: all that a wavefront has, of four and of eight; its first one, its last
+# one; all but a single key of the last block
+@pytest.mark.parametrize("case", [(1, 20, 128, 2, 64, (1,)), (1, 20, 128, 2, 32, (0, 2, 3)), (2, 16, 100, 2, 128, (3,)), (1, 33, 512, 2, 64, (2, 10)), (1, 33, 512, 3, 64, (2,)),
+                                  (1, 33, 512, 3, 32, (0, 1, 2, 3, 4, 5, 6, 7, 9)), (1, 17, 400, 2, 64, (12,)), (1, 17, 300, 2, 128, (0, 5)), (1, 17, 257, 2, 64, tuple(range(8)))], ids=str)
+def test_attention_f32_of_few_queries_and_keys_without_weight(gpu, case):
+    """Scores of minus infinity, from keys of minus infinity and queries that are positive there, while others are finite: exactly no weight.
+    Against 64 bits; bound as above, over the keys that have a weight."""
+    B, Sq, Sk, H, D, blocks = case
+    r = rng(Sq + Sk + len(blocks))
+    q, k, v = (r.standard_normal((B, n, H * D)).astype(np.float32) for n in (Sq, Sk, Sk))
+    weight = np.ones(Sk, bool)
+    for b in blocks:
+        weight[32 * b:32 * b + 32] = False
+    q[:, :, ::D] = np.abs(q[:, :, ::D]) + np.float32(0.5)
+    masked = k.copy()
+    masked[:, ~weight, ::D] = -np.inf
+    scale = 1.0 / np.sqrt(D)
+    split = lambda t: t.astype(np.float64).reshape(B, -1, H, D).transpose(0, 2, 1, 3)  # noqa: E731
+    q6, k6, v6 = split(q), split(k[:, weight]), split(v[:, weight])
+    s = scale * (q6 @ k6.transpose(0, 1, 3, 2))
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    u = 2.0 ** -24
+    e = (D + 2) * u * (scale * (np.abs(q6) @ np.abs(k6).transpose(0, 1, 3, 2))).max(-1, keepdims=True) + 2 * u * (s.max(-1, keepdims=True) - s).max(-1, keepdims=True)
+    merge = lambda t: t.transpose(0, 2, 1, 3).reshape(B, Sq, H * D)  # noqa: E731
+    want, bound = merge(p @ v6), merge((4 * e + (2 * Sk + 12) * u) * (p @ np.abs(v6)))
+    assert (np.abs(oc.attention(gpu, q, masked, v, H, scale) - want) <= bound).all()
+
+
 @pytest.mark.parametrize("case", [(1, 384, 384, 12, 64), (2, 31, 257, 3, 64), (1, 70, 129, 2, 32), (1, 64, 160, 5, 32), (1, 45, 513, 2, 128),
                                   (1, 1, 1, 1, 64), (3, 33, 32, 2, 64), (1, 600, 600, 16, 64)], ids=str)
 def test_attention_f16_blocks_and_wavefronts(gpu, cpu, case):
