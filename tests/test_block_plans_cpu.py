@@ -6,6 +6,7 @@ import subprocess
 
 import pytest
 
+import test_gpu_ops
 from test_untracked_reads import CSRC, HIPCC
 
 COMMON = r"""
@@ -137,3 +138,29 @@ def test_expansions_read_inside_the_workgroups_lds(f32):
     plans = f32(problems)
     assert all(p is not None and p[5] > 0 for p in plans)
     assert not [q for q, p in zip(problems, plans) if p[6]]
+
+
+def _cases(name):
+    mark, = (m for m in getattr(test_gpu_ops, name).pytestmark if m.name == "parametrize")
+    return mark.args[1]
+
+
+def test_the_fp32_tests_reach_every_kernel(f32):
+    """The cases of the tests on the GPU are for the kernels that the planner's estimate sends them to: if it is fitted anew, they may need others."""
+    cases = _cases("test_inverted_residual_block_fp32") + _cases("test_inverted_residual_block_fp32_kernels")
+    plans = f32([(n, cin, h, w, ch, cout, stride, *pads, expand) for n, cin, h, w, ch, cout, stride, pads, expand, _, _ in cases])
+    got = {(c[6], p[0], p[2], p[3], p[4] > 1) for c, p in zip(cases, plans)}  # stride, k-steps, blocks of pixels, wavefronts, in parts
+    want = {(s, kc, nb, g, parts) for s in (1, 2) for kc in (24, 40) for nb in (1, 2) for g in (4, 8) for parts in (False, True)}
+    want -= {(2, 40, 2, 8, False), (2, 40, 2, 8, True)}  # no room for eight wavefronts, or never the fastest
+    want |= {(s, 8, 2, 4, parts) for s in (1, 2) for parts in (False, True)} - {(2, 8, 2, 4, False)} | {(2, 8, 2, 8, False), (1, 0, 2, 4, False), (2, 0, 2, 4, False)}
+    assert want <= got, sorted(want - got)
+
+
+def test_the_fp16_tests_reach_every_kernel(f16):
+    cases = [c for name in ("", "_in_parts", "_kernels") for c in _cases("test_inverted_residual_block_fp16" + name)]
+    plans = f16([(n, cin, h, w, ch, cout, stride, 1, 1, expand) for n, cin, h, w, ch, cout, stride, expand, _ in cases])
+    got = {(c[6], p[0], p[3] > 1) for c, p in zip(cases, plans)}  # stride, steps of input channels, in parts
+    want = {(s, kc, parts) for s in (1, 2) for kc in (0, 1, 2, 4, 6, 10) for parts in (False, True)}
+    assert want <= got, sorted(want - got)
+    in_parts = len(_cases("test_inverted_residual_block_fp16"))
+    assert all(p[3] > 1 for p in plans[in_parts:in_parts + len(_cases("test_inverted_residual_block_fp16_in_parts"))])

@@ -1830,6 +1830,25 @@ def test_inverted_residual_block_fp16_in_parts(n, cin, h, w, ch, cout, stride, e
     test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, residual)
 
 
+@pytest.mark.parametrize("n,cin,h,w,ch,cout,stride,expand,residual", [
+    (64, 24, 20, 21, 144, 24, 1, True, True),    # whole channels: every number of steps of input channels, both strides
+    (64, 24, 30, 31, 144, 24, 2, True, False),
+    (1, 40, 7, 7, 240, 72, 2, True, False),
+    (48, 88, 14, 13, 528, 96, 1, True, False),
+    (24, 88, 30, 31, 528, 96, 2, True, False),
+    (2, 120, 7, 6, 240, 328, 1, True, False),
+    (2, 120, 7, 6, 240, 328, 2, True, False),
+    (1, 16, 7, 9, 960, 24, 1, True, False),      # ... and in parts
+    (1, 16, 7, 9, 960, 24, 2, True, False),
+    (1, 64, 7, 7, 384, 64, 2, True, False),
+    (1, 136, 7, 7, 272, 104, 2, True, False),
+    (2, 192, 7, 7, 192, 16, 2, False, False),
+])
+def test_inverted_residual_block_fp16_kernels(n, cin, h, w, ch, cout, stride, expand, residual):
+    """With the cases of the two tests above, each of the kernels."""
+    test_inverted_residual_block_fp16(n, cin, h, w, ch, cout, stride, expand, residual)
+
+
 @pytest.mark.parametrize("n,cin,h,w,ch,cout,stride,pads,expand,residual,acts", [
     (1, 8, 5, 7, 16, 8, 1, (1, 1), True, False, (3, 3, 5)),      # less than a tile, one group of hidden channels
     (1, 16, 33, 17, 96, 24, 2, (1, 1), True, False, (3, 3, 5)),  # ragged tiles, half a block of output channels
@@ -1904,6 +1923,44 @@ def test_inverted_residual_block_fp32(n, cin, h, w, ch, cout, stride, pads, expa
             setattr(other, name, value)
         assert not lib.dnnrtExecBlockApplies(handle, C.byref(other)) and lib.dnnrtExecRunBlock(handle, C.byref(other)) != 0, bad
     lib.dnnrtDestroy(handle)
+
+
+@pytest.mark.parametrize("n,cin,h,w,ch,cout,stride,pads,expand,residual,acts", [
+    # tiles of 32 pixels with 40 to 160 input channels: four and eight wavefronts, whole channels and parts
+    (48, 40, 14, 13, 240, 72, 1, (1, 1), True, False, (3, 3, 5)),
+    (8, 64, 14, 13, 384, 64, 1, (1, 1), True, True, (3, 3, 5)),
+    (12, 40, 20, 21, 240, 72, 1, (1, 1), True, False, (3, 3, 1)),
+    (12, 64, 14, 13, 384, 96, 1, (1, 1), True, False, (3, 3, 5)),
+    (48, 96, 20, 21, 576, 96, 2, (1, 1), True, False, (3, 3, 5)),
+    (24, 96, 14, 13, 576, 96, 2, (1, 1), True, False, (3, 3, 5)),
+    (6, 40, 56, 57, 240, 72, 2, (1, 1), True, False, (3, 3, 5)),
+    (16, 64, 20, 21, 384, 64, 2, (1, 1), True, True, (3, 3, 5)),
+    (48, 8, 14, 13, 48, 160, 1, (1, 1), True, False, (3, 3, 5)),  # two steps of 40: the others are read and not used
+    (6, 96, 14, 13, 576, 160, 1, (1, 1), True, False, (3, 3, 5)),
+    (12, 120, 14, 13, 240, 328, 1, (1, 1), True, False, (3, 3, 5)),
+    (16, 160, 7, 7, 960, 160, 1, (1, 1), True, True, (3, 3, 5)),
+    (32, 8, 20, 21, 48, 160, 2, (1, 1), True, False, (3, 3, 5)),
+    (24, 96, 14, 13, 576, 160, 2, (1, 1), True, False, (3, 3, 5)),
+    # tiles of 16 pixels, eight wavefronts
+    (12, 40, 14, 13, 240, 72, 1, (1, 1), True, False, (3, 3, 5)),
+    (6, 64, 14, 13, 384, 64, 1, (1, 1), True, True, (3, 3, 5)),
+    (12, 40, 28, 28, 240, 72, 2, (1, 1), True, False, (3, 3, 5)),
+    (8, 96, 14, 13, 576, 96, 2, (1, 1), True, False, (3, 3, 5)),
+    (6, 120, 14, 13, 240, 328, 1, (1, 1), True, False, (3, 3, 5)),
+    (8, 160, 7, 7, 960, 160, 1, (1, 1), True, False, (3, 3, 5)),
+    (12, 120, 14, 13, 240, 328, 2, (1, 1), True, False, (3, 3, 5)),
+    (6, 120, 14, 13, 240, 328, 2, (1, 1), True, False, (3, 3, 5)),
+    # four, whole channels
+    (6, 40, 28, 28, 240, 72, 1, (1, 1), True, False, (3, 3, 5)),
+    (24, 40, 28, 28, 240, 72, 2, (1, 1), True, False, (3, 3, 5)),
+    (2, 8, 7, 7, 48, 160, 1, (1, 1), True, False, (3, 3, 5)),
+    (2, 8, 7, 7, 48, 160, 2, (1, 1), True, False, (3, 3, 5)),
+    (1, 24, 7, 7, 144, 24, 2, (1, 1), True, False, (3, 3, 5)),
+    (3, 32, 9, 8, 32, 16, 2, (1, 1), False, False, (0, 3, 5)),
+])
+def test_inverted_residual_block_fp32_kernels(n, cin, h, w, ch, cout, stride, pads, expand, residual, acts):
+    """With the cases above, each of the kernels in each of the ways that the planner launches it."""
+    test_inverted_residual_block_fp32(n, cin, h, w, ch, cout, stride, pads, expand, residual, acts)
 
 
 @pytest.mark.parametrize("case", [
