@@ -26,11 +26,10 @@
 // a half wavefronts per SIMD; where they are few, the chain of a launch: 3500 cycles until the patch is there, 2500 for the
 // filters, 5000 to 8000 a round, 3000 for the result, 6000 to 11000 for a hand-over (160 -> 960 -> 160 at 7x7, batch 64, four parts).
 //
-// Measured against the three calls at batch 64 (us): 16 -> 96 -> 24 channels, 112x112 stride 2: 104 -> 55; 24 -> 144 -> 24 at
-// 56x56: 85 -> 42; 24 -> 144 -> 32 stride 2: 52 -> 29; 32 -> 192 -> 32 at 28x28: 34 -> 17; 64 -> 384 -> 64 at 14x14: 34 -> 15.5;
-// 96 -> 576 -> 96: 38 -> 22; 32 -> 16 behind a depthwise layer at 112x112, no expansion: 49 -> 37; 160 -> 960 -> 160 at 7x7 30 -> 20.3
-// (30.5 uncut).  MobileNetV2, whole channels and cut: batch 1 249 -> 213, 4 296 -> 243, 8 315 -> 255, 16 358 -> 283, 32 378 -> 350,
-// 64 510 -> 482.
+// Measured against the three calls at batch 64 (us): 16 -> 96 -> 24 channels, 112x112 stride 2: 104 -> 53; 24 -> 144 -> 24 at
+// 56x56: 85 -> 42; 24 -> 144 -> 32 stride 2: 52 -> 28.5; 32 -> 192 -> 32 at 28x28: 34 -> 17; 64 -> 384 -> 64 at 14x14: 34 -> 15;
+// 96 -> 576 -> 96: 38 -> 22; 32 -> 16 behind a depthwise layer at 112x112, no expansion: 49 -> 36; 160 -> 960 -> 160 at 7x7 30 -> 19
+// (30.5 uncut).  MobileNetV2 with whole channels only and as it is: batch 1 249 -> 211, 8 315 -> 249, 32 378 -> 343, 64 485 -> 444.
 #include "conv_f16.h"
 #include "dnnrt_exec.h"
 #include "partials.h"

@@ -21,7 +21,7 @@
 // 4100, expansion 4000, depthwise 600, projection 1200, sums in LDS 2000, hand-over 5600 (2200 until the counter is back, the
 // nine parts 3400), stores 1200.
 //
-// Measured against the three calls, whole MobileNetV2 in a replayed graph (us): batch 1 252 -> 191, 2 284 -> 208, 4 332 -> 259,
+// Measured against the three calls, whole MobileNetV2 in a replayed graph (us): batch 1 254 -> 190, 2 284 -> 208, 4 332 -> 259,
 // 8 413 -> 342, 16 556 -> 473, 32 800 -> 648, 64 1334 -> 1105.  Blocks alone at batch 1: 16 -> 96 -> 24 at 112x112 stride 2 8.5,
 // 24 -> 144 -> 24 at 56x56 9.3, 32 -> 192 -> 32 at 28x28 7.8, 64 -> 384 -> 64 at 14x14 9.2, 160 -> 960 -> 160 at 7x7 12.7.  Tiles of
 // 64 pixels were slower than 32 at every batch (24 -> 144 -> 24, batch 64: 112 against 89).
@@ -74,7 +74,7 @@ constexpr int block32_ss(int s, int nb) { return s == 1 ? (nb == 1 ? 52 : 84) : 
 constexpr int block32_kg(int kc) { return kc <= 8 ? 2 : 8; }  // k-steps of a chunk
 // Floats from the patch on that a workgroup's LDS holds at least: an expansion reads its chunks ahead through all of the template's k-steps, also
 // where the block has fewer, and up to 15 pixels past a channel's end.  What lies there is read and not used.  (Reads that stop with the
-// block's own steps took 191 us for a MobileNetV2 at batch 1 instead of 188.5.)
+// block's own steps took 191 us for a MobileNetV2 at batch 1 where these take 188.5.)
 constexpr int block32_reach(int kc, int xs) { return kc > 0 ? 4 * kc * xs + 15 : 0; }
 constexpr int block32_s2(int nb) { return nb == 1 ? 24 : 40; }  // between those of the depthwise results, as the patch's
 

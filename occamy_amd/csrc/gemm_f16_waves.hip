@@ -5,7 +5,7 @@
 // their round trip per 64 k, every operand read by two wavefronts.  Here each of the four wavefronts owns the whole tile, 64 columns
 // and 64 or 32 rows, for a quarter of the reduction: a ring of two or three stages of 32 k that nobody else touches, so no
 // barrier, every operand read once, 16 MFMAs per stage and wavefront from 12 reads; the four sums meet in LDS at the end, where each lane gets eight
-// neighbouring columns of two rows, bias and residual having been requested before the first load.
+// neighbouring columns of two rows or one, bias and residual having been requested behind the ring's first loads.
 //
 // Time of a workgroup, 384 x 768 x 2304 (us): set-up 0.5, first data 1.0, six stages 2.5, sums 0.6, epilogue and code fetched on the way 1.0.
 // Rings of four stages gained in the loop what they lost waiting for the first data; 96 rows per tile cost 1.2 more per

@@ -4,8 +4,8 @@
 // Tiles of 64 columns and 64 or 32 rows; each of a workgroup's four wavefronts owns the whole tile for a quarter of the reduction,
 // on v_mfma_f32_32x32x2f32.  Its operands go from global memory straight into a ring of two stages of 16 k that nobody
 // else touches: no barrier, every operand read from LDS once (32 MFMAs per stage from 12 reads), nothing staged in registers.  The
-// four sums meet in LDS, where each lane gets four neighbouring columns of some rows; bias and residual were requested before the
-// first load.
+// four sums meet in LDS, where each lane gets four neighbouring columns of some rows; bias and residual were requested behind the
+// ring's first loads.
 //
 // What bounds it: the matrix pipes (a stage is 2048 or 1024 cycles of each SIMD's) and, with the one to a few tiles per compute
 // unit of a few hundred rows, what stands around them: launch, first data, sums and epilogue 4 us, and the hand-over of the split
@@ -307,9 +307,10 @@ bool launch_gemm_f32_waves(const dnnrtContext *ctx, const IgemmArgs &a, bool &la
   // 768 k or as much work as that: 300 x 768 x 768 9.0 us there, 10.6 here; 384 x 768 x 768 13.1 there, 11.3 here; 40 x 3072 x 768 10.4, 13.5;
   // 77 x 3072 x 768 14.5 either way.
   if (ceil_div(a.M, 32) * ceil_div(a.Ncols, 32) * a.Kdim <= (int64_t)ctx->num_cu * 768) return true;
-  // Estimated microseconds: a stage of 16 k takes each of a workgroup's four wavefronts 0.95, with tiles of 32 rows 0.5 (the matrix
-  // pipes: two workgroups on a compute unit take twice that), everything around them 4, a split tile's hand-over 2.3 and 0.25 per
-  // part (0.12).  The tiles left over after the last full round are split.
+  // Estimated microseconds: a stage of 16 k takes each of a workgroup's four wavefronts 0.95, with tiles of 32 rows 0.52 (the matrix
+  // pipes: two workgroups on a compute unit take twice that), everything around them 4 and, with 32 rows, 1 more for every further
+  // workgroup that a compute unit takes, a split tile's hand-over 2.3 and 0.25 per part (0.125).  The tiles left over after the last full
+  // round are split.
   const int stages = a.Kdim / F32W_BK;
   Waves32Plan pl{};
   double best = 0;
